@@ -248,6 +248,8 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
   k.B = args->dims.B; k.H = args->dims.H; k.M = args->dims.M; k.N = args->dims.N;
   k.sm_scale = args->sm_scale;
   k.n_mtiles = (args->dims.M + fox::kFwdBM - 1) / fox::kFwdBM;
+  k.groups = fox::order_groups(k.B * k.H, k.M, k.N, args->dims.D);
+  k.even = fox::even_tiles(k.M, k.N);
   k.splits = 1;
   k.stream = k.n_mtiles == 1 && (int64_t)k.B * k.H * k.N * args->dims.D * 4 >= g_stream_min_kv_bytes.load(std::memory_order_relaxed);
   if (workspace) {

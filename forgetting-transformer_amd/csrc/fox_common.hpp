@@ -426,18 +426,36 @@ __device__ __forceinline__ f32x16 acc_init(const float* t, int row0, int g) {
 // the bias.
 __device__ __forceinline__ float nonzero_scale(float s) { return fabsf(s) < 1e-30f ? 1e-30f : s; }
 
-// Workgroup id -> (bh, tile) with every tile of one (batch, head) on one XCD (the
-// hardware deals consecutive workgroup ids round-robin over 8 XCDs, each with its
-// own L2), heaviest tiles (largest index under a causal mask) first.
-__device__ __forceinline__ void decode_block(int wid, int n_tiles, int n_bh, int& bh, int& tile) {
-  if ((n_bh & 7) == 0) {
-    const int xcd = wid & 7, seq = wid >> 3;
-    bh = (seq / n_tiles) * 8 + xcd;
-    tile = n_tiles - 1 - (seq % n_tiles);
-  } else {
-    bh = wid / n_tiles;
-    tile = n_tiles - 1 - (wid % n_tiles);
+// Workgroup id -> (bh, tile).  Every tile of one (batch, head) goes to one XCD when the count allows it (the hardware
+// deals consecutive workgroup ids round-robin over the 8 XCDs, each with its own L2).  Within an XCD the (batch, head)
+// pairs are taken in `groups` groups of nearly equal size, and inside a group the tiles come heaviest first (largest index
+// under a causal mask) with the pairs of the group in turn.  One pair after the other would start the last pair's
+// heaviest tile when the chip is about to run empty; all pairs at once would stream more K and V than an L2 holds.
+// order_groups() on the host picks the number of groups.
+// `fold`: when the whole grid is resident at two workgroups per CU, the second workgroup of a CU is the one that arrives
+// kCus ids after the first.  Taken in the same order both would be heavy on one CU and both light on another; from
+// workgroup kCus on the list is therefore walked from its light end (forward B1 H16 T4096 D128: 109 -> 84 us, dQ 152 -> 116 us).
+constexpr int kXcds = 8, kCus = 256;
+__device__ __forceinline__ void decode_block(int wid, int n_tiles, int n_bh, int groups, bool fold, int& bh, int& tile) {
+  const bool by_xcd = n_bh % kXcds == 0;
+  const int nb = by_xcd ? n_bh / kXcds : n_bh, cus = by_xcd ? kCus / kXcds : kCus;
+  const int total = n_tiles * nb;
+  int r = by_xcd ? wid / kXcds : wid;
+  if (fold && r >= cus && total <= 2 * cus) r = total - 1 - (r - cus);
+  int b;
+  if (groups == 1) {   // the usual case of a small grid, where the divisions below would show
+    const int t = r / nb;
+    b = r - t * nb;
+    tile = n_tiles - 1 - t;
+  } else {             // the first nb % groups groups hold one pair more than the others
+    const int small = nb / groups, extra = nb % groups, big_end = extra * (small + 1) * n_tiles;
+    const bool big = r < big_end;
+    const int size = big ? small + 1 : small;
+    const int q = big ? r : r - big_end, grp = q / (size * n_tiles), in = q - grp * size * n_tiles;
+    b = (big ? 0 : extra * (small + 1)) + grp * size + in % size;
+    tile = n_tiles - 1 - in / size;
   }
+  bh = by_xcd ? b * kXcds + wid % kXcds : b;
 }
 
 // Adaptive Computation Pruning, query-side bound: the first key block of width BN

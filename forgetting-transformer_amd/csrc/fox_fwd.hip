@@ -262,11 +262,11 @@ __global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
   int bh, mt, sp = 0;
   if constexpr (SPLIT) {  // (query tile, key split) pairs take the place of query tiles
     int mts;
-    decode_block(blockIdx.x, a.n_mtiles * a.splits, a.B * a.H, bh, mts);
+    decode_block(blockIdx.x, a.n_mtiles * a.splits, a.B * a.H, a.groups, !a.even, bh, mts);
     mt = mts / a.splits;
     sp = mts % a.splits;
   } else {
-    decode_block(blockIdx.x, a.n_mtiles, a.B * a.H, bh, mt);
+    decode_block(blockIdx.x, a.n_mtiles, a.B * a.H, a.groups, !a.even, bh, mt);
   }
   const int b = bh / a.H, h = bh % a.H;
   const int M = a.M, N = a.N, p_seq = N - M;
@@ -637,7 +637,8 @@ hipError_t launch_fwd(const FwdK& a, int D, int dtype, hipStream_t s) {
 
 // Number of key splits the forward uses for a shape: 1 unless the grid of query tiles
 // alone leaves most of the chip idle while each workgroup has a long key loop (chunked
-// prefill, decode).  Splits are sized to give every CU about two workgroups; the streaming
+// prefill, decode).  Splits are sized to give every CU at most two workgroups: one workgroup more would
+// run in a second round of its own (B2 H16 M333 N5333 D128: six splits, 576 workgroups, 60 us; five, 480, 50 us).  The streaming
 // kernel of the single-query case keeps no tile in LDS and takes about eight per CU, at
 // least 512 keys each.
 int fwd_key_splits(int B, int H, int M, int N) {
@@ -651,7 +652,7 @@ int fwd_key_splits(int B, int H, int M, int N) {
   const int64_t wgs = (int64_t)((M + kFwdBM - 1) / kFwdBM) * B * H;
   const int key_tiles = (N + kFwdBN - 1) / kFwdBN;
   if (wgs >= 512 || key_tiles < 16) return 1;
-  int splits = (int)((512 + wgs - 1) / wgs);
+  int splits = (int)(512 / wgs);
   splits = splits > key_tiles / 8 ? key_tiles / 8 : splits;
   splits = splits > 32 ? 32 : splits;
   return splits < 1 ? 1 : splits;

@@ -31,6 +31,8 @@ struct FwdK {
   int B, H, M, N;
   float sm_scale;
   int n_mtiles;
+  int groups;      // (batch, head) groups of the launch order (order_groups)
+  bool even;       // the tiles weigh about the same (even_tiles)
   int splits;      // key splits of the forward (1 = none)
   float* ws_o;     // (splits, B, H, M, D) partial accumulators
   float* ws_ml;    // (splits, B, H, M, 2) partial row maximum and row sum
@@ -50,6 +52,8 @@ struct BwdK {
   int B, H, M, N;
   float sm_scale;
   int n_tiles;
+  int groups;      // (batch, head) groups of the launch order (order_groups), set by the launchers
+  bool even;       // the tiles weigh about the same (even_tiles), set by the launchers
   int cls;         // kClassAll, or the class of key tiles this dK/dV launch handles (fox_common.hpp)
   int light_limit; // distance from the diagonal, in keys, that separates the two classes
   int32_t* q_first_block;  // optional (B,H,ceil(M/kFwdBM)): first key block (of kFwdBN keys) each query tile of the dQ kernel visits
@@ -97,6 +101,24 @@ constexpr int kFwdBM = 128;
 constexpr int kFwdBN = 64;
 constexpr int kKvBN = 128;   // key rows per workgroup in the dK/dV kernel
 constexpr int kKvBM = 128;   // query rows per step in the dK/dV kernel
+
+// Groups of (batch, head) pairs in the launch order of the attention kernels (decode_block).  A group ends with its
+// lightest tiles, so the larger the last group, the less of the chip idles while the final heavy tiles finish; the
+// smaller a group, the better its K and V stay in an XCD's 4 MiB L2.  The line lies at 8 MiB of K and V per group and XCD,
+// with at least two pairs.  Forward time against one pair after the other, D = 128, B*H = 64, for 2 / 4 / 8 pairs a group:
+// T = 4096 (2 MiB a pair) 0.890 / 0.877 / 0.886, T = 8192 0.971 / 0.968 / 0.994, T = 16384 0.971 / 0.986 / 1.064; D = 64, B*H = 128,
+// T = 1024, for 4 / 8 / 16: 0.842 / 0.789 / 0.781.  With many more keys than queries the tiles weigh about the same and
+// only the caches count: one pair after the other (dK/dV at M = 128, N = 32768: 2.52 ms, in groups of two 2.65 ms).
+inline bool even_tiles(int M, int N) { return (int64_t)2 * M < N; }
+inline int order_groups(int n_bh, int M, int N, int D) {
+  const bool by_xcd = n_bh % 8 == 0;
+  const int nb = by_xcd ? n_bh / 8 : n_bh;
+  int64_t per = ((int64_t)8 << 20) / ((int64_t)N * D * 4);
+  if (per < 2) per = 2;
+  if (even_tiles(M, N)) per = 1;
+  const int64_t groups = nb / (by_xcd ? per : per * 8);
+  return groups < 1 ? 1 : (int)groups;
+}
 
 hipError_t launch_fwd(const FwdK& a, int D, int dtype, hipStream_t s);
 int fwd_key_splits(int B, int H, int M, int N);
