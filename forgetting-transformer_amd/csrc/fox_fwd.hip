@@ -638,7 +638,9 @@ hipError_t launch_fwd(const FwdK& a, int D, int dtype, hipStream_t s) {
 // Number of key splits the forward uses for a shape: 1 unless the grid of query tiles
 // alone leaves most of the chip idle while each workgroup has a long key loop (chunked
 // prefill, decode).  Splits are sized to give every CU at most two workgroups: one workgroup more would
-// run in a second round of its own (B2 H16 M333 N5333 D128: six splits, 576 workgroups, 60 us; five, 480, 50 us).  The streaming
+// run in a second round of its own (B2 H16 M333 N5333 D128: six splits, 576 workgroups, 60 us; five, 480, 50 us).  Between one
+// and two tiles per CU, tiles of equal weight are halved (the two rounds then even out what a CU with two tiles and one with a single
+// tile differ by); under a causal triangle the folded launch order evens that out already.  The streaming
 // kernel of the single-query case keeps no tile in LDS and takes about eight per CU, at
 // least 512 keys each.
 int fwd_key_splits(int B, int H, int M, int N) {
@@ -651,8 +653,8 @@ int fwd_key_splits(int B, int H, int M, int N) {
   }
   const int64_t wgs = (int64_t)((M + kFwdBM - 1) / kFwdBM) * B * H;
   const int key_tiles = (N + kFwdBN - 1) / kFwdBN;
-  if (wgs >= 512 || key_tiles < 16) return 1;
-  int splits = (int)(512 / wgs);
+  if (wgs >= 2 * kCus || key_tiles < 16) return 1;
+  int splits = wgs > kCus && even_tiles(M, N) ? 2 : (int)(2 * kCus / wgs);
   splits = splits > key_tiles / 8 ? key_tiles / 8 : splits;
   splits = splits > 32 ? 32 : splits;
   return splits < 1 ? 1 : splits;
