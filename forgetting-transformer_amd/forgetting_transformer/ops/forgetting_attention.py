@@ -21,7 +21,7 @@ from typing import Literal, Optional, Union
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 
 __all__ = ["forgetting_attention", "forgetting_attention_from_logits", "forgetting_attention_norm_gate",
            "qk_norm_threshold", "record_pruning_bounds", "ForgettingAttention", "ForgettingAttentionFromLogits",
@@ -475,6 +475,13 @@ def _backward(ctx, do):
     return dq, dk, dv, dgate
 
 
+def _native_threshold(threshold, q, head_first):
+    """A number becomes the cached (B, H) tensor of it, which is what the native path takes; anything else passes through."""
+    if type(threshold) in (float, int) and isinstance(q, torch.Tensor) and q.is_cuda and q.dim() == 4:
+        return _constant_threshold(float(threshold), q.shape[0], q.shape[1 if head_first else 2], q.device)
+    return threshold
+
+
 def forgetting_attention(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -510,6 +517,11 @@ def forgetting_attention(
     Returns:
         out: same shape, layout and dtype as q.
     """
+    if _bound_records is None:   # the native path; None: not a call for it (invalid, or tensors that need a copy first)
+        out = _native.load().attention(q, k, v, log_fgate, head_first, seq_start, sm_scale,
+                                       _native_threshold(adaptive_threshold, q, head_first), False)
+        if out is not None:
+            return out
     for name, entry in dict(q=q, k=k, v=v).items():
         assert entry.dtype in [torch.float16, torch.bfloat16], (
             f"Only torch.float16 or torch.bfloat16 are supported for q/k/v, but got {entry.dtype} for {name}.")
@@ -544,6 +556,11 @@ def forgetting_attention_from_logits(
     stores, ``modeling_forgetting_transformer.py:356-357``); gradients flow to q, k, v and
     fgate_logit through ``out`` only.
     """
+    if _bound_records is None:
+        out = _native.load().attention(q, k, v, fgate_logit, head_first, seq_start, sm_scale,
+                                       _native_threshold(adaptive_threshold, q, head_first), True)
+        if out is not None:
+            return out
     for name, entry in dict(q=q, k=k, v=v).items():
         assert entry.dtype in [torch.float16, torch.bfloat16], (
             f"Only torch.float16 or torch.bfloat16 are supported for q/k/v, but got {entry.dtype} for {name}.")
@@ -589,6 +606,12 @@ def forgetting_attention_norm_gate(
     ``forgetting_attention_from_logits`` and the result is ``(y, log_fgate)``: the whole chain from the layer's
     gate projection to the input of its output projection in one scan kernel and one attention kernel.
     """
+    if _bound_records is None and (gate is None or activation in _NORM_ACTS):
+        out = _native.load().attention_norm_gate(q, k, v, log_fgate, gate, norm_weight,
+                                                 _lib.ACT_NONE if gate is None else _NORM_ACTS[activation], eps, head_first, seq_start,
+                                                 sm_scale, _native_threshold(adaptive_threshold, q, head_first), fgate_is_logit)
+        if out is not None:
+            return out
     for name, entry in dict(q=q, k=k, v=v).items():
         assert entry.dtype in [torch.float16, torch.bfloat16], (
             f"Only torch.float16 or torch.bfloat16 are supported for q/k/v, but got {entry.dtype} for {name}.")

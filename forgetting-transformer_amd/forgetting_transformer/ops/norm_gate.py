@@ -18,7 +18,7 @@ from typing import Optional
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 from .forgetting_attention import _DTYPES, _stream
 
 __all__ = ["group_norm_gated", "GroupNormGated", "group_norm", "rms_norm", "GroupNormPlain"]
@@ -139,6 +139,10 @@ def group_norm_gated(x: torch.Tensor, g: torch.Tensor, weight: torch.Tensor, bia
     x, g: (..., num_groups * D) bfloat16/float16; weight: (num_groups * D,).  The FoX layer calls it with
     ``is_rms_norm=True, activation="sigmoid", num_groups=heads``.
     """
+    if bias is None and residual is None and not prenorm and not residual_in_fp32 and is_rms_norm and activation in _ACTS and g is not None:
+        y = _native.load().norm(x, g, weight, _ACTS[activation], eps, num_groups)   # None: not a call for the native path
+        if y is not None:
+            return y
     return GroupNormGated.apply(x, g, weight, bias, activation, residual, eps, prenorm, residual_in_fp32, is_rms_norm,
                                 num_groups)
 
@@ -151,6 +155,10 @@ def group_norm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
     The FoX layer's QK-norm: ``GroupNorm(num_groups=heads, hidden_size, is_rms_norm=True)`` on the (B, T, H*D)
     projections (``modeling_forgetting_transformer.py:264-265, 314-316``).
     """
+    if bias is None and residual is None and not prenorm and not residual_in_fp32 and is_rms_norm:
+        y = _native.load().norm(x, None, weight, _lib.ACT_NONE, eps, num_groups)
+        if y is not None:
+            return y
     return GroupNormPlain.apply(x, weight, bias, residual, eps, prenorm, residual_in_fp32, is_rms_norm, num_groups)
 
 
@@ -162,4 +170,4 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]
     The FoX layer's QK-norm with weights shared across heads: ``RMSNorm(head_dim)`` on (B, T, H, D)
     (``modeling_forgetting_transformer.py:261-262, 323-325``); the last dimension must be 16, 32, 64 or 128.
     """
-    return GroupNormPlain.apply(x, weight, bias, residual, eps, prenorm, residual_in_fp32, True, 1)
+    return group_norm(x, weight, bias, residual, eps, prenorm, residual_in_fp32, True, 1)

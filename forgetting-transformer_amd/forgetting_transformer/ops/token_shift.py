@@ -14,7 +14,7 @@ import ctypes as C
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 from .forgetting_attention import _DTYPES, _stream, maybe_contiguous
 
 __all__ = ["token_shift", "TokenShift"]
@@ -92,4 +92,5 @@ def token_shift(x: torch.Tensor, prev_weight: torch.Tensor, curr_weight: torch.T
     x: ``(B, T, H, D)`` bfloat16/float16; weights: ``(B, T, H)`` float32.  Differentiable
     with respect to all three arguments.
     """
-    return TokenShift.apply(x, prev_weight, curr_weight)
+    out = _native.load().token_shift(x, prev_weight, curr_weight)   # None: not a call for the native path
+    return TokenShift.apply(x, prev_weight, curr_weight) if out is None else out

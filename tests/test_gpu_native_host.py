@@ -1,0 +1,109 @@
+"""GPU tests of the native host path (csrc/fox_torch.cpp) against the general Python path, which the same inputs take through the
+autograd nodes directly: the two launch the same kernels, so every output and gradient must agree bit for bit, in both
+layouts, with every optional argument, and for inputs the native path hands back (tensors that need a copy first)."""
+from importlib import import_module
+
+import pytest
+import torch
+
+from conftest import make_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ft():
+    assert torch.cuda.is_available(), "these tests need the MI355X"
+    import forgetting_transformer
+    return forgetting_transformer
+
+
+def _grads(out, leaves, do):
+    return (out.detach(),) + torch.autograd.grad(out, leaves, do)
+
+
+def _equal(a, b):
+    for x, y in zip(a, b):
+        assert x.shape == y.shape and x.dtype == y.dtype and torch.equal(x, y)
+
+
+@pytest.mark.parametrize("head_first", [True, False])
+@pytest.mark.parametrize("logit", [False, True])
+@pytest.mark.parametrize("thr,seq,M", [(None, None, 130), ("auto", [3, 60], 130), (-5.0, None, 200), ("per_head", [0, 7], 1), ("table", None, 77)])
+def test_attention(ft, head_first, logit, thr, seq, M):
+    from forgetting_transformer.ops import _native
+    F = import_module("forgetting_transformer.ops.forgetting_attention")
+    B, H, N, D = 2, 3, 200, 64
+    q, k, v, g, do, ss = make_inputs(B, H, M, N, D, device="cuda", head_first=head_first, seq_start=seq, seed=M, gate_mean=1.0)
+    if logit:
+        g = (g * 3 + 2).bfloat16()
+    t = {"per_head": torch.linspace(-9, -3, H, device="cuda"), "table": torch.full((B, H), -4.0, device="cuda")}.get(thr, thr)
+    leaves = [x.requires_grad_() for x in (q, k, v, g)]
+    assert _native.load().attention(q, k, v, g, head_first, ss, None, F._native_threshold(t, q, head_first), logit) is not None
+    fn = ft.forgetting_attention_from_logits if logit else ft.forgetting_attention
+    out = fn(q, k, v, g, head_first=head_first, seq_start=ss, adaptive_threshold=t)
+    a = [x if head_first else x.transpose(1, 2) for x in (q, k, v, g)]
+    node = F.ForgettingAttentionFromLogits if logit else F.ForgettingAttention
+    ref = node.apply(*a, ss, None, t) if logit else node.apply(*a, ss, True, None, t)
+    back = lambda x: x if head_first else x.transpose(1, 2)
+    if logit:
+        assert torch.equal(out[1], back(ref[1])) and not out[1].requires_grad
+        out, ref = out[0], ref[0]
+    _equal(_grads(out, leaves, do), _grads(back(ref), leaves, do))
+    with torch.no_grad():
+        plain = fn(q, k, v, g, head_first=head_first, seq_start=ss, adaptive_threshold=t)
+    assert torch.equal(plain[0] if logit else plain, out) and not (plain[0] if logit else plain).requires_grad
+
+
+@pytest.mark.parametrize("head_first", [True, False])
+@pytest.mark.parametrize("gated,M", [(True, 130), (False, 130), (True, 1)])
+def test_attention_norm_gate(ft, head_first, gated, M):
+    from forgetting_transformer.ops import _lib
+    F = import_module("forgetting_transformer.ops.forgetting_attention")
+    B, H, N, D = 2, 3, 200, 64
+    q, k, v, g, do, ss = make_inputs(B, H, M, N, D, device="cuda", head_first=False, seed=M)
+    gate = torch.randn(B, M, H, D, device="cuda").bfloat16() if gated else None
+    swap = (lambda x: x.transpose(1, 2)) if head_first else (lambda x: x)   # head-first views of (B, T, H * D) memory, as the layer has them
+    w = torch.rand(H * D, device="cuda", requires_grad=True)
+    leaves = [x.requires_grad_() for x in (q, k, v, g) + ((gate,) if gated else ())] + [w]
+    args = [swap(x) for x in (q, k, v, g)]
+    y = ft.forgetting_attention_norm_gate(*args, swap(gate) if gated else None, w, head_first=head_first)
+    hf = [x.transpose(1, 2) for x in (q, k, v, g)] + [gate.transpose(1, 2) if gated else None]
+    ref = F.ForgettingAttentionNormGate.apply(*hf, w, None, None, None, _lib.ACT_SIGMOID if gated else _lib.ACT_NONE, 1e-6, False)
+    _equal(_grads(swap(y), leaves, do), _grads(ref.transpose(1, 2), leaves, do))
+
+
+def test_norms_and_shift(ft):
+    from forgetting_transformer.ops import _lib
+    from forgetting_transformer.ops.norm_gate import GroupNormGated, GroupNormPlain
+    from forgetting_transformer.ops.token_shift import TokenShift
+    x, g = (torch.randn(2, 50, 192, device="cuda").bfloat16().requires_grad_() for _ in range(2))
+    w = torch.rand(192, device="cuda").bfloat16().requires_grad_()
+    do = torch.randn_like(x)
+    _equal(_grads(ft.group_norm(x, w, is_rms_norm=True, num_groups=3), [x, w], do),
+           _grads(GroupNormPlain.apply(x, w, None, None, 1e-5, False, False, True, 3), [x, w], do))
+    _equal(_grads(ft.group_norm_gated(x, g, w, is_rms_norm=True, num_groups=3), [x, g, w], do),
+           _grads(GroupNormGated.apply(x, g, w, None, "swish", None, 1e-6, False, False, True, 3), [x, g, w], do))
+    x4 = x.detach().view(2, 50, 3, 64).requires_grad_()
+    p, c = (torch.rand(2, 50, 3, device="cuda").requires_grad_() for _ in range(2))
+    _equal(_grads(ft.token_shift(x4, p, c), [x4, p, c], do.view_as(x4)), _grads(TokenShift.apply(x4, p, c), [x4, p, c], do.view_as(x4)))
+
+
+def test_calls_the_native_path_hands_back(ft):
+    """Misaligned and non-unit-stride inputs are copied by the general path, other streams and a second backward behave as before."""
+    q, k, v, g, do, _ = make_inputs(1, 2, 90, 90, 32, device="cuda", seed=1)
+    want = ft.forgetting_attention(q, k, v, g, head_first=True)
+    odd = torch.empty(1, 2, 90, 33, device="cuda", dtype=q.dtype)[..., :32].copy_(q)
+    assert torch.equal(ft.forgetting_attention(odd, k, v, g, head_first=True), want)
+    assert torch.equal(ft.forgetting_attention(q, k, v, g, head_first=True, seq_start=torch.zeros(1, dtype=torch.int32, device="cuda")), want)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        other = ft.forgetting_attention(q, k, v, g, head_first=True)
+    torch.cuda.current_stream().wait_stream(s)
+    assert torch.equal(other, want)
+    leaves = [x.requires_grad_() for x in (q, k, v, g)]
+    out = ft.forgetting_attention(q, k, v, g, head_first=True)
+    _equal(torch.autograd.grad(out, leaves, do, retain_graph=True), torch.autograd.grad(out, leaves, do))
+    with pytest.raises(RuntimeError, match="backward through the graph a second time"):
+        torch.autograd.grad(out, leaves, do)
