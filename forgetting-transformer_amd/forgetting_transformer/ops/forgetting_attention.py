@@ -251,7 +251,10 @@ def _heads_adjacent(x: torch.Tensor) -> torch.Tensor:
     elements per token, the layout of the layer's (batch, time, hidden) tensors.  Copies only when needed."""
     B, H, M, D = x.shape
     ok = x.stride() == (M * H * D, D, H * D, 1) and x.data_ptr() % 16 == 0
-    return x if ok else x.transpose(1, 2).contiguous().transpose(1, 2)
+    if ok:
+        return x
+    # (contiguous() would keep any stride on an axis of length 1, and the kernels get the strides as they are)
+    return torch.empty((B, M, H, D), dtype=x.dtype, device=x.device).transpose(1, 2).copy_(x)
 
 
 _GATE_DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16, torch.float32: _lib.DTYPE_FP32}
