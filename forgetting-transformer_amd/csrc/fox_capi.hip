@@ -413,6 +413,13 @@ int fox_auto_threshold(const fox_dims* dims, const fox_view* q, const fox_view* 
                    "fox_auto_threshold");
 }
 
+int fox_qk_norm_threshold(const float* q_weight, const float* k_weight, int32_t H, int32_t D, double seq_len, double tolerance, float* thr,
+                          void* stream) {
+  if (!q_weight || !k_weight || !thr) return fail(FOX_E_ARG, "q_weight, k_weight and thr must not be NULL");
+  if (H <= 0 || D <= 0) return fail(FOX_E_ARG, "H and D must be positive (got %d, %d)", H, D);
+  return check_hip(fox::launch_qk_norm_threshold(q_weight, k_weight, H, D, seq_len, tolerance, thr, (hipStream_t)stream), "fox_qk_norm_threshold");
+}
+
 int fox_attn_fwd_workspace_bytes(const fox_dims* dims, int64_t* bytes) {
   FOX_TRY(check_dims(dims));
   if (!bytes) return fail(FOX_E_ARG, "bytes is NULL");

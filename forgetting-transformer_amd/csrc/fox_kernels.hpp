@@ -75,6 +75,7 @@ struct ShiftK {
   float* dcurr_w;
   int64_t x_sb, x_st, x_sh, w_sb, w_st, w_sh;
   int B, T, H;
+  int strip;   // time steps per thread, set by the launcher
 };
 
 // Gated per-head RMS norm: x, g, y, dy, dx, dg are (R rows, G heads, D) 16-bit, heads and head dim
@@ -94,6 +95,7 @@ struct NormGateK {
   int64_t R;
   int G;
   float eps;
+  int cols, rows_per_lane;   // how the backward is cut (norm_bwd_plan), set by the launcher
 };
 
 // Tile sizes (see fox_tile_config in the public header)
@@ -128,7 +130,6 @@ bool dkdv_split_supports(int D);   // head dims the split (kClassLight) variant 
 hipError_t launch_bwd_dq(const BwdK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_fwd_decode(const FwdK& a, int D, int dtype, hipStream_t s);  // M == 1, without the merge of the splits
 hipError_t launch_norm_gate(const NormGateK& a, int D, int dtype, bool bwd, int act, hipStream_t s);  // act: FOX_ACT_*
-int64_t norm_gate_strips(int64_t rows);
 int64_t norm_gate_workspace_rows(int64_t rows);
 hipError_t launch_shift_fwd(const ShiftK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_shift_bwd(const ShiftK& a, int D, int dtype, hipStream_t s);
@@ -142,6 +143,7 @@ hipError_t launch_gate_cumsum_bwd(const float* dc, const void* logits, int dtype
 hipError_t launch_cumsum_bwd(const float* dc, float* dg, int64_t db, int64_t dh, int64_t dn, const int64_t* seq_start, int B, int H,
                              int N, hipStream_t s);
 hipError_t launch_mfma_probe(const void* operands, float* sink, int workgroups, int iters, hipStream_t s);  // fox_probe.hip
+hipError_t launch_qk_norm_threshold(const float* wq, const float* wk, int H, int D, double seq_len, double tolerance, float* thr, hipStream_t s);
 hipError_t launch_auto_threshold(const View& q, const View& k, int B, int H, int M, int N, int D, int dtype, float sm_scale,
                                  float* thr, uint32_t* scratch, hipStream_t s);
 

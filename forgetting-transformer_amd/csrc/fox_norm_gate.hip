@@ -13,8 +13,8 @@
 //
 // Both are pure streams over HBM.  A (row, head) group of D elements is spread over D/8 lanes, 16
 // bytes each; the two row reductions are shuffles inside that lane group.  In the backward every
-// thread keeps one (head, 8 elements) column and walks a strip of rows, so the weight gradient is
-// accumulated in registers and leaves as one partial per strip; a second kernel adds the partials in
+// thread keeps one (head, 8 elements) column and walks rows of a strip, so the weight gradient is
+// accumulated in registers and leaves as one partial per workgroup; a second kernel adds the partials in
 // a fixed order (no atomics: the result does not depend on scheduling).
 #include "fox_common.hpp"
 #include "fox_kernels.hpp"
@@ -74,21 +74,25 @@ __global__ __launch_bounds__(256) void norm_gate_fwd_kernel(const NormGateK a) {
   }
 }
 
-constexpr int kNormStrip = 32;  // rows per thread in the backward
-
+// Backward.  A workgroup covers `cols` (head, 8 elements) columns -- all of them up to 256 -- times R = blockDim / cols row lanes,
+// and walks `rows_per_lane` rows per lane (every R-th row of its strip), so that a wave reads whole token rows, the weight
+// gradient is accumulated in registers over the rows of a lane, through LDS over the R lanes, and leaves as one partial
+// row per workgroup.  The kernel streams (5 x 2 bytes per element, 3 x 2 without a gate); what bounds a small call is how much of it is in
+// flight, so the rows per lane follow from the size (norm_bwd_plan).  Both launches together: at 32 rows per thread whatever the size,
+// 4096 rows of 12 x 64 made 48 workgroups and took 34.4 us gated and 21.0 us plain, now 12.1 and 9.2 us; 65536 rows of 16 x 128
+// stay at 32 rows (262 and 150 us, 5.1 and 5.4 TB/s); 1 M rows of one 128-element head 183 -> 142 us (fewer partials).
 template <typename Tr, int D, int ACT>
 __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const NormGateK a) {
   constexpr int CH = D / 8;
-  const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int chunk = (int)(gid % CH);
-  const int64_t col = gid / CH;
-  const int h = (int)(col % a.G);
-  const int64_t strip = col / a.G;
-  const int64_t r0 = strip * kNormStrip;
-  const bool live = r0 < a.R;
-  const int64_t r1 = live ? min((int64_t)a.R, r0 + kNormStrip) : r0;
-  const int hh = live ? h : 0;
-  const int64_t off = hh * (int64_t)D + chunk * 8;
+  __shared__ __align__(16) float dw_s[256][8];
+  const int tid = threadIdx.x, rl = tid / a.cols, cl = tid - rl * a.cols;
+  const int R = blockDim.x / a.cols;                    // row lanes (threads beyond R * cols idle)
+  const int col = blockIdx.y * a.cols + cl;
+  const bool live = rl < R && col < a.G * CH;
+  const int hh = live ? col / CH : 0;
+  const int64_t off = live ? (int64_t)col * 8 : 0;
+  const int64_t r0 = (int64_t)blockIdx.x * R * a.rows_per_lane;
+  const int64_t r1 = min((int64_t)a.R, r0 + (int64_t)R * a.rows_per_lane);
   float w[8], dw[8];
   {
     const f32x4 w0 = *reinterpret_cast<const f32x4*>(a.w + off), w1 = *reinterpret_cast<const f32x4*>(a.w + off + 4);
@@ -99,12 +103,12 @@ __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const NormGateK a) {
   for (int e = 0; e < 8; ++e) dw[e] = 0.f;
 
   constexpr int U = 4;  // rows in flight
-  for (int64_t rb = r0; rb < r1; rb += U) {
+  for (int64_t rb = r0 + rl; live && rb < r1; rb += U * R) {   // (the lanes of a (row, head) group enter and leave together)
     u32x4 xv[U], gv[U], dyv[U];
     float rs[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t r = min(rb + u, r1 - 1);
+      const int64_t r = min(rb + u * R, r1 - 1);
       xv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a.x + r * a.x_sr + off));
       if (ACT != kActNone) gv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a.g + r * a.g_sr + off));
       dyv[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a.dy + r * a.dy_sr + off));
@@ -112,8 +116,8 @@ __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const NormGateK a) {
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t r = rb + u;
-      if (r < r1) {  // uniform over the lanes of a (head, strip) group
+      const int64_t r = rb + u * R;
+      if (r < r1) {
         float x[8], g[8], dy[8], dx[8], dg[8], wdy[8];
         unpack8v<Tr>(xv[u], x);
         if (ACT != kActNone) unpack8v<Tr>(gv[u], g);
@@ -155,35 +159,53 @@ __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const NormGateK a) {
       }
     }
   }
-  if (live) {
-    float* p = a.dw_partial + strip * (int64_t)a.G * D + off;
+  if (R > 1) {   // add the row lanes in order
+#pragma unroll
+    for (int e = 0; e < 8; ++e) dw_s[tid][e] = dw[e];
+    __syncthreads();
+    const float* flat = &dw_s[0][0];
+    float* p = a.dw_partial + (int64_t)blockIdx.x * a.G * D;   // (R > 1: one workgroup holds all columns)
+    for (int j = tid; j < a.cols * 8; j += blockDim.x) {
+      float sum = flat[j];
+#pragma unroll 8
+      for (int q = 1; q < R; ++q) sum += flat[q * a.cols * 8 + j];
+      p[j] = sum;
+    }
+  } else if (live) {
+    float* p = a.dw_partial + (int64_t)blockIdx.x * a.G * D + off;
     const f32x4 lo = {dw[0], dw[1], dw[2], dw[3]}, hi = {dw[4], dw[5], dw[6], dw[7]};
     *reinterpret_cast<f32x4*>(p) = lo;
     *reinterpret_cast<f32x4*>(p + 4) = hi;
   }
 }
 
-// dst[group][j] = sum of src[s][j] over the rows s of the group (per_group consecutive rows), added in
-// index order.  Two passes (strips -> groups of kReduceGroup strips -> total) turn the partial weight
-// gradients into dw with enough parallelism and a summation order that does not depend on scheduling.
-constexpr int kReduceGroup = 32;
-__global__ __launch_bounds__(256) void reduce_rows_kernel(const float* __restrict__ src, float* __restrict__ dst, int64_t n_rows,
-                                                          int width, int per_group) {
-  const int j = blockIdx.x * 256 + threadIdx.x;
-  if (j >= width) return;
-  const int64_t s0 = (int64_t)blockIdx.y * per_group;
-  const int64_t s1 = min(n_rows, s0 + per_group);
+// dst[group][j] = sum of src[s][j] over the `per_group` consecutive rows s of the group, in a fixed order: 64 columns per
+// workgroup, one per lane, its 16 waves taking every 16th row; the waves' sums are added in order.  Up to kReduceRows rows
+// are added in one launch, more in two (groups of kReduceRows, then the groups' sums).
+constexpr int kReduceRows = 512;
+__global__ __launch_bounds__(1024) void reduce_rows_kernel(const float* __restrict__ src, float* __restrict__ dst, int64_t n_rows,
+                                                           int width, int per_group) {
+  __shared__ float part[16][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = blockIdx.x * 64 + lane;
+  const int64_t s0 = (int64_t)blockIdx.y * per_group, s1 = min(n_rows, s0 + per_group);
   float acc = 0.f;
-  int64_t s = s0;
-  for (; s + 8 <= s1; s += 8) {
-    float v[8];
+  if (j < width) {
+    int64_t s = s0 + wave;
+    for (; s + 7 * 16 < s1; s += 8 * 16) {
+      float v[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = src[(s + u) * width + j];
+      for (int u = 0; u < 8; ++u) v[u] = src[(s + 16 * u) * width + j];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) acc += v[u];
+      for (int u = 0; u < 8; ++u) acc += v[u];
+    }
+    for (; s < s1; s += 16) acc += src[s * width + j];
   }
-  for (; s < s1; ++s) acc += src[s * width + j];
-  dst[(int64_t)blockIdx.y * width + j] = acc;
+  part[wave][lane] = acc;
+  __syncthreads();
+  if (wave == 0 && j < width) {
+    for (int q = 1; q < 16; ++q) acc += part[q][lane];
+    dst[(int64_t)blockIdx.y * width + j] = acc;
+  }
 }
 
 #define FOX_NG_INST(TR, DD)                                                   \
@@ -197,11 +219,32 @@ __global__ __launch_bounds__(256) void reduce_rows_kernel(const float* __restric
 FOX_NG_INST_ALL(Bf16)
 FOX_NG_INST_ALL(Fp16)
 
-int64_t norm_gate_strips(int64_t rows) { return (rows + kNormStrip - 1) / kNormStrip; }
-// rows of G*D floats the backward needs as workspace: one per strip plus one per group of strips
+// How the backward of `rows` rows of G heads is cut: columns per workgroup, row lanes, rows per lane, workgroups along the rows.
+struct NormBwdPlan {
+  int cols, lanes, rows_per_lane;
+  int64_t strips;
+};
+constexpr int kNormRowsPerLane = 32;   // at most
+static NormBwdPlan norm_bwd_plan(int64_t rows, int G, int D) {
+  NormBwdPlan p;
+  const int all = G * (D / 8), chunks = (all + 255) / 256;
+  p.cols = all < 256 ? all : 256;
+  p.lanes = 256 / p.cols;
+  // about four workgroups per CU, at least four rows per lane (what it keeps in flight)
+  int64_t per = rows * chunks / ((int64_t)p.lanes * 4 * kCus);
+  per = per < 4 ? 4 : per > kNormRowsPerLane ? kNormRowsPerLane : per;
+  p.rows_per_lane = (int)per;
+  p.strips = (rows + p.lanes * per - 1) / (p.lanes * per);
+  return p;
+}
+// Rows of G*D floats the backward needs as workspace, an upper bound over G and D: one per workgroup along the rows (with at least
+// kNormRowsPerLane rows each, or about 4 * kCus of them for small calls) plus one per group of kReduceRows of those; what it
+// adds for the groups is generous (callers were told one per 32).
 int64_t norm_gate_workspace_rows(int64_t rows) {
-  const int64_t strips = norm_gate_strips(rows);
-  return strips + (strips + kReduceGroup - 1) / kReduceGroup;
+  int64_t strips = (rows + kNormRowsPerLane - 1) / kNormRowsPerLane;
+  const int64_t small = (rows + 3) / 4 < 8 * kCus ? (rows + 3) / 4 : 8 * kCus;
+  strips = strips > small ? strips : small;
+  return strips + (strips + 31) / 32;
 }
 
 template <typename Tr, int D>
@@ -215,19 +258,24 @@ static hipError_t norm_gate_d(const NormGateK& a, bool bwd, int act, hipStream_t
     else hipLaunchKernelGGL((norm_gate_fwd_kernel<Tr, D, kActSigmoid>), grid, dim3(256), 0, s, a);
     return hipGetLastError();
   }
-  const int64_t strips = norm_gate_strips(a.R);
-  const int64_t threads = strips * a.G * CH;
-  const dim3 grid((unsigned)((threads + 255) / 256));
-  if (act == kActSwish) hipLaunchKernelGGL((norm_gate_bwd_kernel<Tr, D, kActSwish>), grid, dim3(256), 0, s, a);
-  else if (act == kActNone) hipLaunchKernelGGL((norm_gate_bwd_kernel<Tr, D, kActNone>), grid, dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((norm_gate_bwd_kernel<Tr, D, kActSigmoid>), grid, dim3(256), 0, s, a);
+  const NormBwdPlan p = norm_bwd_plan(a.R, a.G, D);
+  NormGateK k = a;
+  k.cols = p.cols;
+  k.rows_per_lane = p.rows_per_lane;
+  const dim3 grid((unsigned)p.strips, (unsigned)((a.G * CH + p.cols - 1) / p.cols)), block((unsigned)((p.cols * p.lanes + 63) / 64 * 64));
+  if (act == kActSwish) hipLaunchKernelGGL((norm_gate_bwd_kernel<Tr, D, kActSwish>), grid, block, 0, s, k);
+  else if (act == kActNone) hipLaunchKernelGGL((norm_gate_bwd_kernel<Tr, D, kActNone>), grid, block, 0, s, k);
+  else hipLaunchKernelGGL((norm_gate_bwd_kernel<Tr, D, kActSigmoid>), grid, block, 0, s, k);
   const int width = a.G * D;
-  const int64_t groups = (strips + kReduceGroup - 1) / kReduceGroup;
-  float* stage = a.dw_partial + strips * width;  // second part of the workspace
-  hipLaunchKernelGGL(reduce_rows_kernel, dim3((unsigned)((width + 255) / 256), (unsigned)groups), dim3(256), 0, s, a.dw_partial,
-                     stage, strips, width, kReduceGroup);
-  hipLaunchKernelGGL(reduce_rows_kernel, dim3((unsigned)((width + 255) / 256), 1u), dim3(256), 0, s, stage, a.dw, groups, width,
-                     (int)groups);
+  const int64_t groups = (p.strips + kReduceRows - 1) / kReduceRows;
+  const dim3 columns((unsigned)((width + 63) / 64));
+  if (groups == 1) {
+    hipLaunchKernelGGL(reduce_rows_kernel, columns, dim3(1024), 0, s, a.dw_partial, a.dw, p.strips, width, (int)p.strips);
+    return hipGetLastError();
+  }
+  float* stage = a.dw_partial + p.strips * width;  // second part of the workspace
+  hipLaunchKernelGGL(reduce_rows_kernel, dim3(columns.x, (unsigned)groups), dim3(1024), 0, s, a.dw_partial, stage, p.strips, width, kReduceRows);
+  hipLaunchKernelGGL(reduce_rows_kernel, columns, dim3(1024), 0, s, stage, a.dw, groups, width, (int)groups);
   return hipGetLastError();
 }
 

@@ -8,7 +8,7 @@
 // (reference: model/forgetting_transformer/token_shift.py:21-71 forward, :83-156 backward)
 //
 // Both are pure streams over HBM.  A thread owns 8 consecutive head-dim elements
-// (one 16-byte vector) of one (batch, head) column and walks a strip of kStrip time
+// (one 16-byte vector) of one (batch, head) column and walks a strip of time
 // steps with the neighbouring row carried in registers, so every element is fetched
 // once (plus one halo row per strip) and consecutive lanes cover consecutive memory
 // of the (H*D)-element token row.  (strip, head, chunk) triples are flattened over
@@ -18,7 +18,10 @@
 
 namespace fox {
 
-constexpr int kStrip = 32;  // time steps per thread
+// Time steps per thread: long enough that the halo row costs little, short enough that the call has some four workgroups per CU
+// to keep in flight.  At 32 whatever the size, B2 T2048 H12 D64 made 48 workgroups and took 9.0 us forward and 19.2 us
+// backward, now 3.8 and 5.2 us; B4 T16384 H16 D128 stays at 32 (86 and 148 us).
+constexpr int kMaxStrip = 32, kMinStrip = 4;
 
 template <typename Tr>
 __device__ __forceinline__ void unpack8(const u32x4& v, float (&f)[8]) {
@@ -38,9 +41,9 @@ __global__ __launch_bounds__(256) void shift_fwd_kernel(const ShiftK a) {
   const int h = (int)(col % a.H);
   const int strip = (int)(col / a.H);
   const int b = blockIdx.y;
-  const int t0 = strip * kStrip;
+  const int t0 = strip * a.strip;
   if (t0 >= a.T) return;
-  const int t1 = min(a.T, t0 + kStrip);
+  const int t1 = min(a.T, t0 + a.strip);
   const uint16_t* xp = a.x + b * a.x_sb + h * a.x_sh + chunk * 8;
   uint16_t* op = a.out + b * a.x_sb + h * a.x_sh + chunk * 8;
   const float* pw = a.prev_w + b * a.w_sb + h * a.w_sh;
@@ -85,10 +88,10 @@ __global__ __launch_bounds__(256) void shift_bwd_kernel(const ShiftK a) {
   const int h = (int)(col % a.H);
   const int strip = (int)(col / a.H);
   const int b = blockIdx.y;
-  const int t0 = strip * kStrip;
+  const int t0 = strip * a.strip;
   // no early return: the lanes of one (head, strip) reduce together, and whole groups leave together
   const bool live = t0 < a.T;
-  const int t1 = live ? min(a.T, t0 + kStrip) : t0;
+  const int t1 = live ? min(a.T, t0 + a.strip) : t0;
   const int hh = live ? h : 0;
   const uint16_t* xp = a.x + b * a.x_sb + hh * a.x_sh + chunk * 8;
   const uint16_t* gp = a.dout + b * a.x_sb + hh * a.x_sh + chunk * 8;
@@ -173,8 +176,11 @@ FOX_INSTANTIATE_SHIFT(Bf16)
 FOX_INSTANTIATE_SHIFT(Fp16)
 
 template <typename Tr, bool BWD>
-static hipError_t shift_t(const ShiftK& a, int D, hipStream_t s) {
-  const int64_t strips = (a.T + kStrip - 1) / kStrip;
+static hipError_t shift_t(const ShiftK& a0, int D, hipStream_t s) {
+  ShiftK a = a0;
+  const int64_t per = (int64_t)a.B * a.T * a.H * (D / 8) / ((int64_t)256 * 4 * kCus);
+  a.strip = per < kMinStrip ? kMinStrip : per > kMaxStrip ? kMaxStrip : (int)per;
+  const int64_t strips = (a.T + a.strip - 1) / a.strip;
   const int64_t threads = strips * a.H * (D / 8);
   const dim3 grid((unsigned)((threads + 255) / 256), (unsigned)a.B);
 #define FOX_SHIFT_CASE(DD)                                                                   \

@@ -601,7 +601,31 @@ PyObject* py_token_shift(PyObject*, PyObject* const* o, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// qk_norm_threshold(q_weight, k_weight, num_heads, head_dim, seq_len, tolerance, shared)
+PyObject* py_qk_norm_threshold(PyObject*, PyObject* const* o, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 7, "qk_norm_threshold takes 7 arguments");
+  const Tensor *q = tensor_of(o[0]), *k = tensor_of(o[1]);
+  const long H = PyLong_AsLong(o[2]), D = PyLong_AsLong(o[3]);
+  const double T = PyFloat_AsDouble(o[4]), tolerance = PyFloat_AsDouble(o[5]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    return none();
+  }
+  const bool shared = o[6] == Py_True;
+  if (!q || !k || H < 1 || D < 1 || !(T > 0) || !on_current_gpu(*q) || k->device() != q->device() || q->dim() != 1 || q->sizes() != k->sizes() ||
+      q->size(0) != (shared ? D : H * D) || q->scalar_type() != at::kFloat || k->scalar_type() != at::kFloat || !q->is_contiguous() || !k->is_contiguous())
+    return none();
+  const at::NoGradGuard no_grad;
+  Tensor thr = shared ? at::empty({}, q->options()) : at::empty({H}, q->options());
+  check(fox_qk_norm_threshold(q->const_data_ptr<float>(), k->const_data_ptr<float>(), shared ? 1 : (int32_t)H, (int32_t)D, T, tolerance,
+                              thr.mutable_data_ptr<float>(), stream_of(*q)), "fox_qk_norm_threshold");
+  return THPVariable_Wrap(thr);
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"qk_norm_threshold", (PyCFunction)(void (*)(void))py_qk_norm_threshold, METH_FASTCALL, nullptr},
     {"attention", (PyCFunction)(void (*)(void))py_attention, METH_FASTCALL, nullptr},
     {"attention_norm_gate", (PyCFunction)(void (*)(void))py_attention_norm_gate, METH_FASTCALL, nullptr},
     {"norm", (PyCFunction)(void (*)(void))py_norm, METH_FASTCALL, nullptr},

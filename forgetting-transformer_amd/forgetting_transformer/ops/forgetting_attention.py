@@ -633,7 +633,6 @@ def forgetting_attention_norm_gate(
     return out if head_first else out.transpose(1, 2)
 
 
-@torch.no_grad()
 def qk_norm_threshold(q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, num_heads: int, head_dim: int,
                       seq_len: int, log_pruning_tolerance: float, share_param_across_head: bool = False) -> torch.Tensor:
     """``adaptive_threshold`` for queries and keys that went through an RMS QK-norm, from the norm weights alone.
@@ -645,6 +644,18 @@ def qk_norm_threshold(q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, 
     ``forgetting_attention`` broadcasts over the batch; with ``share_param_across_head`` the weights are
     ``(head_dim,)`` and the result is a 0-d tensor.  No pass over q and k is needed (unlike ``"auto"``).
     """
+    thr = _native.load().qk_norm_threshold(q_norm_weight, k_norm_weight, num_heads, head_dim, seq_len, log_pruning_tolerance,
+                                           share_param_across_head)
+    if thr is not None:
+        return thr
+    return _qk_norm_threshold_general(q_norm_weight, k_norm_weight, num_heads, head_dim, seq_len, log_pruning_tolerance,
+                                      share_param_across_head)
+
+
+@torch.no_grad()
+def _qk_norm_threshold_general(q_norm_weight, k_norm_weight, num_heads, head_dim, seq_len, log_pruning_tolerance,
+                               share_param_across_head):
+    """The same rule in tensor operations, for weights the kernel does not take (other dtypes, host tensors)."""
     if share_param_across_head:
         assert q_norm_weight.shape == k_norm_weight.shape == (head_dim,)
         bound = q_norm_weight.abs().max() * k_norm_weight.abs().max() * math.sqrt(head_dim)

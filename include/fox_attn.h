@@ -135,6 +135,14 @@ int fox_gate_cumsum_bwd(const float* dc, const void* logits, int32_t logits_dtyp
 int fox_auto_threshold(const fox_dims* dims, const fox_view* q, const fox_view* k, float sm_scale, float* thr,
                        uint32_t* scratch, void* stream);
 
+/*
+ * thr[h] = -(2 * max_d|q_weight[h,d]| * max_d|k_weight[h,d]| * sqrt(D) + log(seq_len)) + tolerance for H heads of D contiguous
+ * fp32 norm weights, every operation rounded to fp32: the pruning threshold the layer derives from its QK-norm weights
+ * (model/forgetting_transformer/modeling_forgetting_transformer.py:366-380); weights shared across heads are H = 1.
+ */
+int fox_qk_norm_threshold(const float* q_weight, const float* k_weight, int32_t H, int32_t D, double seq_len, double tolerance,
+                          float* thr, void* stream);
+
 typedef struct fox_fwd_args {
   fox_dims dims;
   fox_view q, k, v, o;        /* o is written */

@@ -107,3 +107,53 @@ def test_calls_the_native_path_hands_back(ft):
     _equal(torch.autograd.grad(out, leaves, do, retain_graph=True), torch.autograd.grad(out, leaves, do))
     with pytest.raises(RuntimeError, match="backward through the graph a second time"):
         torch.autograd.grad(out, leaves, do)
+
+
+@pytest.mark.parametrize("H,D,shared", [(1, 16, False), (5, 64, False), (12, 128, False), (3, 32, True)])
+def test_qk_norm_threshold(ft, H, D, shared):
+    """The kernel against the tensor expression it replaces, rounding for rounding."""
+    general = import_module("forgetting_transformer.ops.forgetting_attention")._qk_norm_threshold_general
+    n = D if shared else H * D
+    wq, wk = (torch.randn(n, device="cuda", requires_grad=True) for _ in range(2))
+    got = ft.qk_norm_threshold(wq, wk, H, D, 1777, -10.0, shared)
+    want = general(wq, wk, H, D, 1777, -10.0, shared)
+    assert torch.equal(got, want) and got.shape == want.shape and not got.requires_grad
+    with torch.no_grad():
+        wk[n - 1] = float("nan")
+    assert torch.equal(ft.qk_norm_threshold(wq, wk, H, D, 1777, -10.0, shared).isnan(), general(wq, wk, H, D, 1777, -10.0, shared).isnan())
+
+
+@pytest.mark.parametrize("rows,G,D", [(1, 1, 16), (3, 3, 64), (700, 12, 64), (5000, 5, 32), (4097, 33, 64), (40000, 2, 16), (33001, 1, 128)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_norm_backward_plans(ft, rows, G, D, gated):
+    """Backward of the norms over the ways it is cut: one or several column blocks, row lanes, rows per lane, one or two passes over the
+    partial weight gradients.  dweight sums `rows` products of O(1) 16-bit values: fp32 rounding of the partial sums gives
+    about sqrt(rows) * 2^-24 of its scale, well below the 1e-4 asked; dx and dg are one rounding to bf16 (2^-8 of their own scale)."""
+    from oracle import fox_oracle as O
+    gen = torch.Generator(device="cuda").manual_seed(rows + G)
+    rnd = lambda: torch.randn(rows, G * D, generator=gen, device="cuda").bfloat16()
+    x, g, do = rnd().requires_grad_(), rnd().requires_grad_() if gated else None, rnd()
+    w = (torch.rand(G * D, generator=gen, device="cuda") + 0.5).requires_grad_()
+    leaves = [x, w] + ([g] if gated else [])
+    y = ft.group_norm_gated(x, g, w, None, "sigmoid", is_rms_norm=True, num_groups=G) if gated else ft.group_norm(x, w, is_rms_norm=True, num_groups=G)
+    got = torch.autograd.grad(y, leaves, do)
+    ref = [t.detach().double().requires_grad_() for t in leaves]
+    yr = O.group_norm_gated_ref(ref[0], ref[2], ref[1], G, 1e-6, "sigmoid") if gated else O.group_norm_ref(ref[0], ref[1], G, 1e-5)
+    want = torch.autograd.grad(yr, ref, do.double())
+    for name, a, b, tol in zip(("dx", "dw", "dg"), got, want, (2 ** -8, 1e-4, 2 ** -8)):
+        assert (a.double() - b).abs().max() <= tol * b.abs().max(), name
+
+
+@pytest.mark.parametrize("B,T,H,D", [(1, 1, 1, 16), (2, 3, 5, 64), (1, 257, 3, 128), (2, 4001, 12, 64), (1, 20000, 16, 64)])
+def test_token_shift_strips(ft, B, T, H, D):
+    """Token shift over the strip lengths a size selects, last strips of one step included (fp32 reference, one rounding to bf16)."""
+    from oracle import fox_oracle as O
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(B, T, H, D, generator=gen, device="cuda").bfloat16().requires_grad_()
+    p, c = (torch.rand(B, T, H, generator=gen, device="cuda").requires_grad_() for _ in range(2))
+    do = torch.randn(B, T, H, D, generator=gen, device="cuda").bfloat16()
+    out = ft.token_shift(x, p, c)
+    ref = [t.detach().float().requires_grad_() for t in (x, p, c)]
+    out_ref = O.token_shift_ref(*ref)
+    for a, b in zip((out,) + torch.autograd.grad(out, [x, p, c], do), (out_ref,) + torch.autograd.grad(out_ref, ref, do.float())):
+        assert (a.float() - b).abs().max() <= 2 ** -8 * b.abs().max()
