@@ -6,6 +6,7 @@
 // that it can handle them, allocates the results, calls include/fox_attn.h and, when a gradient can be asked for, records a
 // C++ autograd node.  It returns None for anything else -- invalid arguments, tensors that need a copy first, another
 // current device -- and the Python function then goes through its general path, which raises the documented errors.
+#include <ATen/TracerMode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -420,7 +421,11 @@ struct ShiftNode : public torch::autograd::Function<ShiftNode> {
 const Tensor* tensor_of(PyObject* o) {
   if (!THPVariable_Check(o)) return nullptr;
   const Tensor& t = THPVariable_Unpack(o);
-  return t.key_set().has(c10::DispatchKey::Python) ? nullptr : &t;   // a subclass with its own dispatch has no plain storage
+  // a subclass with its own dispatch and the wrappers of functional transforms have no plain storage; a dual tensor's tangent
+  // and a trace would be lost: all of these go through the general path, which handles or refuses them
+  if (t.key_set().has(c10::DispatchKey::Python) || !t.has_storage() || t._fw_grad(0).defined() || at::tracer::impl::is_dispatch_enabled())
+    return nullptr;
+  return &t;
 }
 
 bool on_current_gpu(const Tensor& t) { return t.is_cuda() && t.device().index() == c10::hip::current_device(); }

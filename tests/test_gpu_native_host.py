@@ -157,3 +157,11 @@ def test_token_shift_strips(ft, B, T, H, D):
     out_ref = O.token_shift_ref(*ref)
     for a, b in zip((out,) + torch.autograd.grad(out, [x, p, c], do), (out_ref,) + torch.autograd.grad(out_ref, ref, do.float())):
         assert (a.float() - b).abs().max() <= 2 ** -8 * b.abs().max()
+
+
+def test_forward_mode_is_refused(ft):
+    """The operators have no forward-mode rule: a dual tensor raises, its tangent is not dropped."""
+    import torch.autograd.forward_ad as fwd
+    q, k, v, g, _, _ = make_inputs(1, 2, 70, 70, 64, device="cuda", head_first=True, seed=3)
+    with fwd.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
+        ft.forgetting_attention(fwd.make_dual(q, torch.ones_like(q)), k, v, g, head_first=True)
