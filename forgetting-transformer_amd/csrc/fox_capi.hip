@@ -446,6 +446,77 @@ int fox_attn_fwd_noalloc(const fox_fwd_args* args, void* stream) {
   return fwd_impl(args, ws, need, stream, "fox_attn_fwd_noalloc");
 }
 
+int fox_attn_decode_workspace_bytes(const fox_dims* dims, int64_t* bytes) {
+  FOX_TRY(check_dims(dims));
+  if (!bytes) return fail(FOX_E_ARG, "bytes is NULL");
+  if (dims->M != 1) return fail(FOX_E_ARG, "fox_attn_decode takes one query row (M = %d)", dims->M);
+  const int splits = fox::decode_splits(dims->B, dims->H, dims->N, dims->D);
+  *bytes = splits <= 1 ? 0 : (int64_t)splits * dims->B * dims->H * (int64_t)(dims->D * sizeof(float) + sizeof(fox::DecodePartial));
+  return FOX_OK;
+}
+
+int fox_attn_decode(const fox_fwd_args* args, const float* g, int64_t g_sb, int64_t g_sh, int64_t g_sn, void* stream) {
+  if (!args || !g) return fail(FOX_E_ARG, "args and g must not be NULL");
+  FOX_TRY(check_dims(&args->dims));
+  if (args->dims.M != 1) return fail(FOX_E_ARG, "fox_attn_decode takes one query row (M = %d)", args->dims.M);
+  if (args->threshold || args->first_block) return fail(FOX_E_ARG, "fox_attn_decode does not prune: threshold and first_block must be NULL");
+  FOX_TRY(check_view(&args->q, "q"));
+  FOX_TRY(check_view(&args->k, "k"));
+  FOX_TRY(check_view(&args->v, "v"));
+  FOX_TRY(check_view(&args->o, "o"));
+  FOX_TRY(check_extent(&args->k, args->dims.N, args->dims.D, "k"));
+  FOX_TRY(check_extent(&args->v, args->dims.N, args->dims.D, "v"));
+  fox::DecodeK k{};
+  k.q = to_view(args->q);
+  k.k = to_view(args->k);
+  k.v = to_view(args->v);
+  k.o = to_view(args->o);
+  k.g = g; k.g_sb = g_sb; k.g_sh = g_sh; k.g_sn = g_sn;
+  k.lse = args->lse;
+  k.seq_start = args->seq_start;
+  k.B = args->dims.B; k.H = args->dims.H; k.N = args->dims.N;
+  k.sm_scale = args->sm_scale;
+  k.splits = 1;
+  if (args->workspace) {
+    int64_t need = 0;
+    FOX_TRY(fox_attn_decode_workspace_bytes(&args->dims, &need));
+    if (need > 0) {
+      if (args->workspace_bytes < need) return fail(FOX_E_ARG, "workspace too small: %lld < %lld bytes", (long long)args->workspace_bytes, (long long)need);
+      if (((uintptr_t)args->workspace & 15) != 0) return fail(FOX_E_ALIGN, "workspace must be 16-byte aligned");
+      k.splits = fox::decode_splits(k.B, k.H, k.N, args->dims.D);
+      k.ws_o = (float*)args->workspace;
+      k.ws_p = (fox::DecodePartial*)(k.ws_o + (int64_t)k.splits * k.B * k.H * args->dims.D);   // (D is a multiple of 4: 16-byte aligned)
+    }
+  }
+  return check_hip(fox::launch_decode_gates(k, args->dims.D, args->dims.dtype, (hipStream_t)stream), "fox_attn_decode");
+}
+
+int fox_cache_append(const fox_cache_append_args* args, void* stream) {
+  if (!args) return fail(FOX_E_ARG, "args is NULL");
+  if (args->B <= 0 || args->H <= 0 || args->T <= 0 || args->old < 0) return fail(FOX_E_ARG, "B, H, T must be positive and old non-negative");
+  if (args->D <= 0 || args->D % 8) return fail(FOX_E_ARG, "head dim must be a multiple of 8 (got %d)", args->D);
+  const int64_t total = (int64_t)args->B * args->H * args->T * (args->D / 8);
+  if (args->T > (1 << 30) || total > 0x7fffffffLL) return fail(FOX_E_ARG, "too many tokens for one call");
+  FOX_TRY(check_view(&args->k, "k"));
+  FOX_TRY(check_view(&args->v, "v"));
+  FOX_TRY(check_view(&args->k_buf, "k_buf"));
+  FOX_TRY(check_view(&args->v_buf, "v_buf"));
+  if (!args->g || !args->g_buf) return fail(FOX_E_ARG, "g and g_buf must not be NULL");
+  fox::CacheAppendK k{};
+  k.k = to_view(args->k);
+  k.v = to_view(args->v);
+  k.k_buf = to_view(args->k_buf);
+  k.v_buf = to_view(args->v_buf);
+  k.g = args->g;
+  k.g_buf = args->g_buf;
+  k.g_sb = args->g_stride_b; k.g_sh = args->g_stride_h; k.g_sn = args->g_stride_n;
+  k.gb_sb = args->g_buf_stride_b; k.gb_sh = args->g_buf_stride_h; k.gb_sn = args->g_buf_stride_n;
+  k.old = args->old;
+  k.H = args->H; k.T = args->T; k.D = args->D;
+  k.total = (uint32_t)total;
+  return check_hip(fox::launch_cache_append(k, (hipStream_t)stream), "fox_cache_append");
+}
+
 int fox_attn_bwd_delta(const fox_bwd_args* args, void* stream) {
   fox::BwdK k;
   FOX_TRY(make_bwd(args, k, false));

@@ -234,4 +234,286 @@ hipError_t launch_fwd_decode(const FwdK& a, int D, int dtype, hipStream_t s) {
   return dtype == 0 ? launch_decode_t<Bf16>(a, D, s) : launch_decode_t<Fp16>(a, D, s);
 }
 
+// ---------------------------------------------------------------------------
+// The same step straight from the log forget gates: no cumulative sum of the whole row in front of it.
+//
+// The score of key n needs the sum of the gates behind it, not the two ends of a sum from the row's start.  Every wave owns
+// a contiguous run of keys, walks it from its end and carries that sum (fp64, rounded once per key) relative to the end of
+// its own run; the runs' totals then shift the partial maxima where partials are merged: four waves in LDS, splits in
+// decode_combine_kernel.  A gate is read once, by the wave that reads its key; the row scan this replaces (one workgroup per
+// row, a chain of barriers per 8192 keys) took 20 us of a 600 us step at B16 H16 N32768 D128 and 5.7 us of 36 at
+// B1 H12 N1500 D64.  Bound by HBM where the cache is long, by one round trip per batch where it is short.
+template <typename Tr, int D>
+__global__ __launch_bounds__(256) void decode_gates_kernel(const DecodeK a) {
+  constexpr int LPR = D / 8;      // lanes per key row
+  constexpr int KPL = 64 / LPR;   // keys per wave load instruction
+  constexpr int U = 8;            // loads of K and of V in flight per lane
+  constexpr int KPB = KPL * U;    // keys per wave and batch
+  constexpr int GB = (KPB + 63) / 64;   // gates per lane and batch
+  static_assert(KPB == kDecodeBatchKeys<D>, "the host counts batches with the same size");
+  __shared__ float part_m[4], part_l[4];
+  __shared__ double part_g[4];
+  __shared__ __align__(16) float part_acc[4][D];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ch = lane % LPR, r = lane / LPR;
+  const int sp = blockIdx.x % a.splits, bh = blockIdx.x / a.splits;
+  const int b = bh / a.H, h = bh % a.H;
+  const int N = a.N;
+  const float* gp = a.g + b * a.g_sb + h * a.g_sh;
+  const uint16_t* qp = a.q.ptr + b * a.q.sb + h * a.q.sh;
+  const uint16_t* kp = a.k.ptr + b * a.k.sb + h * a.k.sh + ch * 8;
+  const uint16_t* vp = a.v.ptr + b * a.v.sb + h * a.v.sh + ch * 8;
+
+  int lo = 0;
+  if (a.seq_start) {
+    const int64_t s64 = a.seq_start[b];
+    lo = (int)(s64 < 0 ? 0 : (s64 > N ? N : s64));
+  }
+  // run gw of the splits * 4 runs, counted from the last key: whole batches, the first one excepted
+  const int runs = a.splits * 4, gw = sp * 4 + wave;
+  int per = (N - lo + runs - 1) / runs;
+  per = (per + KPB - 1) / KPB * KPB;
+  const int64_t back = (int64_t)gw * per;
+  const int k1 = back < N - lo ? N - (int)back : lo, k0 = k1 - lo > per ? k1 - per : lo;
+
+  float qf[8];
+  {
+    const float qk_scale = a.sm_scale * kLog2e;
+    unpack8f<Tr>(*reinterpret_cast<const u32x4*>(qp + ch * 8), qf);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) qf[e] *= qk_scale;
+  }
+  float m = -3.0e38f, l = 0.f;  // finite floor: a group that has seen no key yet yields exp2(-inf) = 0
+  float acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+  double behind = 0.0;          // sum of the run's gates behind the batch
+
+  for (int end = k1; end > k0; end -= KPB) {   // keys end - KPB .. end - 1, those left of k0 masked
+    float gx[GB];
+#pragma unroll
+    for (int s = 0; s < GB; ++s) {             // lane j of group s holds the gate of key end - 1 - 64 s - j
+      const int j = 64 * s + lane, n = end - 1 - j;
+      gx[s] = gp[(int64_t)max(n, k0) * a.g_sn];
+      if (j >= KPB || n < k0) gx[s] = 0.f;
+    }
+    u32x4 kx[U], vx[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int n = max(end - KPB + u * KPL + r, k0);   // keys left of the run read its first row and are masked below
+      kx[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kp + (int64_t)n * a.k.st));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int n = max(end - KPB + u * KPL + r, k0);
+      vx[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vp + (int64_t)n * a.v.st));
+    }
+    float bias[GB];   // log2e * sum of the gates behind the key whose gate this lane holds
+#pragma unroll
+    for (int s = 0; s < GB; ++s) {
+      double incl = (double)gx[s];
+#pragma unroll
+      for (int off = 1; off < kWave; off <<= 1) {
+        const double up = __shfl_up(incl, off);
+        if (lane >= off) incl += up;
+      }
+      const double excl = __shfl_up(incl, 1);   // (not incl - gate: a gate may be -inf)
+      bias[s] = (float)(lane > 0 ? behind + excl : behind) * kLog2e;
+      behind += __shfl(incl, kWave - 1);
+    }
+    float sc[U];
+    float bmax = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float kf[8];
+      unpack8f<Tr>(kx[u], kf);
+      float dot = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dot = fmaf(qf[e], kf[e], dot);
+      dot = row_sum<LPR>(dot);
+      const int j = KPB - 1 - u * KPL;   // key u * KPL + r of the batch sits j - r keys before its end
+      const float x = dot + __shfl(bias[j / 64], (j - r) & 63);
+      sc[u] = (end - KPB + u * KPL + r >= k0) ? x : -INFINITY;
+      bmax = fmaxf(bmax, sc[u]);
+    }
+    const float m_new = fmaxf(m, bmax);
+    const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+    m = m_new;
+    l *= alpha;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] *= alpha;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float p = __builtin_amdgcn_exp2f(sc[u] - m);
+      l += p;
+      float vf[8];
+      unpack8f<Tr>(vx[u], vf);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = fmaf(p, vf[e], acc[e]);
+    }
+  }
+
+  // merge the KPL row groups of the wave, then the four waves, each shifted by the gates of the runs behind its own
+#pragma unroll
+  for (int off = LPR; off < 64; off <<= 1) {
+    const float m2 = __shfl_xor(m, off), l2 = __shfl_xor(l, off);
+    float acc2[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc2[e] = __shfl_xor(acc[e], off);
+    merge_state(m, l, acc, m2, l2, acc2);
+  }
+  if (r == 0) {
+    if (ch == 0) { part_m[wave] = m; part_l[wave] = l; part_g[wave] = behind; }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) part_acc[wave][ch * 8 + e] = acc[e];
+  }
+  __syncthreads();
+  if (tid >= LPR) return;
+  m = part_m[0];
+  l = part_l[0];
+  double shift = part_g[0];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = part_acc[0][ch * 8 + e];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) {
+    float acc2[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc2[e] = part_acc[w][ch * 8 + e];
+    merge_state(m, l, acc, part_m[w] + (float)shift * kLog2e, part_l[w], acc2);
+    shift += part_g[w];
+  }
+
+  if (a.splits > 1) {  // partial result of this split: accumulator, maximum and sum relative to its last key, sum of its gates
+    const int64_t row = (int64_t)bh * a.splits + sp;
+    float* wo = a.ws_o + row * D + ch * 8;
+    const f32x4 w0 = {acc[0], acc[1], acc[2], acc[3]}, w1 = {acc[4], acc[5], acc[6], acc[7]};
+    *reinterpret_cast<f32x4*>(wo) = w0;
+    *reinterpret_cast<f32x4*>(wo + 4) = w1;
+    if (ch == 0) a.ws_p[row] = DecodePartial{shift, m, l};
+    return;
+  }
+  const bool empty = lo >= N;  // every key is left padding: o = 0, lse = -inf (:679-685)
+  const float inv = empty ? 0.f : 1.0f / l;
+  uint16_t* op = const_cast<uint16_t*>(a.o.ptr) + b * a.o.sb + h * a.o.sh + ch * 8;
+  u32x4 w;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) w[e] = Tr::pack2(acc[2 * e] * inv, acc[2 * e + 1] * inv);
+  *reinterpret_cast<u32x4*>(op) = w;
+  if (ch == 0 && a.lse) a.lse[bh] = empty ? -INFINITY : m * kLn2 + __logf(l);
+}
+
+// Merge of the splits of decode_gates_kernel: one workgroup per (batch, head), every partial in flight at once (at most
+// kDecodeMaxSplits of them, one round trip; a thread that walks the splits one after the other pays one per split).
+template <typename Tr, int D>
+__global__ __launch_bounds__(256) void decode_combine_kernel(const DecodeK a) {
+  constexpr int TPR = D / 4, GROUPS = 256 / TPR, PER = (kDecodeMaxSplits + GROUPS - 1) / GROUPS;
+  __shared__ float weight[kDecodeMaxSplits];
+  __shared__ float l_tot, m_tot;
+  __shared__ __align__(16) float part[GROUPS][D];
+  const int tid = threadIdx.x, bh = blockIdx.x, b = bh / a.H, h = bh % a.H, splits = a.splits;
+  const int grp = tid / TPR, d = (tid % TPR) * 4;
+  const float* wo = a.ws_o + (int64_t)bh * splits * D + d;
+  f32x4 x[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) x[i] = *reinterpret_cast<const f32x4*>(wo + (int64_t)min(grp + i * GROUPS, splits - 1) * D);
+  if (tid < kWave) {   // one lane per split (counted from the last keys): its maximum moves by the gates of the splits behind it
+    const DecodePartial p = a.ws_p[(int64_t)bh * splits + min(tid, splits - 1)];
+    double incl = tid < splits ? p.g : 0.0;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const double up = __shfl_up(incl, off);
+      if (tid >= off) incl += up;
+    }
+    const double excl = __shfl_up(incl, 1);
+    const float m = tid == 0 ? p.m : tid < splits ? p.m + (float)excl * kLog2e : -INFINITY;
+    float mx = m;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    const float w = __builtin_amdgcn_exp2f(m - mx);
+    float l = p.l * w;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
+    weight[tid] = w;
+    if (tid == 0) { l_tot = l; m_tot = mx; }
+  }
+  __syncthreads();
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < PER; ++i)
+    if (grp + i * GROUPS < splits) acc += x[i] * weight[grp + i * GROUPS];
+  *reinterpret_cast<f32x4*>(&part[grp][d]) = acc;
+  __syncthreads();
+  if (tid >= TPR) return;
+  acc = *reinterpret_cast<const f32x4*>(&part[0][d]);
+  const int used = min(GROUPS, splits);
+  for (int i = 1; i < used; ++i) acc += *reinterpret_cast<const f32x4*>(&part[i][d]);
+  const bool empty = a.seq_start && a.seq_start[b] >= a.N;
+  const float inv = empty ? 0.f : 1.0f / l_tot;
+  uint16_t* op = const_cast<uint16_t*>(a.o.ptr) + b * a.o.sb + h * a.o.sh + d;
+  u32x2 w;
+  w[0] = Tr::pack2(acc[0] * inv, acc[1] * inv);
+  w[1] = Tr::pack2(acc[2] * inv, acc[3] * inv);
+  *reinterpret_cast<u32x2*>(op) = w;
+  if (d == 0 && a.lse) a.lse[bh] = empty ? -INFINITY : m_tot * kLn2 + __logf(l_tot);
+}
+
+template <typename Tr, int D>
+static hipError_t launch_decode_gates_d(const DecodeK& a, hipStream_t s) {
+  hipLaunchKernelGGL((decode_gates_kernel<Tr, D>), dim3((unsigned)(a.splits * a.B * a.H)), dim3(256), 0, s, a);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || a.splits <= 1) return e;
+  hipLaunchKernelGGL((decode_combine_kernel<Tr, D>), dim3((unsigned)(a.B * a.H)), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+template <typename Tr>
+static hipError_t launch_decode_gates_t(const DecodeK& a, int D, hipStream_t s) {
+  switch (D) {
+    case 16: return launch_decode_gates_d<Tr, 16>(a, s);
+    case 32: return launch_decode_gates_d<Tr, 32>(a, s);
+    case 64: return launch_decode_gates_d<Tr, 64>(a, s);
+    case 128: return launch_decode_gates_d<Tr, 128>(a, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_decode_gates(const DecodeK& a, int D, int dtype, hipStream_t s) {
+  return dtype == 0 ? launch_decode_gates_t<Bf16>(a, D, s) : launch_decode_gates_t<Fp16>(a, D, s);
+}
+
+// Splits of launch_decode_gates: about eight workgroups per CU, but no wave with less than a whole batch of keys (16 KiB of K and V):
+// a step over a short cache is a chain of round trips, one per batch a wave walks.  B1 H12 N1500 D64: two splits 7.9 us
+// (three batches a wave), six 4.6.
+int decode_splits(int B, int H, int N, int D) {
+  const int64_t bh = (int64_t)B * H, batches = ((int64_t)N * D + 16383) / 16384;   // four waves' batches
+  int64_t splits = (2048 + bh - 1) / bh;
+  splits = splits > batches ? batches : splits;
+  splits = splits > kDecodeMaxSplits ? kDecodeMaxSplits : splits;
+  return splits < 1 ? 1 : (int)splits;
+}
+
+// ---------------------------------------------------------------------------
+// New tokens into a layer's cache: keys, values and log gates in one launch.  One 16-byte piece of K and the same piece of V per
+// thread, the thread with a row's first piece also moves its gate.  For one token per sequence the launches are the cost
+// (B1 H12 D64: three strided copies 6.1 us of kernels plus their host time, this kernel 2.3); a prompt is a plain stream.
+__global__ __launch_bounds__(256) void cache_append_kernel(const CacheAppendK a) {
+  const uint32_t idx = blockIdx.x * 256u + threadIdx.x, pieces = (uint32_t)a.D / 8u;
+  if (idx >= a.total) return;
+  const uint32_t row = idx / pieces, ch = idx - row * pieces, bh = row / (uint32_t)a.T, t = row - bh * (uint32_t)a.T;
+  const uint32_t b = bh / (uint32_t)a.H, h = bh - b * (uint32_t)a.H;
+  auto at = [&](const View& v, int64_t t0) { return v.ptr + b * v.sb + h * v.sh + (t0 + t) * v.st + ch * 8; };
+  const u32x4 kx = *reinterpret_cast<const u32x4*>(at(a.k, 0)), vx = *reinterpret_cast<const u32x4*>(at(a.v, 0));
+  float gx = 0.f;
+  if (ch == 0) gx = a.g[b * a.g_sb + h * a.g_sh + t * a.g_sn];
+  *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(at(a.k_buf, a.old))) = kx;
+  *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(at(a.v_buf, a.old))) = vx;
+  if (ch == 0) a.g_buf[b * a.gb_sb + h * a.gb_sh + (a.old + t) * a.gb_sn] = gx;
+}
+
+hipError_t launch_cache_append(const CacheAppendK& a, hipStream_t s) {
+  hipLaunchKernelGGL(cache_append_kernel, dim3((a.total + 255u) / 256u), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
 }  // namespace fox

@@ -40,6 +40,36 @@ struct FwdK {
   bool stream;     // K and V tiles are read once and not again soon: load them with the non-temporal hint
 };
 
+// Single-query forward from the log gates (decode_gates_kernel).
+struct DecodePartial {   // of one key split: sum of its gates, maximum (log2 domain, relative to its last key) and row sum
+  double g;
+  float m, l;
+};
+struct DecodeK {
+  View q, k, v, o;
+  const float* g;            // log gates, element strides below
+  int64_t g_sb, g_sh, g_sn;
+  float* lse;                // (B,H) or null
+  const int64_t* seq_start;
+  int B, H, N;
+  float sm_scale;
+  int splits;
+  float* ws_o;               // (B, H, splits, D) partial accumulators
+  DecodePartial* ws_p;       // (B, H, splits)
+};
+constexpr int kDecodeMaxSplits = 64;                     // one lane of a wave each in the merge
+template <int D> constexpr int kDecodeBatchKeys = 4096 / D;   // keys a wave holds in flight: 8 KiB of K and 8 KiB of V
+
+// New tokens into a layer's key, value and gate buffers: rows old .. old + T - 1 of every (batch, head).
+struct CacheAppendK {
+  View k, v, k_buf, v_buf;
+  const float* g;
+  float* g_buf;
+  int64_t g_sb, g_sh, g_sn, gb_sb, gb_sh, gb_sn, old;
+  int H, T, D;
+  uint32_t total;   // 16-byte pieces of K: B * H * T * D / 8
+};
+
 struct BwdK {
   View q, k, v, o, d_o, dq, dk, dv;
   const float* c;
@@ -129,6 +159,9 @@ hipError_t launch_bwd_dkdv(const BwdK& a, int D, int dtype, hipStream_t s);   //
 bool dkdv_split_supports(int D);   // head dims the split (kClassLight) variant of the dK/dV kernel exists for
 hipError_t launch_bwd_dq(const BwdK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_fwd_decode(const FwdK& a, int D, int dtype, hipStream_t s);  // M == 1, without the merge of the splits
+hipError_t launch_decode_gates(const DecodeK& a, int D, int dtype, hipStream_t s);
+hipError_t launch_cache_append(const CacheAppendK& a, hipStream_t s);
+int decode_splits(int B, int H, int N, int D);
 hipError_t launch_norm_gate(const NormGateK& a, int D, int dtype, bool bwd, int act, hipStream_t s);  // act: FOX_ACT_*
 int64_t norm_gate_workspace_rows(int64_t rows);
 hipError_t launch_shift_fwd(const ShiftK& a, int D, int dtype, hipStream_t s);

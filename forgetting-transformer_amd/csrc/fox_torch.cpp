@@ -8,6 +8,7 @@
 // current device -- and the Python function then goes through its general path, which raises the documented errors.
 #include <ATen/TracerMode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/InferenceMode.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -154,6 +155,31 @@ Forward run_forward(Attention& a, const Tensor& q, const Tensor& k, const Tensor
     f.out = f.out.transpose(1, 2);
   }
   return f;
+}
+
+// One query row without a graph or a threshold: nobody needs the cumulative sums, so the kernel takes the gates themselves.
+bool decodes_from_gates(const Attention& a) {
+  return a.M == 1 && !a.is_logit && !a.auto_threshold && !a.threshold.defined() && !a.epilogue;
+}
+Tensor run_decode(const Attention& a, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g) {
+  fox_fwd_args args{};
+  args.dims = a.dims(q);
+  int64_t ws_bytes = 0;
+  check(fox_attn_decode_workspace_bytes(&args.dims, &ws_bytes), "fox_attn_decode_workspace_bytes");
+  Tensor out = at::empty_like(q), ws;
+  args.q = view_of(q, a.head_first);
+  args.k = view_of(k, a.head_first);
+  args.v = view_of(v, a.head_first);
+  args.o = view_of(out, a.head_first);
+  args.seq_start = a.seq_ptr();
+  args.sm_scale = (float)a.sm_scale;
+  if (ws_bytes > 0) {
+    ws = empty_bytes_like(q, ws_bytes);
+    args.workspace = ws.mutable_data_ptr();
+    args.workspace_bytes = ws_bytes;
+  }
+  check(fox_attn_decode(&args, g.const_data_ptr<float>(), g.stride(0), a.gs_h(g), a.gs_n(g), stream_of(q)), "fox_attn_decode");
+  return out;
 }
 
 // dq, dk, dv and the gradient of the gates, in the layout of the inputs
@@ -508,6 +534,7 @@ PyObject* finish_attention(Attention& a, const Tensor& q, const Tensor& k, const
     out = AttentionNode::apply(q, k, v, g, some(gate), some(weight), &a);
   } else {
     const at::NoGradGuard no_grad;
+    if (decodes_from_gates(a)) return THPVariable_Wrap(run_decode(a, q, k, v, g));
     Forward f = run_forward(a, q, k, v, g);
     out.push_back(f.out);
     if (a.is_logit) out.push_back(a.head_first ? f.log_fgate : f.log_fgate.transpose(1, 2));
@@ -629,7 +656,57 @@ PyObject* py_qk_norm_threshold(PyObject*, PyObject* const* o, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// cache_append(k_buf, v_buf, g_buf, k, v, g, old) -> views of the filled part of the three buffers
+PyObject* py_cache_append(PyObject*, PyObject* const* o, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 7, "cache_append takes 7 arguments");
+  const Tensor* t[6];
+  for (int i = 0; i < 6; ++i) {
+    t[i] = tensor_of(o[i]);
+    if (!t[i] || t[i]->dim() != (i % 3 == 2 ? 3 : 4) || t[i]->numel() == 0 || !on_current_gpu(*t[i])) return none();
+    if (i % 3 == 2 ? t[i]->scalar_type() != at::kFloat : !sixteen_bit(*t[i]) || !vectors_ok(*t[i])) return none();
+    // what the copies of the general path would record or refuse, or may not do in one pass
+    if (at::GradMode::is_enabled() && t[i]->requires_grad()) return none();
+    if (i < 3 && t[i]->is_inference() && !c10::InferenceMode::is_enabled()) return none();
+    if (i >= 3 && (t[i]->storage().is_alias_of(t[0]->storage()) || t[i]->storage().is_alias_of(t[1]->storage()) ||
+                   t[i]->storage().is_alias_of(t[2]->storage())))
+      return none();
+  }
+  const Tensor &kb = *t[0], &vb = *t[1], &gb = *t[2], &k = *t[3], &v = *t[4], &g = *t[5];
+  const int64_t old = PyLong_AsLongLong(o[6]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    return none();
+  }
+  const int64_t B = k.size(0), H = k.size(1), T = k.size(2), D = k.size(3);
+  if (v.sizes() != k.sizes() || g.sizes() != k.sizes().slice(0, 3) || kb.sizes() != vb.sizes() || gb.sizes() != kb.sizes().slice(0, 3) ||
+      kb.size(0) != B || kb.size(1) != H || kb.size(3) != D || kb.scalar_type() != k.scalar_type() || vb.scalar_type() != v.scalar_type() ||
+      D % 8 || old < 0 || old + T > kb.size(2) || T > (1 << 30) || B * H * T * (D / 8) > INT32_MAX)
+    return none();
+  fox_cache_append_args a{};
+  a.B = (int32_t)B; a.H = (int32_t)H; a.T = (int32_t)T; a.D = (int32_t)D;
+  a.old = old;
+  a.k = view_of(k, true);
+  a.v = view_of(v, true);
+  a.g = g.const_data_ptr<float>();
+  a.g_stride_b = g.stride(0); a.g_stride_h = g.stride(1); a.g_stride_n = g.stride(2);
+  a.k_buf = view_of(kb, true);
+  a.v_buf = view_of(vb, true);
+  a.g_buf = gb.mutable_data_ptr<float>();
+  a.g_buf_stride_b = gb.stride(0); a.g_buf_stride_h = gb.stride(1); a.g_buf_stride_n = gb.stride(2);
+  check(fox_cache_append(&a, stream_of(k)), "fox_cache_append");
+  PyObject* out = PyTuple_New(3);
+  if (!out) return nullptr;
+  for (int i = 0; i < 3; ++i) {
+    if (!t[i]->is_inference()) t[i]->unsafeGetTensorImpl()->bump_version();   // an in-place write, as copy_ is
+    PyTuple_SET_ITEM(out, i, THPVariable_Wrap(t[i]->narrow(2, 0, old + T)));
+  }
+  return out;
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
+    {"cache_append", (PyCFunction)(void (*)(void))py_cache_append, METH_FASTCALL, nullptr},
     {"qk_norm_threshold", (PyCFunction)(void (*)(void))py_qk_norm_threshold, METH_FASTCALL, nullptr},
     {"attention", (PyCFunction)(void (*)(void))py_attention, METH_FASTCALL, nullptr},
     {"attention_norm_gate", (PyCFunction)(void (*)(void))py_attention_norm_gate, METH_FASTCALL, nullptr},

@@ -15,13 +15,16 @@ back views of the filled part.  The views have the reference's shapes; their (ba
 are ``capacity`` rows apart instead of ``seq_len``, which ``forgetting_attention`` takes as it takes
 any strided input.  When a layer runs out of capacity its buffers are reallocated ``growth`` times
 larger (amortised constant cost per token); with ``max_length`` given they are allocated once at that
-size and never move.  Depends on nothing but torch.
+size and never move.  On the GPU the new tokens are copied by one kernel (``fox_cache_append``); elsewhere, and for tensors
+that kernel does not take, by torch.
 """
 from __future__ import annotations
 
 from typing import Any, Dict, List, Optional, Tuple
 
 import torch
+
+from .ops import _native
 
 __all__ = ["FgateDynamicCache"]
 
@@ -82,6 +85,11 @@ class FgateDynamicCache:
             self._seen_tokens += new
         old = self.get_seq_length(layer_idx)
         self._reserve(layer_idx, old + new, key_states, value_states, log_fgate_states)
+        if key_states.is_cuda:
+            views = _native.load().cache_append(*self._buffers(layer_idx), key_states, value_states, log_fgate_states, old)
+            if views is not None:
+                self.key_cache[layer_idx], self.value_cache[layer_idx], self.log_fgate_cache[layer_idx] = views
+                return views
         self._key_buf[layer_idx][:, :, old:old + new].copy_(key_states)
         self._value_buf[layer_idx][:, :, old:old + new].copy_(value_states)
         self._log_fgate_buf[layer_idx][:, :, old:old + new].copy_(log_fgate_states)

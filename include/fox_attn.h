@@ -188,6 +188,33 @@ int fox_attn_fwd_workspace_bytes(const fox_dims* dims, int64_t* bytes);
  */
 int fox_attn_fwd_noalloc(const fox_fwd_args* args, void* stream);
 
+/*
+ * One query row against the keys (M == 1) straight from the log forget gates, without fox_cumsum_fwd in front:
+ * what fox_cumsum_fwd + fox_attn_fwd compute, for callers that keep no log_lambda (generation).  g is (B,H,N) fp32 with
+ * element strides; log_lambda is ignored, lse may be NULL, threshold and first_block must be NULL.  workspace holds
+ * fox_attn_decode_workspace_bytes() bytes, NULL = one workgroup per (batch, head).
+ */
+int fox_attn_decode(const fox_fwd_args* args, const float* g, int64_t g_stride_b, int64_t g_stride_h, int64_t g_stride_n,
+                    void* stream);
+int fox_attn_decode_workspace_bytes(const fox_dims* dims, int64_t* bytes);
+
+/*
+ * New tokens into a decode cache (fgate_cache.py:107-116 concatenates instead): k, v (B,H,T,D) 16-bit and g (B,H,T) fp32 go
+ * to rows old .. old + T - 1 of the buffers.  D is a multiple of 8; the caller makes sure the buffers have the rows and that
+ * sources and destinations do not overlap.
+ */
+typedef struct fox_cache_append_args {
+  int32_t B, H, T, D;
+  int64_t old;
+  fox_view k, v;
+  const float* g;
+  int64_t g_stride_b, g_stride_h, g_stride_n;
+  fox_view k_buf, v_buf;
+  float* g_buf;
+  int64_t g_buf_stride_b, g_buf_stride_h, g_buf_stride_n;
+} fox_cache_append_args;
+int fox_cache_append(const fox_cache_append_args* args, void* stream);
+
 typedef struct fox_bwd_args {
   fox_dims dims;
   fox_view q, k, v, o, d_o;   /* inputs */

@@ -1,0 +1,66 @@
+"""The kernels of token-by-token generation: one query row straight from the log gates (no graph, no threshold), its merge of key
+splits, and the append of new tokens to the cache."""
+import pytest
+import torch
+
+from conftest import assert_parity, make_inputs
+from oracle import fox_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def ft():
+    assert torch.cuda.is_available(), "these tests need the MI355X"
+    import forgetting_transformer
+    return forgetting_transformer
+
+
+# a batch of keys per wave is 4096 / D, a workgroup takes four: one key, edges of a batch and of a workgroup's share, several
+# batches per wave (no more splits to give), one split (many heads)
+@pytest.mark.parametrize("B,H,N,D", [(1, 1, 1, 64), (1, 3, 63, 64), (2, 2, 65, 64), (1, 2, 255, 64), (1, 2, 257, 64), (1, 12, 1500, 64),
+                                     (2, 3, 33, 128), (1, 2, 129, 128), (2, 2, 9001, 128), (1, 2, 1025, 16), (2, 2, 70000, 16),
+                                     (3, 5, 700, 32), (1, 1, 40000, 64), (16, 130, 300, 32)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("gate_mean", [3.0, -1.0])
+def test_single_query(ft, B, H, N, D, dtype, gate_mean):
+    ss = [(N * i) // (2 * B) for i in range(B)]
+    ss[-1] = N if B > 2 else N - 1                     # a row with nothing to see, or only its own key
+    q, k, v, g, _, ss = make_inputs(B, H, 1, N, D, dtype=dtype, device="cuda", head_first=True, seq_start=ss, seed=N + D, gate_mean=gate_mean)
+    ref = O.forgetting_attention_ref(q, k, v, g, head_first=True, seq_start=ss)
+    with torch.no_grad():
+        out = ft.forgetting_attention(q, k, v, g, head_first=True, seq_start=ss)
+        swap = [x.transpose(1, 2).contiguous() for x in (q, k, v, g)]
+        other = ft.forgetting_attention(*swap, seq_start=ss)
+    assert_parity("out", out, ref)
+    assert torch.equal(other.transpose(1, 2), out)     # strided gates and rows: the same arithmetic
+
+
+def test_single_query_behind_a_closed_gate(ft):
+    """A log gate of -inf hides every key left of it and nothing else."""
+    q, k, v, g, _, _ = make_inputs(1, 2, 1, 3000, 64, device="cuda", head_first=True, seed=5, gate_mean=2.0)
+    g[:, :, 1234] = float("-inf")
+    with torch.no_grad():
+        out = ft.forgetting_attention(q, k, v, g, head_first=True)
+        ref = O.forgetting_attention_ref(q, k[:, :, 1234:], v[:, :, 1234:], g[:, :, 1234:].clamp(min=-50), head_first=True)
+    assert_parity("out", out, ref)
+
+
+@pytest.mark.parametrize("D,T,dtype", [(64, 1, torch.bfloat16), (128, 1, torch.float16), (16, 7, torch.bfloat16), (40, 300, torch.float16),
+                                       (12, 3, torch.bfloat16), (64, 2, torch.float32)])
+def test_cache_append(ft, D, T, dtype):
+    """Appending against concatenation, from strided sources; head dims and types the kernel does not take go through torch."""
+    B, H = 2, 3
+    rnd = lambda n: torch.randn(B, n, H, D, device="cuda").to(dtype).transpose(1, 2)
+    gates = lambda n: -torch.rand(B, n, H, device="cuda").transpose(1, 2)
+    cache, parts = ft.FgateDynamicCache(min_capacity=64), []
+    for n in (T, 5, T):
+        parts.append((rnd(n), rnd(n), gates(n)))
+        got = cache.update(*parts[-1], 0)
+        for a, b, c in zip(got, zip(*parts), cache[0]):
+            assert torch.equal(a, torch.cat(b, dim=2)) and c.data_ptr() == a.data_ptr()
+    version = cache._key_buf[0]._version
+    cache.crop(T + 5)
+    with torch.inference_mode():
+        got = cache.update(*parts[2], 0)
+    assert torch.equal(got[1], torch.cat([p[1] for p in parts], dim=2)) and cache._key_buf[0]._version > version
