@@ -13,17 +13,20 @@
 
 namespace fox {
 
-constexpr int kScanThreads = 1024;  // one workgroup per row: few rows, long rows, so the workgroup is as wide as it gets
-
 // Scan of one row: element idx is produced by load(idx) and the running sum up to and including
 // it is handed to store(idx, sum).  REVERSE walks the row from its last element to its first.
-// A span of 8 x 1024 elements moves between memory and LDS with consecutive lanes on consecutive
+// A span of 8 x NT elements moves between memory and LDS with consecutive lanes on consecutive
 // elements (whole cache lines per wave instruction, whatever the caller's stride), and between LDS and
 // registers with eight consecutive elements per thread, the order the scan wants.
-template <bool REVERSE, typename Load, typename Store>
+// Bound by latency: one workgroup per row, few rows.  A long row gets the widest workgroup there is; a row that a single span of
+// fewer waves covers gets just those (scan_threads), and the barriers between sixteen waves and the chain over their totals go.
+// Rows of 77 to 2048 elements: 5.1 us a call with 1024 threads, 3.9 with as many as the row needs.  Rows cut over several
+// workgroups, each adding up what lies in front of its piece, were slower wherever there were enough of them to count (64 rows of 16384 8.5 -> 10.4
+// us, 256 rows of 32768 17 -> 28 us).
+template <bool REVERSE, int NT, typename Load, typename Store>
 __device__ __forceinline__ void scan_row(int N, Load load, Store store) {
-  constexpr int PER = 8, NT = kScanThreads, SPAN = PER * NT;
-  __shared__ double wave_tot[NT / kWave];
+  constexpr int PER = 8, SPAN = PER * NT, WAVES = NT / kWave;
+  __shared__ double wave_tot[WAVES];
   __shared__ __align__(16) float stage[SPAN];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   double carry = 0.0;
@@ -61,7 +64,7 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store) {
     __syncthreads();
     double before = carry, total = 0.0;
 #pragma unroll
-    for (int w = 0; w < NT / kWave; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       const double t = wave_tot[w];
       if (w < wave) before += t;
       total += t;
@@ -89,8 +92,10 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store) {
   }
 }
 
-template <bool REVERSE>
-__global__ __launch_bounds__(kScanThreads) void scan_kernel(const float* __restrict__ in, int64_t sb, int64_t sh, int64_t sn,
+inline int scan_threads(int N) { return N <= 8 * 64 ? 64 : N <= 8 * 256 ? 256 : 1024; }
+
+template <bool REVERSE, int NT>
+__global__ __launch_bounds__(NT) void scan_kernel(const float* __restrict__ in, int64_t sb, int64_t sh, int64_t sn,
                                                    const int64_t* __restrict__ seq_start, float* __restrict__ out, int64_t ob,
                                                    int64_t oh, int64_t on, int H, int N) {
   const int bh = blockIdx.x, b = bh / H, h = bh % H;
@@ -104,7 +109,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_kernel(const float* __restr
   // Reverse: the gradient of every gate up to and including position seq is the sum of all dc, zero in exact
   // arithmetic (those gates shift every cumulative sum the kernels see by the same amount, or are zeroed by the
   // forward); it is stored as an exact zero instead of the rounding noise of that sum.
-  scan_row<REVERSE>(
+  scan_row<REVERSE, NT>(
       N, [&](int idx) { return (REVERSE || idx >= seq) ? src[(int64_t)idx * sn] : 0.f; },
       [&](int idx, float sum) { dst[(int64_t)idx * on] = (REVERSE && idx <= seq) ? 0.f : sum; });
 }
@@ -138,8 +143,8 @@ __device__ __forceinline__ float log_sigmoid(float x) {
 
 // c[n] = sum_{seq_start <= l <= n} logsigmoid(x[l]) in one pass over the logits; optionally also
 // stores log_fgate[n] = logsigmoid(x[n]) (the decode cache of the FoX layer keeps it).
-template <int DT>
-__global__ __launch_bounds__(kScanThreads) void gate_scan_fwd_kernel(const void* __restrict__ logits, int64_t sb, int64_t sh, int64_t sn,
+template <int DT, int NT>
+__global__ __launch_bounds__(NT) void gate_scan_fwd_kernel(const void* __restrict__ logits, int64_t sb, int64_t sh, int64_t sn,
                                                             const int64_t* __restrict__ seq_start,
                                                             float* __restrict__ log_fgate, float* __restrict__ out, int H,
                                                             int N) {
@@ -152,7 +157,7 @@ __global__ __launch_bounds__(kScanThreads) void gate_scan_fwd_kernel(const void*
     const int64_t s64 = seq_start[b];
     seq = (int)(s64 < 0 ? 0 : (s64 > N ? N : s64));
   }
-  scan_row<false>(
+  scan_row<false, NT>(
       N,
       [&](int idx) {
         const float x = load_logit<DT>(logits, base + (int64_t)idx * sn);
@@ -165,8 +170,8 @@ __global__ __launch_bounds__(kScanThreads) void gate_scan_fwd_kernel(const void*
 
 // dlogit[l] = (sum_{n>=l} dc[n]) * d logsigmoid(x_l)/dx = dg[l] * (1 - sigmoid(x_l)), stored in the
 // dtype and layout of the logits.
-template <int DT>
-__global__ __launch_bounds__(kScanThreads) void gate_scan_bwd_kernel(const float* __restrict__ dc, const void* __restrict__ logits,
+template <int DT, int NT>
+__global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(const float* __restrict__ dc, const void* __restrict__ logits,
                                                             int64_t sb, int64_t sh, int64_t sn, const int64_t* __restrict__ seq_start,
                                                             void* __restrict__ dlogits, int64_t db, int64_t dh, int64_t dn, int H,
                                                             int N) {
@@ -178,7 +183,7 @@ __global__ __launch_bounds__(kScanThreads) void gate_scan_bwd_kernel(const float
     const int64_t s64 = seq_start[b];
     seq = (int)(s64 < 0 ? 0 : (s64 > N ? N : s64));
   }
-  scan_row<true>(
+  scan_row<true, NT>(
       N, [&](int idx) { return src[idx]; },
       [&](int idx, float sum) {
         const float x = load_logit<DT>(logits, lbase + (int64_t)idx * sn);
@@ -189,13 +194,20 @@ __global__ __launch_bounds__(kScanThreads) void gate_scan_bwd_kernel(const float
       });
 }
 
+// KERNEL<ARG, threads for rows of N elements>, one workgroup per row of the B x H.
+#define FOX_LAUNCH_SCAN(KERNEL, ARG, ...)                                                                      \
+  switch (scan_threads(N)) {                                                                                    \
+    case 64: hipLaunchKernelGGL((KERNEL<ARG, 64>), dim3((unsigned)(B * H)), dim3(64), 0, s, __VA_ARGS__); break;    \
+    case 256: hipLaunchKernelGGL((KERNEL<ARG, 256>), dim3((unsigned)(B * H)), dim3(256), 0, s, __VA_ARGS__); break; \
+    default: hipLaunchKernelGGL((KERNEL<ARG, 1024>), dim3((unsigned)(B * H)), dim3(1024), 0, s, __VA_ARGS__);       \
+  }
+
 hipError_t launch_gate_cumsum_fwd(const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn, const int64_t* seq_start,
                                   float* log_fgate, float* c, int B, int H, int N, hipStream_t s) {
-  const dim3 grid((unsigned)(B * H));
   switch (dtype) {
-    case 0: hipLaunchKernelGGL(gate_scan_fwd_kernel<0>, grid, dim3(kScanThreads), 0, s, logits, sb, sh, sn, seq_start, log_fgate, c, H, N); break;
-    case 1: hipLaunchKernelGGL(gate_scan_fwd_kernel<1>, grid, dim3(kScanThreads), 0, s, logits, sb, sh, sn, seq_start, log_fgate, c, H, N); break;
-    case 2: hipLaunchKernelGGL(gate_scan_fwd_kernel<2>, grid, dim3(kScanThreads), 0, s, logits, sb, sh, sn, seq_start, log_fgate, c, H, N); break;
+    case 0: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 0, logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
+    case 1: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 1, logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
+    case 2: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 2, logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -204,11 +216,10 @@ hipError_t launch_gate_cumsum_fwd(const void* logits, int dtype, int64_t sb, int
 hipError_t launch_gate_cumsum_bwd(const float* dc, const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn,
                                   const int64_t* seq_start, void* dlogits, int64_t db, int64_t dh, int64_t dn, int B, int H, int N,
                                   hipStream_t s) {
-  const dim3 grid((unsigned)(B * H));
   switch (dtype) {
-    case 0: hipLaunchKernelGGL(gate_scan_bwd_kernel<0>, grid, dim3(kScanThreads), 0, s, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, H, N); break;
-    case 1: hipLaunchKernelGGL(gate_scan_bwd_kernel<1>, grid, dim3(kScanThreads), 0, s, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, H, N); break;
-    case 2: hipLaunchKernelGGL(gate_scan_bwd_kernel<2>, grid, dim3(kScanThreads), 0, s, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, H, N); break;
+    case 0: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 0, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, H, N) break;
+    case 1: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 1, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, H, N) break;
+    case 2: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 2, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, H, N) break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -216,15 +227,15 @@ hipError_t launch_gate_cumsum_bwd(const float* dc, const void* logits, int dtype
 
 hipError_t launch_cumsum_fwd(const float* g, int64_t sb, int64_t sh, int64_t sn, const int64_t* seq_start, float* c, int B,
                              int H, int N, hipStream_t s) {
-  hipLaunchKernelGGL(scan_kernel<false>, dim3((unsigned)(B * H)), dim3(kScanThreads), 0, s, g, sb, sh, sn, seq_start, c,
-                     (int64_t)H * N, (int64_t)N, (int64_t)1, H, N);
+  FOX_LAUNCH_SCAN(scan_kernel, false, g, sb, sh, sn, seq_start, c,
+                     (int64_t)H * N, (int64_t)N, (int64_t)1, H, N)
   return hipGetLastError();
 }
 
 hipError_t launch_cumsum_bwd(const float* dc, float* dg, int64_t db, int64_t dh, int64_t dn, const int64_t* seq_start, int B, int H,
                              int N, hipStream_t s) {
-  hipLaunchKernelGGL(scan_kernel<true>, dim3((unsigned)(B * H)), dim3(kScanThreads), 0, s, dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
-                     seq_start, dg, db, dh, dn, H, N);
+  FOX_LAUNCH_SCAN(scan_kernel, true, dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
+                     seq_start, dg, db, dh, dn, H, N)
   return hipGetLastError();
 }
 

@@ -609,6 +609,37 @@ def test_cumsum_kernels(fa):
     assert torch.equal(dg_t, dg)
 
 
+@pytest.mark.parametrize("N", [1, 64, 511, 512, 513, 2047, 2048, 2049, 8193])   # one, four and sixteen waves a row, one span and two
+def test_cumsum_kernels_at_the_edges_of_their_workgroups(fa, N):
+    from forgetting_transformer.ops import _lib
+    lib = _lib.load()
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    B, H = 2, 3
+    x = (torch.randn(B, N, H, device="cuda") * 2).transpose(1, 2)
+    g = F.logsigmoid(x.double())
+    ss = torch.tensor([0, N // 3], device="cuda")
+    keep = torch.arange(N, device="cuda") >= ss[:, None, None]
+    c, c_gate, lg, dg = (torch.full((B, H, N), float("nan"), device="cuda") for _ in range(4))
+    g32 = g.float()
+    _lib.check(lib.fox_cumsum_fwd(g32.data_ptr(), *g32.stride(), ss.data_ptr(), c.data_ptr(), B, H, N, stream), "cumsum_fwd")
+    ref = torch.where(keep, g32.double(), 0.0).cumsum(-1)
+    assert ((c.double() - ref).abs() <= 6e-8 * ref.abs()).all()           # fp64 sums rounded once
+    _lib.check(lib.fox_gate_cumsum_fwd(x.data_ptr(), 2, *x.stride(), ss.data_ptr(), lg.data_ptr(), c_gate.data_ptr(), B, H, N, stream),
+               "gate_cumsum_fwd")
+    ref = torch.where(keep, lg.double(), 0.0).cumsum(-1)                 # of the log gates that it stored itself
+    assert ((c_gate.double() - ref).abs() <= 6e-8 * ref.abs()).all() and (lg.double() - g).abs().max() <= 1e-6 * g.abs().max()
+    dc = torch.randn(B, H, N, device="cuda")
+    sums = dc.double().flip(-1).cumsum(-1).flip(-1)
+    dead = torch.arange(N, device="cuda") <= ss[:, None, None]
+    _lib.check(lib.fox_cumsum_bwd(dc.data_ptr(), dg.data_ptr(), 0, 0, 0, ss.data_ptr(), B, H, N, stream), "cumsum_bwd")
+    assert ((dg.double() - sums.masked_fill(dead, 0.0)).abs() <= 6e-8 * sums.abs() + 1e-12).all()
+    dx = torch.full((B, H, N), float("nan"), device="cuda")
+    _lib.check(lib.fox_gate_cumsum_bwd(dc.data_ptr(), x.data_ptr(), 2, *x.stride(), ss.data_ptr(), dx.data_ptr(), *dx.stride(), B, H, N,
+                                       stream), "gate_cumsum_bwd")
+    ref = sums.masked_fill(dead, 0.0) * torch.sigmoid(-x.double())
+    assert ((dx.double() - ref).abs() <= 2e-6 * ref.abs() + 1e-12).all()   # hardware exp and reciprocal: a few ulp
+
+
 def test_mfma_probe_runs(fa):
     """The measuring-stick loop of the power report: launches, returns, leaves its sink alone."""
     from forgetting_transformer.ops import _lib
