@@ -234,6 +234,8 @@ hipError_t launch_fwd_decode(const FwdK& a, int D, int dtype, hipStream_t s) {
   return dtype == 0 ? launch_decode_t<Bf16>(a, D, s) : launch_decode_t<Fp16>(a, D, s);
 }
 
+static int64_t decode_batches(int N, int D) { return ((int64_t)N * D + 16383) / 16384; }   // batches of keys, four waves each
+
 // ---------------------------------------------------------------------------
 // The same step straight from the log forget gates: no cumulative sum of the whole row in front of it.
 //
@@ -243,17 +245,17 @@ hipError_t launch_fwd_decode(const FwdK& a, int D, int dtype, hipStream_t s) {
 // decode_combine_kernel.  A gate is read once, by the wave that reads its key; the row scan this replaces (one workgroup per
 // row, a chain of barriers per 8192 keys) took 20 us of a 600 us step at B16 H16 N32768 D128 and 5.7 us of 36 at
 // B1 H12 N1500 D64.  Bound by HBM where the cache is long, by one round trip per batch where it is short.
-template <typename Tr, int D>
-__global__ __launch_bounds__(256) void decode_gates_kernel(const DecodeK a) {
+template <typename Tr, int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void decode_gates_kernel(const DecodeK a) {
   constexpr int LPR = D / 8;      // lanes per key row
   constexpr int KPL = 64 / LPR;   // keys per wave load instruction
   constexpr int U = 8;            // loads of K and of V in flight per lane
   constexpr int KPB = KPL * U;    // keys per wave and batch
   constexpr int GB = (KPB + 63) / 64;   // gates per lane and batch
   static_assert(KPB == kDecodeBatchKeys<D>, "the host counts batches with the same size");
-  __shared__ float part_m[4], part_l[4];
-  __shared__ double part_g[4];
-  __shared__ __align__(16) float part_acc[4][D];
+  __shared__ float part_m[WAVES], part_l[WAVES];
+  __shared__ double part_g[WAVES];
+  __shared__ __align__(16) float part_acc[WAVES][D];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ch = lane % LPR, r = lane / LPR;
@@ -270,8 +272,8 @@ __global__ __launch_bounds__(256) void decode_gates_kernel(const DecodeK a) {
     const int64_t s64 = a.seq_start[b];
     lo = (int)(s64 < 0 ? 0 : (s64 > N ? N : s64));
   }
-  // run gw of the splits * 4 runs, counted from the last key: whole batches, the first one excepted
-  const int runs = a.splits * 4, gw = sp * 4 + wave;
+  // run gw of the splits * WAVES runs, counted from the last key: whole batches, the first one excepted
+  const int runs = a.splits * WAVES, gw = sp * WAVES + wave;
   int per = (N - lo + runs - 1) / runs;
   per = (per + KPB - 1) / KPB * KPB;
   const int64_t back = (int64_t)gw * per;
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(256) void decode_gates_kernel(const DecodeK a) {
     }
   }
 
-  // merge the KPL row groups of the wave, then the four waves, each shifted by the gates of the runs behind its own
+  // merge the KPL row groups of the wave, then the waves, each shifted by the gates of the runs behind its own
 #pragma unroll
   for (int off = LPR; off < 64; off <<= 1) {
     const float m2 = __shfl_xor(m, off), l2 = __shfl_xor(l, off);
@@ -376,7 +378,7 @@ __global__ __launch_bounds__(256) void decode_gates_kernel(const DecodeK a) {
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = part_acc[0][ch * 8 + e];
 #pragma unroll
-  for (int w = 1; w < 4; ++w) {
+  for (int w = 1; w < WAVES; ++w) {
     float acc2[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc2[e] = part_acc[w][ch * 8 + e];
@@ -458,9 +460,21 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecodeK a) {
   if (d == 0 && a.lse) a.lse[bh] = empty ? -INFINITY : m_tot * kLn2 + __logf(l_tot);
 }
 
+// Whether one workgroup of sixteen waves takes a (batch, head) whole, which saves the merge of splits and its launch.  The line
+// lies where a CU's share of the bandwidth costs more than the merge: D 64, splits of four waves and merge against one
+// workgroup, us: B1 H12 N300 (2 batches) 7.9 / 6.8, N1500 (6 batches) 8.2 / 12.0.  With half a workgroup per CU or more the
+// splits share those CUs anyway: B8 H16 N700 (3) 10.7 / 9.5, B16 H16 N700 13.6 / 11.7, B8 H16 N2048 (8) 17.0 / 17.5.
+static bool decode_one_workgroup(int64_t bh, int64_t batches) {
+  return bh < 2 * kCus && batches > 1 && batches <= (bh >= kCus / 2 ? 4 : 2);
+}
+
 template <typename Tr, int D>
 static hipError_t launch_decode_gates_d(const DecodeK& a, hipStream_t s) {
-  hipLaunchKernelGGL((decode_gates_kernel<Tr, D>), dim3((unsigned)(a.splits * a.B * a.H)), dim3(256), 0, s, a);
+  if (decode_one_workgroup((int64_t)a.B * a.H, decode_batches(a.N, D))) {
+    hipLaunchKernelGGL((decode_gates_kernel<Tr, D, 16>), dim3((unsigned)(a.B * a.H)), dim3(1024), 0, s, a);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL((decode_gates_kernel<Tr, D, 4>), dim3((unsigned)(a.splits * a.B * a.H)), dim3(256), 0, s, a);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.splits <= 1) return e;
   hipLaunchKernelGGL((decode_combine_kernel<Tr, D>), dim3((unsigned)(a.B * a.H)), dim3(256), 0, s, a);
@@ -486,7 +500,8 @@ hipError_t launch_decode_gates(const DecodeK& a, int D, int dtype, hipStream_t s
 // a step over a short cache is a chain of round trips, one per batch a wave walks.  B1 H12 N1500 D64: two splits 7.9 us
 // (three batches a wave), six 4.6.
 int decode_splits(int B, int H, int N, int D) {
-  const int64_t bh = (int64_t)B * H, batches = ((int64_t)N * D + 16383) / 16384;   // four waves' batches
+  const int64_t bh = (int64_t)B * H, batches = decode_batches(N, D);
+  if (decode_one_workgroup(bh, batches)) return 1;
   int64_t splits = (2048 + bh - 1) / bh;
   splits = splits > batches ? batches : splits;
   splits = splits > kDecodeMaxSplits ? kDecodeMaxSplits : splits;

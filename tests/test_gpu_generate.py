@@ -36,14 +36,29 @@ def test_single_query(ft, B, H, N, D, dtype, gate_mean):
     assert torch.equal(other.transpose(1, 2), out)     # strided gates and rows: the same arithmetic
 
 
-def test_single_query_behind_a_closed_gate(ft):
+@pytest.mark.parametrize("N,at", [(3000, 1234), (300, 100), (300, 299)])
+def test_single_query_behind_a_closed_gate(ft, N, at):
     """A log gate of -inf hides every key left of it and nothing else."""
-    q, k, v, g, _, _ = make_inputs(1, 2, 1, 3000, 64, device="cuda", head_first=True, seed=5, gate_mean=2.0)
-    g[:, :, 1234] = float("-inf")
+    q, k, v, g, _, _ = make_inputs(1, 2, 1, N, 64, device="cuda", head_first=True, seed=5, gate_mean=2.0)
+    g[:, :, at] = float("-inf")
     with torch.no_grad():
         out = ft.forgetting_attention(q, k, v, g, head_first=True)
-        ref = O.forgetting_attention_ref(q, k[:, :, 1234:], v[:, :, 1234:], g[:, :, 1234:].clamp(min=-50), head_first=True)
+        ref = O.forgetting_attention_ref(q, k[:, :, at:], v[:, :, at:], g[:, :, at:].clamp(min=-50), head_first=True)
     assert_parity("out", out, ref)
+
+
+# one workgroup of sixteen waves takes a (batch, head) whole: two batches of keys with few heads, up to four with many, and
+# the first sizes beyond
+@pytest.mark.parametrize("B,H,N,D", [(2, 3, 257, 64), (2, 3, 512, 64), (2, 3, 513, 64), (1, 3, 129, 128), (2, 2, 2048, 16), (2, 2, 600, 32),
+                                     (4, 32, 1024, 64), (4, 32, 1025, 64), (5, 26, 300, 128), (8, 63, 2047, 32), (8, 64, 700, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_single_query_in_one_workgroup(ft, B, H, N, D, dtype):
+    ss = [(N * i) // B for i in range(B)]
+    ss[-1] = N if B > 2 else N - 1
+    q, k, v, g, _, ss = make_inputs(B, H, 1, N, D, dtype=dtype, device="cuda", head_first=True, seq_start=ss, seed=N + D, gate_mean=1.0)
+    with torch.no_grad():
+        out = ft.forgetting_attention(q, k, v, g, head_first=True, seq_start=ss)
+    assert_parity("out", out, O.forgetting_attention_ref(q, k, v, g, head_first=True, seq_start=ss))
 
 
 @pytest.mark.parametrize("D,T,dtype", [(64, 1, torch.bfloat16), (128, 1, torch.float16), (16, 7, torch.bfloat16), (40, 300, torch.float16),
