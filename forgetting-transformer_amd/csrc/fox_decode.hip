@@ -464,15 +464,18 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecodeK a) {
 // lies where a CU's share of the bandwidth costs more than the merge: D 64, splits of four waves and merge against one
 // workgroup, us: B1 H12 N300 (2 batches) 7.9 / 6.8, N1500 (6 batches) 8.2 / 12.0.  With half a workgroup per CU or more the
 // splits share those CUs anyway: B8 H16 N700 (3) 10.7 / 9.5, B16 H16 N700 13.6 / 11.7, B8 H16 N2048 (8) 17.0 / 17.5.
-static bool decode_one_workgroup(int64_t bh, int64_t batches) {
-  return bh < 2 * kCus && batches > 1 && batches <= (bh >= kCus / 2 ? 4 : 2);
+// Head dim 16 needs one register more than sixteen waves leave a lane.
+static bool decode_one_workgroup(int64_t bh, int64_t batches, int D) {
+  return D >= 32 && bh < 2 * kCus && batches > 1 && batches <= (bh >= kCus / 2 ? 4 : 2);
 }
 
 template <typename Tr, int D>
 static hipError_t launch_decode_gates_d(const DecodeK& a, hipStream_t s) {
-  if (decode_one_workgroup((int64_t)a.B * a.H, decode_batches(a.N, D))) {
-    hipLaunchKernelGGL((decode_gates_kernel<Tr, D, 16>), dim3((unsigned)(a.B * a.H)), dim3(1024), 0, s, a);
-    return hipGetLastError();
+  if constexpr (D >= 32) {
+    if (decode_one_workgroup((int64_t)a.B * a.H, decode_batches(a.N, D), D)) {
+      hipLaunchKernelGGL((decode_gates_kernel<Tr, D, 16>), dim3((unsigned)(a.B * a.H)), dim3(1024), 0, s, a);
+      return hipGetLastError();
+    }
   }
   hipLaunchKernelGGL((decode_gates_kernel<Tr, D, 4>), dim3((unsigned)(a.splits * a.B * a.H)), dim3(256), 0, s, a);
   const hipError_t e = hipGetLastError();
@@ -501,7 +504,7 @@ hipError_t launch_decode_gates(const DecodeK& a, int D, int dtype, hipStream_t s
 // (three batches a wave), six 4.6.
 int decode_splits(int B, int H, int N, int D) {
   const int64_t bh = (int64_t)B * H, batches = decode_batches(N, D);
-  if (decode_one_workgroup(bh, batches)) return 1;
+  if (decode_one_workgroup(bh, batches, D)) return 1;
   int64_t splits = (2048 + bh - 1) / bh;
   splits = splits > batches ? batches : splits;
   splits = splits > kDecodeMaxSplits ? kDecodeMaxSplits : splits;
