@@ -263,10 +263,12 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
       k.ws_ml = k.ws_o + (int64_t)k.splits * k.B * k.H * k.M * args->dims.D;
     }
   }
+  const bool split_shape = k.M == 1 || k.splits > 1;
+  k.pair = fox::fwd_pairs(k.B, k.H, k.M, k.N, args->dims.D, k.thr != nullptr, k.splits);
+  if (k.pair) k.splits = 1;
   if (epi) {
     const int D = args->dims.D;
-    if (k.M == 1 || k.splits > 1) {
-      // two passes: the plain forward, then the norm over o as (B*M rows, H heads)
+    if (split_shape) {
       const fox_view* vs[3] = {&args->o, &epi->y, &epi->gate};
       for (int i = 0; i < 3; ++i) {
         if (i == 2 && epi->activation == FOX_ACT_NONE) break;
@@ -274,6 +276,9 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
           return fail(FOX_E_ARG, "%s: a key-split or single-query shape needs o, gate and y with adjacent heads "
                                  "(stride_h == D, stride_b == M * stride_t)", what);
       }
+    }
+    if (split_shape && !k.pair) {
+      // two passes: the plain forward, then the norm over o as (B*M rows, H heads)
       FOX_TRY(check_hip(fox::launch_fwd(k, D, args->dims.dtype, (hipStream_t)stream), what));
       fox::NormGateK n{};
       n.x = (const uint16_t*)args->o.ptr; n.x_sr = args->o.stride_t;

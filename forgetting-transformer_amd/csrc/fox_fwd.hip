@@ -243,22 +243,36 @@ constexpr int kFwdWaves = D <= 64 ? 3 : 2;
 // STREAM: the variant for shapes with a single query tile per (batch, head): every K and V tile is read by exactly one
 // workgroup, so the tile loads carry the non-temporal hint (with it the chunked-prefill shape B16 M128 N32768 H16 D128
 // takes 0.62 ms instead of 0.71).  Where tiles are shared by the workgroups of several query tiles the hint costs 16-28 %.
-template <typename Tr, int D, bool SPLIT, bool EPI = false, bool STREAM = false>
-__global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
+//
+// PAIR: the variant for grids of few query tiles (fwd_pairs below).  A workgroup has two groups of four waves with their own
+// tile buffers; they take the key tiles of the same 128 query rows in turn, each with its own running maximum and sum, and group 0
+// merges the two states from LDS before the epilogue.  The walk of the heaviest tile, which is what such a grid waits for, is half
+// as long, and a CU with a single query tile has two waves per SIMD (B1 H16 T3001 D128, scan included: 67.7 -> 57.6 us).  Both groups pass the same barriers: the trip counts of
+// the loops are those of group 0, and a step for which group 1 has no tile left moves and computes nothing.
+template <typename Tr, int D, bool SPLIT, bool EPI, bool STREAM, bool PAIR>
+__device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's only argument
+  static_assert(!(PAIR && (SPLIT || STREAM)), "the paired variant is for whole walks over shared tiles");
+  static_assert(!PAIR || D >= 32, "group 1's accumulators are handed over in its tile buffers");
+  constexpr int GROUPS = PAIR ? 2 : 1;
   static_assert(!(SPLIT && EPI), "partial results of a key split are not normalised");
   static_assert(!(STREAM && EPI), "no streaming variant with the epilogue");
   constexpr int AUX = STREAM ? kLoadNonTemporal : 0;
   constexpr int BM = kFwdBM, BN = kFwdBN;
   constexpr int KK = D / 16, DB = (D + 31) / 32, NB = BN / 32;
   static_assert(BM == 128, "four waves of 32 rows");
-  __shared__ __align__(16) char k_tile0[Tile<D>::bytes(BN)];
-  __shared__ __align__(16) char k_tile1[Tile<D>::bytes(BN)];
-  __shared__ __align__(16) char v_tile0[Tile<D>::bytes(BN)];
-  __shared__ __align__(16) char v_tile1[Tile<D>::bytes(BN)];
-  __shared__ __align__(16) float cn_s0[BN];
-  __shared__ __align__(16) float cn_s1[BN];
+  __shared__ __align__(16) char k_tile0_s[GROUPS * Tile<D>::bytes(BN)];
+  __shared__ __align__(16) char k_tile1_s[GROUPS * Tile<D>::bytes(BN)];
+  __shared__ __align__(16) char v_tile0_s[GROUPS * Tile<D>::bytes(BN)];
+  __shared__ __align__(16) char v_tile1_s[GROUPS * Tile<D>::bytes(BN)];
+  __shared__ __align__(16) float cn_s0_s[GROUPS * BN];
+  __shared__ __align__(16) float cn_s1_s[GROUPS * BN];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 5, i = lane & 31;
+  const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), grp = PAIR ? wave_id >> 2 : 0;
+  const int tid = PAIR ? threadIdx.x & 255 : threadIdx.x, wave = PAIR ? wave_id & 3 : wave_id;   // within the group
+  const int lane = tid & 63, g = lane >> 5, i = lane & 31;
+  char *k_tile0 = k_tile0_s + grp * Tile<D>::bytes(BN), *k_tile1 = k_tile1_s + grp * Tile<D>::bytes(BN);
+  char *v_tile0 = v_tile0_s + grp * Tile<D>::bytes(BN), *v_tile1 = v_tile1_s + grp * Tile<D>::bytes(BN);
+  float *cn_s0 = cn_s0_s + grp * BN, *cn_s1 = cn_s1_s + grp * BN;
   int bh, mt, sp = 0;
   if constexpr (SPLIT) {  // (query tile, key split) pairs take the place of query tiles
     int mts;
@@ -266,7 +280,7 @@ __global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
     mt = mts / a.splits;
     sp = mts % a.splits;
   } else {
-    decode_block(blockIdx.x, a.n_mtiles, a.B * a.H, a.groups, !a.even, bh, mt);
+    decode_block(blockIdx.x, a.n_mtiles, a.B * a.H, a.groups, !a.even && !PAIR, bh, mt);   // paired: one workgroup per CU
   }
   const int b = bh / a.H, h = bh % a.H;
   const int M = a.M, N = a.N, p_seq = N - M;
@@ -292,14 +306,21 @@ __global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
   // visit (the one under the end of the diagonal) does not depend on the pruning bound, so it goes
   // first; then Q, then the per-row and per-key terms; the bound search's loads queue behind them.
   const DirectTileLoader<D, BN, 4, AUX> kld(a.k.st, wave, lane), vld(a.v.st, wave, lane);
-  const int n0_first = hi > 0 ? ((hi - 1) / BN) * BN : 0;
-  const bool early = !SPLIT && hi > (min(seq, hi) / BN) * BN && (n0_first + BN - 1 > a0 || !(qk_scale > 0.f));
+  int n0_first = hi > 0 ? ((hi - 1) / BN) * BN : 0;
+  bool early = !SPLIT && hi > (min(seq, hi) / BN) * BN && (n0_first + BN - 1 > a0 || !(qk_scale > 0.f));
   // The tile before it is requested as well when nothing can exclude it: it still reaches the workgroup's first row
   // (the pruning bound never cuts there) and lies right of seq_start.  Under pruning a workgroup visits two or
   // three tiles, and every round trip taken out of that chain counts.
   const int n0_second = n0_first - BN;
-  const bool early2 = early && n0_second >= (a0 / BN) * BN && n0_second >= (min(seq, hi) / BN) * BN &&
+  bool early2 = early && n0_second >= (a0 / BN) * BN && n0_second >= (min(seq, hi) / BN) * BN &&
                       (n0_second + BN - 1 > a0 || !(qk_scale > 0.f));
+  if constexpr (PAIR) {   // group 1's first tile is the second of the walk
+    if (grp) {
+      early = early2;
+      n0_first = n0_second;
+    }
+    early2 = false;
+  }
   if (early) {
     kld.issue(kp, a.k.st, n0_first, N, k_tile0);
     vld.issue(vp, a.v.st, n0_first, N, v_tile0);
@@ -400,37 +421,41 @@ __global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
   const int t_stop = n_tiles - n_diag;
   auto tile_n0 = [&](int t) { return lo + t * BN; };   // start of the tile at loop position t
   if (n_diag > 0) {
-    if (!early) issue(tile_n0(n_tiles - 1), k_tile0, v_tile0);
+    if (!early && n_tiles - 1 - grp >= t_stop) issue(tile_n0(n_tiles - 1 - grp), k_tile0, v_tile0);
     if (tid < BN) cn_s0[tid] = cn_term();
     if (early2) { cn_raw = cn_raw2; cn_ok = cn_ok2; }
   }
   bool requested = early2;  // buffers 1 already hold (or await) the next tile
-  for (int t = n_tiles - 1; t >= t_stop; t -= 2) {
+  for (int tu = n_tiles - 1; tu >= t_stop; tu -= 2 * GROUPS) {
+    const int t = tu - grp, t1 = t - GROUPS, t2 = t - 2 * GROUPS;   // this group's tile and its next two
     // even step: consume buffers 0, fill buffers 1
     wait_vmem_all();
     __syncthreads();
-    if (t - 1 >= t_stop && !requested) issue(tile_n0(t - 1), k_tile1, v_tile1);
+    if (t1 >= t_stop && !requested) issue(tile_n0(t1), k_tile1, v_tile1);
     requested = false;
-    compute(tile_n0(t), k_tile0, v_tile0, cn_s0);
-    if (t - 1 < t_stop) break;
+    if (!PAIR || t >= t_stop) compute(tile_n0(t), k_tile0, v_tile0, cn_s0);
+    if (tu - GROUPS < t_stop) break;
     if (tid < BN) cn_s1[tid] = cn_term();
     // odd step: consume buffers 1, fill buffers 0
     wait_vmem_all();
     __syncthreads();
-    if (t - 2 >= t_stop) issue(tile_n0(t - 2), k_tile0, v_tile0);
-    compute(tile_n0(t - 1), k_tile1, v_tile1, cn_s1);
-    if (t - 2 >= t_stop && tid < BN) cn_s0[tid] = cn_term();
+    if (t2 >= t_stop) issue(tile_n0(t2), k_tile0, v_tile0);
+    if (!PAIR || t1 >= t_stop) compute(tile_n0(t1), k_tile1, v_tile1, cn_s1);
+    if (t2 >= t_stop && tid < BN) cn_s0[tid] = cn_term();
   }
 
-  const int n_int = t_stop;  // interior tile j (0 = nearest to the diagonal) starts at key lo + (n_int-1-j)*BN
-  if (n_int > 0) {
+  if (t_stop > 0) {
+    // this group's interior tile j (0 = nearest to the diagonal); n_steps is the count of group 0, the larger one
+    const int n_int = (t_stop - grp + GROUPS - 1) / GROUPS, n_steps = (t_stop + GROUPS - 1) / GROUPS;
+    auto int_n0 = [&](int j) { return lo + (t_stop - 1 - grp - GROUPS * j) * BN; };
     auto issue_k = [&](int j, char* kt) {
-      const int n0 = lo + (n_int - 1 - j) * BN;
+      const int n0 = int_n0(j);
       issue_cn(n0);
       kld.issue(kp, a.k.st, n0, N, kt);
     };
-    auto issue_v = [&](int j, char* vt) { vld.issue(vp, a.v.st, lo + (n_int - 1 - j) * BN, N, vt); };
+    auto issue_v = [&](int j, char* vt) { vld.issue(vp, a.v.st, int_n0(j), N, vt); };
     // K runs one tile ahead of V: iteration j computes S(j+1) and P(j) V(j).
+    static_assert(kMinPipelinedTiles >= GROUPS, "every group has an interior tile here");
     __syncthreads();  // phase 1 is done with every buffer
     issue_k(0, k_tile0);
     if (tid < BN) cn_s0[tid] = cn_term();
@@ -451,8 +476,9 @@ __global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
     // tile: the loads then write zeros into the free buffer).
     auto pipelined_tile = [&](int j, const char* k_nx, const char* v_cur, const float* cn_nx, char* k_fill, char* v_fill,
                               f32x16 (&s_cur)[NB], f32x16 (&s_nx)[NB]) {
+      if (PAIR && j >= n_int) return;   // group 0 has one tile more
       const bool more_k = j + 2 < n_int, more_v = j + 1 < n_int;
-      const int nk = more_k ? lo + (n_int - 3 - j) * BN : lo, nv = more_v ? lo + (n_int - 2 - j) * BN : lo;
+      const int nk = more_k ? int_n0(j + 2) : lo, nv = more_v ? int_n0(j + 1) : lo;
       if (more_k) issue_cn(nk);
       const uint16_t *k_src = kp + (int64_t)nk * a.k.st, *v_src = vp + (int64_t)nv * a.v.st;
       const int k_bytes = kld.extent(a.k.st, nk, more_k ? N : nk), v_bytes = vld.extent(a.v.st, nv, more_v ? N : nv);
@@ -460,14 +486,14 @@ __global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
       if (wave_has_rows) fwd_tile_pipelined<Tr, D>(k_nx, v_cur, cn_nx, qreg, oacc, m_i, l_i, qk_scale, lane, s_cur, s_nx, dma);
       else dma.all();  // a wave without query rows only moves its share of the tiles
     };
-    for (int j = 0; j < n_int; j += 2) {
+    for (int j = 0; j < n_steps; j += 2) {
       // even iteration: K(j+1) in k_tile1 with its key terms in cn_s1, V(j) in v_tile0.  The key
       // terms of tile j+1 go to LDS before the barrier: their buffer was last read two iterations ago.
       wait_vmem_all();
       if (j + 1 < n_int && tid < BN) cn_s1[tid] = cn_term();
       __syncthreads();
       pipelined_tile(j, k_tile1, v_tile0, cn_s1, k_tile0, v_tile1, s_a, s_b);
-      if (j + 1 >= n_int) break;
+      if (j + 1 >= n_steps) break;
       // odd iteration: K(j+2) in k_tile0 with its key terms in cn_s0, V(j+1) in v_tile1
       wait_vmem_all();
       if (j + 2 < n_int && tid < BN) cn_s0[tid] = cn_term();
@@ -477,7 +503,33 @@ __global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
   }
 
   // epilogue
-  const float l_tot = half_sum(l_i);
+  float l_tot = half_sum(l_i);
+  if constexpr (PAIR) {   // group 1 leaves its state in its tile buffers (one per wave), group 0 takes it up and goes on alone
+    __shared__ float pair_m[256], pair_l[256];
+    static_assert(16 * DB * kWave * 4 <= Tile<D>::bytes(BN), "a wave's accumulators fit one tile buffer");
+    const int next = Tile<D>::bytes(BN);
+    float* there = reinterpret_cast<float*>((wave == 0 ? k_tile0_s : wave == 1 ? k_tile1_s : wave == 2 ? v_tile0_s : v_tile1_s) + next);
+    wait_vmem_all();
+    __syncthreads();
+    if (grp) {
+      pair_m[tid] = m_i;
+      pair_l[tid] = l_tot;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) there[(16 * db + r) * kWave + lane] = oacc[db][r];
+    }
+    __syncthreads();
+    if (grp) return;   // (no barrier below)
+    const float m2 = pair_m[tid], mx = fmaxf(m_i, m2);
+    const float w0 = __builtin_amdgcn_exp2f(m_i - mx), w1 = __builtin_amdgcn_exp2f(m2 - mx);
+    m_i = mx;
+    l_tot = l_tot * w0 + pair_l[tid] * w1;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) oacc[db][r] = oacc[db][r] * w0 + there[(16 * db + r) * kWave + lane] * w1;
+  }
   if constexpr (SPLIT) {
     // partial result of this key split: unnormalised accumulator, row maximum (log2 domain,
     // including the row term) and row sum; fox::combine_kernel merges the splits
@@ -506,8 +558,10 @@ __global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
   if (m < M && g == 0) a.lse[(int64_t)bh * M + m] = empty ? -INFINITY : (m_i + cm2) * kLn2 + __logf(l_tot);
   // o leaves through LDS (the tile buffers are free now, one per wave) so that the global stores are whole rows
   static_assert(kStoreStageBytes<D> <= Tile<D>::bytes(BN), "one wave stages in one tile buffer");
-  wait_vmem_all();  // whatever was requested last (possibly an empty tile) has landed
-  __syncthreads();  // every wave is done with the last tile
+  if constexpr (!PAIR) {
+    wait_vmem_all();  // whatever was requested last (possibly an empty tile) has landed
+    __syncthreads();  // every wave is done with the last tile
+  }
   char* stage = wave == 0 ? k_tile0 : wave == 1 ? k_tile1 : wave == 2 ? v_tile0 : v_tile1;
   if constexpr (EPI) {  // the layer's output norm and gate, applied while the rows are on their way out
     // The epilogue's arguments are fetched from the kernel argument block only here, through a pointer the
@@ -525,6 +579,20 @@ __global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
     store_rows_via_lds<Tr, D>(stage, oacc, inv, op, a.o.st, m0 + 32 * wave, M, lane);
   }
   asm volatile("" ::"v"(l2_touch));   // the value is never used; this keeps the load
+}
+
+// (the bodies for the device pass only: on the host side a kernel is a stub, and the tile code's device builtins do not resolve there)
+template <typename Tr, int D, bool SPLIT, bool EPI = false, bool STREAM = false>
+__global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
+#ifdef __HIP_DEVICE_COMPILE__
+  fwd_body<Tr, D, SPLIT, EPI, STREAM, false>(a);
+#endif
+}
+template <typename Tr, int D, bool EPI>
+__global__ __launch_bounds__(512, 2) void fwd_pair_kernel(const FwdK a) {
+#ifdef __HIP_DEVICE_COMPILE__
+  fwd_body<Tr, D, false, EPI, false, true>(a);
+#endif
 }
 
 // Merge the partial results of the key splits of one query row:
@@ -590,6 +658,12 @@ constexpr int kStreamMaxQueryTiles = 1;
   template __global__ void fwd_kernel<TR, 32, true, false, true>(const FwdK);   \
   template __global__ void fwd_kernel<TR, 64, true, false, true>(const FwdK);   \
   template __global__ void fwd_kernel<TR, 128, true, false, true>(const FwdK);  \
+  template __global__ void fwd_pair_kernel<TR, 32, false>(const FwdK);   \
+  template __global__ void fwd_pair_kernel<TR, 64, false>(const FwdK);   \
+  template __global__ void fwd_pair_kernel<TR, 128, false>(const FwdK);  \
+  template __global__ void fwd_pair_kernel<TR, 32, true>(const FwdK);    \
+  template __global__ void fwd_pair_kernel<TR, 64, true>(const FwdK);    \
+  template __global__ void fwd_pair_kernel<TR, 128, true>(const FwdK);   \
   template __global__ void combine_kernel<TR, 16>(const FwdK);           \
   template __global__ void combine_kernel<TR, 32>(const FwdK);           \
   template __global__ void combine_kernel<TR, 64>(const FwdK);           \
@@ -606,6 +680,13 @@ static hipError_t launch_fwd_d(const FwdK& a, int dtype, hipStream_t s) {
     if (e != hipSuccess || a.splits <= 1) return e;
   } else if (a.splits <= 1) {
     const dim3 grid((unsigned)(a.n_mtiles * a.B * a.H));
+    if constexpr (D >= 32) {
+      if (a.pair && !stream) {
+        if (a.epi.y.ptr) hipLaunchKernelGGL((fwd_pair_kernel<Tr, D, true>), grid, dim3(512), 0, s, a);
+        else hipLaunchKernelGGL((fwd_pair_kernel<Tr, D, false>), grid, dim3(512), 0, s, a);
+        return hipGetLastError();
+      }
+    }
     if (a.epi.y.ptr) hipLaunchKernelGGL((fwd_kernel<Tr, D, false, true>), grid, dim3(256), 0, s, a);
     else if (stream) hipLaunchKernelGGL((fwd_kernel<Tr, D, false, false, true>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((fwd_kernel<Tr, D, false>), grid, dim3(256), 0, s, a);
@@ -633,6 +714,24 @@ static hipError_t launch_fwd_t(const FwdK& a, int D, int dtype, hipStream_t s) {
 
 hipError_t launch_fwd(const FwdK& a, int D, int dtype, hipStream_t s) {
   return dtype == 0 ? launch_fwd_t<Bf16>(a, D, dtype, s) : launch_fwd_t<Fp16>(a, D, dtype, s);
+}
+
+// Whether the forward takes the paired variant (fwd_pair_kernel): less than two query tiles per CU under a causal triangle, where the
+// heaviest tile's walk sets the time.  Measured forward with its scan, us, one group / paired.
+// - Unsplit grids beyond one tile per CU lose a little throughput (the merge, one workgroup's start and end with nothing beside it)
+//   and gain the tail: worth it from a walk of 16 keys per tile beyond one per CU on.  D 64: 280 tiles N1200 26.0 / 21.8, 322 tiles N2900
+//   49.4 / 39.9, 384 tiles N1024 23.3 / 24.1, N3001 48.6 / 39.5.  D 128: 280 tiles N1200 32.3 / 29.1, 384 tiles N1024 31.2 / 34.4, N2048
+//   50.2 / 47.3, N3001 67.7 / 57.6.  Two full tiles per CU are balanced by the folded order (D 128 N2048 55.9 / 59.2, N4096 94.1 / 91.7),
+//   more make no tail that matters (768 tiles N4096 121 / 129).
+// - Smaller grids with fewer keys than are split: from 512 keys on.  D 64: N300 11.6 / 12.0, N512 15.6 / 14.5, N777 19.3 / 17.1.
+// - Two key splits cost a pass over fp32 partials and a merge launch, which pays for longer walks only.  D 128 and 64: B2 H12 N1024
+//   33.2 / 25.3 and 24.6 / 19.4, B1 H16 N2048 44.3 / 38.2 and 34.3 / 29.3, B1 H10 N2900 53.4 / 55.1 and 38.2 / 39.0.
+// - Under a pruning threshold the walks are short whatever the shape; head dim 16 has no room to hand the accumulators over.
+bool fwd_pairs(int B, int H, int M, int N, int D, bool pruned, int splits) {
+  const int64_t wgs = (int64_t)((M + kFwdBM - 1) / kFwdBM) * B * H;
+  if (D < 32 || pruned || even_tiles(M, N) || wgs >= 2 * kCus || N < 512) return false;
+  if (splits > 1) return splits == 2 && N <= 2560;
+  return N >= 16 * (wgs - kCus);
 }
 
 // Number of key splits the forward uses for a shape: 1 unless the grid of query tiles

@@ -34,6 +34,7 @@ struct FwdK {
   int groups;      // (batch, head) groups of the launch order (order_groups)
   bool even;       // the tiles weigh about the same (even_tiles)
   int splits;      // key splits of the forward (1 = none)
+  bool pair;       // two groups of waves share every query tile's walk (fwd_pairs)
   float* ws_o;     // (splits, B, H, M, D) partial accumulators
   float* ws_ml;    // (splits, B, H, M, 2) partial row maximum and row sum
   FwdEpilogue epi; // only for splits == 1 and M > 1 (the launcher rejects it otherwise)
@@ -154,6 +155,7 @@ inline int order_groups(int n_bh, int M, int N, int D) {
 
 hipError_t launch_fwd(const FwdK& a, int D, int dtype, hipStream_t s);
 int fwd_key_splits(int B, int H, int M, int N);
+bool fwd_pairs(int B, int H, int M, int N, int D, bool pruned, int splits);
 hipError_t launch_bwd_delta(const BwdK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_bwd_dkdv(const BwdK& a, int D, int dtype, hipStream_t s);   // a.cls selects the variant and its tiles
 bool dkdv_split_supports(int D);   // head dims the split (kClassLight) variant of the dK/dV kernel exists for

@@ -5,6 +5,8 @@ wrong pair shows."""
 import pytest
 import torch
 
+from conftest import assert_parity, make_inputs
+from oracle import fox_oracle as O
 from test_gpu_parity import fa, run_case  # noqa: F401  (fa is a fixture)
 
 pytestmark = pytest.mark.gpu
@@ -23,3 +25,28 @@ def test_launch_order(fa, B, H, T, D):
 @pytest.mark.parametrize("B,H,M,N,D", [(2, 16, 333, 1100, 32), (1, 8, 129, 3000, 64), (3, 7, 300, 2000, 16)])
 def test_key_splits(fa, B, H, M, N, D):
     run_case(fa, B, H, M, N, D, seed=M + N, gate_mean=2.0)
+
+
+# few query tiles: two groups of waves share a tile's walk.  Walks of one tile (group 1 has none), of odd and even length, with three,
+# four and five interior tiles (where the pipelined path begins), with left padding inside the walk and without a diagonal-free part
+@pytest.mark.parametrize("B,H,M,N", [(1, 2, 257, 513), (2, 3, 512, 512), (1, 3, 449, 577), (1, 3, 513, 576), (2, 2, 640, 640),
+                                     (1, 2, 300, 512), (1, 3, 900, 1025), (1, 5, 1500, 1533), (3, 5, 777, 777), (1, 16, 2100, 2100)])
+@pytest.mark.parametrize("D,dtype", [(32, torch.bfloat16), (64, torch.float16), (128, torch.bfloat16)])
+def test_paired_forward(fa, B, H, M, N, D, dtype):
+    run_case(fa, B, H, M, N, D, dtype=dtype, seed=M + D, gate_mean=2.0)
+    run_case(fa, B, H, M, N, D, dtype=dtype, seed=M + D, gate_mean=0.0, head_first=False, seq_start=[(N * (2 * b + 1)) // (2 * B) for b in range(B)])
+
+
+@pytest.mark.parametrize("D", [32, 128])
+def test_paired_forward_with_a_negative_scale(fa, D):   # every tile takes the masked path
+    run_case(fa, 1, 2, 700, 900, D, seed=3, gate_mean=2.0, sm_scale=-0.1)
+
+
+# grids beyond one tile per CU and in place of two key splits, at their edges: the output alone
+@pytest.mark.parametrize("B,H,T", [(2, 16, 1500), (1, 17, 1921), (3, 10, 1024), (1, 12, 2560)])
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.float16)])
+def test_paired_forward_of_larger_grids(fa, B, H, T, D, dtype):
+    q, k, v, g, _, ss = make_inputs(B, H, T, T, D, dtype=dtype, device="cuda", head_first=False, seed=T, gate_mean=2.0)
+    with torch.no_grad():
+        out = fa(q, k, v, g)
+    assert_parity("out", out, O.forgetting_attention_ref(q, k, v, g))

@@ -82,6 +82,16 @@ def test_kernels_do_not_spill():
         assert u["ScratchSize"] == 0, (name, u)
 
 
+def test_paired_forward_fits_a_cu():
+    """Eight waves at two per SIMD, nothing in scratch, both groups' tiles in the LDS of one CU."""
+    import json
+    usage = json.loads(_lib.LIB_PATH.with_name("kernel_resources.json").read_text())
+    pairs = {n: u for n, u in usage.items() if "fwd_pair_kernelI" in n}
+    assert len(pairs) == 12
+    for name, u in pairs.items():
+        assert u["ScratchSize"] == 0 and u["VGPRs Spill"] == 0 and u["Occupancy"] >= 2 and u["LDS Size"] <= 160 * 1024, (name, u)
+
+
 def test_tile_config():
     for d in (16, 32, 64, 128):
         bm, bn, kbn, kbm = _lib.tile_config(d)
