@@ -467,22 +467,27 @@ bool needs_graph(std::initializer_list<const Tensor*> ts) {
 
 PyObject* none() { Py_RETURN_NONE; }
 
+// The truth value of a Python flag, whatever type it comes in (bool, 0/1, numpy.bool_); false: it has none.
+bool flag(PyObject* o, bool& value) {
+  const int r = PyObject_IsTrue(o);
+  if (r < 0) PyErr_Clear();   // the general path raises it again
+  value = r > 0;
+  return r >= 0;
+}
+
 std::optional<Tensor> some(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
 
 // Fills `a` from the arguments both attention entry points share; false: not a call for the native path.
 bool parse_attention(Attention& a, const Tensor* q, const Tensor* k, const Tensor* v, const Tensor* g, PyObject* head_first,
-                     PyObject* seq_start, PyObject* sm_scale, PyObject* threshold, bool is_logit) {
+                     PyObject* seq_start, PyObject* sm_scale, PyObject* threshold, PyObject* is_logit) {
   if (!q || !k || !v || !g) return false;
   if (q->dim() != 4 || k->dim() != 4 || v->dim() != 4 || g->dim() != 3) return false;
   if (!on_current_gpu(*q) || k->device() != q->device() || v->device() != q->device() || g->device() != q->device()) return false;
   const auto dt = q->scalar_type();
   if (!sixteen_bit(*q) || k->scalar_type() != dt || v->scalar_type() != dt) return false;
-  if (is_logit ? gate_dtype(*g) < 0 : g->scalar_type() != at::kFloat) return false;
-  const int hf = PyObject_IsTrue(head_first);
-  if (hf < 0) return false;
-  a.head_first = hf != 0;
-  a.is_logit = is_logit;
-  const int ih = hf ? 1 : 2, it = hf ? 2 : 1;
+  if (!flag(is_logit, a.is_logit) || !flag(head_first, a.head_first)) return false;
+  if (a.is_logit ? gate_dtype(*g) < 0 : g->scalar_type() != at::kFloat) return false;
+  const int ih = a.head_first ? 1 : 2, it = a.head_first ? 2 : 1;
   a.B = q->size(0);
   a.H = q->size(ih);
   a.M = q->size(it);
@@ -553,7 +558,7 @@ PyObject* py_attention(PyObject*, PyObject* const* o, Py_ssize_t n) {
   TORCH_CHECK(n == 9, "attention takes 9 arguments");
   Attention a;
   const Tensor *q = tensor_of(o[0]), *k = tensor_of(o[1]), *v = tensor_of(o[2]), *g = tensor_of(o[3]);
-  if (!parse_attention(a, q, k, v, g, o[4], o[5], o[6], o[7], o[8] == Py_True)) return none();
+  if (!parse_attention(a, q, k, v, g, o[4], o[5], o[6], o[7], o[8])) return none();
   return finish_attention(a, *q, *k, *v, *g, Tensor(), Tensor());
   END_HANDLE_TH_ERRORS
 }
@@ -564,7 +569,7 @@ PyObject* py_attention_norm_gate(PyObject*, PyObject* const* o, Py_ssize_t n) {
   TORCH_CHECK(n == 13, "attention_norm_gate takes 13 arguments");
   Attention a;
   const Tensor *q = tensor_of(o[0]), *k = tensor_of(o[1]), *v = tensor_of(o[2]), *g = tensor_of(o[3]), *w = tensor_of(o[5]);
-  if (!parse_attention(a, q, k, v, g, o[8], o[9], o[10], o[11], o[12] == Py_True)) return none();
+  if (!parse_attention(a, q, k, v, g, o[8], o[9], o[10], o[11], o[12])) return none();
   Tensor gate;
   if (o[4] != Py_None) {
     const Tensor* t = tensor_of(o[4]);
@@ -644,7 +649,8 @@ PyObject* py_qk_norm_threshold(PyObject*, PyObject* const* o, Py_ssize_t n) {
     PyErr_Clear();
     return none();
   }
-  const bool shared = o[6] == Py_True;
+  bool shared = false;
+  if (!flag(o[6], shared)) return none();
   if (!q || !k || H < 1 || D < 1 || !(T > 0) || !on_current_gpu(*q) || k->device() != q->device() || q->dim() != 1 || q->sizes() != k->sizes() ||
       q->size(0) != (shared ? D : H * D) || q->scalar_type() != at::kFloat || k->scalar_type() != at::kFloat || !q->is_contiguous() || !k->is_contiguous())
     return none();

@@ -3,6 +3,7 @@ autograd nodes directly: the two launch the same kernels, so every output and gr
 layouts, with every optional argument, and for inputs the native path hands back (tensors that need a copy first)."""
 from importlib import import_module
 
+import numpy as np
 import pytest
 import torch
 
@@ -165,3 +166,35 @@ def test_forward_mode_is_refused(ft):
     q, k, v, g, _, _ = make_inputs(1, 2, 70, 70, 64, device="cuda", head_first=True, seed=3)
     with fwd.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
         ft.forgetting_attention(fwd.make_dual(q, torch.ones_like(q)), k, v, g, head_first=True)
+
+
+@pytest.mark.parametrize("true,false", [(1, 0), (np.True_, np.False_)])
+def test_flags_count_by_their_truth_value(ft, true, false):
+    """Configurations hold switches as 0/1 or numpy.bool_: they mean what `if flag` means, also with fp32 logits, where nothing in the
+    types tells logits from log gates."""
+    q, k, v, _, _, _ = make_inputs(1, 2, 70, 70, 64, device="cuda", head_first=False, seed=11)
+    logits, w = torch.randn(1, 70, 2, device="cuda") + 1, torch.rand(128, device="cuda") + 0.5
+    call = lambda **kw: ft.forgetting_attention_norm_gate(q, k, v, kw.pop("g", logits), None, w, **kw)
+    want, got = call(fgate_is_logit=True), call(fgate_is_logit=true, head_first=false)
+    assert isinstance(got, tuple) and len(got) == 2
+    _equal(got, want)
+    log_gates = torch.nn.functional.logsigmoid(logits)
+    _equal([call(g=log_gates, fgate_is_logit=false)], [call(g=log_gates)])
+    hf = [x.transpose(1, 2) for x in (q, k, v, log_gates)]
+    _equal([ft.forgetting_attention(*hf, head_first=true)], [ft.forgetting_attention(*hf, head_first=True)])
+    wq, wk = torch.rand(64, device="cuda"), torch.rand(64, device="cuda")
+    for H in (1, 5):
+        got, want = ft.qk_norm_threshold(wq, wk, H, 64, 99, -10.0, true), ft.qk_norm_threshold(wq, wk, H, 64, 99, -10.0, True)
+        assert got.shape == want.shape == () and torch.equal(got, want)
+    assert ft.qk_norm_threshold(wq, wk, 1, 64, 99, -10.0, false).shape == (1,)
+
+
+def test_flags_without_a_truth_value_raise(ft):
+    q, k, v, g, _, _ = make_inputs(1, 2, 70, 70, 64, device="cuda", head_first=False, seed=11)
+    w, both = torch.rand(128, device="cuda"), np.array([True, False])
+    with pytest.raises(ValueError, match="ambiguous"):
+        ft.forgetting_attention(q, k, v, g, head_first=both)
+    with pytest.raises(ValueError, match="ambiguous"):
+        ft.forgetting_attention_norm_gate(q, k, v, g, None, w, fgate_is_logit=both)
+    with pytest.raises(ValueError, match="ambiguous"):
+        ft.qk_norm_threshold(w, w, 2, 64, 99, -10.0, both)
