@@ -271,7 +271,8 @@ def _fwd_workspace_bytes(B, H, M, N, D, dtype_code):
 
 @functools.lru_cache(maxsize=64)
 def _cached_constant_threshold(value, B, H, device):
-    t = torch.full((B, H), value, dtype=torch.float, device=device)
+    with torch.inference_mode(False):   # later calls may save it for a backward, which refuses inference tensors
+        t = torch.full((B, H), value, dtype=torch.float, device=device)
     # the fill has finished before the tensor enters the cache: whichever stream reads it later needs no ordering
     torch.cuda.current_stream(device).synchronize()
     return t

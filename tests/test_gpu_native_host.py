@@ -198,3 +198,17 @@ def test_flags_without_a_truth_value_raise(ft):
         ft.forgetting_attention_norm_gate(q, k, v, g, None, w, fgate_is_logit=both)
     with pytest.raises(ValueError, match="ambiguous"):
         ft.qk_norm_threshold(w, w, 2, 64, 99, -10.0, both)
+
+
+@pytest.mark.parametrize("thr", [-7.125, -7])   # values no other test uses: the first call with each is the one under inference mode
+def test_a_number_as_threshold_in_inference_mode_then_training(ft, thr):
+    """The (B, H) tensor made of a number serves later calls too: evaluating first must not leave a tensor training cannot save."""
+    F = import_module("forgetting_transformer.ops.forgetting_attention")
+    q, k, v, g, do, _ = make_inputs(1, 3, 150, 150, 64, device="cuda", head_first=True, seed=4, gate_mean=1.0)
+    with torch.inference_mode():
+        first = ft.forgetting_attention(q, k, v, g, head_first=True, adaptive_threshold=thr)
+    leaves = [x.requires_grad_() for x in (q, k, v, g)]
+    out = ft.forgetting_attention(*leaves, head_first=True, adaptive_threshold=thr)
+    assert torch.equal(out, first)
+    ref = F.ForgettingAttention.apply(*leaves, None, True, None, thr)
+    _equal(_grads(out, leaves, do), _grads(ref, leaves, do))
