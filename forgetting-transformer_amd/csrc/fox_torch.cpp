@@ -442,7 +442,8 @@ struct ShiftNode : public torch::autograd::Function<ShiftNode> {
 
 // ---------------------------------------------------------------------------------------------------------------
 // Python entry points (METH_FASTCALL: the arguments come as a plain array).  Each returns None when the call is not one it
-// handles.
+// handles.  The interpreter lock is free while they allocate, launch and build the graph: a launch may wait for room in a
+// queue, and threads that drive other streams or devices must not wait with it (the argument array keeps its objects alive).
 // ---------------------------------------------------------------------------------------------------------------
 const Tensor* tensor_of(PyObject* o) {
   if (!THPVariable_Check(o)) return nullptr;
@@ -535,14 +536,20 @@ bool parse_attention(Attention& a, const Tensor* q, const Tensor* k, const Tenso
 PyObject* finish_attention(Attention& a, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& gate,
                            const Tensor& weight) {
   variable_list out;
-  if (needs_graph({&q, &k, &v, &g, &gate, &weight})) {
-    out = AttentionNode::apply(q, k, v, g, some(gate), some(weight), &a);
-  } else {
-    const at::NoGradGuard no_grad;
-    if (decodes_from_gates(a)) return THPVariable_Wrap(run_decode(a, q, k, v, g));
-    Forward f = run_forward(a, q, k, v, g);
-    out.push_back(f.out);
-    if (a.is_logit) out.push_back(a.head_first ? f.log_fgate : f.log_fgate.transpose(1, 2));
+  {
+    const pybind11::gil_scoped_release no_gil;
+    if (needs_graph({&q, &k, &v, &g, &gate, &weight})) {
+      out = AttentionNode::apply(q, k, v, g, some(gate), some(weight), &a);
+    } else {
+      const at::NoGradGuard no_grad;
+      if (decodes_from_gates(a)) {
+        out.push_back(run_decode(a, q, k, v, g));
+      } else {
+        Forward f = run_forward(a, q, k, v, g);
+        out.push_back(f.out);
+        if (a.is_logit) out.push_back(a.head_first ? f.log_fgate : f.log_fgate.transpose(1, 2));
+      }
+    }
   }
   if (!a.is_logit) return THPVariable_Wrap(out[0]);
   PyObject* pair = PyTuple_New(2);
@@ -614,10 +621,18 @@ PyObject* py_norm(PyObject*, PyObject* const* o, Py_ssize_t n) {
   const int64_t width = x->size(-1);
   if (G < 1 || width % G || !head_dim_ok(width / G)) return none();
   if (w->dim() != 1 || w->size(0) != width || w->device() != x->device() || !w->is_floating_point()) return none();
-  if (needs_graph({x, &gate, w})) return THPVariable_Wrap(NormNode::apply(*x, some(gate), *w, (int64_t)act, eps, (int64_t)G));
-  const at::NoGradGuard no_grad;
-  Tensor rstd;
-  return THPVariable_Wrap(NormNode::run(*x, gate, w->detach().to(at::kFloat).contiguous(), (int)act, eps, G, rstd));
+  Tensor y;
+  {
+    const pybind11::gil_scoped_release no_gil;
+    if (needs_graph({x, &gate, w})) {
+      y = NormNode::apply(*x, some(gate), *w, (int64_t)act, eps, (int64_t)G);
+    } else {
+      const at::NoGradGuard no_grad;
+      Tensor rstd;
+      y = NormNode::run(*x, gate, w->detach().to(at::kFloat).contiguous(), (int)act, eps, G, rstd);
+    }
+  }
+  return THPVariable_Wrap(y);
   END_HANDLE_TH_ERRORS
 }
 
@@ -632,9 +647,17 @@ PyObject* py_token_shift(PyObject*, PyObject* const* o, Py_ssize_t n) {
   if (p->scalar_type() != at::kFloat || c->scalar_type() != at::kFloat || p->device() != x->device() || c->device() != x->device()) return none();
   if (p->sizes() != x->sizes().slice(0, 3) || c->sizes() != p->sizes() || p->strides() != c->strides() || !p->is_non_overlapping_and_dense())
     return none();
-  if (needs_graph({x, p, c})) return THPVariable_Wrap(ShiftNode::apply(*x, *p, *c));
-  const at::NoGradGuard no_grad;
-  return THPVariable_Wrap(ShiftNode::run(*x, *p, *c));
+  Tensor out;
+  {
+    const pybind11::gil_scoped_release no_gil;
+    if (needs_graph({x, p, c})) {
+      out = ShiftNode::apply(*x, *p, *c);
+    } else {
+      const at::NoGradGuard no_grad;
+      out = ShiftNode::run(*x, *p, *c);
+    }
+  }
+  return THPVariable_Wrap(out);
   END_HANDLE_TH_ERRORS
 }
 
@@ -654,10 +677,14 @@ PyObject* py_qk_norm_threshold(PyObject*, PyObject* const* o, Py_ssize_t n) {
   if (!q || !k || H < 1 || D < 1 || !(T > 0) || !on_current_gpu(*q) || k->device() != q->device() || q->dim() != 1 || q->sizes() != k->sizes() ||
       q->size(0) != (shared ? D : H * D) || q->scalar_type() != at::kFloat || k->scalar_type() != at::kFloat || !q->is_contiguous() || !k->is_contiguous())
     return none();
-  const at::NoGradGuard no_grad;
-  Tensor thr = shared ? at::empty({}, q->options()) : at::empty({H}, q->options());
-  check(fox_qk_norm_threshold(q->const_data_ptr<float>(), k->const_data_ptr<float>(), shared ? 1 : (int32_t)H, (int32_t)D, T, tolerance,
-                              thr.mutable_data_ptr<float>(), stream_of(*q)), "fox_qk_norm_threshold");
+  Tensor thr;
+  {
+    const pybind11::gil_scoped_release no_gil;
+    const at::NoGradGuard no_grad;
+    thr = shared ? at::empty({}, q->options()) : at::empty({H}, q->options());
+    check(fox_qk_norm_threshold(q->const_data_ptr<float>(), k->const_data_ptr<float>(), shared ? 1 : (int32_t)H, (int32_t)D, T, tolerance,
+                                thr.mutable_data_ptr<float>(), stream_of(*q)), "fox_qk_norm_threshold");
+  }
   return THPVariable_Wrap(thr);
   END_HANDLE_TH_ERRORS
 }
@@ -700,7 +727,10 @@ PyObject* py_cache_append(PyObject*, PyObject* const* o, Py_ssize_t n) {
   a.v_buf = view_of(vb, true);
   a.g_buf = gb.mutable_data_ptr<float>();
   a.g_buf_stride_b = gb.stride(0); a.g_buf_stride_h = gb.stride(1); a.g_buf_stride_n = gb.stride(2);
-  check(fox_cache_append(&a, stream_of(k)), "fox_cache_append");
+  {
+    const pybind11::gil_scoped_release no_gil;
+    check(fox_cache_append(&a, stream_of(k)), "fox_cache_append");
+  }
   PyObject* out = PyTuple_New(3);
   if (!out) return nullptr;
   for (int i = 0; i < 3; ++i) {

@@ -1,6 +1,7 @@
 """GPU tests of the native host path (csrc/fox_torch.cpp) against the general Python path, which the same inputs take through the
 autograd nodes directly: the two launch the same kernels, so every output and gradient must agree bit for bit, in both
 layouts, with every optional argument, and for inputs the native path hands back (tensors that need a copy first)."""
+import time
 from importlib import import_module
 
 import numpy as np
@@ -212,3 +213,57 @@ def test_a_number_as_threshold_in_inference_mode_then_training(ft, thr):
     assert torch.equal(out, first)
     ref = F.ForgettingAttention.apply(*leaves, None, True, None, thr)
     _equal(_grads(out, leaves, do), _grads(ref, leaves, do))
+
+
+def test_other_threads_run_while_an_operator_is_called(ft):
+    """The interpreter lock is free during allocation and launches.  With a switch interval that never expires, another thread gets
+    its turn only when the calling thread gives the lock up by itself; nothing else in the loops below does."""
+    import sys
+    import threading
+    q, k, v, g, _, _ = make_inputs(1, 2, 64, 64, 64, device="cuda", head_first=True, seed=2)
+    x, w, p = torch.randn(1, 64, 2, 64, device="cuda").bfloat16(), torch.rand(128, device="cuda"), torch.rand(1, 64, 2, device="cuda")
+    cache = [torch.zeros(1, 2, 128, 64, device="cuda").bfloat16(), torch.zeros(1, 2, 128, 64, device="cuda").bfloat16(),
+             torch.zeros(1, 2, 128, device="cuda")]
+    from forgetting_transformer.ops import _native
+    ext = _native.load()
+    x2 = x.view(1, 64, 128)
+    calls = {"attention": (ext.attention, (q, k, v, g, True, None, None, None, False)),
+             "decode": (ext.attention, (q[:, :, :1], k, v, g, True, None, None, None, False)),
+             "attention_norm_gate": (ext.attention_norm_gate, (q, k, v, g, None, w, 2, 1e-6, True, None, None, None, False)),
+             "norm": (ext.norm, (x2, None, w, 2, 1e-6, 2)), "token_shift": (ext.token_shift, (x, p, p)),
+             "qk_norm_threshold": (ext.qk_norm_threshold, (w, w, 2, 64, 99, -10.0, False)),
+             "cache_append": (ext.cache_append, (*cache, k, v, g, 0))}
+    interval, ready = sys.getswitchinterval(), threading.Event()
+    stuck = []
+    with torch.no_grad():
+        for name, (fn, args) in calls.items():
+            assert fn(*args) is not None, name
+            torch.cuda.synchronize()
+            turns, stop = [0], [False]
+            ready.clear()
+
+            def other():
+                ready.set()
+                while not stop[0]:
+                    turns[0] += 1
+                    time.sleep(0)       # gives the lock back after every turn
+
+            thread = threading.Thread(target=other)
+            try:
+                sys.setswitchinterval(1000.0)
+                thread.start()
+                ready.wait()
+                time.sleep(0.05)        # it waits for the lock by now, with the interval above
+                before = turns[0]
+                for _ in range(3000):
+                    fn(*args)
+                    if turns[0] > before:
+                        break
+                else:
+                    stuck.append(name)
+            finally:
+                stop[0] = True
+                sys.setswitchinterval(interval)
+                thread.join()
+            torch.cuda.synchronize()
+    assert not stuck, stuck
