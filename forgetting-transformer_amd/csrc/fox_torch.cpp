@@ -8,6 +8,7 @@
 // current device -- and the Python function then goes through its general path, which raises the documented errors.
 #include <ATen/TracerMode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/InferenceMode.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -445,12 +446,17 @@ struct ShiftNode : public torch::autograd::Function<ShiftNode> {
 // handles.  The interpreter lock is free while they allocate, launch and build the graph: a launch may wait for room in a
 // queue, and threads that drive other streams or devices must not wait with it (the argument array keeps its objects alive).
 // ---------------------------------------------------------------------------------------------------------------
+// Whether a function transform (vmap, grad, jvp, ...) is active on this thread.  The operators have no rules for them, and the
+// general path's autograd nodes refuse to run under one, whether or not their tensors are wrapped.
+bool under_transform() { return c10::impl::tls_local_dispatch_key_set().included_.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode); }
+
 const Tensor* tensor_of(PyObject* o) {
   if (!THPVariable_Check(o)) return nullptr;
   const Tensor& t = THPVariable_Unpack(o);
   // a subclass with its own dispatch and the wrappers of functional transforms have no plain storage; a dual tensor's tangent
   // and a trace would be lost: all of these go through the general path, which handles or refuses them
-  if (t.key_set().has(c10::DispatchKey::Python) || !t.has_storage() || t._fw_grad(0).defined() || at::tracer::impl::is_dispatch_enabled())
+  if (t.key_set().has(c10::DispatchKey::Python) || !t.has_storage() || t._fw_grad(0).defined() || at::tracer::impl::is_dispatch_enabled() ||
+      under_transform())
     return nullptr;
   return &t;
 }

@@ -267,3 +267,22 @@ def test_other_threads_run_while_an_operator_is_called(ft):
                 thread.join()
             torch.cuda.synchronize()
     assert not stuck, stuck
+
+
+def test_function_transforms_are_refused(ft):
+    """No operator has rules for functorch's transforms: a call under one raises, whether its tensors are the transformed ones or
+    are only closed over."""
+    q, k, v, g, _, _ = make_inputs(1, 2, 70, 70, 64, device="cuda", head_first=True, seed=3)
+    x, w, p = torch.randn(2, 30, 128, device="cuda").bfloat16(), torch.rand(128, device="cuda"), torch.rand(2, 30, 2, device="cuda")
+    x4 = x.view(2, 30, 2, 64)
+    calls = [lambda t: ft.forgetting_attention(q + t.to(q.dtype) if t is not None else q, k, v, g, head_first=True),
+             lambda t: ft.forgetting_attention_norm_gate(q + t.to(q.dtype) if t is not None else q, k, v, g, None, w, head_first=True),
+             lambda t: ft.group_norm(x + t.to(x.dtype) if t is not None else x, w, is_rms_norm=True, num_groups=2),
+             lambda t: ft.token_shift(x4 + t.to(x.dtype) if t is not None else x4, p, p)]
+    ts = torch.zeros(3, device="cuda")
+    for call in calls:
+        for used in (True, False):
+            with pytest.raises(RuntimeError, match="setup_context"):
+                torch.func.vmap(lambda t: call(t if used else None).sum() + t)(ts)
+            with pytest.raises(RuntimeError, match="setup_context"):
+                torch.func.grad(lambda t: call(t if used else None).float().sum() + t)(ts[0])
