@@ -451,9 +451,9 @@ struct ShiftNode : public torch::autograd::Function<ShiftNode> {
 bool under_transform() { return c10::impl::tls_local_dispatch_key_set().included_.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode); }
 
 const Tensor* tensor_of(PyObject* o) {
-  if (!THPVariable_Check(o)) return nullptr;
+  if (!THPVariable_CheckExact(o)) return nullptr;   // Tensor or Parameter: the general path's results keep other subclasses
   const Tensor& t = THPVariable_Unpack(o);
-  // a subclass with its own dispatch and the wrappers of functional transforms have no plain storage; a dual tensor's tangent
+  // tensors with a dispatch of their own and the wrappers of functional transforms have no plain storage; a dual tensor's tangent
   // and a trace would be lost: all of these go through the general path, which handles or refuses them
   if (t.key_set().has(c10::DispatchKey::Python) || !t.has_storage() || t._fw_grad(0).defined() || at::tracer::impl::is_dispatch_enabled() ||
       under_transform())

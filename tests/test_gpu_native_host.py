@@ -286,3 +286,22 @@ def test_function_transforms_are_refused(ft):
                 torch.func.vmap(lambda t: call(t if used else None).sum() + t)(ts)
             with pytest.raises(RuntimeError, match="setup_context"):
                 torch.func.grad(lambda t: call(t if used else None).float().sum() + t)(ts[0])
+
+
+class _Tagged(torch.Tensor):
+    """A subclass without a dispatch of its own: what torch calls __torch_function__ keeps the type."""
+
+
+def test_tensor_subclasses_keep_their_type(ft):
+    """As the general path does, a result laid out like a subclass instance is one."""
+    from forgetting_transformer.ops.token_shift import TokenShift
+    F = import_module("forgetting_transformer.ops.forgetting_attention")
+    q, k, v, g, _, _ = make_inputs(1, 2, 70, 70, 64, device="cuda", head_first=True, seed=3)
+    tagged = q.as_subclass(_Tagged)
+    out, ref = ft.forgetting_attention(tagged, k, v, g, head_first=True), F.ForgettingAttention.apply(tagged, k, v, g, None, True, None, None)
+    assert type(out) is type(ref) is _Tagged and torch.equal(out, ref)
+    x, p = q.transpose(1, 2).contiguous().as_subclass(_Tagged), torch.rand(1, 70, 2, device="cuda")
+    out, ref = ft.token_shift(x, p, p), TokenShift.apply(x, p, p)
+    assert type(out) is type(ref) is _Tagged and torch.equal(out, ref)
+    par = torch.nn.Parameter(q)
+    assert type(ft.forgetting_attention(par, k, v, g, head_first=True)) is torch.Tensor
