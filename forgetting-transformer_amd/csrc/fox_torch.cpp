@@ -446,9 +446,13 @@ struct ShiftNode : public torch::autograd::Function<ShiftNode> {
 // handles.  The interpreter lock is free while they allocate, launch and build the graph: a launch may wait for room in a
 // queue, and threads that drive other streams or devices must not wait with it (the argument array keeps its objects alive).
 // ---------------------------------------------------------------------------------------------------------------
-// Whether a function transform (vmap, grad, jvp, ...) is active on this thread.  The operators have no rules for them, and the
-// general path's autograd nodes refuse to run under one, whether or not their tensors are wrapped.
-bool under_transform() { return c10::impl::tls_local_dispatch_key_set().included_.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode); }
+// Whether this thread runs under a function transform (vmap, grad, jvp, ...) or a Python dispatch mode.  The operators have no
+// rules for transforms, and the general path's autograd nodes refuse to run under one, whether or not their tensors are wrapped;
+// a mode sees, replaces or refuses the tensor operations of the general path.
+bool under_transform_or_mode() {
+  const auto keys = c10::impl::tls_local_dispatch_key_set().included_;
+  return keys.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || keys.has(c10::DispatchKey::Python);
+}
 
 const Tensor* tensor_of(PyObject* o) {
   if (!THPVariable_CheckExact(o)) return nullptr;   // Tensor or Parameter: the general path's results keep other subclasses
@@ -456,7 +460,7 @@ const Tensor* tensor_of(PyObject* o) {
   // tensors with a dispatch of their own and the wrappers of functional transforms have no plain storage; a dual tensor's tangent
   // and a trace would be lost: all of these go through the general path, which handles or refuses them
   if (t.key_set().has(c10::DispatchKey::Python) || !t.has_storage() || t._fw_grad(0).defined() || at::tracer::impl::is_dispatch_enabled() ||
-      under_transform())
+      under_transform_or_mode())
     return nullptr;
   return &t;
 }

@@ -305,3 +305,22 @@ def test_tensor_subclasses_keep_their_type(ft):
     assert type(out) is type(ref) is _Tagged and torch.equal(out, ref)
     par = torch.nn.Parameter(q)
     assert type(ft.forgetting_attention(par, k, v, g, head_first=True)) is torch.Tensor
+
+
+def test_dispatch_modes_see_the_calls_operations(ft):
+    """Under a dispatch mode the general path runs, whose allocations and copies the mode can see, refuse or replace."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Names(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    cache, names = ft.FgateDynamicCache(max_length=8), []
+    new = [torch.randn(1, 2, 3, 64, device="cuda").bfloat16() for _ in range(2)] + [torch.randn(1, 2, 3, device="cuda")]
+    cache.update(*new, 0)
+    with Names():
+        got = cache.update(*new, 0)
+    assert sum("copy_" in n for n in names) == 3
+    for a, b in zip(got, new):
+        assert torch.equal(a, torch.cat([b, b], dim=2))
