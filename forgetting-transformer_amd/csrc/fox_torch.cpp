@@ -318,7 +318,9 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
     if (!grads[0].defined()) return variable_list(7);
     Tensor d_o = grads[0], dgate, dweight;
     if (s[9].defined()) {   // the norm's backward first: its dx is the gradient of o
-      const Tensor &gate = s[8], dy = make_heads_adjacent(grads[0], a.head_first);
+      // (saved-tensor hooks may hand o and the gate back in another layout)
+      const Tensor o = make_heads_adjacent(s[4], a.head_first), dy = make_heads_adjacent(grads[0], a.head_first);
+      const Tensor gate = s[8].defined() ? make_heads_adjacent(s[8], a.head_first) : Tensor();
       auto rows_like = [&](void) {
         Tensor t = at::empty({a.B, a.M, a.H, a.D}, q.options());
         return a.head_first ? t.transpose(1, 2) : t;
@@ -326,7 +328,7 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
       d_o = rows_like();
       if (gate.defined()) dgate = rows_like();
       Tensor dw;
-      run_norm_backward(s[4], gate, s[9], s[10], dy, a.B * a.M, a.H, a.D, (int)d["act"].toInt(), d["eps"].toDouble(), d_o, dgate, dw);
+      run_norm_backward(o, gate, s[9], s[10], dy, a.B * a.M, a.H, a.D, (int)d["act"].toInt(), d["eps"].toDouble(), d_o, dgate, dw);
       dweight = dw.to((at::ScalarType)d["wtype"].toInt());
     }
     variable_list r = run_backward(a, q, k, s[2], s[3], s[4], s[5], d_o);

@@ -228,7 +228,8 @@ class ForgettingAttentionNormGate(torch.autograd.Function):
         B, H, M, D = q.shape
         rows, width = B * M, H * D
         lib = _lib.load()
-        dy = _heads_adjacent(dy)
+        dy, o = _heads_adjacent(dy), _heads_adjacent(o)   # (saved-tensor hooks may hand o and the gate back in another layout)
+        gate = _heads_adjacent(gate) if gated else None
         do = torch.empty((B, M, H, D), dtype=q.dtype, device=q.device).transpose(1, 2)
         dgate = torch.empty((B, M, H, D), dtype=q.dtype, device=q.device).transpose(1, 2) if gated else None
         dw = torch.empty((width,), dtype=torch.float32, device=q.device)

@@ -324,3 +324,36 @@ def test_dispatch_modes_see_the_calls_operations(ft):
     assert sum("copy_" in n for n in names) == 3
     for a, b in zip(got, new):
         assert torch.equal(a, torch.cat([b, b], dim=2))
+
+
+def _repacked(t):   # as a copy to pinned host memory and back leaves it: the values, in a plain contiguous tensor
+    return torch.empty(t.shape, dtype=t.dtype, device=t.device).copy_(t)
+
+
+@pytest.mark.parametrize("head_first", [True, False])
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("general", [True, False])
+def test_saved_tensors_that_come_back_in_another_layout(ft, head_first, gated, general):
+    """Saved-tensor hooks may hand back tensors with other strides: the gradients are the same."""
+    from forgetting_transformer.ops import _lib
+    F = import_module("forgetting_transformer.ops.forgetting_attention")
+    B, H, T, D = 2, 3, 90, 32
+    swap = (lambda x: x.transpose(1, 2)) if head_first else (lambda x: x)
+    q, k, v, gate, do = (swap(torch.randn(B, T, H, D, device="cuda").bfloat16()) for _ in range(5))
+    logits, w = swap(torch.randn(B, T, H, device="cuda") + 2), torch.rand(H * D, device="cuda") + 0.5
+    leaves = [x.requires_grad_() for x in (q, k, v, logits, w) + ((gate,) if gated else ())]
+
+    def grads():
+        if general:
+            hf = [x if head_first else x.transpose(1, 2) for x in (q, k, v, logits, gate)]
+            y = F.ForgettingAttentionNormGate.apply(*hf[:4], hf[4] if gated else None, w, None, None, None,
+                                                    _lib.ACT_SIGMOID if gated else _lib.ACT_NONE, 1e-6, True)[0]
+            y = y if head_first else y.transpose(1, 2)
+        else:
+            y = ft.forgetting_attention_norm_gate(q, k, v, logits, gate if gated else None, w, head_first=head_first, fgate_is_logit=True)[0]
+        return lambda: torch.autograd.grad(y, leaves, do)
+
+    want = grads()()
+    with torch.autograd.graph.saved_tensors_hooks(_repacked, lambda t: t):
+        later = grads()
+    _equal(later(), want)
