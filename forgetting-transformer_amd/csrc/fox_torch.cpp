@@ -279,6 +279,11 @@ Tensor make_heads_adjacent(const Tensor& t, bool head_first) {
   return c.copy_(t);
 }
 
+// Saved-tensor hooks may hand a tensor back with other strides than it was saved with; each backward brings what it reads into
+// the layout that its kernel assumes.
+Tensor packed(const Tensor& t) { return t.defined() ? t.contiguous() : t; }
+Tensor vectors(const Tensor& t) { return vectors_ok(t) ? t : t.contiguous(); }
+
 struct AttentionNode : public torch::autograd::Function<AttentionNode> {
   static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g,
                                const std::optional<Tensor>& gate, const std::optional<Tensor>& weight, Attention* a) {
@@ -302,7 +307,7 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
     auto& d = ctx->saved_data;
-    const Tensor &q = s[0], &k = s[1];
+    const Tensor q = vectors(s[0]), k = vectors(s[1]), v = vectors(s[2]);
     Attention a;
     a.head_first = d["hf"].toBool();
     a.is_logit = d["logit"].toBool();
@@ -312,13 +317,12 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
     a.M = q.size(a.head_first ? 2 : 1);
     a.N = k.size(a.head_first ? 2 : 1);
     a.D = q.size(3);
-    a.seq_start = s[6];
-    a.threshold = s[7];
+    a.seq_start = packed(s[6]);
+    a.threshold = packed(s[7]);
     const c10::DeviceGuard guard(q.device());
     if (!grads[0].defined()) return variable_list(7);
     Tensor d_o = grads[0], dgate, dweight;
     if (s[9].defined()) {   // the norm's backward first: its dx is the gradient of o
-      // (saved-tensor hooks may hand o and the gate back in another layout)
       const Tensor o = make_heads_adjacent(s[4], a.head_first), dy = make_heads_adjacent(grads[0], a.head_first);
       const Tensor gate = s[8].defined() ? make_heads_adjacent(s[8], a.head_first) : Tensor();
       auto rows_like = [&](void) {
@@ -328,10 +332,10 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
       d_o = rows_like();
       if (gate.defined()) dgate = rows_like();
       Tensor dw;
-      run_norm_backward(o, gate, s[9], s[10], dy, a.B * a.M, a.H, a.D, (int)d["act"].toInt(), d["eps"].toDouble(), d_o, dgate, dw);
+      run_norm_backward(o, gate, packed(s[9]), packed(s[10]), dy, a.B * a.M, a.H, a.D, (int)d["act"].toInt(), d["eps"].toDouble(), d_o, dgate, dw);
       dweight = dw.to((at::ScalarType)d["wtype"].toInt());
     }
-    variable_list r = run_backward(a, q, k, s[2], s[3], s[4], s[5], d_o);
+    variable_list r = run_backward(a, q, k, v, s[3], vectors(s[4]), packed(s[5]), d_o);
     return {r[0], r[1], r[2], r[3], dgate, dweight, Tensor()};
   }
 };
@@ -382,14 +386,14 @@ struct NormNode : public torch::autograd::Function<NormNode> {
     const variable_list s = ctx->get_saved_variables();
     auto& d = ctx->saved_data;
     if (!grads[0].defined()) return variable_list(6);
-    const Tensor &x = s[0], &gate = s[1];
+    const Tensor x = packed(s[0]), gate = packed(s[1]);
     const c10::DeviceGuard guard(x.device());
     const int64_t G = d["G"].toInt(), width = x.size(-1);
     Tensor dy = grads[0];
     if (!dy.is_contiguous() || !vectors_ok(dy)) dy = dy.contiguous();
     Tensor dx = at::empty_like(x), dg, dw;
     if (gate.defined()) dg = at::empty_like(gate);
-    run_norm_backward(x, gate, s[2], s[3], dy, x.numel() / width, G, width / G, (int)d["act"].toInt(), d["eps"].toDouble(), dx, dg, dw);
+    run_norm_backward(x, gate, packed(s[2]), packed(s[3]), dy, x.numel() / width, G, width / G, (int)d["act"].toInt(), d["eps"].toDouble(), dx, dg, dw);
     return {dx, dg, dw.to((at::ScalarType)d["wtype"].toInt()), Tensor(), Tensor(), Tensor()};
   }
 };
@@ -427,13 +431,16 @@ struct ShiftNode : public torch::autograd::Function<ShiftNode> {
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
     if (!grads[0].defined()) return variable_list(3);
-    const Tensor& x = s[0];
+    // one set of strides for x, dout and dx, one for the weights and their gradients
+    const Tensor x = s[0].is_non_overlapping_and_dense() ? vectors(s[0]) : s[0].contiguous();
+    const bool weights_ok = s[1].strides() == s[2].strides() && s[1].is_non_overlapping_and_dense();
+    const Tensor prev_w = weights_ok ? s[1] : s[1].contiguous(), curr_w = weights_ok ? s[2] : s[2].contiguous();
     const c10::DeviceGuard guard(x.device());
     Tensor dout = grads[0];
     if (dout.strides() != x.strides() || (reinterpret_cast<uintptr_t>(dout.const_data_ptr()) & 15))
-      dout = at::empty_like(x).copy_(dout);   // the kernels share one set of strides
-    Tensor dx = at::empty_like(x), dprev = at::empty_like(s[1]), dcurr = at::empty_like(s[2]);
-    fox_shift_args a = args(x, s[1], s[2]);
+      dout = at::empty_like(x).copy_(dout);
+    Tensor dx = at::empty_like(x), dprev = at::empty_like(prev_w), dcurr = at::empty_like(curr_w);
+    fox_shift_args a = args(x, prev_w, curr_w);
     a.dout = dout.const_data_ptr();
     a.dx = dx.mutable_data_ptr();
     a.dprev_weight = dprev.mutable_data_ptr<float>();

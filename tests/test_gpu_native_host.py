@@ -357,3 +357,46 @@ def test_saved_tensors_that_come_back_in_another_layout(ft, head_first, gated, g
     with torch.autograd.graph.saved_tensors_hooks(_repacked, lambda t: t):
         later = grads()
     _equal(later(), want)
+
+
+def _padded(t):       # the values, with gaps behind every row
+    if t.dim() < 2:
+        return t
+    return torch.empty((*t.shape[:-1], t.shape[-1] + 8), dtype=t.dtype, device=t.device)[..., :t.shape[-1]].copy_(t)
+
+
+def _turned(t):       # the values, with the last axis outermost in memory
+    return torch.empty((t.shape[-1], *t.shape[:-1]), dtype=t.dtype, device=t.device).movedim(0, -1).copy_(t) if t.dim() > 1 else t
+
+
+def _some_turned(t):  # of tensors with the same shape only every second one
+    _some_turned.calls = getattr(_some_turned, "calls", 0) + 1
+    return _turned(t) if _some_turned.calls % 2 else t
+
+
+@pytest.mark.parametrize("pack", [_repacked, _padded, _turned, _some_turned])
+@pytest.mark.parametrize("head_first", [True, False])
+def test_every_backward_with_saved_tensors_in_other_layouts(ft, pack, head_first):
+    B, T, H, D = 2, 45, 3, 32
+    rnd = lambda *s: torch.randn(*s, device="cuda").bfloat16().requires_grad_()
+    x, gate, k, v = rnd(B, T, H * D), rnd(B, T, H * D), rnd(B, T, H, D), rnd(B, T, H, D)
+    w, p, c = torch.rand(H * D, device="cuda", requires_grad=True), *(torch.rand(B, T, H, device="cuda", requires_grad=True) for _ in range(2))
+    logits, do = torch.randn(B, T, H, device="cuda", requires_grad=True), torch.randn(B, T, H, D, device="cuda").bfloat16()
+    thr, ss = torch.full((B, H), -9.0, device="cuda"), torch.tensor([0, 7], device="cuda")
+    leaves = [x, gate, k, v, w, p, c, logits]
+
+    def grads():
+        q = ft.group_norm_gated(x, gate, w, is_rms_norm=True, num_groups=H).view(B, T, H, D)
+        ks = ft.token_shift(k, p, c)
+        if head_first:
+            out, _ = ft.forgetting_attention_from_logits(q.transpose(1, 2), ks.transpose(1, 2), v.transpose(1, 2), logits.transpose(1, 2),
+                                                         head_first=True, seq_start=ss, adaptive_threshold=thr)
+            out = out.transpose(1, 2)
+        else:
+            out = ft.forgetting_attention(q, ks, v, torch.nn.functional.logsigmoid(logits), seq_start=ss, adaptive_threshold=thr)
+        return lambda: torch.autograd.grad(out, leaves, do)
+
+    want = grads()()
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+        later = grads()
+    _equal(later(), want)
