@@ -16,6 +16,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/extension.h>
 
+#include <atomic>
 #include <cmath>
 #include <optional>
 
@@ -183,6 +184,26 @@ Tensor run_decode(const Attention& a, const Tensor& q, const Tensor& k, const Te
   return out;
 }
 
+// The list that takes the pruning bounds of every backward while record_pruning_bounds() is active; the interpreter lock guards it.
+PyObject* g_bounds = nullptr;
+std::atomic<bool> g_bounds_on{false};
+
+// Room for the bounds of one backward, handed to the kernels and to the list.
+void record_bounds(const Attention& a, const Tensor& q, fox_bwd_args& args) {
+  int32_t block_m = 0, block_n = 0, kv_n = 0, kv_m = 0;
+  check(fox_tile_config(args.dims.D, &block_m, &block_n, &kv_n, &kv_m), "fox_tile_config");
+  const auto ints = q.options().dtype(at::kInt);
+  Tensor first = at::zeros({a.B, a.H, (a.M + block_m - 1) / block_m}, ints), end = at::full({a.B, a.H, (a.N + 63) / 64}, -1, ints);
+  const pybind11::gil_scoped_acquire gil;
+  if (!g_bounds) return;
+  args.q_first_block = first.mutable_data_ptr<int32_t>();
+  args.kv_end_row = end.mutable_data_ptr<int32_t>();
+  pybind11::dict d;
+  d["dq_first_block"] = pybind11::reinterpret_steal<pybind11::object>(THPVariable_Wrap(first));
+  d["kv_end_row"] = pybind11::reinterpret_steal<pybind11::object>(THPVariable_Wrap(end));
+  pybind11::reinterpret_borrow<pybind11::list>(g_bounds).append(d);   // (keeps both tensors alive past the launches)
+}
+
 // dq, dk, dv and the gradient of the gates, in the layout of the inputs
 variable_list run_backward(const Attention& a, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& o,
                            const Tensor& rows, Tensor d_o) {
@@ -215,6 +236,7 @@ variable_list run_backward(const Attention& a, const Tensor& q, const Tensor& k,
   args.delta = t;
   args.drow = t + n_l;
   args.dlog_lambda = t + 2 * n_l;
+  if (a.threshold.defined() && g_bounds_on.load(std::memory_order_relaxed)) record_bounds(a, q, args);
   if (!a.is_logit) {
     args.dlog_fgate = dg.mutable_data_ptr<float>();
     args.dlog_fgate_stride_b = dg.stride(0);
@@ -760,7 +782,22 @@ PyObject* py_cache_append(PyObject*, PyObject* const* o, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// record_bounds(list or None)
+PyObject* py_record_bounds(PyObject*, PyObject* list) {
+  if (list != Py_None && !PyList_Check(list)) {
+    PyErr_SetString(PyExc_TypeError, "record_bounds takes a list or None");
+    return nullptr;
+  }
+  PyObject* old = g_bounds;
+  g_bounds = list == Py_None ? nullptr : list;
+  Py_XINCREF(g_bounds);
+  g_bounds_on.store(g_bounds != nullptr, std::memory_order_relaxed);
+  Py_XDECREF(old);
+  Py_RETURN_NONE;
+}
+
 PyMethodDef methods[] = {
+    {"record_bounds", (PyCFunction)py_record_bounds, METH_O, nullptr},
     {"cache_append", (PyCFunction)(void (*)(void))py_cache_append, METH_FASTCALL, nullptr},
     {"qk_norm_threshold", (PyCFunction)(void (*)(void))py_qk_norm_threshold, METH_FASTCALL, nullptr},
     {"attention", (PyCFunction)(void (*)(void))py_attention, METH_FASTCALL, nullptr},

@@ -15,6 +15,7 @@ from ._lib import LIB_PATH
 EXT_PATH = LIB_PATH.with_name("_fox_torch.so")
 
 _ext = None
+_bounds = None   # the list of an active record_pruning_bounds()
 _lock = threading.Lock()
 
 
@@ -32,5 +33,15 @@ def load():
             spec = importlib.util.spec_from_loader("_fox_torch", loader)
             module = importlib.util.module_from_spec(spec)
             loader.exec_module(module)
+            module.record_bounds(_bounds)
             _ext = module
     return _ext
+
+
+def record_bounds(records) -> None:
+    """Have the native nodes' backwards add their pruning bounds to ``records`` (None: to nothing)."""
+    global _bounds
+    with _lock:
+        _bounds = records
+        if _ext is not None:
+            _ext.record_bounds(records)

@@ -87,10 +87,12 @@ def record_pruning_bounds():
     query row where the dK/dV walk below them stops).  Not thread-safe; meant for tests and diagnostics."""
     global _bound_records
     prev, _bound_records = _bound_records, []
+    _native.record_bounds(_bound_records)   # for backwards whose forward ran before the block
     try:
         yield _bound_records
     finally:
         _bound_records = prev
+        _native.record_bounds(prev)
 
 
 _current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)   # the binding without its Python wrappers

@@ -400,3 +400,26 @@ def test_every_backward_with_saved_tensors_in_other_layouts(ft, pack, head_first
     with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
         later = grads()
     _equal(later(), want)
+
+
+@pytest.mark.parametrize("head_first", [True, False])
+def test_bounds_of_a_backward_whose_forward_ran_before_the_recording(ft, head_first):
+    """record_pruning_bounds collects every backward made inside the block, whichever path its forward took."""
+    F = import_module("forgetting_transformer.ops.forgetting_attention")
+    B, H, T, D = 1, 2, 700, 64
+    q, k, v, g, do, _ = make_inputs(B, H, T, T, D, device="cuda", head_first=head_first, seed=6, gate_mean=-1.0)
+    leaves = [x.requires_grad_() for x in (q, k, v, g)]
+    call = lambda: ft.forgetting_attention(*leaves, head_first=head_first, adaptive_threshold=-12.0)
+    with F.record_pruning_bounds() as want:
+        torch.autograd.grad(call(), leaves, do)
+    out = call()
+    with F.record_pruning_bounds() as got:
+        torch.autograd.grad(out, leaves, do, retain_graph=True)
+    torch.autograd.grad(out, leaves, do)          # after the block: nothing is recorded
+    assert len(want) == 2 and len(got) == 1 and set(got[0]) == {"dq_first_block", "kv_end_row"}
+    for name, t in got[0].items():
+        assert t.dtype == torch.int32 and torch.equal(t, want[1][name])
+    plain = ft.forgetting_attention(*leaves, head_first=head_first)
+    with F.record_pruning_bounds() as got:       # no threshold, no bounds
+        torch.autograd.grad(plain, leaves, do)
+    assert got == []
