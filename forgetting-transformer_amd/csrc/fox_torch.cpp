@@ -707,6 +707,8 @@ PyObject* py_qk_norm_threshold(PyObject*, PyObject* const* o, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK(n == 7, "qk_norm_threshold takes 7 arguments");
   const Tensor *q = tensor_of(o[0]), *k = tensor_of(o[1]);
+  // (a tensor as tolerance would have to be read back from the device here; the general path adds it)
+  if (!PyFloat_Check(o[5]) && !PyLong_Check(o[5])) return none();
   const long H = PyLong_AsLong(o[2]), D = PyLong_AsLong(o[3]);
   const double T = PyFloat_AsDouble(o[4]), tolerance = PyFloat_AsDouble(o[5]);
   if (PyErr_Occurred()) {

@@ -2,6 +2,7 @@
 autograd nodes directly: the two launch the same kernels, so every output and gradient must agree bit for bit, in both
 layouts, with every optional argument, and for inputs the native path hands back (tensors that need a copy first)."""
 import time
+import warnings
 from importlib import import_module
 
 import numpy as np
@@ -423,3 +424,23 @@ def test_bounds_of_a_backward_whose_forward_ran_before_the_recording(ft, head_fi
     with F.record_pruning_bounds() as got:       # no threshold, no bounds
         torch.autograd.grad(plain, leaves, do)
     assert got == []
+
+
+def test_qk_norm_threshold_with_a_tensor_tolerance(ft):
+    """A tolerance that is a tensor is added as one: per head, without waiting for the device, and under stream capture."""
+    H, D = 4, 64
+    wq, wk = torch.randn(H * D, device="cuda"), torch.randn(H * D, device="cuda")
+    base = ft.qk_norm_threshold(wq, wk, H, D, 512, 0.0)
+    tol = torch.tensor(-10.0, device="cuda")
+    rows = torch.linspace(-12, -9, H, device="cuda")
+    assert torch.equal(ft.qk_norm_threshold(wq, wk, H, D, 512, rows), base + rows)
+    mode = torch.cuda.get_sync_debug_mode()
+    torch.cuda.set_sync_debug_mode("warn")
+    try:
+        with warnings.catch_warnings(record=True) as seen:
+            warnings.simplefilter("always")
+            got = ft.qk_norm_threshold(wq, wk, H, D, 512, tol)
+    finally:
+        torch.cuda.set_sync_debug_mode(mode)
+    assert torch.equal(got, base + tol) and not [w for w in seen if "synchroniz" in str(w.message)]
+    assert torch.equal(ft.qk_norm_threshold(wq, wk, H, D, 512, np.float32(-10.0)), base + tol)
