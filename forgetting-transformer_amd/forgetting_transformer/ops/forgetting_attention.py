@@ -648,10 +648,11 @@ def qk_norm_threshold(q_norm_weight: torch.Tensor, k_norm_weight: torch.Tensor, 
     ``forgetting_attention`` broadcasts over the batch; with ``share_param_across_head`` the weights are
     ``(head_dim,)`` and the result is a 0-d tensor.  No pass over q and k is needed (unlike ``"auto"``).
     """
-    thr = _native.load().qk_norm_threshold(q_norm_weight, k_norm_weight, num_heads, head_dim, seq_len, log_pruning_tolerance,
-                                           share_param_across_head)
-    if thr is not None:
-        return thr
+    if q_norm_weight.is_cuda:   # (on the host the rule needs no library)
+        thr = _native.load().qk_norm_threshold(q_norm_weight, k_norm_weight, num_heads, head_dim, seq_len, log_pruning_tolerance,
+                                               share_param_across_head)
+        if thr is not None:
+            return thr
     return _qk_norm_threshold_general(q_norm_weight, k_norm_weight, num_heads, head_dim, seq_len, log_pruning_tolerance,
                                       share_param_across_head)
 

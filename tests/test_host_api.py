@@ -368,3 +368,16 @@ def test_noalloc_rejects_shapes_beyond_its_array():
     args = _lib.FwdArgs(dims)
     rc = lib.fox_attn_fwd_noalloc(C.byref(args), None)
     assert rc == -1 and b"64" in lib.fox_last_error() and b"scratch" in lib.fox_last_error()
+
+
+def test_qk_norm_threshold_on_the_host_needs_no_library(monkeypatch):
+    """The rule in tensor operations, wherever the weights live; a checkout that is not built (or a torch without HIP) has it too."""
+    import forgetting_transformer as ft
+    from forgetting_transformer.ops import _native
+    monkeypatch.setattr(_native, "_ext", None)
+    monkeypatch.setattr(_native, "EXT_PATH", _native.EXT_PATH.with_name("absent.so"))
+    w = torch.linspace(-2.0, 1.0, 32)
+    got = ft.qk_norm_threshold(w, w, 2, 16, 100, -10.0)
+    top = w.view(2, 16).abs().amax(-1).double()
+    want = -(2 * top * top * 4.0 + math.log(100)) - 10.0
+    assert torch.allclose(got.double(), want, rtol=1e-6, atol=0)     # five fp32 operations, 6e-8 each
