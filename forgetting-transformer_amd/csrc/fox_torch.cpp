@@ -552,6 +552,7 @@ bool parse_attention(Attention& a, const Tensor* q, const Tensor* k, const Tenso
     } else {
       const Tensor* t = tensor_of(threshold);
       if (!t || t->scalar_type() != at::kFloat || t->device() != q->device() || t->dim() > 2) return false;
+      if (at::GradMode::is_enabled() && t->requires_grad()) return false;   // an input of the node there, with no gradient
       if (t->dim() == 2 && t->size(0) == a.B && t->size(1) == a.H && t->is_contiguous()) {
         a.threshold = t->detach();
       } else {

@@ -444,3 +444,14 @@ def test_qk_norm_threshold_with_a_tensor_tolerance(ft):
         torch.cuda.set_sync_debug_mode(mode)
     assert torch.equal(got, base + tol) and not [w for w in seen if "synchroniz" in str(w.message)]
     assert torch.equal(ft.qk_norm_threshold(wq, wk, H, D, 512, np.float32(-10.0)), base + tol)
+
+
+@pytest.mark.parametrize("M", [1, 70])
+def test_a_threshold_that_requires_grad(ft, M):
+    """A trainable threshold has no gradient but makes the result part of a graph: backward runs and leaves it without one."""
+    q, k, v, g, do, _ = make_inputs(1, 2, M, 70, 64, device="cuda", head_first=True, seed=3)
+    thr = torch.full((2,), -20.0, device="cuda", requires_grad=True)
+    out = ft.forgetting_attention(q, k, v, g, head_first=True, adaptive_threshold=thr)
+    assert out.requires_grad and torch.autograd.grad(out, [thr], do, allow_unused=True) == (None,)
+    with torch.no_grad():
+        assert torch.equal(ft.forgetting_attention(q, k, v, g, head_first=True, adaptive_threshold=thr), out)
