@@ -221,6 +221,23 @@ int make_norm_gate(const fox_norm_gate_args* a, fox::NormGateK& k, bool bwd) {
   return FOX_OK;
 }
 
+// What the forward does with a shape: the key splits its size asks for (only with scratch to hold their partial results), and whether
+// it runs as the paired kernel, which takes the place of the splits.
+struct FwdPlan {
+  int wanted, splits;
+  bool pair;
+};
+FwdPlan plan_fwd(const fox_dims& d, bool pruned, bool scratch) {
+  FwdPlan p;
+  p.wanted = scratch ? fox::fwd_key_splits(d.B, d.H, d.M, d.N) : 1;
+  p.pair = fox::fwd_pairs(d.B, d.H, d.M, d.N, d.D, pruned, p.wanted);
+  p.splits = p.pair ? 1 : p.wanted;
+  return p;
+}
+int64_t split_bytes(const fox_dims& d, int splits) {
+  return splits <= 1 ? 0 : (int64_t)splits * d.B * d.H * d.M * (d.D + 2) * (int64_t)sizeof(float);
+}
+
 // The forward with its key-split scratch passed separately: the caller's workspace (fox_attn_fwd) or the
 // library's own array (fox_attn_fwd_noalloc).  workspace == NULL never splits keys.
 // epi: the norm-and-gate epilogue (already validated), or NULL.  With an epilogue, shapes the unsplit kernel does
@@ -250,22 +267,20 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
   k.n_mtiles = (args->dims.M + fox::kFwdBM - 1) / fox::kFwdBM;
   k.groups = fox::order_groups(k.B * k.H, k.M, k.N, args->dims.D);
   k.even = fox::even_tiles(k.M, k.N);
-  k.splits = 1;
+  const FwdPlan plan = plan_fwd(args->dims, k.thr != nullptr, workspace != nullptr);
+  k.splits = plan.splits;
+  k.pair = plan.pair;
   k.stream = k.n_mtiles == 1 && (int64_t)k.B * k.H * k.N * args->dims.D * 4 >= g_stream_min_kv_bytes.load(std::memory_order_relaxed);
   if (workspace) {
-    const int splits = fox::fwd_key_splits(k.B, k.H, k.M, k.N);
-    const int64_t need = splits <= 1 ? 0 : (int64_t)splits * k.B * k.H * k.M * (args->dims.D + 2) * (int64_t)sizeof(float);
+    const int64_t need = split_bytes(args->dims, plan.wanted);
     if (need > 0) {
       if (workspace_bytes < need) return fail(FOX_E_ARG, "workspace too small: %lld < %lld bytes", (long long)workspace_bytes, (long long)need);
       if (((uintptr_t)workspace & 15) != 0) return fail(FOX_E_ALIGN, "workspace must be 16-byte aligned");
-      k.splits = splits;
       k.ws_o = (float*)workspace;
       k.ws_ml = k.ws_o + (int64_t)k.splits * k.B * k.H * k.M * args->dims.D;
     }
   }
-  const bool split_shape = k.M == 1 || k.splits > 1;
-  k.pair = fox::fwd_pairs(k.B, k.H, k.M, k.N, args->dims.D, k.thr != nullptr, k.splits);
-  if (k.pair) k.splits = 1;
+  const bool split_shape = k.M == 1 || plan.wanted > 1;
   if (epi) {
     const int D = args->dims.D;
     if (split_shape) {
@@ -428,8 +443,16 @@ int fox_qk_norm_threshold(const float* q_weight, const float* k_weight, int32_t 
 int fox_attn_fwd_workspace_bytes(const fox_dims* dims, int64_t* bytes) {
   FOX_TRY(check_dims(dims));
   if (!bytes) return fail(FOX_E_ARG, "bytes is NULL");
-  const int splits = fox::fwd_key_splits(dims->B, dims->H, dims->M, dims->N);
-  *bytes = splits <= 1 ? 0 : (int64_t)splits * dims->B * dims->H * dims->M * (dims->D + 2) * (int64_t)sizeof(float);
+  *bytes = split_bytes(*dims, fox::fwd_key_splits(dims->B, dims->H, dims->M, dims->N));
+  return FOX_OK;
+}
+
+int fox_attn_fwd_plan(const fox_dims* dims, int32_t pruned, int32_t* key_splits, int32_t* paired, int64_t* workspace_bytes) {
+  FOX_TRY(check_dims(dims));
+  const FwdPlan p = plan_fwd(*dims, pruned != 0, true);
+  if (key_splits) *key_splits = p.splits;
+  if (paired) *paired = p.pair;
+  if (workspace_bytes) *workspace_bytes = split_bytes(*dims, p.splits);
   return FOX_OK;
 }
 

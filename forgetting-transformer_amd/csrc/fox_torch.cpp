@@ -82,7 +82,7 @@ struct Attention {   // one call, in the caller's layout
 struct Forward {     // what a forward leaves behind
   Tensor out;        // o, or y with an epilogue
   Tensor o, log_fgate, rstd;
-  Tensor rows;       // fp32: log_lambda (B,H,N), then at lse_at() the log-normaliser (B,H,M), then key-split scratch
+  Tensor rows;       // fp32: log_lambda (B,H,N), then at lse_at() the log-normaliser (B,H,M)
 };
 
 int64_t lse_at(const Attention& a) { return (a.B * a.H * a.N + 3) / 4 * 4; }
@@ -107,11 +107,13 @@ Forward run_forward(Attention& a, const Tensor& q, const Tensor& k, const Tensor
     check(fox_auto_threshold(&dims, &qv, &kv, (float)a.sm_scale, a.threshold.mutable_data_ptr<float>(),
                              (uint32_t*)scratch.mutable_data_ptr(), stream), "fox_auto_threshold");
   }
-  // log_lambda (B,H,N), the log-normaliser (B,H,M) and the key-split scratch come from one allocation
+  // log_lambda (B,H,N) and the log-normaliser (B,H,M) come from one allocation, which the backward keeps; key splits have their own
   int64_t ws_bytes = 0;
-  check(fox_attn_fwd_workspace_bytes(&dims, &ws_bytes), "fox_attn_fwd_workspace_bytes");
-  const int64_t at_l = lse_at(a), at_ws = at_l + (a.B * a.H * a.M + 3) / 4 * 4;   // (the scratch stays 16-byte aligned)
-  f.rows = empty_floats(q, at_ws + ws_bytes / 4);
+  check(fox_attn_fwd_plan(&dims, a.threshold.defined(), nullptr, nullptr, &ws_bytes), "fox_attn_fwd_plan");
+  const int64_t at_l = lse_at(a);
+  f.rows = empty_floats(q, at_l + a.B * a.H * a.M);
+  Tensor ws;
+  if (ws_bytes > 0) ws = empty_bytes_like(q, ws_bytes);
   float* base = f.rows.mutable_data_ptr<float>();
   if (a.is_logit) {   // logsigmoid fused into the scan; the fp32 log gates are a by-product
     f.log_fgate = at::empty({a.B, a.H, a.N}, q.options().dtype(at::kFloat));
@@ -131,7 +133,7 @@ Forward run_forward(Attention& a, const Tensor& q, const Tensor& k, const Tensor
   args.seq_start = a.seq_ptr();
   args.threshold = a.thr_ptr();
   args.sm_scale = (float)a.sm_scale;
-  args.workspace = ws_bytes > 0 ? base + at_ws : nullptr;
+  args.workspace = ws_bytes > 0 ? ws.mutable_data_ptr() : nullptr;
   args.workspace_bytes = ws_bytes;
   if (!a.epilogue) {
     f.out = f.o = at::empty_like(q);

@@ -135,6 +135,7 @@ SIGNATURES = {
     "fox_attn_fwd_noalloc": (C.c_int, [C.POINTER(FwdArgs), C.c_void_p]),
     "fox_attn_fwd_norm_gate": (C.c_int, [C.POINTER(FwdArgs), C.POINTER(FwdEpilogue), C.c_void_p]),
     "fox_attn_fwd_workspace_bytes": (C.c_int, [C.POINTER(Dims), C.POINTER(C.c_int64)]),
+    "fox_attn_fwd_plan": (C.c_int, [C.POINTER(Dims), C.c_int32, C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.POINTER(C.c_int64)]),
     "fox_attn_decode": (C.c_int, [C.POINTER(FwdArgs), C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p]),
     "fox_attn_decode_workspace_bytes": (C.c_int, [C.POINTER(Dims), C.POINTER(C.c_int64)]),
     "fox_cache_append": (C.c_int, [C.c_void_p, C.c_void_p]),   # fox_cache_append_args, filled by the host extension

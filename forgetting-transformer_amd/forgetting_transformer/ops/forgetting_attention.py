@@ -264,11 +264,11 @@ _GATE_DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16,
 
 
 @functools.lru_cache(maxsize=256)
-def _fwd_workspace_bytes(B, H, M, N, D, dtype_code):
-    """Bytes of key-split scratch the forward wants for a shape (0 = the shape is not split); asked once per shape."""
+def _fwd_workspace_bytes(B, H, M, N, D, dtype_code, pruned):
+    """Bytes of key-split scratch the forward uses for a shape (0 = the shape is not split); asked once per shape."""
     need = C.c_int64(0)
-    _lib.check(_lib.load().fox_attn_fwd_workspace_bytes(C.byref(_lib.Dims(B, H, M, N, D, dtype_code)), C.byref(need)),
-               "fox_attn_fwd_workspace_bytes")
+    _lib.check(_lib.load().fox_attn_fwd_plan(C.byref(_lib.Dims(B, H, M, N, D, dtype_code)), pruned, None, None, C.byref(need)),
+               "fox_attn_fwd_plan")
     return need.value
 
 
@@ -367,13 +367,14 @@ def _forward(ctx, gate_is_logit, q, k, v, log_fgate, seq_start, causal, sm_scale
             _lib.check(lib.fox_auto_threshold(C.byref(dims), C.byref(qv), C.byref(kv), sm_scale,
                                               _ptr(adaptive_threshold), _ptr(scratch), stream), "fox_auto_threshold")
 
-        # log_lambda (B,H,N), the log-normaliser L (B,H,M) and the key-split scratch come from one allocation
-        ws_bytes = _fwd_workspace_bytes(B, H, M, N, D, dims.dtype)
-        n_c, n_l = (B * H * N + 3) // 4 * 4, (B * H * M + 3) // 4 * 4    # floats; the scratch behind them stays 16-byte aligned
-        buf = torch.empty(n_c + n_l + ws_bytes // 4, dtype=torch.float32, device=device)
+        # log_lambda (B,H,N) and the log-normaliser L (B,H,M) come from one allocation, which the backward keeps; key splits have
+        # their own
+        ws_bytes = _fwd_workspace_bytes(B, H, M, N, D, dims.dtype, int(adaptive_threshold is not None))
+        n_c = (B * H * N + 3) // 4 * 4
+        buf = torch.empty(n_c + B * H * M, dtype=torch.float32, device=device)
         log_lambda = buf[:B * H * N].view(B, H, N)
-        L = buf[n_c:n_c + B * H * M].view(B, H, M)
-        workspace = buf[n_c + n_l:] if ws_bytes > 0 else None
+        L = buf[n_c:].view(B, H, M)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes > 0 else None
 
         # c = cumsum(log_fgate) with gates left of seq_start zeroed, one fused kernel
         if gate_is_logit:  # logsigmoid fused into the scan; the fp32 log gates are a by-product

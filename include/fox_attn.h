@@ -175,6 +175,14 @@ int fox_attn_fwd(const fox_fwd_args* args, void* stream);
 int fox_attn_fwd_workspace_bytes(const fox_dims* dims, int64_t* bytes);
 
 /*
+ * What fox_attn_fwd does with a shape when it may split: the number of key splits (1 = none), whether two groups of waves
+ * share every query tile's walk instead, and the scratch this uses.  It depends on whether a threshold is given (pruned);
+ * fox_attn_fwd_workspace_bytes() covers both.  Where *workspace_bytes is 0, a call with workspace = NULL does the same.
+ * Any of the three results may be NULL.
+ */
+int fox_attn_fwd_plan(const fox_dims* dims, int32_t pruned, int32_t* key_splits, int32_t* paired, int64_t* workspace_bytes);
+
+/*
  * fox_attn_fwd for callers that cannot allocate device memory or bring a workspace: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the reference.  Same
  * arguments and results as fox_attn_fwd (bit for bit), except that args->workspace / workspace_bytes are

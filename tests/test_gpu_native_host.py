@@ -455,3 +455,28 @@ def test_a_threshold_that_requires_grad(ft, M):
     assert out.requires_grad and torch.autograd.grad(out, [thr], do, allow_unused=True) == (None,)
     with torch.no_grad():
         assert torch.equal(ft.forgetting_attention(q, k, v, g, head_first=True, adaptive_threshold=thr), out)
+
+
+# grids the paired kernel takes instead of two key splits, grids that stay split, and one that is neither
+@pytest.mark.parametrize("B,H,M,N,D", [(2, 12, 1024, 1024, 128), (2, 16, 333, 5333, 128), (4, 32, 1024, 1024, 64)])
+@pytest.mark.parametrize("epilogue,general", [(False, False), (True, False), (False, True)])
+def test_no_scratch_is_kept_for_the_backward(ft, B, H, M, N, D, epilogue, general):
+    """What a forward leaves behind is its results: the scratch of key splits is gone when the call returns."""
+    F = import_module("forgetting_transformer.ops.forgetting_attention")
+    q, k, v, g, do, _ = make_inputs(B, H, M, N, D, device="cuda", head_first=True, seed=1, gate_mean=1.0)
+    for x in (q, k, v, g):
+        x.requires_grad_()
+    w = torch.rand(H * D, device="cuda")
+    def call():
+        if general:
+            return F.ForgettingAttention.apply(q, k, v, g, None, True, None, None)
+        return ft.forgetting_attention_norm_gate(q, k, v, g, None, w, head_first=True) if epilogue else ft.forgetting_attention(q, k, v, g, head_first=True)
+    call()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    out = call()
+    kept = torch.cuda.memory_allocated() - before
+    rows = B * H * M * D * 2
+    need = rows + 4 * B * H * (M + N) + ((rows + 4 * B * H * M) if epilogue else 0)
+    assert kept <= need + (2 << 20) + 8 * 512, (kept, need)     # (the allocator hands out large blocks with up to 1 MiB left over)
+    del out
