@@ -1,5 +1,7 @@
 """The kernels of token-by-token generation: one query row straight from the log gates (no graph, no threshold), its merge of key
 splits, and the append of new tokens to the cache."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -59,6 +61,40 @@ def test_single_query_in_one_workgroup(ft, B, H, N, D, dtype):
     with torch.no_grad():
         out = ft.forgetting_attention(q, k, v, g, head_first=True, seq_start=ss)
     assert_parity("out", out, O.forgetting_attention_ref(q, k, v, g, head_first=True, seq_start=ss))
+
+
+# through the C ABI: splits and their merge, one workgroup of sixteen waves, one key; with the scratch and without (one workgroup of
+# four waves walks the whole cache), with lse and without, gates with strides; the last sequence is all padding
+@pytest.mark.parametrize("B,H,N,D", [(3, 2, 5000, 64), (3, 2, 400, 64), (2, 3, 9001, 128), (2, 2, 3000, 16), (3, 40, 700, 32), (2, 1, 1, 64)])
+def test_decode_entry_point(ft, B, H, N, D):
+    from forgetting_transformer.ops import _lib
+    from forgetting_transformer.ops.forgetting_attention import _view
+    lib, stream = _lib.load(), C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ss = [(N * i) // (2 * B) for i in range(B - 1)] + [N]
+    q, k, v, g, _, ss = make_inputs(B, H, 1, N, D, device="cuda", head_first=True, seq_start=ss, seed=N, gate_mean=3.0)
+    gates = g.transpose(1, 2).contiguous().transpose(1, 2)       # (B, H, N) with the heads adjacent
+    dims, need = _lib.Dims(B, H, 1, N, D, _lib.DTYPE_BF16), C.c_int64(0)
+    _lib.check(lib.fox_attn_decode_workspace_bytes(C.byref(dims), C.byref(need)), "fox_attn_decode_workspace_bytes")
+    scores = (k.double() @ q.double().transpose(-1, -2)).squeeze(-1) / D ** 0.5
+    scores += g.double().flip(-1).cumsum(-1).flip(-1) - g.double()          # the gates behind each key
+    scores = scores.masked_fill(torch.arange(N, device="cuda") < ss[:, None, None], float("-inf"))
+    lse_ref = scores.logsumexp(-1)
+    ref = O.forgetting_attention_ref(q, k, v, g, head_first=True, seq_start=ss)
+    for scratch in (True, False):
+        for with_lse in (True, False):
+            ws = torch.empty(max(need.value, 16), dtype=torch.uint8, device="cuda")
+            o, lse = torch.full_like(q, float("nan")), torch.full((B, H), float("nan"), device="cuda")
+            args = _lib.FwdArgs(dims, _view(q), _view(k), _view(v), _view(o), None, lse.data_ptr() if with_lse else None, ss.data_ptr(), None,
+                                1.0 / D ** 0.5, None, ws.data_ptr() if scratch and need.value else None, need.value if scratch else 0)
+            _lib.check(lib.fox_attn_decode(C.byref(args), gates.data_ptr(), *gates.stride(), stream), "fox_attn_decode")
+            assert_parity("out", o, ref, context=(scratch, with_lse))
+            assert (o[-1] == 0).all()
+            if not with_lse:
+                assert lse.isnan().all()
+                continue
+            assert (lse[-1] == float("-inf")).all()
+            # fp32: D products summed (scores of a few units), the bias of the keys that count (tens at most) rounded once, 2^x and log
+            assert (lse[:-1].double() - lse_ref[:-1]).abs().max() <= 2e-5, (scratch, (lse[:-1].double() - lse_ref[:-1]).abs().max())
 
 
 @pytest.mark.parametrize("D,T,dtype", [(64, 1, torch.bfloat16), (128, 1, torch.float16), (16, 7, torch.bfloat16), (40, 300, torch.float16),

@@ -480,3 +480,80 @@ def test_no_scratch_is_kept_for_the_backward(ft, B, H, M, N, D, epilogue, genera
     need = rows + 4 * B * H * (M + N) + ((rows + 4 * B * H * M) if epilogue else 0)
     assert kept <= need + (2 << 20) + 8 * 512, (kept, need)     # (the allocator hands out large blocks with up to 1 MiB left over)
     del out
+
+
+def _layer_step(ft, x, k, v, logits, w):
+    B, T, H, D = k.shape
+    q = ft.group_norm(x, w, is_rms_norm=True, num_groups=H).view(B, T, H, D)
+    return ft.forgetting_attention_norm_gate(q, k, v, logits, None, w, fgate_is_logit=True, adaptive_threshold=-20.0)[0]
+
+
+@pytest.mark.parametrize("reentrant", [True, False])
+def test_under_activation_checkpointing(ft, reentrant):
+    from torch.utils.checkpoint import checkpoint
+    B, T, H, D = 2, 130, 3, 64
+    rnd = lambda *s: torch.randn(*s, device="cuda").bfloat16().requires_grad_()
+    leaves = [rnd(B, T, H * D), rnd(B, T, H, D), rnd(B, T, H, D), torch.randn(B, T, H, device="cuda", requires_grad=True),
+              torch.rand(H * D, device="cuda", requires_grad=True)]
+    do = torch.randn(B, T, H, D, device="cuda").bfloat16()
+    grads = []
+    for again in (False, True):
+        y = checkpoint(_layer_step, ft, *leaves, use_reentrant=reentrant) if again else _layer_step(ft, *leaves)
+        grads.append([y.detach()] + [g.clone() for g in _backward_into_leaves(y, leaves, do)])
+    _equal(*grads)
+
+
+def _backward_into_leaves(y, leaves, do):
+    for t in leaves:
+        t.grad = None
+    y.backward(do)
+    return [t.grad for t in leaves]
+
+
+def test_steps_on_several_threads_and_streams(ft):
+    """Forward and backward from four threads at once, each on its own stream and device buffers, against the same steps one by one."""
+    import threading
+    B, T, H, D = 1, 300, 2, 64
+    def inputs(i):
+        gen = torch.Generator(device="cuda").manual_seed(i)
+        rnd = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+        return [rnd(B, T + i, H * D).bfloat16(), rnd(B, T + i, H, D).bfloat16(), rnd(B, T + i, H, D).bfloat16(), rnd(B, T + i, H) + 1,
+                rnd(H * D).abs() + 0.5], rnd(B, T + i, H, D).bfloat16()
+    def step(i):
+        leaves, do = inputs(i)
+        leaves = [t.requires_grad_() for t in leaves]
+        y = _layer_step(ft, *leaves)
+        return [y.detach()] + list(torch.autograd.grad(y, leaves, do))
+    want = [step(i) for i in range(4)]
+    torch.cuda.synchronize()
+    got, errors = [[None] * 5 for _ in range(4)], []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for r in range(5):
+                    got[i][r] = step(i)
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:   # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for i in range(4):
+        for r in range(5):
+            _equal(got[i][r], want[i])
+
+
+@pytest.mark.filterwarnings("ignore")   # the tracer's remarks
+def test_traces_are_refused(ft):
+    """The general path's shape checks refuse the tracer's sizes; the native path must not turn the result into a constant instead."""
+    q, k, v, g, _, _ = make_inputs(1, 2, 70, 70, 64, device="cuda", head_first=True, seed=3)
+    with pytest.raises(AssertionError, match="head dims"):
+        torch.jit.trace(lambda a, b, c, d: ft.forgetting_attention(a, b, c, d, head_first=True), (q, k, v, g), check_trace=False)
+    x, w = torch.randn(2, 30, 128, device="cuda").bfloat16(), torch.rand(128, device="cuda")
+    with pytest.raises(AssertionError, match="group size"):
+        torch.jit.trace(lambda a, b: ft.group_norm(a, b, is_rms_norm=True, num_groups=2), (x, w), check_trace=False)

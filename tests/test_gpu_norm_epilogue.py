@@ -105,6 +105,20 @@ def test_activations_layouts_and_left_padding(ops, activation, head_first, seq):
     _run_case(ops, 2, 4, 257, 257, 64, torch.bfloat16, activation, head_first=head_first, seq=seq, seed=3)
 
 
+# the paired forward with the norm in its epilogue: grids of fewer tiles than are split, one that took two key splits before
+# (192 tiles), with a ragged last tile, and one beyond a tile per CU
+@pytest.mark.parametrize("D,dtype", [(32, torch.bfloat16), (64, torch.float16), (64, torch.bfloat16), (128, torch.bfloat16), (32, torch.float16),
+                                     (128, torch.float16)])
+@pytest.mark.parametrize("B,H,M,N,activation,head_first,seq", [(2, 3, 600, 600, "sigmoid", False, [0, 333]), (1, 3, 700, 900, None, True, None),
+                                                               (2, 12, 1000, 1024, "swish", True, None), (1, 17, 2000, 2000, "sigmoid", False, None)])
+def test_in_the_paired_forward(ops, B, H, M, N, D, dtype, activation, head_first, seq):
+    from forgetting_transformer.ops import _lib
+    paired = C.c_int32(0)
+    _lib.check(_lib.load().fox_attn_fwd_plan(C.byref(_lib.Dims(B, H, M, N, D, 0)), 0, None, C.byref(paired), None), "fox_attn_fwd_plan")
+    assert paired.value
+    _run_case(ops, B, H, M, N, D, dtype, activation, head_first=head_first, seq=seq, seed=M + D)
+
+
 def test_with_pruning_threshold(ops):
     _run_case(ops, 1, 2, 1024, 1024, 128, torch.bfloat16, "sigmoid", head_first=False, seq=None, thr=-8.0, seed=5)
 

@@ -2,6 +2,8 @@
 the variants that a shape selects, each at the sizes where its bookkeeping has an edge.  Every case is compared with the
 oracle over all (batch, head) pairs at the operator's bar, so a tile that is visited twice, never, or for the
 wrong pair shows."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -42,11 +44,32 @@ def test_paired_forward_with_a_negative_scale(fa, D):   # every tile takes the m
     run_case(fa, 1, 2, 700, 900, D, seed=3, gate_mean=2.0, sm_scale=-0.1)
 
 
-# grids beyond one tile per CU and in place of two key splits, at their edges: the output alone
-@pytest.mark.parametrize("B,H,T", [(2, 16, 1500), (1, 17, 1921), (3, 10, 1024), (1, 12, 2560)])
+# grids beyond one tile per CU and in place of two key splits, on both sides of the rule: the output alone.  384 tiles are paired
+# from 2048 keys on, 511 from 4080 on, 512 never; 240 and 252 tiles would take two splits, which the pairing replaces up to 2560 keys
+@pytest.mark.parametrize("B,H,T,paired", [(2, 16, 1500, False), (1, 17, 1921, True), (3, 10, 1024, True), (1, 12, 2560, True), (1, 12, 2561, False),
+                                          (1, 24, 2047, False), (1, 24, 2048, True), (2, 16, 2048, False), (1, 7, 9300, True)])
 @pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.float16)])
-def test_paired_forward_of_larger_grids(fa, B, H, T, D, dtype):
+def test_paired_forward_of_larger_grids(fa, B, H, T, paired, D, dtype):
+    from forgetting_transformer.ops import _lib
+    lib, plan = _lib.load(), C.c_int32(-1)
+    dims = _lib.Dims(B, H, T, T, D, int(dtype == torch.float16))
+    _lib.check(lib.fox_attn_fwd_plan(C.byref(dims), 0, None, C.byref(plan), None), "fox_attn_fwd_plan")
+    assert plan.value == paired
     q, k, v, g, _, ss = make_inputs(B, H, T, T, D, dtype=dtype, device="cuda", head_first=False, seed=T, gate_mean=2.0)
     with torch.no_grad():
         out = fa(q, k, v, g)
     assert_parity("out", out, O.forgetting_attention_ref(q, k, v, g))
+
+
+@pytest.mark.parametrize("B,H,T,D", [(3, 10, 1024, 64), (1, 3, 600, 32), (1, 17, 1921, 128)])
+def test_paired_forward_with_and_without_scratch(fa, B, H, T, D):
+    """The plan asks for no scratch where the paired kernel runs; a caller that brings what key splits would need gets the same
+    results, bit for bit."""
+    from test_zz_no_alloc import _fwd_pair
+    from forgetting_transformer.ops import _lib
+    from forgetting_transformer.ops.forgetting_attention import _view
+    lib = _lib.load()
+    (own, noalloc), _, (q, k, v, g, _) = _fwd_pair(lib, _lib, _view, B, H, T, T, D, seed=5)
+    with torch.no_grad():
+        out = fa(q, k, v, g, head_first=True)
+    assert torch.equal(out, own[0]) and torch.equal(out, noalloc[0]) and torch.equal(own[1], noalloc[1])

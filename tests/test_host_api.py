@@ -381,3 +381,34 @@ def test_qk_norm_threshold_on_the_host_needs_no_library(monkeypatch):
     top = w.view(2, 16).abs().amax(-1).double()
     want = -(2 * top * top * 4.0 + math.log(100)) - 10.0
     assert torch.allclose(got.double(), want, rtol=1e-6, atol=0)     # five fp32 operations, 6e-8 each
+
+
+def test_forward_plan():
+    """What a shape is given: key splits with scratch, or the paired kernel with none; never both, never more than the older query says."""
+    lib = _lib.load()
+    splits, paired, need, most = C.c_int32(), C.c_int32(), C.c_int64(), C.c_int64()
+
+    def plan(B, H, M, N, D, pruned=0):
+        dims = _lib.Dims(B, H, M, N, D, 0)
+        assert lib.fox_attn_fwd_plan(C.byref(dims), pruned, C.byref(splits), C.byref(paired), C.byref(need)) == 0
+        assert lib.fox_attn_fwd_workspace_bytes(C.byref(dims), C.byref(most)) == 0
+        assert need.value in (0, most.value) and (need.value > 0) == (splits.value > 1) and not (paired.value and splits.value > 1)
+        assert need.value == (B * H * M * splits.value * (D + 2) * 4 if splits.value > 1 else 0)
+        return splits.value, bool(paired.value)
+
+    assert plan(2, 12, 1024, 1024, 128) == (1, True) and plan(2, 12, 1024, 1024, 128, pruned=1) == (2, False)
+    assert plan(2, 12, 1024, 1024, 16) == (2, False)                  # no paired kernel for this head dim
+    assert plan(1, 2, 511, 511, 64) == (1, False) and plan(1, 2, 512, 512, 64) == (1, True)
+    assert plan(1, 24, 2048, 2048, 64) == (1, True) and plan(1, 24, 2047, 2047, 64) == (1, False)
+    assert plan(2, 16, 2048, 2048, 64) == (1, False) and plan(4, 16, 16384, 16384, 128) == (1, False)
+    assert plan(16, 16, 128, 32768, 128) == (2, False) and plan(2, 16, 333, 5333, 128) == (5, False)
+    assert plan(1, 12, 1, 1500, 64)[1] is False
+    for M, N in ((1, 1), (1, 4096), (128, 600), (300, 600), (301, 600), (1000, 1000), (1025, 2560), (1025, 2561), (8192, 8192)):
+        for H in (1, 7, 16, 33, 40, 64):
+            for D in (16, 32, 64, 128):
+                for pruned in (0, 1):
+                    _, pair = plan(1, H, M, N, D, pruned)
+                    assert not (pair and (pruned or D == 16))
+    assert lib.fox_attn_fwd_plan(C.byref(_lib.Dims(1, 1, 1, 100, 48, 0)), 0, None, None, None) == -1
+    assert lib.fox_attn_fwd_plan(None, 0, None, None, None) == -1
+    assert lib.fox_attn_fwd_plan(C.byref(_lib.Dims(1, 1, 1, 100, 64, 0)), 0, None, None, None) == 0
