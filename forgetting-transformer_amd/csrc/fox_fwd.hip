@@ -681,7 +681,7 @@ static hipError_t launch_fwd_d(const FwdK& a, int dtype, hipStream_t s) {
   } else if (a.splits <= 1) {
     const dim3 grid((unsigned)(a.n_mtiles * a.B * a.H));
     if constexpr (D >= 32) {
-      if (a.pair && !stream) {
+      if (a.pair) {   // (two query tiles at least: never a streaming shape)
         if (a.epi.y.ptr) hipLaunchKernelGGL((fwd_pair_kernel<Tr, D, true>), grid, dim3(512), 0, s, a);
         else hipLaunchKernelGGL((fwd_pair_kernel<Tr, D, false>), grid, dim3(512), 0, s, a);
         return hipGetLastError();
