@@ -281,12 +281,18 @@ def _cached_constant_threshold(value, B, H, device):
     return t
 
 
+_key_included = torch._C._dispatch_tls_is_dispatch_key_included
+_TRANSFORM_OR_MODE = (torch._C.DispatchKey.FuncTorchDynamicLayerFrontMode, torch._C.DispatchKey.Python)
+
+
 def _constant_threshold(value, B, H, device):
     """(B, H) fp32 tensor holding one float threshold: the same values as as_tensor + broadcast_to of the reference
     (:104-109), filled on the device once per (value, shape, device) instead of once per call.  Read-only.
     Under stream capture the tensor is filled by a kernel of the captured graph instead (a tensor created during
-    capture lives in the graph's memory pool and holds nothing until the graph runs, so it must not be cached)."""
-    if device.type != "cuda" or torch.cuda.is_current_stream_capturing():   # (CPU tensors are rejected further down)
+    capture lives in the graph's memory pool and holds nothing until the graph runs, so it must not be cached); nor is
+    one cached that a function transform wraps or a dispatch mode may replace."""
+    # (CPU tensors are rejected further down)
+    if device.type != "cuda" or torch.cuda.is_current_stream_capturing() or any(map(_key_included, _TRANSFORM_OR_MODE)):
         return torch.full((B, H), value, dtype=torch.float, device=device)
     return _cached_constant_threshold(value, B, H, device)
 

@@ -557,3 +557,22 @@ def test_traces_are_refused(ft):
     x, w = torch.randn(2, 30, 128, device="cuda").bfloat16(), torch.rand(128, device="cuda")
     with pytest.raises(AssertionError, match="group size"):
         torch.jit.trace(lambda a, b: ft.group_norm(a, b, is_rms_norm=True, num_groups=2), (x, w), check_trace=False)
+
+
+@pytest.mark.parametrize("first,thr", [("transform", -9.0625), ("mode", -9.1875)])   # numbers no other test uses
+def test_a_number_as_threshold_under_a_transform_or_mode_first(ft, first, thr):
+    """The tensor made of a number serves later calls: one that a transform wrapped, or a mode replaced, must not stay behind."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    F = import_module("forgetting_transformer.ops.forgetting_attention")
+    q, k, v, g, _, _ = make_inputs(1, 2, 300, 300, 64, device="cuda", head_first=True, seed=3, gate_mean=-1.0)
+    want = ft.forgetting_attention(q, k, v, g, head_first=True, adaptive_threshold=torch.full((1, 2), thr, device="cuda"))
+    call = lambda: ft.forgetting_attention(q, k, v, g, head_first=True, adaptive_threshold=thr)
+    if first == "transform":
+        with pytest.raises(RuntimeError, match="setup_context"):
+            torch.func.grad(lambda t: call().float().sum() + t)(torch.zeros((), device="cuda"))
+    else:
+        with FakeTensorMode():       # (what a call does there before anything looks at its tensors)
+            F._native_threshold(thr, q, True)
+    got = F._native_threshold(thr, q, True)
+    assert type(got) is torch.Tensor and got.data_ptr() != 0 and (got == thr).all()
+    assert torch.equal(call(), want)
