@@ -206,9 +206,10 @@ void record_bounds(const Attention& a, const Tensor& q, fox_bwd_args& args) {
   pybind11::reinterpret_borrow<pybind11::list>(g_bounds).append(d);   // (keeps both tensors alive past the launches)
 }
 
-// dq, dk, dv and the gradient of the gates, in the layout of the inputs
-variable_list run_backward(const Attention& a, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, const Tensor& o,
-                           const Tensor& rows, Tensor d_o) {
+// dq, dk, dv and the gradient of the gates, in the layout of the inputs.  g: the gate logits, undefined for log gates, of which the
+// backward needs the strides only
+variable_list run_backward(const Attention& a, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g, at::IntArrayRef g_strides,
+                           const Tensor& o, const Tensor& rows, Tensor d_o) {
   if (!vectors_ok(d_o)) d_o = d_o.contiguous();
   void* stream = stream_of(q);
   const int64_t n_c = a.B * a.H * a.N, n_l = a.B * a.H * a.M;
@@ -216,10 +217,8 @@ variable_list run_backward(const Attention& a, const Tensor& q, const Tensor& k,
   Tensor tmp = empty_floats(q, 2 * n_l + n_c);
   float* t = tmp.mutable_data_ptr<float>();
   Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
-  // in the layout of the caller's gates when they are a permuted dense tensor: autograd takes the gradient as it is
   Tensor dg = a.is_logit ? at::empty_like(g)
-              : g.is_non_overlapping_and_dense() ? at::empty_strided(g.sizes(), g.strides(), g.options())
-                                                 : at::empty(g.sizes(), g.options());
+                         : at::empty_strided({a.B, a.head_first ? a.H : a.N, a.head_first ? a.N : a.H}, g_strides, tmp.options());
   fox_bwd_args args{};
   args.dims = a.dims(q);
   args.q = view_of(q, a.head_first);
@@ -312,7 +311,7 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
   static variable_list forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& g,
                                const std::optional<Tensor>& gate, const std::optional<Tensor>& weight, Attention* a) {
     Forward f = run_forward(*a, q, k, v, g);
-    ctx->save_for_backward({q, k, v, g, f.o, f.rows, a->seq_start, a->threshold, a->gate, a->weight, f.rstd});
+    ctx->save_for_backward({q, k, v, a->is_logit ? g : Tensor(), f.o, f.rows, a->seq_start, a->threshold, a->gate, a->weight, f.rstd});
     auto& d = ctx->saved_data;
     d["hf"] = a->head_first;
     d["logit"] = a->is_logit;
@@ -322,7 +321,12 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
       d["eps"] = a->eps;
       d["wtype"] = (int64_t)weight->scalar_type();
     }
-    if (!a->is_logit) return {f.out};
+    if (!a->is_logit) {
+      // the gradient in the layout of the caller's gates when they are a permuted dense tensor: autograd takes it as it is
+      if (g.is_non_overlapping_and_dense()) d["gs"] = g.strides();
+      else d["gs"] = at::IntArrayRef{g.size(1) * g.size(2), g.size(2), 1};
+      return {f.out};
+    }
     Tensor log_fgate = a->head_first ? f.log_fgate : f.log_fgate.transpose(1, 2);
     ctx->mark_non_differentiable({log_fgate});
     return {f.out, log_fgate};
@@ -359,7 +363,8 @@ struct AttentionNode : public torch::autograd::Function<AttentionNode> {
       run_norm_backward(o, gate, packed(s[9]), packed(s[10]), dy, a.B * a.M, a.H, a.D, (int)d["act"].toInt(), d["eps"].toDouble(), d_o, dgate, dw);
       dweight = dw.to((at::ScalarType)d["wtype"].toInt());
     }
-    variable_list r = run_backward(a, q, k, v, s[3], vectors(s[4]), packed(s[5]), d_o);
+    const std::vector<int64_t> g_strides = a.is_logit ? std::vector<int64_t>() : d["gs"].toIntVector();
+    variable_list r = run_backward(a, q, k, v, s[3], g_strides, vectors(s[4]), packed(s[5]), d_o);
     return {r[0], r[1], r[2], r[3], dgate, dweight, Tensor()};
   }
 };

@@ -576,3 +576,34 @@ def test_a_number_as_threshold_under_a_transform_or_mode_first(ft, first, thr):
     got = F._native_threshold(thr, q, True)
     assert type(got) is torch.Tensor and got.data_ptr() != 0 and (got == thr).all()
     assert torch.equal(call(), want)
+
+
+@pytest.mark.parametrize("logits", [False, True])
+def test_gates_changed_between_forward_and_backward(ft, logits):
+    """The backward does not read log gates, so their buffer is free again after the forward; logits it does read."""
+    q, k, v, g, do, _ = make_inputs(1, 2, 70, 70, 64, device="cuda", head_first=True, seed=3)
+    leaves = [x.requires_grad_() for x in (q, k, v)]
+
+    def call():
+        return ft.forgetting_attention_from_logits(*leaves, g, head_first=True)[0] if logits else ft.forgetting_attention(*leaves, g, head_first=True)
+
+    want, out = torch.autograd.grad(call(), leaves, do), call()
+    g.zero_()
+    if logits:
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            torch.autograd.grad(out, leaves, do)
+    else:
+        _equal(torch.autograd.grad(out, leaves, do), want)
+
+
+def test_log_gates_are_not_kept_for_the_backward(ft):
+    B, H, T, D = 1, 16, 1 << 16, 16
+    q, k, v, g, _, _ = make_inputs(B, H, 128, T, D, device="cuda", head_first=True, seed=3)
+    q.requires_grad_()
+    g_bytes = g.numel() * 4
+    out = ft.forgetting_attention(q, k, v, g, head_first=True)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    del g
+    assert before - torch.cuda.memory_allocated() >= g_bytes
+    del out
