@@ -495,10 +495,11 @@ bool under_transform_or_mode() {
 const Tensor* tensor_of(PyObject* o) {
   if (!THPVariable_CheckExact(o)) return nullptr;   // Tensor or Parameter: the general path's results keep other subclasses
   const Tensor& t = THPVariable_Unpack(o);
-  // tensors with a dispatch of their own and the wrappers of functional transforms have no plain storage; a dual tensor's tangent
-  // and a trace would be lost: all of these go through the general path, which handles or refuses them
-  if (t.key_set().has(c10::DispatchKey::Python) || !t.has_storage() || t._fw_grad(0).defined() || at::tracer::impl::is_dispatch_enabled() ||
-      under_transform_or_mode())
+  // tensors with a dispatch of their own and the wrappers of functional transforms have no plain storage, negated views and zero
+  // tensors hold other values than their memory; a dual tensor's tangent and a trace would be lost: all of these go through the
+  // general path, which handles or refuses them
+  if (t.key_set().has(c10::DispatchKey::Python) || !t.has_storage() || t.is_neg() || t._is_zerotensor() ||
+      t._fw_grad(0).defined() || at::tracer::impl::is_dispatch_enabled() || under_transform_or_mode())
     return nullptr;
   return &t;
 }

@@ -607,3 +607,13 @@ def test_log_gates_are_not_kept_for_the_backward(ft):
     del g
     assert before - torch.cuda.memory_allocated() >= g_bytes
     del out
+
+
+def test_a_negated_view_joins_the_cache_with_its_values(ft):
+    """The imaginary part of a conjugate is a view that stands for the negated memory."""
+    z = torch.complex(torch.randn(1, 2, 3, device="cuda"), torch.randn(1, 2, 3, device="cuda"))
+    g = z.conj().imag
+    assert g.is_neg()
+    k = torch.randn(1, 2, 3, 64, device="cuda").bfloat16()
+    got = ft.FgateDynamicCache().update(k, k, g, 0)
+    assert torch.equal(got[2], -z.imag)
