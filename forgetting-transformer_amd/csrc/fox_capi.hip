@@ -316,7 +316,9 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
 
 extern "C" {
 
-int fox_version(void) { return 201; }  // 0.2.x: fox_bwd_args and the scan entry points differ from 0.1.0; 0.2.1 adds fox_set_stream_min_kv_bytes and fox_probe_mfma
+// 0.2.x: fox_bwd_args and the scan entry points differ from 0.1.0; 0.2.1 adds fox_set_stream_min_kv_bytes and fox_probe_mfma, 0.2.2
+// fox_attn_decode, fox_cache_append, fox_qk_norm_threshold and fox_attn_fwd_plan
+int fox_version(void) { return 202; }
 
 const char* fox_last_error(void) { return g_err; }
 
