@@ -713,7 +713,7 @@ static hipError_t delta_t(const BwdK& a, int D, hipStream_t s) {
 template <typename Tr>
 static hipError_t dkdv_t(const BwdK& a0, int D, hipStream_t s) {
   BwdK a = a0;
-  a.groups = order_groups(a.B * a.H, a.M, a.N, D);
+  a.groups = order_groups(a.B * a.H, (a.N + kKvBN - 1) / kKvBN, a.M, a.N, D, a.k.st, a.thr != nullptr);
   a.even = even_tiles(a.M, a.N);
   if (a.cls == kClassLight) {  // the split variant: 64 keys per workgroup
     if (!dkdv_split_supports(D)) return hipErrorInvalidValue;
@@ -735,9 +735,9 @@ static hipError_t dkdv_t(const BwdK& a0, int D, hipStream_t s) {
 template <typename Tr>
 static hipError_t dq_t(const BwdK& a0, int D, hipStream_t s) {
   BwdK a = a0;
-  a.groups = order_groups(a.B * a.H, a.M, a.N, D);
-  a.even = even_tiles(a.M, a.N);
   a.n_tiles = (a.M + kFwdBM - 1) / kFwdBM;
+  a.groups = order_groups(a.B * a.H, a.n_tiles, a.M, a.N, D, a.k.st, a.thr != nullptr);
+  a.even = even_tiles(a.M, a.N);
   const dim3 grid((unsigned)(a.n_tiles * a.B * a.H));
   FOX_DISPATCH_D(dq_kernel, grid, 0)
   return hipGetLastError();

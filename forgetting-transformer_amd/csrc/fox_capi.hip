@@ -265,7 +265,7 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
   k.B = args->dims.B; k.H = args->dims.H; k.M = args->dims.M; k.N = args->dims.N;
   k.sm_scale = args->sm_scale;
   k.n_mtiles = (args->dims.M + fox::kFwdBM - 1) / fox::kFwdBM;
-  k.groups = fox::order_groups(k.B * k.H, k.M, k.N, args->dims.D);
+  k.groups = fox::order_groups(k.B * k.H, k.n_mtiles, k.M, k.N, args->dims.D, k.k.st, k.thr != nullptr);
   k.even = fox::even_tiles(k.M, k.N);
   const FwdPlan plan = plan_fwd(args->dims, k.thr != nullptr, workspace != nullptr);
   k.splits = plan.splits;

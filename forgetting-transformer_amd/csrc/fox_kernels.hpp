@@ -142,11 +142,26 @@ constexpr int kKvBM = 128;   // query rows per step in the dK/dV kernel
 // T = 4096 (2 MiB a pair) 0.890 / 0.877 / 0.886, T = 8192 0.971 / 0.968 / 0.994, T = 16384 0.971 / 0.986 / 1.064; D = 64, B*H = 128,
 // T = 1024, for 4 / 8 / 16: 0.842 / 0.789 / 0.781.  With many more keys than queries the tiles weigh about the same and
 // only the caches count: one pair after the other (dK/dV at M = 128, N = 32768: 2.52 ms, in groups of two 2.65 ms).
-inline bool even_tiles(int M, int N) { return (int64_t)2 * M < N; }
-inline int order_groups(int n_bh, int M, int N, int D) {
+// Below D = 64 with the heads of a token side by side, a row is a part of a 128-byte line that it shares with the heads next to it.
+// - Without a threshold a row counts as the whole line, whose other heads run on other XCDs: by its own bytes D = 16, B4 T4096 H64 got 32
+//   pairs a group, forward 478 -> 600 us and backward 1.09 -> 1.37 ms against one pair after the other (now 435 us and 1.04 ms).  Under a
+//   threshold the walks are short and large groups cost nothing (D = 16, B8 H16 T2048 "auto", groups by bytes over one pair after the
+//   other: forward 1.10, backward 1.12 of its rate).
+// - Where 8 does not divide the pairs, one pair after the other puts tile t of pair b on XCD (b * tiles + t) % 8: pairs 8 / gcd(tiles, 8) apart
+//   meet on an XCD, and when they share lines that is worth more than groups can give to the short walks under a threshold.  At -10, groups
+//   over that order, forward / backward rate: D = 16 with 64 tiles B4 H15 0.83 / 0.65, with 60 (every second pair) B9 H12 0.85 / 0.69, with 54 1.02 / 1.01;
+//   D = 32 with 64 tiles B4 H15 0.90 / 0.81, with 60 1.07 / 1.05.  Up to four tiles per CU groups are the faster ones anyway.
+constexpr bool even_tiles(int M, int N) { return (int64_t)2 * M < N; }
+constexpr int order_groups(int n_bh, int tiles, int M, int N, int D, int64_t row_stride, bool pruned) {
   const bool by_xcd = n_bh % 8 == 0;
   const int nb = by_xcd ? n_bh / 8 : n_bh;
-  int64_t per = ((int64_t)8 << 20) / ((int64_t)N * D * 4);
+  const int64_t line = row_stride < 64 ? row_stride : 64;   // in elements
+  if (pruned && !by_xcd && (int64_t)tiles * n_bh > 4 * 256) {
+    const int apart = tiles % 8 == 0 ? 1 : tiles % 4 == 0 ? 2 : tiles % 2 == 0 ? 4 : 8;
+    if (apart * D < line) return nb;
+  }
+  const int64_t row = pruned || D > line ? D : line;
+  int64_t per = ((int64_t)8 << 20) / (N * row * 4);
   if (per < 2) per = 2;
   if (even_tiles(M, N)) per = 1;
   const int64_t groups = nb / (by_xcd ? per : per * 8);

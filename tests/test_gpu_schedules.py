@@ -23,6 +23,13 @@ def test_launch_order(fa, B, H, T, D):
     run_case(fa, B, H, T, T, D, seed=H + T, gate_mean=1.0)
 
 
+# rows shorter than a cache line with the heads of a token side by side: two groups; one pair after the other under a threshold
+@pytest.mark.parametrize("B,H,T,D,thr", [(1, 512, 1030, 16, None), (1, 131, 1020, 16, -10.0), (1, 91, 1500, 16, -10.0), (3, 45, 1024, 32, -6.0)])
+def test_launch_order_of_shared_lines(fa, B, H, T, D, thr):
+    torch.cuda.empty_cache()
+    run_case(fa, B, H, T, T, D, seed=H + T, gate_mean=1.0, head_first=False, thr=thr)
+
+
 # few query rows behind many keys: key splits that fill the chip once, also where one split more would not fit
 @pytest.mark.parametrize("B,H,M,N,D", [(2, 16, 333, 1100, 32), (1, 8, 129, 3000, 64), (3, 7, 300, 2000, 16)])
 def test_key_splits(fa, B, H, M, N, D):

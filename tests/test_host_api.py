@@ -412,3 +412,25 @@ def test_forward_plan():
     assert lib.fox_attn_fwd_plan(C.byref(_lib.Dims(1, 1, 1, 100, 48, 0)), 0, None, None, None) == -1
     assert lib.fox_attn_fwd_plan(None, 0, None, None, None) == -1
     assert lib.fox_attn_fwd_plan(C.byref(_lib.Dims(1, 1, 1, 100, 64, 0)), 0, None, None, None) == 0
+
+
+def test_launch_order_groups(tmp_path):
+    """Groups in the launch order of the attention kernels: what a row takes in cache counts, and where pairs that share lines meet on an
+    XCD a threshold takes them one after the other (the order changes time only, so no result would show a wrong one)."""
+    import shutil
+    import subprocess
+    hipcc = shutil.which("hipcc") or shutil.which("/opt/rocm/bin/hipcc")
+    if hipcc is None:
+        pytest.skip("no hipcc")
+    # (pairs, tiles, rows, keys, head dim, row stride in elements, threshold) -> groups
+    cases = {(256, 32, 4096, 4096, 16, 64 * 16, 0): 4, (256, 32, 4096, 4096, 16, 16, 0): 1, (256, 32, 4096, 4096, 16, 64 * 16, 1): 1,   # 8 divides the pairs
+             (256, 32, 4096, 4096, 32, 64 * 32, 0): 4, (256, 32, 4096, 4096, 64, 64 * 64, 0): 4, (64, 128, 16384, 16384, 128, 2048, 1): 4,
+             (60, 64, 8192, 8192, 16, 15 * 16, 1): 60, (60, 60, 7680, 7680, 16, 15 * 16, 1): 60, (60, 54, 6912, 6912, 16, 15 * 16, 1): 1,   # it does not
+             (60, 64, 8192, 8192, 32, 15 * 32, 1): 60, (60, 60, 7680, 7680, 32, 15 * 32, 1): 1, (60, 64, 8192, 8192, 64, 15 * 64, 1): 1,
+             (60, 64, 8192, 8192, 128, 15 * 128, 1): 3, (60, 64, 8192, 8192, 16, 16, 1): 1, (60, 64, 8192, 8192, 16, 15 * 16, 0): 1,
+             (60, 16, 2048, 2048, 16, 15 * 16, 1): 1, (9, 1, 128, 32768, 16, 9 * 16, 0): 1, (32, 1, 128, 32768, 128, 128, 0): 4}
+    src = tmp_path / "order.hip"
+    src.write_text('#include "fox_kernels.hpp"\n' + "".join(
+        f"static_assert(fox::order_groups({', '.join(map(str, c[:6]))}, {'true' if c[6] else 'false'}) == {n});\n" for c, n in cases.items()))
+    csrc = ROOT / "forgetting-transformer_amd" / "csrc"
+    subprocess.run([hipcc, "-std=c++17", "--cuda-host-only", "-fsyntax-only", "-Wno-unused-command-line-argument", f"-I{csrc}", str(src)], check=True)
