@@ -74,24 +74,30 @@ __global__ __launch_bounds__(256) void norm_gate_fwd_kernel(const NormGateK a) {
   }
 }
 
-// Backward.  A workgroup covers `cols` (head, 8 elements) columns -- all of them up to 256 -- times R = blockDim / cols row lanes,
+// Backward.  A workgroup covers the `cols` (head, 8 elements) columns times R = blockDim / cols row lanes,
 // and walks `rows_per_lane` rows per lane (every R-th row of its strip), so that a wave reads whole token rows, the weight
 // gradient is accumulated in registers over the rows of a lane, through LDS over the R lanes, and leaves as one partial
 // row per workgroup.  The kernel streams (5 x 2 bytes per element, 3 x 2 without a gate); what bounds a small call is how much of it is in
 // flight, so the rows per lane follow from the size (norm_bwd_plan).  Both launches together: at 32 rows per thread whatever the size,
 // 4096 rows of 12 x 64 made 48 workgroups and took 34.4 us gated and 21.0 us plain, now 12.1 and 9.2 us; 65536 rows of 16 x 128
 // stay at 32 rows (262 and 150 us, 5.1 and 5.4 TB/s); 1 M rows of one 128-element head 183 -> 142 us (fewer partials).
+// More than 256 columns: one row lane, and the (strip, column) pairs are dealt out in order, so that the workgroups of the same rows run
+// side by side and no lane idles (workgroups of 256 columns, all strips of the first columns in front: 32768 rows of 32 x 128 303 instead of 263 us).
 template <typename Tr, int D, int ACT>
 __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const NormGateK a) {
   constexpr int CH = D / 8;
   __shared__ __align__(16) float dw_s[256][8];
-  const int tid = threadIdx.x, rl = tid / a.cols, cl = tid - rl * a.cols;
-  const int R = blockDim.x / a.cols;                    // row lanes (threads beyond R * cols idle)
-  const int col = blockIdx.y * a.cols + cl;
-  const bool live = rl < R && col < a.G * CH;
+  const int tid = threadIdx.x;
+  const bool wide = a.cols > 256;
+  const int64_t flat = (int64_t)blockIdx.x * 256 + tid;
+  const int64_t strip = wide ? flat / a.cols : blockIdx.x;
+  const int rl = wide ? 0 : tid / a.cols;
+  const int col = wide ? (int)(flat - strip * a.cols) : tid - rl * a.cols;
+  const int R = wide ? 1 : blockDim.x / a.cols;         // row lanes (threads beyond R * cols idle)
+  const bool live = rl < R && strip * R * a.rows_per_lane < a.R;
   const int hh = live ? col / CH : 0;
   const int64_t off = live ? (int64_t)col * 8 : 0;
-  const int64_t r0 = (int64_t)blockIdx.x * R * a.rows_per_lane;
+  const int64_t r0 = strip * R * a.rows_per_lane;
   const int64_t r1 = min((int64_t)a.R, r0 + (int64_t)R * a.rows_per_lane);
   float w[8], dw[8];
   {
@@ -164,7 +170,7 @@ __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const NormGateK a) {
     for (int e = 0; e < 8; ++e) dw_s[tid][e] = dw[e];
     __syncthreads();
     const float* flat = &dw_s[0][0];
-    float* p = a.dw_partial + (int64_t)blockIdx.x * a.G * D;   // (R > 1: one workgroup holds all columns)
+    float* p = a.dw_partial + strip * a.G * D;
     for (int j = tid; j < a.cols * 8; j += blockDim.x) {
       float sum = flat[j];
 #pragma unroll 8
@@ -172,7 +178,7 @@ __global__ __launch_bounds__(256) void norm_gate_bwd_kernel(const NormGateK a) {
       p[j] = sum;
     }
   } else if (live) {
-    float* p = a.dw_partial + (int64_t)blockIdx.x * a.G * D + off;
+    float* p = a.dw_partial + strip * a.G * D + off;
     const f32x4 lo = {dw[0], dw[1], dw[2], dw[3]}, hi = {dw[4], dw[5], dw[6], dw[7]};
     *reinterpret_cast<f32x4*>(p) = lo;
     *reinterpret_cast<f32x4*>(p + 4) = hi;
@@ -219,7 +225,7 @@ __global__ __launch_bounds__(1024) void reduce_rows_kernel(const float* __restri
 FOX_NG_INST_ALL(Bf16)
 FOX_NG_INST_ALL(Fp16)
 
-// How the backward of `rows` rows of G heads is cut: columns per workgroup, row lanes, rows per lane, workgroups along the rows.
+// How the backward of `rows` rows of G heads is cut: columns, row lanes, rows per lane, strips of lanes * rows_per_lane rows (one partial each).
 struct NormBwdPlan {
   int cols, lanes, rows_per_lane;
   int64_t strips;
@@ -227,11 +233,10 @@ struct NormBwdPlan {
 constexpr int kNormRowsPerLane = 32;   // at most
 static NormBwdPlan norm_bwd_plan(int64_t rows, int G, int D) {
   NormBwdPlan p;
-  const int all = G * (D / 8), chunks = (all + 255) / 256;
-  p.cols = all < 256 ? all : 256;
-  p.lanes = 256 / p.cols;
+  p.cols = G * (D / 8);
+  p.lanes = p.cols > 256 ? 1 : 256 / p.cols;
   // about four workgroups per CU, at least four rows per lane (what it keeps in flight)
-  int64_t per = rows * chunks / ((int64_t)p.lanes * 4 * kCus);
+  int64_t per = rows * ((p.cols + 255) / 256) / ((int64_t)p.lanes * 4 * kCus);
   per = per < 4 ? 4 : per > kNormRowsPerLane ? kNormRowsPerLane : per;
   p.rows_per_lane = (int)per;
   p.strips = (rows + p.lanes * per - 1) / (p.lanes * per);
@@ -262,7 +267,8 @@ static hipError_t norm_gate_d(const NormGateK& a, bool bwd, int act, hipStream_t
   NormGateK k = a;
   k.cols = p.cols;
   k.rows_per_lane = p.rows_per_lane;
-  const dim3 grid((unsigned)p.strips, (unsigned)((a.G * CH + p.cols - 1) / p.cols)), block((unsigned)((p.cols * p.lanes + 63) / 64 * 64));
+  const bool wide = p.cols > 256;
+  const dim3 grid((unsigned)(wide ? (p.strips * p.cols + 255) / 256 : p.strips)), block(wide ? 256u : (unsigned)((p.cols * p.lanes + 63) / 64 * 64));
   if (act == kActSwish) hipLaunchKernelGGL((norm_gate_bwd_kernel<Tr, D, kActSwish>), grid, block, 0, s, k);
   else if (act == kActNone) hipLaunchKernelGGL((norm_gate_bwd_kernel<Tr, D, kActNone>), grid, block, 0, s, k);
   else hipLaunchKernelGGL((norm_gate_bwd_kernel<Tr, D, kActSigmoid>), grid, block, 0, s, k);

@@ -62,6 +62,13 @@ def test_shapes(gng, shape, G):
     _case(gng, shape, G, torch.bfloat16, "sigmoid", seed=shape[0])
 
 
+# more than 256 columns of 8 elements: the last that one workgroup holds, the first that it does not, strips that end inside a
+# workgroup, rows that end inside a strip
+@pytest.mark.parametrize("rows,G,D", [(130, 16, 128), (130, 17, 128), (1, 20, 128), (77, 33, 128), (259, 40, 64), (5, 129, 16), (2049, 65, 32)])
+def test_wide_rows(gng, rows, G, D):
+    _case(gng, (rows, G * D), G, torch.bfloat16, "sigmoid", seed=rows + G)
+
+
 def test_layer_configuration_and_weight_dtype(gng):
     """The FoX layer's call: (B, T, hidden) bf16, groups = heads, eps 1e-6 (modeling_forgetting_transformer.py:243)."""
     _case(gng, (2, 300, 16 * 128), 16, torch.bfloat16, "sigmoid", seed=2, eps=1e-6, w_dtype=torch.bfloat16)
