@@ -229,7 +229,7 @@ struct FwdPlan {
 };
 FwdPlan plan_fwd(const fox_dims& d, bool pruned, bool scratch) {
   FwdPlan p;
-  p.wanted = scratch ? fox::fwd_key_splits(d.B, d.H, d.M, d.N) : 1;
+  p.wanted = scratch ? fox::fwd_key_splits(d.B, d.H, d.M, d.N, d.D) : 1;
   p.pair = fox::fwd_pairs(d.B, d.H, d.M, d.N, d.D, pruned, p.wanted);
   p.splits = p.pair ? 1 : p.wanted;
   return p;
@@ -445,7 +445,7 @@ int fox_qk_norm_threshold(const float* q_weight, const float* k_weight, int32_t 
 int fox_attn_fwd_workspace_bytes(const fox_dims* dims, int64_t* bytes) {
   FOX_TRY(check_dims(dims));
   if (!bytes) return fail(FOX_E_ARG, "bytes is NULL");
-  *bytes = split_bytes(*dims, fox::fwd_key_splits(dims->B, dims->H, dims->M, dims->N));
+  *bytes = split_bytes(*dims, fox::fwd_key_splits(dims->B, dims->H, dims->M, dims->N, dims->D));
   return FOX_OK;
 }
 

@@ -739,10 +739,12 @@ bool fwd_pairs(int B, int H, int M, int N, int D, bool pruned, int splits) {
 // prefill, decode).  Splits are sized to give every CU at most two workgroups: one workgroup more would
 // run in a second round of its own (B2 H16 M333 N5333 D128: six splits, 576 workgroups, 60 us; five, 480, 50 us).  Between one
 // and two tiles per CU, tiles of equal weight are halved (the two rounds then even out what a CU with two tiles and one with a single
-// tile differ by); under a causal triangle the folded launch order evens that out already.  The streaming
+// tile differ by); under a causal triangle the folded launch order evens that out already.  Head dims up to 64 hold three workgroups on a CU
+// (kFwdWaves): where two splits leave some CUs with a single one, three fill them (B8 H8 M333 N12000 D32 two / three splits 107 / 95 us, N3000 37.9 / 36.5;
+// causal B1 H5 T5333 D64 50.5 / 45.0), but for the causal grids of up to 2560 keys that the paired kernel takes.  The streaming
 // kernel of the single-query case keeps no tile in LDS and takes about eight per CU, at
 // least 512 keys each.
-int fwd_key_splits(int B, int H, int M, int N) {
+int fwd_key_splits(int B, int H, int M, int N, int D) {
   if (M == 1) {
     const int64_t bh = (int64_t)B * H;
     int64_t splits = (2048 + bh - 1) / bh;
@@ -754,6 +756,7 @@ int fwd_key_splits(int B, int H, int M, int N) {
   const int key_tiles = (N + kFwdBN - 1) / kFwdBN;
   if (wgs >= 2 * kCus || key_tiles < 16) return 1;
   int splits = wgs > kCus && even_tiles(M, N) ? 2 : (int)(2 * kCus / wgs);
+  if (D <= 64 && splits == 2 && wgs < kCus && (even_tiles(M, N) || N > 2560)) splits = 3;
   splits = splits > key_tiles / 8 ? key_tiles / 8 : splits;
   splits = splits > 32 ? 32 : splits;
   return splits < 1 ? 1 : splits;

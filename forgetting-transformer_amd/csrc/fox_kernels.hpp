@@ -169,7 +169,7 @@ constexpr int order_groups(int n_bh, int tiles, int M, int N, int D, int64_t row
 }
 
 hipError_t launch_fwd(const FwdK& a, int D, int dtype, hipStream_t s);
-int fwd_key_splits(int B, int H, int M, int N);
+int fwd_key_splits(int B, int H, int M, int N, int D);
 bool fwd_pairs(int B, int H, int M, int N, int D, bool pruned, int splits);
 hipError_t launch_bwd_delta(const BwdK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_bwd_dkdv(const BwdK& a, int D, int dtype, hipStream_t s);   // a.cls selects the variant and its tiles

@@ -36,6 +36,13 @@ def test_key_splits(fa, B, H, M, N, D):
     run_case(fa, B, H, M, N, D, seed=M + N, gate_mean=2.0)
 
 
+# three splits at head dims up to 64 where two would leave some CUs with one workgroup: tiles of equal weight, a causal triangle
+@pytest.mark.parametrize("B,H,M,N", [(8, 8, 333, 1500), (5, 8, 600, 2000), (1, 10, 2600, 2600)])
+@pytest.mark.parametrize("D", [16, 64])
+def test_three_key_splits(fa, B, H, M, N, D):
+    run_case(fa, B, H, M, N, D, seed=M + N, gate_mean=2.0)
+
+
 # few query tiles: two groups of waves share a tile's walk.  Walks of one tile (group 1 has none), of odd and even length, with three,
 # four and five interior tiles (where the pipelined path begins), with left padding inside the walk and without a diagonal-free part
 @pytest.mark.parametrize("B,H,M,N", [(1, 2, 257, 513), (2, 3, 512, 512), (1, 3, 449, 577), (1, 3, 513, 576), (2, 2, 640, 640),

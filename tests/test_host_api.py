@@ -403,6 +403,11 @@ def test_forward_plan():
     assert plan(2, 16, 2048, 2048, 64) == (1, False) and plan(4, 16, 16384, 16384, 128) == (1, False)
     assert plan(16, 16, 128, 32768, 128) == (2, False) and plan(2, 16, 333, 5333, 128) == (5, False)
     assert plan(1, 12, 1, 1500, 64)[1] is False
+    # three workgroups of head dim 64 and less to a CU: three splits instead of two on some, except where the paired kernel takes over
+    for D, n in ((16, 3), (32, 3), (64, 3), (128, 2)):
+        assert plan(8, 8, 333, 5333, D) == (n, False) and plan(1, 9, 2600, 2600, D) == plan(1, 9, 2600, 2600, D, pruned=1) == (n, False)
+        assert plan(8, 8, 500, 5333, D) == (2, False)                 # two splits fill every CU twice
+        assert plan(1, 9, 2560, 2560, D) == ((2, False) if D == 16 else (1, True))
     for M, N in ((1, 1), (1, 4096), (128, 600), (300, 600), (301, 600), (1000, 1000), (1025, 2560), (1025, 2561), (8192, 8192)):
         for H in (1, 7, 16, 33, 40, 64):
             for D in (16, 32, 64, 128):
