@@ -241,7 +241,7 @@ __global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(
   const int kb = DSPLIT ? wave >> 1 : wave;   // block of 32 keys this wave owns
   const int dh = DSPLIT ? wave & 1 : 0;       // half of the head dim it accumulates
   int bh, nt;
-  decode_block(blockIdx.x, a.n_tiles, a.B * a.H, a.groups, !a.even && (D <= 64 || DSPLIT), bh, nt);
+  decode_block(blockIdx.x, a.n_tiles, a.B * a.H, a.groups, !a.even && (D <= 64 || DSPLIT), false, bh, nt);
   nt = a.n_tiles - 1 - nt;  // the first key tiles see the most query rows: start them first
   const int b = bh / a.H, h = bh % a.H;
   const int M = a.M, N = a.N, p_seq = N - M;
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK a) {
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 5, i = lane & 31;
   int bh, mt;
-  decode_block(blockIdx.x, a.n_tiles, a.B * a.H, a.groups, !a.even, bh, mt);
+  decode_block(blockIdx.x, a.n_tiles, a.B * a.H, a.groups, !a.even, true, bh, mt);
   const int b = bh / a.H, h = bh % a.H;
   const int M = a.M, N = a.N, p_seq = N - M;
   const int m0 = mt * BM;

@@ -435,8 +435,12 @@ __device__ __forceinline__ float nonzero_scale(float s) { return fabsf(s) < 1e-3
 // `fold`: when the whole grid is resident at two workgroups per CU, the second workgroup of a CU is the one that arrives
 // kCus ids after the first.  Taken in the same order both would be heavy on one CU and both light on another; from
 // workgroup kCus on the list is therefore walked from its light end (forward B1 H16 T4096 D128: 109 -> 84 us, dQ 152 -> 116 us).
+// `last_first`: the pairs from the last to the first.  The dQ kernel takes them so, between a forward and a dK/dV kernel that start with the
+// first: each of the three then opens on the tensors its predecessor touched last, which are still in the 256 MiB last-level cache.
+// Backward with dQ ascending / descending: B4 T16384 H16 D128 "auto" 731 / 710 us, B16 H16 T4096 D64 "auto" 516 / 491,
+// B4 H32 T4096 D64 at -10 240 / 229, without a threshold 963 / 953.
 constexpr int kXcds = 8, kCus = 256;
-__device__ __forceinline__ void decode_block(int wid, int n_tiles, int n_bh, int groups, bool fold, int& bh, int& tile) {
+__device__ __forceinline__ void decode_block(int wid, int n_tiles, int n_bh, int groups, bool fold, bool last_first, int& bh, int& tile) {
   const bool by_xcd = n_bh % kXcds == 0;
   const int nb = by_xcd ? n_bh / kXcds : n_bh, cus = by_xcd ? kCus / kXcds : kCus;
   const int total = n_tiles * nb;
@@ -455,6 +459,7 @@ __device__ __forceinline__ void decode_block(int wid, int n_tiles, int n_bh, int
     b = (big ? 0 : extra * (small + 1)) + grp * size + in % size;
     tile = n_tiles - 1 - in / size;
   }
+  if (last_first) b = nb - 1 - b;
   bh = by_xcd ? b * kXcds + wid % kXcds : b;
 }
 

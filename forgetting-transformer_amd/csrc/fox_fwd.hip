@@ -276,11 +276,11 @@ __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's o
   int bh, mt, sp = 0;
   if constexpr (SPLIT) {  // (query tile, key split) pairs take the place of query tiles
     int mts;
-    decode_block(blockIdx.x, a.n_mtiles * a.splits, a.B * a.H, a.groups, !a.even, bh, mts);
+    decode_block(blockIdx.x, a.n_mtiles * a.splits, a.B * a.H, a.groups, !a.even, false, bh, mts);
     mt = mts / a.splits;
     sp = mts % a.splits;
   } else {
-    decode_block(blockIdx.x, a.n_mtiles, a.B * a.H, a.groups, !a.even && !PAIR, bh, mt);   // paired: one workgroup per CU
+    decode_block(blockIdx.x, a.n_mtiles, a.B * a.H, a.groups, !a.even && !PAIR, false, bh, mt);   // paired: one workgroup per CU
   }
   const int b = bh / a.H, h = bh % a.H;
   const int M = a.M, N = a.N, p_seq = N - M;
