@@ -242,8 +242,9 @@ int64_t split_bytes(const fox_dims& d, int splits) {
 // library's own array (fox_attn_fwd_noalloc).  workspace == NULL never splits keys.
 // epi: the norm-and-gate epilogue (already validated), or NULL.  With an epilogue, shapes the unsplit kernel does
 // not handle run the plain forward followed by the standalone norm kernel.
+// gates: the forward from the gates (already validated, for a shape it takes), or NULL.
 int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes, void* stream, const char* what,
-             const fox_fwd_epilogue* epi = nullptr) {
+             const fox_fwd_epilogue* epi = nullptr, const fox_gates* gates = nullptr) {
   FOX_TRY(check_dims(&args->dims));
   FOX_TRY(check_view(&args->q, "q"));
   FOX_TRY(check_view(&args->k, "k"));
@@ -251,7 +252,7 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
   if (!(epi && !args->o.ptr)) FOX_TRY(check_view(&args->o, "o"));
   FOX_TRY(check_extent(&args->k, args->dims.N, args->dims.D, "k"));
   FOX_TRY(check_extent(&args->v, args->dims.N, args->dims.D, "v"));
-  if (!args->log_lambda || !args->lse) return fail(FOX_E_ARG, "log_lambda and lse must not be NULL");
+  if (!(args->log_lambda || gates) || !args->lse) return fail(FOX_E_ARG, "log_lambda and lse must not be NULL");
   fox::FwdK k{};
   k.q = to_view(args->q);
   k.k = to_view(args->k);
@@ -267,7 +268,7 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
   k.n_mtiles = (args->dims.M + fox::kFwdBM - 1) / fox::kFwdBM;
   k.groups = fox::order_groups(k.B * k.H, k.n_mtiles, k.M, k.N, args->dims.D, k.k.st, k.thr != nullptr);
   k.even = fox::even_tiles(k.M, k.N);
-  const FwdPlan plan = plan_fwd(args->dims, k.thr != nullptr, workspace != nullptr);
+  const FwdPlan plan = plan_fwd(args->dims, k.thr != nullptr, workspace != nullptr || gates);   // (with gates: pairs in place of splits, or neither)
   k.splits = plan.splits;
   k.pair = plan.pair;
   k.stream = k.n_mtiles == 1 && (int64_t)k.B * k.H * k.N * args->dims.D * 4 >= g_stream_min_kv_bytes.load(std::memory_order_relaxed);
@@ -280,7 +281,7 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
       k.ws_ml = k.ws_o + (int64_t)k.splits * k.B * k.H * k.M * args->dims.D;
     }
   }
-  const bool split_shape = k.M == 1 || plan.wanted > 1;
+  const bool split_shape = k.M == 1 || (plan.wanted > 1 && !gates);
   if (epi) {
     const int D = args->dims.D;
     if (split_shape) {
@@ -309,7 +310,22 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
     k.epi.eps = epi->eps;
     k.epi.act = epi->activation;
   }
-  return check_hip(fox::launch_fwd(k, args->dims.D, args->dims.dtype, (hipStream_t)stream), what);
+  if (!gates) return check_hip(fox::launch_fwd(k, args->dims.D, args->dims.dtype, (hipStream_t)stream), what);
+  k.gates = fox::GateK{gates->g, gates->stride_b, gates->stride_h, gates->stride_n, gates->is_logit ? gates->dtype : fox::kGateLog,
+                       const_cast<float*>(args->log_lambda), gates->log_fgate};
+  return check_hip(fox::launch_fwd_gates(k, args->dims.D, args->dims.dtype, (hipStream_t)stream), what);
+}
+
+int check_epilogue(const fox_fwd_args* args, const fox_fwd_epilogue* epi) {
+  if (!args || !epi) return fail(FOX_E_ARG, "args and epilogue must not be NULL");
+  if (epi->activation != FOX_ACT_SIGMOID && epi->activation != FOX_ACT_SWISH && epi->activation != FOX_ACT_NONE)
+    return fail(FOX_E_ARG, "activation must be FOX_ACT_SIGMOID, FOX_ACT_SWISH or FOX_ACT_NONE (got %d)", epi->activation);
+  FOX_TRY(check_view(&epi->y, "y"));
+  if (epi->activation != FOX_ACT_NONE) FOX_TRY(check_view(&epi->gate, "gate"));
+  if (!epi->weight || !epi->rstd) return fail(FOX_E_ARG, "weight and rstd must not be NULL");
+  if (((uintptr_t)epi->weight & 15) != 0) return fail(FOX_E_ALIGN, "weight must be 16-byte aligned");
+  if (epi->y.ptr == args->o.ptr) return fail(FOX_E_ARG, "y must not alias o");
+  return FOX_OK;
 }
 
 }  // namespace
@@ -317,8 +333,8 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
 extern "C" {
 
 // 0.2.x: fox_bwd_args and the scan entry points differ from 0.1.0; 0.2.1 adds fox_set_stream_min_kv_bytes and fox_probe_mfma, 0.2.2
-// fox_attn_decode, fox_cache_append, fox_qk_norm_threshold and fox_attn_fwd_plan
-int fox_version(void) { return 202; }
+// fox_attn_decode, fox_cache_append, fox_qk_norm_threshold and fox_attn_fwd_plan, 0.2.3 fox_attn_fwd_gates and fox_attn_fwd_takes_gates
+int fox_version(void) { return 203; }
 
 const char* fox_last_error(void) { return g_err; }
 
@@ -343,15 +359,28 @@ int fox_tile_config(int32_t D, int32_t* block_m, int32_t* block_n, int32_t* kv_b
 }
 
 int fox_attn_fwd_norm_gate(const fox_fwd_args* args, const fox_fwd_epilogue* epi, void* stream) {
-  if (!args || !epi) return fail(FOX_E_ARG, "args and epilogue must not be NULL");
-  if (epi->activation != FOX_ACT_SIGMOID && epi->activation != FOX_ACT_SWISH && epi->activation != FOX_ACT_NONE)
-    return fail(FOX_E_ARG, "activation must be FOX_ACT_SIGMOID, FOX_ACT_SWISH or FOX_ACT_NONE (got %d)", epi->activation);
-  FOX_TRY(check_view(&epi->y, "y"));
-  if (epi->activation != FOX_ACT_NONE) FOX_TRY(check_view(&epi->gate, "gate"));
-  if (!epi->weight || !epi->rstd) return fail(FOX_E_ARG, "weight and rstd must not be NULL");
-  if (((uintptr_t)epi->weight & 15) != 0) return fail(FOX_E_ALIGN, "weight must be 16-byte aligned");
-  if (epi->y.ptr == args->o.ptr) return fail(FOX_E_ARG, "y must not alias o");
+  FOX_TRY(check_epilogue(args, epi));
   return fwd_impl(args, args->workspace, args->workspace_bytes, stream, "fox_attn_fwd_norm_gate", epi);
+}
+
+int fox_attn_fwd_takes_gates(const fox_dims* dims, int32_t pruned, int32_t* yes) {
+  FOX_TRY(check_dims(dims));
+  if (!yes) return fail(FOX_E_ARG, "yes is NULL");
+  const FwdPlan p = plan_fwd(*dims, pruned != 0, true);
+  *yes = fox::fwd_scans(dims->B, dims->H, dims->M, dims->N, p.splits);
+  return FOX_OK;
+}
+
+int fox_attn_fwd_gates(const fox_fwd_args* args, const fox_gates* gates, const fox_fwd_epilogue* epi, void* stream) {
+  if (!args || !gates) return fail(FOX_E_ARG, "args and gates must not be NULL");
+  if (epi) FOX_TRY(check_epilogue(args, epi));
+  if (!gates->g) return fail(FOX_E_ARG, "g is NULL");
+  if (gates->is_logit ? gates->dtype < FOX_DTYPE_BF16 || gates->dtype > FOX_DTYPE_FP32 : gates->dtype != FOX_DTYPE_FP32)
+    return fail(FOX_E_ARG, "gates: dtype must be FOX_DTYPE_BF16, FP16 or FP32 for logits and FP32 for log gates (got %d)", gates->dtype);
+  int32_t yes = 0;
+  FOX_TRY(fox_attn_fwd_takes_gates(&args->dims, args->threshold != nullptr, &yes));
+  if (!yes) return fail(FOX_E_ARG, "fox_attn_fwd_gates does not take this shape (fox_attn_fwd_takes_gates)");
+  return fwd_impl(args, nullptr, 0, stream, "fox_attn_fwd_gates", epi, gates);
 }
 
 int fox_norm_gate_fwd(const fox_norm_gate_args* args, void* stream) {

@@ -292,6 +292,53 @@ __device__ __forceinline__ float half_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Forget-gate logits in fp32, bf16 or fp16 (the output of the gate projection of the FoX layer).
+template <int DT>
+__device__ __forceinline__ float load_logit(const void* p, int64_t i) {
+  if constexpr (DT == 2) return reinterpret_cast<const float*>(p)[i];
+  const uint32_t w = reinterpret_cast<const uint16_t*>(p)[i];
+  if constexpr (DT == 0) return Bf16::lo(w);
+  return Fp16::lo(w);
+}
+// logsigmoid(x) = min(x, 0) - log1p(exp(-|x|)), stable on both sides, from the hardware exp / log:
+// log1p(z) for z in (0, 1] is log(u) + (z - (u - 1)) / u with u = fl(1 + z), which repairs the rounding
+// of 1 + z (absolute error ~1e-8, and log1p(z) -> z for tiny z as it must).  The result is clamped to <= 0:
+// a log gate is never positive, and the pruning bounds rely on the cumulative sums not increasing, whatever
+// the last bit of the hardware logarithm does near u = 1.
+__device__ __forceinline__ float log_sigmoid(float x) {
+  const float z = __expf(-fabsf(x));
+  const float u = 1.0f + z;
+  const float l = fmaxf(__logf(u) + __fdividef(z - (u - 1.0f), u), 0.f);
+  return fminf(fminf(x, 0.f) - l, 0.f);
+}
+
+// ---------------------------------------------------------------------------
+// Scan over the 64 lanes of a wave in fp64
+// ---------------------------------------------------------------------------
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double x) {   // x of the lane a DPP control selects; zero where there is none
+  const uint64_t v = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWS, 0xf, true);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, ROWS, 0xf, true);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+// Sum of x over lanes 0 .. own.  Executed by a whole wave.
+__device__ __forceinline__ double wave_scan(double x) {
+  x += dpp_move<0x111, 0xf>(x);   // row_shr 1, 2, 4, 8: within rows of sixteen lanes
+  x += dpp_move<0x112, 0xf>(x);
+  x += dpp_move<0x114, 0xf>(x);
+  x += dpp_move<0x118, 0xf>(x);
+  x += dpp_move<0x142, 0xa>(x);   // row_bcast 15 into rows 1 and 3
+  x += dpp_move<0x143, 0xc>(x);   // row_bcast 31 into rows 2 and 3
+  return x;
+}
+__device__ __forceinline__ double lane_before(double x) { return dpp_move<0x138, 0xf>(x); }   // wave_shr 1; zero in lane 0
+__device__ __forceinline__ double of_lane(double x, int lane) {   // lane: wave-uniform
+  const uint64_t v = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, lane), hi = __builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
 // Store a wave's transposed accumulator block as rows of 16-bit values.  Lane (g, i) holds row i of
 // 32 rows; register r of acc[db] is column 32*db + 8*(r/4) + 4*g + r%4.  Written straight to global
 // memory that is 8 bytes per lane scattered over 32 rows; staged through a wave-private LDS area of

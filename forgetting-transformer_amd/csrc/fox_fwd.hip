@@ -233,6 +233,71 @@ struct TileDma {
   }
 };
 
+// Cumulative sums c[n] = sum of the gates of keys seq .. n (zero left of seq) for n < hi, into LDS.  As in scan_row: coalesced through LDS,
+// consecutive keys per thread, fp64, rounded once.  Positions from `first` to hi are also stored for the backward, as are the log gates of
+// logits.  fetch() requests the gates: it comes before the tile loads, which the counter of loads in flight retires in order, and the barriers
+// below wait for LDS only, so the tiles and Q arrive while the sums are formed.
+template <int NT>
+struct OwnScan {
+  static constexpr int MAX = (kOwnScanMaxKeys / NT + 1) | 1;   // keys per thread: odd, so that a wave's reads fall on different banks
+  float g[MAX];
+
+  static __device__ __forceinline__ void barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+  template <int KIND>
+  __device__ __forceinline__ void fetch_as(const GateK& t, int64_t row, int hi, int tid) {
+#pragma unroll
+    for (int e = 0; e < MAX; ++e) {
+      if (e * NT >= hi) break;
+      const int64_t i = row + min(e * NT + tid, hi - 1) * t.sn;
+      if constexpr (KIND == kGateLog) g[e] = reinterpret_cast<const float*>(t.g)[i];
+      else g[e] = load_logit<KIND>(t.g, i);
+    }
+  }
+  __device__ __forceinline__ void fetch(const GateK& t, int b, int h, int hi, int tid) {
+    const int64_t row = b * t.sb + h * t.sh;
+    if (t.kind == kGateLog) fetch_as<kGateLog>(t, row, hi, tid);
+    else if (t.kind == 0) fetch_as<0>(t, row, hi, tid);
+    else if (t.kind == 1) fetch_as<1>(t, row, hi, tid);
+    else fetch_as<2>(t, row, hi, tid);
+  }
+  __device__ __forceinline__ void run(const GateK& t, float* c_s, int64_t out_row, int hi, int seq, int first, int tid) {
+    __shared__ double wave_tot[NT / kWave];
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+#pragma unroll
+    for (int e = 0; e < MAX; ++e) {
+      if (e * NT >= hi) break;
+      const int n = e * NT + tid;
+      if (t.kind != kGateLog) {
+        g[e] = log_sigmoid(g[e]);
+        if (t.log_fgate && n >= first && n < hi) t.log_fgate[out_row + n] = g[e];
+      }
+      if (n < hi) c_s[n] = n >= seq ? g[e] : 0.f;
+    }
+    barrier();
+    const int per = ((hi + NT - 1) / NT) | 1, n0 = tid * per;
+    double v[MAX], sum = 0.0;
+#pragma unroll
+    for (int e = 0; e < MAX; ++e) {
+      if (e >= per) break;
+      sum += n0 + e < hi ? (double)c_s[n0 + e] : 0.0;
+      v[e] = sum;
+    }
+    const double incl = wave_scan(sum);
+    if (lane == kWave - 1) wave_tot[wave] = incl;
+    barrier();
+    double before = lane_before(incl);
+    for (int w = 0; w < wave; ++w) before += wave_tot[w];
+#pragma unroll
+    for (int e = 0; e < MAX; ++e) {
+      if (e >= per) break;
+      if (n0 + e < hi) c_s[n0 + e] = (float)(before + v[e]);
+    }
+    barrier();
+    if (t.c)
+      for (int n = first + tid; n < hi; n += NT) t.c[out_row + n] = c_s[n];
+  }
+};
+
 // EPI: the variant whose epilogue also applies the layer's output norm and gate (a.epi); a variant of its own so
 // that the plain kernel's register allocation is not touched by it.
 // Waves per SIMD the forward is compiled for: the register budget that goes with it (512 / waves) holds the
@@ -249,13 +314,18 @@ constexpr int kFwdWaves = D <= 64 ? 3 : 2;
 // merges the two states from LDS before the epilogue.  The walk of the heaviest tile, which is what such a grid waits for, is half
 // as long, and a CU with a single query tile has two waves per SIMD (B1 H16 T3001 D128, scan included: 67.7 -> 57.6 us).  Both groups pass the same barriers: the trip counts of
 // the loops are those of group 0, and a step for which group 1 has no tile left moves and computes nothing.
-template <typename Tr, int D, bool SPLIT, bool EPI, bool STREAM, bool PAIR>
+//
+// SCAN: the workgroup forms the cumulative sums of its row itself, from the log gates or their logits, up to its last key, and keeps them in
+// LDS; each writes the part of its own rows for the backward.  Every workgroup of a row repeats the sum of what lies in front of it, so this is for
+// grids of few workgroups per CU (fwd_scans, with the times), where it takes the scan's launch out of the chain.
+template <typename Tr, int D, bool SPLIT, bool EPI, bool STREAM, bool PAIR, bool SCAN>
 __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's only argument
   static_assert(!(PAIR && (SPLIT || STREAM)), "the paired variant is for whole walks over shared tiles");
   static_assert(!PAIR || D >= 32, "group 1's accumulators are handed over in its tile buffers");
   constexpr int GROUPS = PAIR ? 2 : 1;
   static_assert(!(SPLIT && EPI), "partial results of a key split are not normalised");
   static_assert(!(STREAM && EPI), "no streaming variant with the epilogue");
+  static_assert(!(SCAN && (SPLIT || STREAM)), "own sums are for whole walks over shared tiles");
   constexpr int AUX = STREAM ? kLoadNonTemporal : 0;
   constexpr int BM = kFwdBM, BN = kFwdBN;
   constexpr int KK = D / 16, DB = (D + 31) / 32, NB = BN / 32;
@@ -285,7 +355,8 @@ __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's o
   const int b = bh / a.H, h = bh % a.H;
   const int M = a.M, N = a.N, p_seq = N - M;
   const int m0 = mt * BM;
-  const float* c_row = a.c + (int64_t)bh * N;
+  __shared__ float c_s[SCAN ? kOwnScanMaxKeys : 1];
+  const float* c_row = SCAN ? c_s : a.c + (int64_t)bh * N;   // (own sums: [0, hi))
   const uint16_t* qp = a.q.ptr + b * a.q.sb + h * a.q.sh;
   const uint16_t* kp = a.k.ptr + b * a.k.sb + h * a.k.sh;
   const uint16_t* vp = a.v.ptr + b * a.v.sb + h * a.v.sh;
@@ -305,6 +376,8 @@ __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's o
   // Everything the workgroup needs first is requested before anything is waited for.  The first tile to
   // visit (the one under the end of the diagonal) does not depend on the pruning bound, so it goes
   // first; then Q, then the per-row and per-key terms; the bound search's loads queue behind them.
+  OwnScan<GROUPS * 256> scan;
+  if constexpr (SCAN) scan.fetch(a.gates, b, h, hi, threadIdx.x);
   const DirectTileLoader<D, BN, 4, AUX> kld(a.k.st, wave, lane), vld(a.v.st, wave, lane);
   int n0_first = hi > 0 ? ((hi - 1) / BN) * BN : 0;
   bool early = !SPLIT && hi > (min(seq, hi) / BN) * BN && (n0_first + BN - 1 > a0 || !(qk_scale > 0.f));
@@ -331,8 +404,9 @@ __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's o
   }
   u32x4 qreg[KK];
   load_row_operand_regs<D>(qreg, qp, a.q.st, m, M, g);
+  if constexpr (SCAN) scan.run(a.gates, c_s, (int64_t)bh * N, hi, seq, mt == 0 ? 0 : a0, threadIdx.x);
   const float c_ref = c_row[a0];
-  const float c_m = c_row[min(a_m, N - 1)];
+  const float c_m = c_row[min(a_m, (SCAN ? hi : N) - 1)];
   // Under pruning the third tile of the walk (the look-back tile, which is also the next query tile's upper diagonal
   // tile) is wanted more often than not, but its LDS buffer is busy until the first tile is done.  One dword per cache
   // line brings it into L2 now, while the neighbour fetches it as well (pruned forward 0.253 -> 0.246 ms at B4 T16384
@@ -353,16 +427,26 @@ __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's o
   // Key terms of a tile: the load is requested here, the arithmetic on it is done where the value goes to
   // LDS (a tile later), so that nothing waits for the load in between.  Masked keys get -inf through the
   // subtraction.
+  // (Own sums are in LDS already: only the tile is kept.)
   float cn_raw = 0.f;
   bool cn_ok = false;
+  int cn_n0 = 0;
   auto issue_cn = [&](int n0) {
-    if (tid < BN) {
+    cn_n0 = n0;
+    if (!SCAN && tid < BN) {
       const int n = n0 + tid;
       cn_ok = (n < N) & (n >= seq);
       cn_raw = c_row[min(n, N - 1)];
     }
   };
-  auto cn_term = [&]() { return (c_ref - (cn_ok ? cn_raw : INFINITY)) * kLog2e * inv_scale; };
+  auto cn_term = [&]() {
+    if constexpr (SCAN) {
+      const int n = cn_n0 + tid;
+      return (c_ref - (n < N && n >= seq ? c_s[min(n, hi - 1)] : INFINITY)) * kLog2e * inv_scale;
+    } else {
+      return (c_ref - (cn_ok ? cn_raw : INFINITY)) * kLog2e * inv_scale;
+    }
+  };
   auto issue = [&](int n0, char* kt, char* vt) {
     issue_cn(n0);  // small load first: vmcnt retires in order, so it must not queue behind the tile loads
     kld.issue(kp, a.k.st, n0, N, kt);
@@ -371,7 +455,7 @@ __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's o
   if (early) issue_cn(n0_first);
   float cn_raw2 = 0.f;   // key terms of the second early tile: handed to cn_raw once the first tile's are in LDS
   bool cn_ok2 = false;
-  if (early2 && tid < BN) {
+  if (!SCAN && early2 && tid < BN) {
     const int n = n0_second + tid;
     cn_ok2 = (n < N) & (n >= seq);
     cn_raw2 = c_row[min(n, N - 1)];
@@ -423,7 +507,7 @@ __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's o
   if (n_diag > 0) {
     if (!early && n_tiles - 1 - grp >= t_stop) issue(tile_n0(n_tiles - 1 - grp), k_tile0, v_tile0);
     if (tid < BN) cn_s0[tid] = cn_term();
-    if (early2) { cn_raw = cn_raw2; cn_ok = cn_ok2; }
+    if (early2) { cn_raw = cn_raw2; cn_ok = cn_ok2; cn_n0 = n0_second; }
   }
   bool requested = early2;  // buffers 1 already hold (or await) the next tile
   for (int tu = n_tiles - 1; tu >= t_stop; tu -= 2 * GROUPS) {
@@ -585,13 +669,26 @@ __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's o
 template <typename Tr, int D, bool SPLIT, bool EPI = false, bool STREAM = false>
 __global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_kernel(const FwdK a) {
 #ifdef __HIP_DEVICE_COMPILE__
-  fwd_body<Tr, D, SPLIT, EPI, STREAM, false>(a);
+  fwd_body<Tr, D, SPLIT, EPI, STREAM, false, false>(a);
 #endif
 }
 template <typename Tr, int D, bool EPI>
 __global__ __launch_bounds__(512, 2) void fwd_pair_kernel(const FwdK a) {
 #ifdef __HIP_DEVICE_COMPILE__
-  fwd_body<Tr, D, false, EPI, false, true>(a);
+  fwd_body<Tr, D, false, EPI, false, true, false>(a);
+#endif
+}
+// The same two with their own cumulative sums
+template <typename Tr, int D, bool EPI>
+__global__ __launch_bounds__(256, kFwdWaves<D>) void fwd_scan_kernel(const FwdK a) {
+#ifdef __HIP_DEVICE_COMPILE__
+  fwd_body<Tr, D, false, EPI, false, false, true>(a);
+#endif
+}
+template <typename Tr, int D, bool EPI>
+__global__ __launch_bounds__(512, 2) void fwd_scan_pair_kernel(const FwdK a) {
+#ifdef __HIP_DEVICE_COMPILE__
+  fwd_body<Tr, D, false, EPI, false, true, true>(a);
 #endif
 }
 
@@ -664,6 +761,20 @@ constexpr int kStreamMaxQueryTiles = 1;
   template __global__ void fwd_pair_kernel<TR, 32, true>(const FwdK);    \
   template __global__ void fwd_pair_kernel<TR, 64, true>(const FwdK);    \
   template __global__ void fwd_pair_kernel<TR, 128, true>(const FwdK);   \
+  template __global__ void fwd_scan_kernel<TR, 16, false>(const FwdK);   \
+  template __global__ void fwd_scan_kernel<TR, 32, false>(const FwdK);   \
+  template __global__ void fwd_scan_kernel<TR, 64, false>(const FwdK);   \
+  template __global__ void fwd_scan_kernel<TR, 128, false>(const FwdK);  \
+  template __global__ void fwd_scan_kernel<TR, 16, true>(const FwdK);    \
+  template __global__ void fwd_scan_kernel<TR, 32, true>(const FwdK);    \
+  template __global__ void fwd_scan_kernel<TR, 64, true>(const FwdK);    \
+  template __global__ void fwd_scan_kernel<TR, 128, true>(const FwdK);   \
+  template __global__ void fwd_scan_pair_kernel<TR, 32, false>(const FwdK);  \
+  template __global__ void fwd_scan_pair_kernel<TR, 64, false>(const FwdK);  \
+  template __global__ void fwd_scan_pair_kernel<TR, 128, false>(const FwdK); \
+  template __global__ void fwd_scan_pair_kernel<TR, 32, true>(const FwdK);   \
+  template __global__ void fwd_scan_pair_kernel<TR, 64, true>(const FwdK);   \
+  template __global__ void fwd_scan_pair_kernel<TR, 128, true>(const FwdK);  \
   template __global__ void combine_kernel<TR, 16>(const FwdK);           \
   template __global__ void combine_kernel<TR, 32>(const FwdK);           \
   template __global__ void combine_kernel<TR, 64>(const FwdK);           \
@@ -701,6 +812,32 @@ static hipError_t launch_fwd_d(const FwdK& a, int dtype, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <typename Tr, int D>
+static hipError_t launch_fwd_gates_d(const FwdK& a, hipStream_t s) {
+  if (a.M == 1 || a.splits > 1 || a.N > kOwnScanMaxKeys) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(a.n_mtiles * a.B * a.H));
+  if constexpr (D >= 32) {
+    if (a.pair) {
+      if (a.epi.y.ptr) hipLaunchKernelGGL((fwd_scan_pair_kernel<Tr, D, true>), grid, dim3(512), 0, s, a);
+      else hipLaunchKernelGGL((fwd_scan_pair_kernel<Tr, D, false>), grid, dim3(512), 0, s, a);
+      return hipGetLastError();
+    }
+  }
+  if (a.epi.y.ptr) hipLaunchKernelGGL((fwd_scan_kernel<Tr, D, true>), grid, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((fwd_scan_kernel<Tr, D, false>), grid, dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+template <typename Tr>
+static hipError_t launch_fwd_gates_t(const FwdK& a, int D, hipStream_t s) {
+  switch (D) {
+    case 16: return launch_fwd_gates_d<Tr, 16>(a, s);
+    case 32: return launch_fwd_gates_d<Tr, 32>(a, s);
+    case 64: return launch_fwd_gates_d<Tr, 64>(a, s);
+    case 128: return launch_fwd_gates_d<Tr, 128>(a, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 template <typename Tr>
 static hipError_t launch_fwd_t(const FwdK& a, int D, int dtype, hipStream_t s) {
   switch (D) {
@@ -714,6 +851,21 @@ static hipError_t launch_fwd_t(const FwdK& a, int D, int dtype, hipStream_t s) {
 
 hipError_t launch_fwd(const FwdK& a, int D, int dtype, hipStream_t s) {
   return dtype == 0 ? launch_fwd_t<Bf16>(a, D, dtype, s) : launch_fwd_t<Fp16>(a, D, dtype, s);
+}
+
+hipError_t launch_fwd_gates(const FwdK& a, int D, int dtype, hipStream_t s) {
+  return dtype == 0 ? launch_fwd_gates_t<Bf16>(a, D, s) : launch_fwd_gates_t<Fp16>(a, D, s);
+}
+
+// Whether the forward forms the cumulative sums itself (fwd_scan_kernel) instead of reading what a scan left.  The scan is a launch and
+// 3 to 6 us of one workgroup per row; own sums cost a workgroup 1 to 2 us, most of it while its first tiles arrive, but every workgroup.
+// Forward with its scan / with own sums, us.  Resident grids (up to two workgroups per CU), any row: B1 H12 N77 D64 8.9 / 6.9, B4 H12 N512 14.7 / 12.8,
+// B1 H16 N3001 D128 57.0 / 54.2, B2 H12 N2048 D64 at -10 15.0 / 13.5, B1 H16 N3500 D128 at -10 22.9 / 19.7.  Up to four per CU: short rows, B8 H16 N768 D64 22.9 / 21.5,
+// B16 H32 N256 20.8 / 20.5, not long ones (B4 H16 N1500 D128 55.8 / 55.8).  Beyond that every round repeats the sums: B8 H12 N2048 D64 70.6 / 71.4,
+// B16 H16 N3500 475 / 499.
+bool fwd_scans(int B, int H, int M, int N, int splits) {
+  const int64_t wgs = (int64_t)((M + kFwdBM - 1) / kFwdBM) * B * H;
+  return M > 1 && splits <= 1 && N <= kOwnScanMaxKeys && (wgs <= 2 * kCus || (wgs <= 4 * kCus && N <= 1024));
 }
 
 // Whether the forward takes the paired variant (fwd_pair_kernel): less than two query tiles per CU under a causal triangle, where the

@@ -21,6 +21,17 @@ struct FwdEpilogue {
   int act;
 };
 
+// Gates of a forward that forms their cumulative sums itself (fwd_body).
+struct GateK {
+  const void* g;       // log gates (fp32), or logits
+  int64_t sb, sh, sn;  // element strides
+  int kind;            // kGateLog, or the dtype of the logits
+  float* c;            // (B,H,N) or null: the cumulative sums, for a backward
+  float* log_fgate;    // (B,H,N) or null: the log gates of logits
+};
+enum : int { kGateLog = -1 };            // else 0 bf16, 1 fp16, 2 fp32 logits
+constexpr int kOwnScanMaxKeys = 3584;    // what fits beside the tiles in LDS at every head dim and occupancy
+
 struct FwdK {
   View q, k, v, o;
   const float* c;
@@ -39,6 +50,7 @@ struct FwdK {
   float* ws_ml;    // (splits, B, H, M, 2) partial row maximum and row sum
   FwdEpilogue epi; // only for splits == 1 and M > 1 (the launcher rejects it otherwise)
   bool stream;     // K and V tiles are read once and not again soon: load them with the non-temporal hint
+  GateK gates;     // launch_fwd_gates only, which does not read c
 };
 
 // Single-query forward from the log gates (decode_gates_kernel).
@@ -169,6 +181,8 @@ constexpr int order_groups(int n_bh, int tiles, int M, int N, int D, int64_t row
 }
 
 hipError_t launch_fwd(const FwdK& a, int D, int dtype, hipStream_t s);
+hipError_t launch_fwd_gates(const FwdK& a, int D, int dtype, hipStream_t s);   // unsplit, at most kOwnScanMaxKeys keys, M > 1
+bool fwd_scans(int B, int H, int M, int N, int splits);
 int fwd_key_splits(int B, int H, int M, int N, int D);
 bool fwd_pairs(int B, int H, int M, int N, int D, bool pruned, int splits);
 hipError_t launch_bwd_delta(const BwdK& a, int D, int dtype, hipStream_t s);

@@ -125,31 +125,11 @@ __global__ __launch_bounds__(NT) void scan_kernel(const float* __restrict__ in, 
       [&](int idx, float sum) { dst[(int64_t)idx * on] = (REVERSE && idx <= seq) ? 0.f : sum; });
 }
 
-// Forget-gate logits in fp32, bf16 or fp16 (the output of the gate projection of the FoX layer).
-template <int DT>
-__device__ __forceinline__ float load_logit(const void* p, int64_t i) {
-  if constexpr (DT == 2) return reinterpret_cast<const float*>(p)[i];
-  const uint32_t w = reinterpret_cast<const uint16_t*>(p)[i];
-  if constexpr (DT == 0) return Bf16::lo(w);
-  return Fp16::lo(w);
-}
 template <int DT>
 __device__ __forceinline__ void store_logit(void* p, int64_t i, float x) {
   if constexpr (DT == 2) reinterpret_cast<float*>(p)[i] = x;
   else if constexpr (DT == 0) reinterpret_cast<uint16_t*>(p)[i] = (uint16_t)(Bf16::pack2(x, 0.f) & 0xffffu);
   else reinterpret_cast<uint16_t*>(p)[i] = (uint16_t)(Fp16::pack2(x, 0.f) & 0xffffu);
-}
-
-// logsigmoid(x) = min(x, 0) - log1p(exp(-|x|)), stable on both sides, from the hardware exp / log:
-// log1p(z) for z in (0, 1] is log(u) + (z - (u - 1)) / u with u = fl(1 + z), which repairs the rounding
-// of 1 + z (absolute error ~1e-8, and log1p(z) -> z for tiny z as it must).  The result is clamped to <= 0:
-// a log gate is never positive, and the pruning bounds rely on the cumulative sums not increasing, whatever
-// the last bit of the hardware logarithm does near u = 1.
-__device__ __forceinline__ float log_sigmoid(float x) {
-  const float z = __expf(-fabsf(x));
-  const float u = 1.0f + z;
-  const float l = fmaxf(__logf(u) + __fdividef(z - (u - 1.0f), u), 0.f);
-  return fminf(fminf(x, 0.f) - l, 0.f);
 }
 
 // c[n] = sum_{seq_start <= l <= n} logsigmoid(x[l]) in one pass over the logits; optionally also

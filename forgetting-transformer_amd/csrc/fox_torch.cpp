@@ -115,12 +115,20 @@ Forward run_forward(Attention& a, const Tensor& q, const Tensor& k, const Tensor
   Tensor ws;
   if (ws_bytes > 0) ws = empty_bytes_like(q, ws_bytes);
   float* base = f.rows.mutable_data_ptr<float>();
-  if (a.is_logit) {   // logsigmoid fused into the scan; the fp32 log gates are a by-product
+  // short rows and small grids: the forward takes the gates as they are; else their cumulative sums come from a scan in front of it
+  // (logits: with logsigmoid fused in; the fp32 log gates are a by-product)
+  int32_t from_gates = 0;
+  check(fox_attn_fwd_takes_gates(&dims, a.threshold.defined(), &from_gates), "fox_attn_fwd_takes_gates");
+  fox_gates gates{g.const_data_ptr(), a.is_logit, a.is_logit ? gate_dtype(g) : FOX_DTYPE_FP32, g.stride(0), a.gs_h(g), a.gs_n(g), nullptr};
+  if (a.is_logit) {
     f.log_fgate = at::empty({a.B, a.H, a.N}, q.options().dtype(at::kFloat));
-    check(fox_gate_cumsum_fwd(g.const_data_ptr(), gate_dtype(g), g.stride(0), a.gs_h(g), a.gs_n(g), a.seq_ptr(),
-                              f.log_fgate.mutable_data_ptr<float>(), base, dims.B, dims.H, dims.N, stream), "fox_gate_cumsum_fwd");
-  } else {
-    check(fox_cumsum_fwd(g.const_data_ptr<float>(), g.stride(0), a.gs_h(g), a.gs_n(g), a.seq_ptr(), base, dims.B, dims.H, dims.N,
+    gates.log_fgate = f.log_fgate.mutable_data_ptr<float>();
+  }
+  if (!from_gates && a.is_logit) {
+    check(fox_gate_cumsum_fwd(gates.g, gates.dtype, gates.stride_b, gates.stride_h, gates.stride_n, a.seq_ptr(), gates.log_fgate, base, dims.B,
+                              dims.H, dims.N, stream), "fox_gate_cumsum_fwd");
+  } else if (!from_gates) {
+    check(fox_cumsum_fwd(g.const_data_ptr<float>(), gates.stride_b, gates.stride_h, gates.stride_n, a.seq_ptr(), base, dims.B, dims.H, dims.N,
                          stream), "fox_cumsum_fwd");
   }
   fox_fwd_args args{};
@@ -138,7 +146,8 @@ Forward run_forward(Attention& a, const Tensor& q, const Tensor& k, const Tensor
   if (!a.epilogue) {
     f.out = f.o = at::empty_like(q);
     args.o = view_of(f.o, a.head_first);
-    check(fox_attn_fwd(&args, stream), "fox_attn_fwd");
+    if (from_gates) check(fox_attn_fwd_gates(&args, &gates, nullptr, stream), "fox_attn_fwd_gates");
+    else check(fox_attn_fwd(&args, stream), "fox_attn_fwd");
     return f;
   }
   // o and y as rows of heads * head_dim per token: what the norm's backward and the output projection read
@@ -153,7 +162,8 @@ Forward run_forward(Attention& a, const Tensor& q, const Tensor& k, const Tensor
   epi.rstd = f.rstd.mutable_data_ptr<float>();
   epi.eps = (float)a.eps;
   epi.activation = a.act;
-  check(fox_attn_fwd_norm_gate(&args, &epi, stream), "fox_attn_fwd_norm_gate");
+  if (from_gates) check(fox_attn_fwd_gates(&args, &gates, &epi, stream), "fox_attn_fwd_gates");
+  else check(fox_attn_fwd_norm_gate(&args, &epi, stream), "fox_attn_fwd_norm_gate");
   if (a.head_first) {
     f.o = f.o.transpose(1, 2);
     f.out = f.out.transpose(1, 2);

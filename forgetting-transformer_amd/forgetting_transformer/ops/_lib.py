@@ -112,6 +112,15 @@ class FwdEpilogue(C.Structure):
     ]
 
 
+class Gates(C.Structure):
+    _fields_ = [
+        ("g", C.c_void_p),
+        ("is_logit", C.c_int32), ("dtype", C.c_int32),
+        ("stride_b", C.c_int64), ("stride_h", C.c_int64), ("stride_n", C.c_int64),
+        ("log_fgate", C.c_void_p),
+    ]
+
+
 # every symbol include/fox_attn.h declares: name -> (restype, argtypes)
 SIGNATURES = {
     "fox_version": (C.c_int, []),
@@ -138,6 +147,8 @@ SIGNATURES = {
     "fox_attn_fwd_plan": (C.c_int, [C.POINTER(Dims), C.c_int32, C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.POINTER(C.c_int64)]),
     "fox_attn_decode": (C.c_int, [C.POINTER(FwdArgs), C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p]),
     "fox_attn_decode_workspace_bytes": (C.c_int, [C.POINTER(Dims), C.POINTER(C.c_int64)]),
+    "fox_attn_fwd_gates": (C.c_int, [C.POINTER(FwdArgs), C.POINTER(Gates), C.POINTER(FwdEpilogue), C.c_void_p]),
+    "fox_attn_fwd_takes_gates": (C.c_int, [C.POINTER(Dims), C.c_int32, C.POINTER(C.c_int32)]),
     "fox_cache_append": (C.c_int, [C.c_void_p, C.c_void_p]),   # fox_cache_append_args, filled by the host extension
     "fox_attn_bwd_delta": (C.c_int, [C.POINTER(BwdArgs), C.c_void_p]),
     "fox_attn_bwd_dkdv": (C.c_int, [C.POINTER(BwdArgs), C.c_void_p]),

@@ -378,6 +378,21 @@ typedef struct fox_fwd_epilogue {
 
 int fox_attn_fwd_norm_gate(const fox_fwd_args* args, const fox_fwd_epilogue* epilogue, void* stream);
 
+/*
+ * The forward straight from the gates: what fox_cumsum_fwd or fox_gate_cumsum_fwd followed by fox_attn_fwd or, with an epilogue,
+ * fox_attn_fwd_norm_gate compute, in one launch.  Of args, log_lambda is written (NULL = not wanted) and the workspace is not used.
+ * For the shapes that fox_attn_fwd_takes_gates names only, FOX_E_ARG otherwise: every workgroup repeats the sum of the gates in front of its
+ * rows, which pays for short rows and small grids.
+ */
+typedef struct fox_gates {
+  const void* g;                         /* (B,H,N): fp32 log forget gates, or their logits */
+  int32_t is_logit, dtype;               /* dtype: FOX_DTYPE_*, of logits; log gates are FP32 */
+  int64_t stride_b, stride_h, stride_n;  /* in elements */
+  float* log_fgate;                      /* NULL, or (B,H,N) contiguous: the log gates, written from logits */
+} fox_gates;
+int fox_attn_fwd_gates(const fox_fwd_args* args, const fox_gates* gates, const fox_fwd_epilogue* epilogue, void* stream);
+int fox_attn_fwd_takes_gates(const fox_dims* dims, int32_t pruned, int32_t* yes);
+
 #ifdef __cplusplus
 }
 #endif
