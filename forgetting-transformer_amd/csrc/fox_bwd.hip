@@ -8,6 +8,7 @@
 //                  registers as MFMA B operands; dK^T, dV^T accumulators) and
 //                  walks the query tiles below its diagonal; writes dk, dv and
 //                  dc[n] = drow[n - (N - M)] - sum_i dS[i,n].
+//   bwd_kernel   : both kinds of workgroups in one launch, for small grids (bwd_together).
 //   delta_kernel : delta alone (a stage of its own for callers that want it;
 //                  the backward does not launch it).
 // Every kernel only stores: no read-modify-write of anything another kernel wrote,
@@ -223,26 +224,28 @@ __device__ __forceinline__ void dkdv_step_interior(const char* q_tile, const cha
 // waves share 32 keys, each recomputing S and dP and accumulating one half of the head dim of dK and dV, so that
 // the kernel fits in 256 registers; a workgroup is 64 keys x 2 halves with query steps of 64 rows, and two
 // workgroups (two waves per SIMD) share a CU.
-template <typename Tr, int D, bool DSPLIT>
-__global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(const BwdK a) {
+//
+// OWN_DELTA: the body forms delta = sum_d o_id * do_id for the rows of a step itself instead of reading what the dQ kernel left, so
+// that it can run beside it (bwd_kernel).  A wave takes the rows whose dO it has brought into LDS: its own wait is enough to read
+// them, and the barrier that publishes the step's tiles publishes their delta as well.
+template <int D, bool DSPLIT>
+struct DkdvLds {
+  static constexpr int BMQ = DSPLIT ? 64 : kKvBM;
+  char *q_tile0, *q_tile1, *do_tile0, *do_tile1;   // Tile<D>::bytes(BMQ) each
+  float *rc_s0, *rc_s1, *dl_s0, *dl_s1;            // BMQ each
+};
+template <typename Tr, int D, bool DSPLIT, bool OWN_DELTA>
+__device__ __forceinline__ void dkdv_body(const BwdK& a, int bh, int nt, const DkdvLds<D, DSPLIT>& lds) {
   constexpr int BN = DSPLIT ? 64 : kKvBN, BMQ = DSPLIT ? 64 : kKvBM;
   constexpr int KK = D / 16, DB = (D + 31) / 32, NDB = DSPLIT ? DB / 2 : DB, DW = DSPLIT ? D / 2 : D;
   static_assert(!DSPLIT || DB % 2 == 0, "the head dim splits into two halves of whole 32-column blocks");
-  __shared__ __align__(16) char q_tile0[Tile<D>::bytes(BMQ)];
-  __shared__ __align__(16) char q_tile1[Tile<D>::bytes(BMQ)];
-  __shared__ __align__(16) char do_tile0[Tile<D>::bytes(BMQ)];
-  __shared__ __align__(16) char do_tile1[Tile<D>::bytes(BMQ)];
-  __shared__ __align__(16) float rc_s0[BMQ];
-  __shared__ __align__(16) float rc_s1[BMQ];
-  __shared__ __align__(16) float dl_s0[BMQ];
-  __shared__ __align__(16) float dl_s1[BMQ];
+  static_assert(!OWN_DELTA || D <= 64, "the long-loop path and the split variant read delta");
+  char *q_tile0 = lds.q_tile0, *q_tile1 = lds.q_tile1, *do_tile0 = lds.do_tile0, *do_tile1 = lds.do_tile1;
+  float *rc_s0 = lds.rc_s0, *rc_s1 = lds.rc_s1, *dl_s0 = lds.dl_s0, *dl_s1 = lds.dl_s1;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 5, i = lane & 31;
   const int kb = DSPLIT ? wave >> 1 : wave;   // block of 32 keys this wave owns
   const int dh = DSPLIT ? wave & 1 : 0;       // half of the head dim it accumulates
-  int bh, nt;
-  decode_block(blockIdx.x, a.n_tiles, a.B * a.H, a.groups, !a.even && (D <= 64 || DSPLIT), false, bh, nt);
-  nt = a.n_tiles - 1 - nt;  // the first key tiles see the most query rows: start them first
   const int b = bh / a.H, h = bh % a.H;
   const int M = a.M, N = a.N, p_seq = N - M;
   const int n0 = nt * BN;
@@ -254,6 +257,7 @@ __global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(
   }
   const float* lse_row = a.lse + (int64_t)bh * M;
   const float* delta_row = a.delta + (int64_t)bh * M;
+  const uint16_t* op = a.o.ptr + b * a.o.sb + h * a.o.sh;   // (read with OWN_DELTA only)
   const uint16_t* qp = a.q.ptr + b * a.q.sb + h * a.q.sh;
   const uint16_t* kp = a.k.ptr + b * a.k.sb + h * a.k.sh;
   const uint16_t* vp = a.v.ptr + b * a.v.sb + h * a.v.sh;
@@ -274,6 +278,35 @@ __global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(
   // Everything the workgroup needs first is requested before anything is waited for: the tile of the
   // first diagonal step (it does not depend on the pruning bound), K and V, then the per-row terms.
   const DirectTileLoader<D, BMQ> qld(a.q.st, wave, lane), dold(a.d_o.st, wave, lane);
+  // The wave's own rows of a step: its j-th load brings one 1 KiB block of the tile into LDS, 16 bytes per lane in lane order, and o is
+  // fetched in the same order, so that the CH lanes of a row hold matching pieces of o and dO (whole rows: operand-shaped loads move a
+  // quarter of the bytes per clock).
+  constexpr int CH = D / 8, OPER = OWN_DELTA ? DirectTileLoader<D, BMQ>::PER : 0, ORPB = Tile<D>::RPB;
+  static_assert(!OWN_DELTA || DirectTileLoader<D, BMQ>::NBLK % 4 == 0, "every wave has whole blocks of the step");
+  const DirectTileLoader<D, BMQ> old(a.o.st, wave, lane);
+  u32x4 o_raw[OPER > 0 ? OPER : 1];
+  auto issue_o = [&](int ms) {
+    if constexpr (OWN_DELTA) {
+      const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<uint16_t*>(op + (int64_t)ms * a.o.st), 0, old.extent(a.o.st, ms, M), 0x00020000);
+#pragma unroll
+      for (int j = 0; j < OPER; ++j) o_raw[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, old.voff[j], 0, 0));
+    }
+  };
+  auto store_own_delta = [&](const char* dot, float* dl) {   // after the wave's own loads have landed; rows past M are zeros
+    if constexpr (OWN_DELTA) {
+      const int line = lane >> 4, row0 = (line * 16 + ((lane & 15) ^ (line << 2))) / CH;
+#pragma unroll
+      for (int j = 0; j < OPER; ++j) {
+        const u32x4 x = *reinterpret_cast<const u32x4*>(dot + (wave + 4 * j) * Tile<D>::BLOCK_BYTES + 16 * lane);
+        float part = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part += Tr::lo(o_raw[j][e]) * Tr::lo(x[e]) + Tr::hi(o_raw[j][e]) * Tr::hi(x[e]);
+        part = row_sum<CH>(part);
+        if (lane % CH == 0) dl[(wave + 4 * j) * ORPB + row0] = -part;
+      }
+    }
+  };
   const bool early = m_lo < M && p_seq + m_lo < n0 + BN - 1 && !(n0 + BN <= seq);
   if (early) {
     qld.issue(qp, a.q.st, m_lo, M, q_tile1);
@@ -313,7 +346,7 @@ __global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(
       row_ok = mm < M;
       l_raw = lse_row[mc];
       c_raw = c_row[p_seq + mc];
-      d_raw = delta_row[mc];
+      if constexpr (!OWN_DELTA) d_raw = delta_row[mc];
     }
   };
   auto rc_term = [&]() {
@@ -325,8 +358,12 @@ __global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(
     issue_rows(ms);  // small loads first: vmcnt retires in order, so they must not queue behind the tile
     qld.issue(qp, a.q.st, ms, M, qt);
     dold.issue(dop, a.d_o.st, ms, M, dot);
+    issue_o(ms);
   };
-  if (early) issue_rows(m_lo);
+  if (early) {
+    issue_rows(m_lo);
+    issue_o(m_lo);
+  }
   const float colc = (n < N && n >= seq) ? (c_key - c_ref) * kLog2e : INFINITY;
 
   f32x16 dkacc[NDB], dvacc[NDB];
@@ -375,21 +412,28 @@ __global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(
     // between the two buffer sets, starting with set 1 (which the early request above has filled): the next step's
     // tiles are requested before the current one is computed.
     auto step_rows = [&](int idx) { return idx < n_diag ? m_lo + idx * BMQ : m_top - (idx - n_diag) * BMQ; };
+    auto store_rows = [&](const char* dot, float* rc, float* dl) {
+      if (row_lane) {
+        rc[row_slot] = rc_term();
+        if constexpr (!OWN_DELTA) dl[row_slot] = dl_term();
+      }
+      wait_vmem_all();
+      if constexpr (OWN_DELTA) {
+        __builtin_amdgcn_sched_barrier(0);   // the reads below stay behind the wait
+        store_own_delta(dot, dl);
+      }
+    };
     if (n_steps > 0) {
       if (!early) issue(step_rows(0), q_tile1, do_tile1);
-      if (row_lane) { rc_s1[row_slot] = rc_term(); dl_s1[row_slot] = dl_term(); }
+      store_rows(do_tile1, rc_s1, dl_s1);
     }
     for (int idx = 0; idx < n_steps; ++idx) {
       const bool odd = idx & 1;
-      wait_vmem_all();
       __syncthreads();
       if (idx + 1 < n_steps) issue(step_rows(idx + 1), odd ? q_tile1 : q_tile0, odd ? do_tile1 : do_tile0);
       dkdv_step<Tr, D, BMQ, NDB>(odd ? q_tile0 : q_tile1, odd ? do_tile0 : do_tile1, odd ? rc_s0 : rc_s1, odd ? dl_s0 : dl_s1, kreg,
                                  vreg, dkacc, dvacc, csum, p_seq + step_rows(idx), n, n_w0, qk_scale, colc, lane, dh * NDB);
-      if (idx + 1 < n_steps && row_lane) {
-        (odd ? rc_s1 : rc_s0)[row_slot] = rc_term();
-        (odd ? dl_s1 : dl_s0)[row_slot] = dl_term();
-      }
+      if (idx + 1 < n_steps) store_rows(odd ? do_tile1 : do_tile0, odd ? rc_s1 : rc_s0, odd ? dl_s1 : dl_s0);
     }
   } else {
   for (int t = 0; t < n_diag; ++t) {
@@ -456,7 +500,10 @@ __global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(
   // gradient w.r.t. the cumulative sum: the row sum the dQ kernel left for the query row that sits at this key
   // position (none left of the first query row) minus this key's column sum
   if (n < N && g == 0 && dh == 0) {  // (the two waves of a split pair hold the same column sums)
-    const float rtot = n >= p_seq ? a.drow[(int64_t)bh * M + (n - p_seq)] : 0.f;
+    float rtot = 0.f;   // (beside the dQ kernel: the reverse scan adds it)
+    if constexpr (!OWN_DELTA) {
+      if (n >= p_seq) rtot = a.drow[(int64_t)bh * M + (n - p_seq)];
+    }
     a.dc[(int64_t)bh * N + n] = rtot - ctot;
   }
   // dK and dV leave through LDS (the tile buffers are free now) so that the global stores are whole rows (of the
@@ -466,6 +513,25 @@ __global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(
   char* stage = (wave < 2 ? q_tile0 : do_tile0) + (wave & 1) * kStoreStageBytes<DW>;
   store_rows_via_lds<Tr, DW>(stage, dkacc, a.sm_scale, dkp + dh * DW, a.dk.st, n_w0, N, lane);
   store_rows_via_lds<Tr, DW>(stage, dvacc, 1.0f, dvp + dh * DW, a.dv.st, n_w0, N, lane);
+}
+
+template <typename Tr, int D, bool DSPLIT>
+__global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(const BwdK a) {
+  constexpr int BMQ = DkdvLds<D, DSPLIT>::BMQ;
+  __shared__ __align__(16) char q_tile0[Tile<D>::bytes(BMQ)];
+  __shared__ __align__(16) char q_tile1[Tile<D>::bytes(BMQ)];
+  __shared__ __align__(16) char do_tile0[Tile<D>::bytes(BMQ)];
+  __shared__ __align__(16) char do_tile1[Tile<D>::bytes(BMQ)];
+  __shared__ __align__(16) float rc_s0[BMQ];
+  __shared__ __align__(16) float rc_s1[BMQ];
+  __shared__ __align__(16) float dl_s0[BMQ];
+  __shared__ __align__(16) float dl_s1[BMQ];
+#ifdef __HIP_DEVICE_COMPILE__
+  int bh, nt;
+  decode_block(blockIdx.x, a.n_tiles, a.B * a.H, a.groups, !a.even && (D <= 64 || DSPLIT), false, bh, nt);
+  nt = a.n_tiles - 1 - nt;  // the first key tiles see the most query rows: start them first
+  dkdv_body<Tr, D, DSPLIT, false>(a, bh, nt, {q_tile0, q_tile1, do_tile0, do_tile1, rc_s0, rc_s1, dl_s0, dl_s1});
+#endif
 }
 
 // ---------------------------------------------------------------------------
@@ -514,20 +580,19 @@ __device__ __forceinline__ void dq_tile(const char* k_tile, const char* v_tile, 
   }
 }
 
+template <int D>
+struct DqLds {
+  char *k_tile0, *k_tile1, *v_tile0, *v_tile1;   // Tile<D>::bytes(kFwdBN) each
+  float *cn_s0, *cn_s1;                          // kFwdBN each
+};
 template <typename Tr, int D>
-__global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK a) {
+__device__ __forceinline__ void dq_body(const BwdK& a, int bh, int mt, const DqLds<D>& lds) {
   constexpr int BM = kFwdBM, BN = kFwdBN;
   constexpr int KK = D / 16, DB = (D + 31) / 32;
-  __shared__ __align__(16) char k_tile0[Tile<D>::bytes(BN)];
-  __shared__ __align__(16) char k_tile1[Tile<D>::bytes(BN)];
-  __shared__ __align__(16) char v_tile0[Tile<D>::bytes(BN)];
-  __shared__ __align__(16) char v_tile1[Tile<D>::bytes(BN)];
-  __shared__ __align__(16) float cn_s0[BN];
-  __shared__ __align__(16) float cn_s1[BN];
+  char *k_tile0 = lds.k_tile0, *k_tile1 = lds.k_tile1, *v_tile0 = lds.v_tile0, *v_tile1 = lds.v_tile1;
+  float *cn_s0 = lds.cn_s0, *cn_s1 = lds.cn_s1;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 5, i = lane & 31;
-  int bh, mt;
-  decode_block(blockIdx.x, a.n_tiles, a.B * a.H, a.groups, !a.even, true, bh, mt);
   const int b = bh / a.H, h = bh % a.H;
   const int M = a.M, N = a.N, p_seq = N - M;
   const int m0 = mt * BM;
@@ -611,7 +676,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK a) {
     lo = max(lo, t * BN);
   }
   lo = (lo / BN) * BN;
-  if (a.q_first_block && tid == 0) a.q_first_block[(int64_t)bh * a.n_tiles + mt] = lo / BN;
+  if (a.q_first_block && tid == 0) a.q_first_block[(int64_t)bh * ((M + BM - 1) / BM) + mt] = lo / BN;
   const int n_tiles = (hi - lo + BN - 1) / BN;
 
   // rows past M and empty rows (lse = -inf) get rowc = -inf through the subtraction: no load behind a branch
@@ -675,6 +740,57 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK a) {
   store_rows_via_lds<Tr, D>(stage, dqacc, a.sm_scale, dqp, a.dq.st, m0 + 32 * wave, M, lane);
 }
 
+template <typename Tr, int D>
+__global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK a) {
+  __shared__ __align__(16) char k_tile0[Tile<D>::bytes(kFwdBN)];
+  __shared__ __align__(16) char k_tile1[Tile<D>::bytes(kFwdBN)];
+  __shared__ __align__(16) char v_tile0[Tile<D>::bytes(kFwdBN)];
+  __shared__ __align__(16) char v_tile1[Tile<D>::bytes(kFwdBN)];
+  __shared__ __align__(16) float cn_s0[kFwdBN];
+  __shared__ __align__(16) float cn_s1[kFwdBN];
+#ifdef __HIP_DEVICE_COMPILE__
+  int bh, mt;
+  decode_block(blockIdx.x, a.n_tiles, a.B * a.H, a.groups, !a.even, true, bh, mt);
+  dq_body<Tr, D>(a, bh, mt, {k_tile0, k_tile1, v_tile0, v_tile1, cn_s0, cn_s1});
+#endif
+}
+
+// ---------------------------------------------------------------------------
+// The kernel's argument block behind a pointer the compiler cannot see through: each kind of workgroup loads its arguments where it needs
+// them (loaded at entry, those of both would not fit the scalar registers).
+__device__ __forceinline__ const BwdK& own_arguments() {
+  typedef const BwdK __attribute__((address_space(4)))* kernarg;
+  kernarg p = (kernarg)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const BwdK*)p;
+}
+
+// dQ and dK/dV in one launch, for small grids of head dims up to 64: workgroups of either kind side by side, the heaviest of either kind first.
+// One after the other, each of the two kernels waits for its longest walk on a chip that is mostly idle.
+template <typename Tr, int D>
+__global__ __launch_bounds__(256, 2) void bwd_kernel(const BwdK a) {
+  static_assert(D <= 64 && kKvBM >= kFwdBN, "two workgroups of either kind per CU; the dQ walk fits the buffers of the dK/dV walk");
+  __shared__ __align__(16) char tile0[Tile<D>::bytes(kKvBM)];
+  __shared__ __align__(16) char tile1[Tile<D>::bytes(kKvBM)];
+  __shared__ __align__(16) char tile2[Tile<D>::bytes(kKvBM)];
+  __shared__ __align__(16) char tile3[Tile<D>::bytes(kKvBM)];
+  __shared__ __align__(16) float row0[kKvBM];
+  __shared__ __align__(16) float row1[kKvBM];
+  __shared__ __align__(16) float row2[kKvBM];
+  __shared__ __align__(16) float row3[kKvBM];
+#ifdef __HIP_DEVICE_COMPILE__
+  const int q_tiles = (a.M + kFwdBM - 1) / kFwdBM;
+  int bh, t;
+  decode_block(blockIdx.x, 2 * a.n_tiles, a.B * a.H, a.groups, !a.even, false, bh, t);
+  if (t & 1) {
+    const int mt = t / 2 - (a.n_tiles - q_tiles);   // (fewer query tiles than key tiles where M < N)
+    if (mt >= 0) dq_body<Tr, D>(own_arguments(), bh, mt, {tile0, tile1, tile2, tile3, row0, row1});
+  } else {
+    dkdv_body<Tr, D, false, true>(own_arguments(), bh, a.n_tiles - 1 - t / 2, {tile0, tile1, tile2, tile3, row0, row1, row2, row3});
+  }
+#endif
+}
+
 // explicit instantiations: every (dtype, head dim) pair the dispatchers can reach
 #define FOX_INSTANTIATE_BWD(KERNEL, TR)                      \
   template __global__ void KERNEL<TR, 16>(const BwdK);       \
@@ -693,6 +809,9 @@ FOX_INSTANTIATE_DKDV(Bf16)
 FOX_INSTANTIATE_DKDV(Fp16)
 FOX_INSTANTIATE_BWD(dq_kernel, Bf16)
 FOX_INSTANTIATE_BWD(dq_kernel, Fp16)
+#define FOX_INSTANTIATE_BOTH(TR)                               template __global__ void bwd_kernel<TR, 16>(const BwdK);     template __global__ void bwd_kernel<TR, 32>(const BwdK);     template __global__ void bwd_kernel<TR, 64>(const BwdK);
+FOX_INSTANTIATE_BOTH(Bf16)
+FOX_INSTANTIATE_BOTH(Fp16)
 
 // ---------------------------------------------------------------------------
 #define FOX_DISPATCH_D(KERNEL, GRID, SMEM)                                                        \
@@ -743,6 +862,22 @@ static hipError_t dq_t(const BwdK& a0, int D, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <typename Tr>
+static hipError_t bwd_t(const BwdK& a0, int D, hipStream_t s) {
+  BwdK a = a0;
+  a.n_tiles = (a.N + kKvBN - 1) / kKvBN;
+  a.groups = order_groups(a.B * a.H, a.n_tiles, a.M, a.N, D, a.k.st, a.thr != nullptr);
+  a.even = even_tiles(a.M, a.N);
+  const dim3 grid((unsigned)(2 * a.n_tiles * a.B * a.H));
+  switch (D) {
+    case 16: hipLaunchKernelGGL((bwd_kernel<Tr, 16>), grid, dim3(256), 0, s, a); break;
+    case 32: hipLaunchKernelGGL((bwd_kernel<Tr, 32>), grid, dim3(256), 0, s, a); break;
+    case 64: hipLaunchKernelGGL((bwd_kernel<Tr, 64>), grid, dim3(256), 0, s, a); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 bool dkdv_split_supports(int D) { return D == 128; }
 
 hipError_t launch_bwd_delta(const BwdK& a, int D, int dtype, hipStream_t s) {
@@ -750,6 +885,20 @@ hipError_t launch_bwd_delta(const BwdK& a, int D, int dtype, hipStream_t s) {
 }
 hipError_t launch_bwd_dkdv(const BwdK& a, int D, int dtype, hipStream_t s) {
   return dtype == 0 ? dkdv_t<Bf16>(a, D, s) : dkdv_t<Fp16>(a, D, s);
+}
+// Whether dQ and dK/dV go out as one launch (bwd_kernel).  One after the other, each waits for the longest walk of a grid that fills the chip
+// once or less; side by side the two waits are one, and so are two launches and the drain between them.  Backward, one after the other / together, us:
+// D 64 B1 H5 T3000 118 / 80, B2 H8 T2000 82 / 60, B4 H12 T512 31.9 / 27.8, B16 H16 T250 35.0 / 32.0, B2 H12 T2048 at -60 45.4 / 44.4; D 32 B3 H5 T777 34.6 / 29.3,
+// D 16 B4 H16 T1000 42.8 / 33.7.  Against it stand delta, formed anew for every step, and the LDS of the dK/dV walk, which the dQ walk does not
+// need: with more than 512 tiles of either kind at D 64 it goes either way (768: B12 H16 T500 51.2 / 50.3, B16 H24 T250 38.1 / 40.5; 2048: B8 H32 T1000
+// "auto" 87 / 99; 4096: B4 H32 T4096 980 / 1130).  Head dims up to 32 hold three workgroups per CU: 768 tiles B4 H24 T1000 at -10 35.1 / 32.7 and
+// 35.4 / 31.6, 2048 tiles B8 H16 T2048 D16 151 / 200.
+bool bwd_together(const BwdK& a, int D) {
+  if (D > 64 || a.o.st <= 0 || ((int64_t)kKvBM * a.o.st + D) * 2 >= (int64_t)1 << 31) return false;   // o through 32-bit offsets
+  return (int64_t)((a.N + kKvBN - 1) / kKvBN) * a.B * a.H <= (D == 64 ? 2 : 3) * kCus;
+}
+hipError_t launch_bwd(const BwdK& a, int D, int dtype, hipStream_t s) {
+  return dtype == 0 ? bwd_t<Bf16>(a, D, s) : bwd_t<Fp16>(a, D, s);
 }
 hipError_t launch_bwd_dq(const BwdK& a, int D, int dtype, hipStream_t s) {
   return dtype == 0 ? dq_t<Bf16>(a, D, s) : dq_t<Fp16>(a, D, s);

@@ -328,6 +328,28 @@ int check_epilogue(const fox_fwd_args* args, const fox_fwd_epilogue* epi) {
   return FOX_OK;
 }
 
+// dq, dk, dv and dlog_lambda, by the two stages one after the other or side by side in one launch.  In the latter case dlog_lambda
+// lacks the row sums of dS: *drow is where they are, for the scan that follows (null otherwise).
+int bwd_products(const fox_bwd_args* args, void* stream, const float** drow) {
+  fox::BwdK k;
+  FOX_TRY(make_bwd(args, k, true));
+  const fox_dims& d = args->dims;
+  *drow = nullptr;
+  if (!fox::bwd_together(k, d.D)) {
+    FOX_TRY(fox_attn_bwd_dq(args, stream));
+    return fox_attn_bwd_dkdv(args, stream);
+  }
+  FOX_TRY(check_view(&args->dq, "dq"));
+  FOX_TRY(check_view(&args->dk, "dk"));
+  FOX_TRY(check_view(&args->dv, "dv"));
+  k.dq = to_view(args->dq);
+  k.dk = to_view(args->dk);
+  k.dv = to_view(args->dv);
+  FOX_TRY(check_hip(fox::launch_bwd(k, d.D, d.dtype, (hipStream_t)stream), "fox_attn_bwd"));
+  *drow = k.drow;
+  return FOX_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -440,7 +462,7 @@ int fox_gate_cumsum_bwd(const float* dc, const void* logits, int32_t logits_dtyp
   if (logits_dtype < FOX_DTYPE_BF16 || logits_dtype > FOX_DTYPE_FP32) return fail(FOX_E_ARG, "logits_dtype must be FOX_DTYPE_BF16, FP16 or FP32 (got %d)", logits_dtype);
   if ((const void*)dc == dlogits || logits == dlogits) return fail(FOX_E_ARG, "dlogits must not alias dc or logits");
   return check_hip(fox::launch_gate_cumsum_bwd(dc, logits, logits_dtype, sb, sh, sn, seq_start, dlogits, db, dh, dn, B, H, N,
-                                               (hipStream_t)stream),
+                                               nullptr, N, (hipStream_t)stream),
                    "fox_gate_cumsum_bwd");
 }
 
@@ -450,7 +472,7 @@ int fox_cumsum_bwd(const float* dc, float* dg, int64_t dg_sb, int64_t dg_sh, int
   if (B <= 0 || H <= 0 || N <= 0) return fail(FOX_E_ARG, "B, H, N must be positive");
   if (dc == dg) return fail(FOX_E_ARG, "dc and dg must not alias");
   if (dg_sb == 0 && dg_sh == 0 && dg_sn == 0) { dg_sb = (int64_t)H * N; dg_sh = N; dg_sn = 1; }   // contiguous (B,H,N)
-  return check_hip(fox::launch_cumsum_bwd(dc, dg, dg_sb, dg_sh, dg_sn, seq_start, B, H, N, (hipStream_t)stream), "fox_cumsum_bwd");
+  return check_hip(fox::launch_cumsum_bwd(dc, dg, dg_sb, dg_sh, dg_sn, seq_start, B, H, N, nullptr, N, (hipStream_t)stream), "fox_cumsum_bwd");
 }
 
 int fox_auto_threshold(const fox_dims* dims, const fox_view* q, const fox_view* k, float sm_scale, float* thr,
@@ -609,10 +631,26 @@ int fox_attn_bwd_dq(const fox_bwd_args* args, void* stream) {
 int fox_attn_bwd(const fox_bwd_args* args, void* stream) {
   if (!args) return fail(FOX_E_ARG, "args is NULL");
   if (!args->dlog_fgate) return fail(FOX_E_ARG, "dlog_fgate is NULL");
-  FOX_TRY(fox_attn_bwd_dq(args, stream));
-  FOX_TRY(fox_attn_bwd_dkdv(args, stream));
-  return fox_cumsum_bwd(args->dlog_lambda, args->dlog_fgate, args->dlog_fgate_stride_b, args->dlog_fgate_stride_h,
-                        args->dlog_fgate_stride_n, args->seq_start, args->dims.B, args->dims.H, args->dims.N, stream);
+  const float* drow = nullptr;
+  FOX_TRY(bwd_products(args, stream, &drow));
+  if (args->dlog_lambda == args->dlog_fgate) return fail(FOX_E_ARG, "dc and dg must not alias");
+  int64_t sb = args->dlog_fgate_stride_b, sh = args->dlog_fgate_stride_h, sn = args->dlog_fgate_stride_n;
+  if (sb == 0 && sh == 0 && sn == 0) { sb = (int64_t)args->dims.H * args->dims.N; sh = args->dims.N; sn = 1; }   // contiguous (B,H,N)
+  return check_hip(fox::launch_cumsum_bwd(args->dlog_lambda, args->dlog_fgate, sb, sh, sn, args->seq_start, args->dims.B, args->dims.H,
+                                          args->dims.N, drow, args->dims.M, (hipStream_t)stream), "fox_attn_bwd");
+}
+
+int fox_attn_bwd_logits(const fox_bwd_args* args, const void* logits, int32_t logits_dtype, int64_t sb, int64_t sh, int64_t sn, void* dlogits,
+                        int64_t db, int64_t dh, int64_t dn, void* stream) {
+  if (!args) return fail(FOX_E_ARG, "args is NULL");
+  if (!logits || !dlogits) return fail(FOX_E_ARG, "logits and dlogits must not be NULL");
+  if (logits_dtype < FOX_DTYPE_BF16 || logits_dtype > FOX_DTYPE_FP32) return fail(FOX_E_ARG, "logits_dtype must be FOX_DTYPE_BF16, FP16 or FP32 (got %d)", logits_dtype);
+  if ((const void*)args->dlog_lambda == dlogits || logits == dlogits) return fail(FOX_E_ARG, "dlogits must not alias dlog_lambda or logits");
+  const float* drow = nullptr;
+  FOX_TRY(bwd_products(args, stream, &drow));
+  return check_hip(fox::launch_gate_cumsum_bwd(args->dlog_lambda, logits, logits_dtype, sb, sh, sn, args->seq_start, dlogits, db, dh, dn,
+                                               args->dims.B, args->dims.H, args->dims.N, drow, args->dims.M, (hipStream_t)stream),
+                   "fox_attn_bwd_logits");
 }
 
 }  // extern "C"

@@ -21,23 +21,6 @@ namespace fox {
 
 namespace {
 
-// x + (x of the lane selected by a DPP control), as one v_add_f32 with a DPP operand
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float x) {
-  const int y = __builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true);
-  return x + __int_as_float(y);
-}
-
-// Sum over the LPR (2, 4, 8 or 16) consecutive lanes that hold one key row; every lane gets the total.
-template <int LPR>
-__device__ __forceinline__ float row_sum(float x) {
-  x = dpp_add<0xB1>(x);                            // quad_perm [1,0,3,2]
-  if constexpr (LPR >= 4) x = dpp_add<0x4E>(x);    // quad_perm [2,3,0,1]
-  if constexpr (LPR >= 8) x = dpp_add<0x141>(x);   // row_half_mirror: lane i <-> 7 - i of its eight
-  if constexpr (LPR >= 16) x = dpp_add<0x140>(x);  // row_mirror: lane i <-> 15 - i of its sixteen
-  return x;
-}
-
 template <typename Tr>
 __device__ __forceinline__ void unpack8f(const u32x4& v, float (&f)[8]) {
 #pragma unroll

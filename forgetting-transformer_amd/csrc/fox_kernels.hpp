@@ -188,6 +188,8 @@ bool fwd_pairs(int B, int H, int M, int N, int D, bool pruned, int splits);
 hipError_t launch_bwd_delta(const BwdK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_bwd_dkdv(const BwdK& a, int D, int dtype, hipStream_t s);   // a.cls selects the variant and its tiles
 bool dkdv_split_supports(int D);   // head dims the split (kClassLight) variant of the dK/dV kernel exists for
+bool bwd_together(const BwdK& a, int D);
+hipError_t launch_bwd(const BwdK& a, int D, int dtype, hipStream_t s);   // dq_kernel's and dkdv_kernel's work in one launch
 hipError_t launch_bwd_dq(const BwdK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_fwd_decode(const FwdK& a, int D, int dtype, hipStream_t s);  // M == 1, without the merge of the splits
 hipError_t launch_decode_gates(const DecodeK& a, int D, int dtype, hipStream_t s);
@@ -203,9 +205,9 @@ hipError_t launch_gate_cumsum_fwd(const void* logits, int dtype, int64_t sb, int
                                   float* log_fgate, float* c, int B, int H, int N, hipStream_t s);
 hipError_t launch_gate_cumsum_bwd(const float* dc, const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn,
                                   const int64_t* seq_start, void* dlogits, int64_t db, int64_t dh, int64_t dn, int B, int H, int N,
-                                  hipStream_t s);
+                                  const float* drow, int M, hipStream_t s);   // drow: null, or (B,H,M) added to the last M of dc
 hipError_t launch_cumsum_bwd(const float* dc, float* dg, int64_t db, int64_t dh, int64_t dn, const int64_t* seq_start, int B, int H,
-                             int N, hipStream_t s);
+                             int N, const float* drow, int M, hipStream_t s);
 hipError_t launch_mfma_probe(const void* operands, float* sink, int workgroups, int iters, hipStream_t s);  // fox_probe.hip
 hipError_t launch_qk_norm_threshold(const float* wq, const float* wk, int H, int D, double seq_len, double tolerance, float* thr, hipStream_t s);
 hipError_t launch_auto_threshold(const View& q, const View& k, int B, int H, int M, int N, int D, int dtype, float sm_scale,

@@ -104,14 +104,23 @@ inline unsigned scan_blocks(int rows) { return (unsigned)((rows + kXcds - 1) / k
 
 inline int scan_threads(int N) { return N <= 8 * 64 ? 64 : N <= 8 * 256 ? 256 : 1024; }
 
+// Gradient of the cumulative sum at position idx of a row: minus its column sum of dS and, where the backward ran in one launch
+// (drow not null: M row sums, of the last M positions), plus its row sum.  (Every load is issued: none behind a branch of its own.)
+__device__ __forceinline__ float load_dc(const float* dc_row, const float* drow_row, int p_seq, int idx) {
+  if (!drow_row) return dc_row[idx];
+  const float x = dc_row[idx], r = drow_row[max(idx - p_seq, 0)];
+  return idx >= p_seq ? x + r : x;
+}
+
 template <bool REVERSE, int NT>
 __global__ __launch_bounds__(NT) void scan_kernel(const float* __restrict__ in, int64_t sb, int64_t sh, int64_t sn,
                                                    const int64_t* __restrict__ seq_start, float* __restrict__ out, int64_t ob,
-                                                   int64_t oh, int64_t on, int rows, int H, int N) {
+                                                   int64_t oh, int64_t on, int rows, int H, int N, const float* __restrict__ drow, int M) {
   const int bh = scan_row_of_block(rows), b = bh / H, h = bh % H;
   if (bh >= rows) return;
   const float* src = in + b * sb + h * sh;
   float* dst = out + b * ob + h * oh;
+  const float* dr = REVERSE && drow ? drow + (int64_t)bh * M : nullptr;
   int seq = 0;
   if (seq_start) {
     const int64_t s64 = seq_start[b];
@@ -121,7 +130,7 @@ __global__ __launch_bounds__(NT) void scan_kernel(const float* __restrict__ in, 
   // arithmetic (those gates shift every cumulative sum the kernels see by the same amount, or are zeroed by the
   // forward); it is stored as an exact zero instead of the rounding noise of that sum.
   scan_row<REVERSE, NT>(
-      N, [&](int idx) { return (REVERSE || idx >= seq) ? src[(int64_t)idx * sn] : 0.f; },
+      N, [&](int idx) { return REVERSE ? load_dc(src, dr, N - M, idx) : idx >= seq ? src[(int64_t)idx * sn] : 0.f; },
       [&](int idx, float sum) { dst[(int64_t)idx * on] = (REVERSE && idx <= seq) ? 0.f : sum; });
 }
 
@@ -166,10 +175,11 @@ template <int DT, int NT>
 __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(const float* __restrict__ dc, const void* __restrict__ logits,
                                                             int64_t sb, int64_t sh, int64_t sn, const int64_t* __restrict__ seq_start,
                                                             void* __restrict__ dlogits, int64_t db, int64_t dh, int64_t dn,
-                                                            int rows, int H, int N) {
+                                                            int rows, int H, int N, const float* __restrict__ drow, int M) {
   const int bh = scan_row_of_block(rows), b = bh / H, h = bh % H;
   if (bh >= rows) return;
   const float* src = dc + (int64_t)bh * N;
+  const float* dr = drow ? drow + (int64_t)bh * M : nullptr;
   const int64_t lbase = b * sb + h * sh, dbase = b * db + h * dh;
   int seq = 0;
   if (seq_start) {
@@ -177,7 +187,7 @@ __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(const float* __restri
     seq = (int)(s64 < 0 ? 0 : (s64 > N ? N : s64));
   }
   scan_row<true, NT>(
-      N, [&](int idx) { return src[idx]; },
+      N, [&](int idx) { return load_dc(src, dr, N - M, idx); },
       [&](int idx, float sum) {
         const float x = load_logit<DT>(logits, lbase + (int64_t)idx * sn);
         const float z = __expf(-fabsf(x));
@@ -208,11 +218,11 @@ hipError_t launch_gate_cumsum_fwd(const void* logits, int dtype, int64_t sb, int
 
 hipError_t launch_gate_cumsum_bwd(const float* dc, const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn,
                                   const int64_t* seq_start, void* dlogits, int64_t db, int64_t dh, int64_t dn, int B, int H, int N,
-                                  hipStream_t s) {
+                                  const float* drow, int M, hipStream_t s) {
   switch (dtype) {
-    case 0: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 0, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N) break;
-    case 1: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 1, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N) break;
-    case 2: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 2, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N) break;
+    case 0: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 0, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 1: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 1, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 2: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 2, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -221,14 +231,14 @@ hipError_t launch_gate_cumsum_bwd(const float* dc, const void* logits, int dtype
 hipError_t launch_cumsum_fwd(const float* g, int64_t sb, int64_t sh, int64_t sn, const int64_t* seq_start, float* c, int B,
                              int H, int N, hipStream_t s) {
   FOX_LAUNCH_SCAN(scan_kernel, false, g, sb, sh, sn, seq_start, c,
-                     (int64_t)H * N, (int64_t)N, (int64_t)1, B * H, H, N)
+                     (int64_t)H * N, (int64_t)N, (int64_t)1, B * H, H, N, nullptr, N)
   return hipGetLastError();
 }
 
 hipError_t launch_cumsum_bwd(const float* dc, float* dg, int64_t db, int64_t dh, int64_t dn, const int64_t* seq_start, int B, int H,
-                             int N, hipStream_t s) {
+                             int N, const float* drow, int M, hipStream_t s) {
   FOX_LAUNCH_SCAN(scan_kernel, true, dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
-                     seq_start, dg, db, dh, dn, B * H, H, N)
+                     seq_start, dg, db, dh, dn, B * H, H, N, drow, M)
   return hipGetLastError();
 }
 

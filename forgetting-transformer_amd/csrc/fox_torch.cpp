@@ -254,12 +254,9 @@ variable_list run_backward(const Attention& a, const Tensor& q, const Tensor& k,
     args.dlog_fgate_stride_h = a.gs_h(dg);
     args.dlog_fgate_stride_n = a.gs_n(dg);
     check(fox_attn_bwd(&args, stream), "fox_attn_bwd");
-  } else {   // same stages, the last one fused with the derivative of logsigmoid
-    check(fox_attn_bwd_dq(&args, stream), "fox_attn_bwd_dq");
-    check(fox_attn_bwd_dkdv(&args, stream), "fox_attn_bwd_dkdv");
-    check(fox_gate_cumsum_bwd(args.dlog_lambda, g.const_data_ptr(), gate_dtype(g), g.stride(0), a.gs_h(g), a.gs_n(g), a.seq_ptr(),
-                              dg.mutable_data_ptr(), dg.stride(0), a.gs_h(dg), a.gs_n(dg), args.dims.B, args.dims.H, args.dims.N,
-                              stream), "fox_gate_cumsum_bwd");
+  } else {
+    check(fox_attn_bwd_logits(&args, g.const_data_ptr(), gate_dtype(g), g.stride(0), a.gs_h(g), a.gs_n(g), dg.mutable_data_ptr(),
+                              dg.stride(0), a.gs_h(dg), a.gs_n(dg), stream), "fox_attn_bwd_logits");
   }
   return {dq, dk, dv, dg};
 }

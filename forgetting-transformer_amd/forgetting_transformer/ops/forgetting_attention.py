@@ -478,14 +478,10 @@ def _backward(ctx, do):
         if gate_logit is None:
             _lib.check(lib.fox_attn_bwd(C.byref(args), stream), "fox_attn_bwd")
             dgate = dlog_fgate
-        else:  # same stages, the last one fused with the derivative of logsigmoid
-            _lib.check(lib.fox_attn_bwd_dq(C.byref(args), stream), "fox_attn_bwd_dq")
-            _lib.check(lib.fox_attn_bwd_dkdv(C.byref(args), stream), "fox_attn_bwd_dkdv")
+        else:
             dgate = torch.empty_like(gate_logit)
-            _lib.check(lib.fox_gate_cumsum_bwd(_ptr(dlog_lambda), _ptr(gate_logit), _GATE_DTYPES[gate_logit.dtype],
-                                               gate_logit.stride(0), gate_logit.stride(1), gate_logit.stride(2),
-                                               _ptr(seq_start), _ptr(dgate), dgate.stride(0), dgate.stride(1), dgate.stride(2), B, H, N,
-                                               stream), "fox_gate_cumsum_bwd")
+            _lib.check(lib.fox_attn_bwd_logits(C.byref(args), _ptr(gate_logit), _GATE_DTYPES[gate_logit.dtype], *gate_logit.stride(),
+                                               _ptr(dgate), *dgate.stride(), stream), "fox_attn_bwd_logits")
     return dq, dk, dv, dgate
 
 
