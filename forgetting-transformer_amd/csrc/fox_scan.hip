@@ -92,13 +92,13 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store) {
   }
 }
 
-// Row of a workgroup (rows >= `rows`: none).  Workgroups go round-robin over the 8 XCDs; neighbouring rows are given to one XCD, because the
-// rows of a batch's heads share cache lines when the gates lie as (B, T, H): spread over all XCDs, every L2 would write its
-// own part of each line (reverse scan into (B, T, H), rows over all XCDs / neighbours on one: B4 T4096 H32 10.8 / 7.6 us, B4 T16384 H16 19.0 / 17.0; the
-// forward's strided reads wait for their one lane a clock, not for the lines).
-__device__ __forceinline__ int scan_row_of_block(int rows) {
-  const int per = (rows + kXcds - 1) / kXcds, row = (int)(blockIdx.x % kXcds) * per + (int)(blockIdx.x / kXcds);
-  return (int)(blockIdx.x / kXcds) < per ? row : rows;
+// Row of a workgroup (rows >= `rows`: none).  Workgroups go round-robin over the 8 XCDs, and so do the rows: where 8 divides their number the attention
+// kernels put a pair on the same XCD, whose L2 then still holds what the one wrote for the other.  The gate gradients of a batch's heads share cache
+// lines when they lie as (B, T, H): with their rows spread every L2 would write its own part of each line, so those go to one XCD as neighbours
+// (`neighbours`; reverse scan, spread / neighbours: B4 T4096 H32 10.8 / 7.6 us, B4 T16384 H16 19.0 / 17.0; strided reads of the forward scan do not gain).
+__device__ __forceinline__ int scan_row_of_block(int rows, bool neighbours) {
+  const int per = (rows + kXcds - 1) / kXcds, id = blockIdx.x;
+  return neighbours ? id % kXcds * per + id / kXcds : id;   // (the grid is 8 * per workgroups)
 }
 inline unsigned scan_blocks(int rows) { return (unsigned)((rows + kXcds - 1) / kXcds * kXcds); }
 
@@ -116,8 +116,8 @@ template <bool REVERSE, int NT>
 __global__ __launch_bounds__(NT) void scan_kernel(const float* __restrict__ in, int64_t sb, int64_t sh, int64_t sn,
                                                    const int64_t* __restrict__ seq_start, float* __restrict__ out, int64_t ob,
                                                    int64_t oh, int64_t on, int rows, int H, int N, const float* __restrict__ drow, int M) {
-  const int bh = scan_row_of_block(rows), b = bh / H, h = bh % H;
-  if (bh >= rows) return;
+  const int bh = REVERSE ? scan_row_of_block(rows, on != 1) : blockIdx.x, b = bh / H, h = bh % H;
+  if (REVERSE && bh >= rows) return;
   const float* src = in + b * sb + h * sh;
   float* dst = out + b * ob + h * oh;
   const float* dr = REVERSE && drow ? drow + (int64_t)bh * M : nullptr;
@@ -146,10 +146,9 @@ __device__ __forceinline__ void store_logit(void* p, int64_t i, float x) {
 template <int DT, int NT>
 __global__ __launch_bounds__(NT) void gate_scan_fwd_kernel(const void* __restrict__ logits, int64_t sb, int64_t sh, int64_t sn,
                                                             const int64_t* __restrict__ seq_start,
-                                                            float* __restrict__ log_fgate, float* __restrict__ out, int rows,
-                                                            int H, int N) {
-  const int bh = scan_row_of_block(rows), b = bh / H, h = bh % H;
-  if (bh >= rows) return;
+                                                            float* __restrict__ log_fgate, float* __restrict__ out, int H,
+                                                            int N) {
+  const int bh = blockIdx.x, b = bh / H, h = bh % H;
   const int64_t base = b * sb + h * sh;
   float* dst = out + (int64_t)bh * N;
   float* lg = log_fgate ? log_fgate + (int64_t)bh * N : nullptr;
@@ -176,7 +175,7 @@ __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(const float* __restri
                                                             int64_t sb, int64_t sh, int64_t sn, const int64_t* __restrict__ seq_start,
                                                             void* __restrict__ dlogits, int64_t db, int64_t dh, int64_t dn,
                                                             int rows, int H, int N, const float* __restrict__ drow, int M) {
-  const int bh = scan_row_of_block(rows), b = bh / H, h = bh % H;
+  const int bh = scan_row_of_block(rows, dn != 1), b = bh / H, h = bh % H;
   if (bh >= rows) return;
   const float* src = dc + (int64_t)bh * N;
   const float* dr = drow ? drow + (int64_t)bh * M : nullptr;
@@ -197,20 +196,20 @@ __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(const float* __restri
       });
 }
 
-// KERNEL<ARG, threads for rows of N elements>, one workgroup per row of the B x H.
-#define FOX_LAUNCH_SCAN(KERNEL, ARG, ...)                                                                      \
+// KERNEL<ARG, threads for rows of N elements>, BLOCKS workgroups, one per row of the B x H.
+#define FOX_LAUNCH_SCAN(KERNEL, ARG, BLOCKS, ...)                                                                      \
   switch (scan_threads(N)) {                                                                                    \
-    case 64: hipLaunchKernelGGL((KERNEL<ARG, 64>), dim3(scan_blocks(B * H)), dim3(64), 0, s, __VA_ARGS__); break;    \
-    case 256: hipLaunchKernelGGL((KERNEL<ARG, 256>), dim3(scan_blocks(B * H)), dim3(256), 0, s, __VA_ARGS__); break; \
-    default: hipLaunchKernelGGL((KERNEL<ARG, 1024>), dim3(scan_blocks(B * H)), dim3(1024), 0, s, __VA_ARGS__);       \
+    case 64: hipLaunchKernelGGL((KERNEL<ARG, 64>), dim3(BLOCKS), dim3(64), 0, s, __VA_ARGS__); break;    \
+    case 256: hipLaunchKernelGGL((KERNEL<ARG, 256>), dim3(BLOCKS), dim3(256), 0, s, __VA_ARGS__); break; \
+    default: hipLaunchKernelGGL((KERNEL<ARG, 1024>), dim3(BLOCKS), dim3(1024), 0, s, __VA_ARGS__);       \
   }
 
 hipError_t launch_gate_cumsum_fwd(const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn, const int64_t* seq_start,
                                   float* log_fgate, float* c, int B, int H, int N, hipStream_t s) {
   switch (dtype) {
-    case 0: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 0, logits, sb, sh, sn, seq_start, log_fgate, c, B * H, H, N) break;
-    case 1: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 1, logits, sb, sh, sn, seq_start, log_fgate, c, B * H, H, N) break;
-    case 2: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 2, logits, sb, sh, sn, seq_start, log_fgate, c, B * H, H, N) break;
+    case 0: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 0, (unsigned)(B * H), logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
+    case 1: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 1, (unsigned)(B * H), logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
+    case 2: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 2, (unsigned)(B * H), logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -220,9 +219,9 @@ hipError_t launch_gate_cumsum_bwd(const float* dc, const void* logits, int dtype
                                   const int64_t* seq_start, void* dlogits, int64_t db, int64_t dh, int64_t dn, int B, int H, int N,
                                   const float* drow, int M, hipStream_t s) {
   switch (dtype) {
-    case 0: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 0, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
-    case 1: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 1, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
-    case 2: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 2, dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 0: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 0, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 1: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 1, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 2: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 2, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -230,14 +229,14 @@ hipError_t launch_gate_cumsum_bwd(const float* dc, const void* logits, int dtype
 
 hipError_t launch_cumsum_fwd(const float* g, int64_t sb, int64_t sh, int64_t sn, const int64_t* seq_start, float* c, int B,
                              int H, int N, hipStream_t s) {
-  FOX_LAUNCH_SCAN(scan_kernel, false, g, sb, sh, sn, seq_start, c,
+  FOX_LAUNCH_SCAN(scan_kernel, false, (unsigned)(B * H), g, sb, sh, sn, seq_start, c,
                      (int64_t)H * N, (int64_t)N, (int64_t)1, B * H, H, N, nullptr, N)
   return hipGetLastError();
 }
 
 hipError_t launch_cumsum_bwd(const float* dc, float* dg, int64_t db, int64_t dh, int64_t dn, const int64_t* seq_start, int B, int H,
                              int N, const float* drow, int M, hipStream_t s) {
-  FOX_LAUNCH_SCAN(scan_kernel, true, dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
+  FOX_LAUNCH_SCAN(scan_kernel, true, scan_blocks(B * H), dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
                      seq_start, dg, db, dh, dn, B * H, H, N, drow, M)
   return hipGetLastError();
 }
