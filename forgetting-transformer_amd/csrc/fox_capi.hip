@@ -537,6 +537,10 @@ int fox_attn_decode_workspace_bytes(const fox_dims* dims, int64_t* bytes) {
 }
 
 int fox_attn_decode(const fox_fwd_args* args, const float* g, int64_t g_sb, int64_t g_sh, int64_t g_sn, void* stream) {
+  return fox_attn_decode_counted(args, g, g_sb, g_sh, g_sn, nullptr, stream);
+}
+
+int fox_attn_decode_counted(const fox_fwd_args* args, const float* g, int64_t g_sb, int64_t g_sh, int64_t g_sn, uint32_t* arrived, void* stream) {
   if (!args || !g) return fail(FOX_E_ARG, "args and g must not be NULL");
   FOX_TRY(check_dims(&args->dims));
   if (args->dims.M != 1) return fail(FOX_E_ARG, "fox_attn_decode takes one query row (M = %d)", args->dims.M);
@@ -567,6 +571,7 @@ int fox_attn_decode(const fox_fwd_args* args, const float* g, int64_t g_sb, int6
       k.splits = fox::decode_splits(k.B, k.H, k.N, args->dims.D);
       k.ws_o = (float*)args->workspace;
       k.ws_p = (fox::DecodePartial*)(k.ws_o + (int64_t)k.splits * k.B * k.H * args->dims.D);   // (D is a multiple of 4: 16-byte aligned)
+      if (fox::decode_merges(k.B, k.H, k.splits)) k.arrived = arrived;
     }
   }
   return check_hip(fox::launch_decode_gates(k, args->dims.D, args->dims.dtype, (hipStream_t)stream), "fox_attn_decode");

@@ -219,6 +219,67 @@ hipError_t launch_fwd_decode(const FwdK& a, int D, int dtype, hipStream_t s) {
 
 static int64_t decode_batches(int N, int D) { return ((int64_t)N * D + 16383) / 16384; }   // batches of keys, four waves each
 
+// Merge of the splits of decode_gates_kernel by 256 threads per (batch, head), every partial in flight at once (at most
+// kDecodeMaxSplits of them, one round trip; a thread that walks the splits one after the other pays one per split).
+// AGENT: the partials come from workgroups of the same launch.
+template <typename Tr, int D, bool AGENT>
+__device__ __forceinline__ void decode_merge(const DecodeK& a, int bh) {
+  constexpr int TPR = D / 4, GROUPS = 256 / TPR, PER = (kDecodeMaxSplits + GROUPS - 1) / GROUPS;
+  __shared__ float weight[kDecodeMaxSplits];
+  __shared__ float l_tot, m_tot;
+  __shared__ __align__(16) float part[GROUPS][D];
+  const int tid = threadIdx.x, b = bh / a.H, h = bh % a.H, splits = a.splits;
+  const int grp = tid / TPR, d = (tid % TPR) * 4;
+  const float* wo = a.ws_o + (int64_t)bh * splits * D + d;
+  f32x4 x[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const float* p = wo + (int64_t)min(grp + i * GROUPS, splits - 1) * D;
+    if constexpr (AGENT) x[i] = f32x4{load_agent(p), load_agent(p + 1), load_agent(p + 2), load_agent(p + 3)};
+    else x[i] = *reinterpret_cast<const f32x4*>(p);
+  }
+  if (tid < kWave) {   // one lane per split (counted from the last keys): its maximum moves by the gates of the splits behind it
+    const DecodePartial* from = a.ws_p + (int64_t)bh * splits + min(tid, splits - 1);
+    const DecodePartial p = AGENT ? DecodePartial{load_agent(&from->g), load_agent(&from->m), load_agent(&from->l)} : *from;
+    double incl = tid < splits ? p.g : 0.0;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const double up = __shfl_up(incl, off);
+      if (tid >= off) incl += up;
+    }
+    const double excl = __shfl_up(incl, 1);
+    const float m = tid == 0 ? p.m : tid < splits ? p.m + (float)excl * kLog2e : -INFINITY;
+    float mx = m;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+    const float w = __builtin_amdgcn_exp2f(m - mx);
+    float l = p.l * w;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
+    weight[tid] = w;
+    if (tid == 0) { l_tot = l; m_tot = mx; }
+  }
+  __syncthreads();
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < PER; ++i)
+    if (grp + i * GROUPS < splits) acc += x[i] * weight[grp + i * GROUPS];
+  *reinterpret_cast<f32x4*>(&part[grp][d]) = acc;
+  __syncthreads();
+  if (tid >= TPR) return;
+  acc = *reinterpret_cast<const f32x4*>(&part[0][d]);
+  const int used = min(GROUPS, splits);
+  for (int i = 1; i < used; ++i) acc += *reinterpret_cast<const f32x4*>(&part[i][d]);
+  const bool empty = a.seq_start && a.seq_start[b] >= a.N;
+  const float inv = empty ? 0.f : 1.0f / l_tot;
+  uint16_t* op = const_cast<uint16_t*>(a.o.ptr) + b * a.o.sb + h * a.o.sh + d;
+  u32x2 w;
+  w[0] = Tr::pack2(acc[0] * inv, acc[1] * inv);
+  w[1] = Tr::pack2(acc[2] * inv, acc[3] * inv);
+  *reinterpret_cast<u32x2*>(op) = w;
+  if (d == 0 && a.lse) a.lse[bh] = empty ? -INFINITY : m_tot * kLn2 + __logf(l_tot);
+}
+
 // ---------------------------------------------------------------------------
 // The same step straight from the log forget gates: no cumulative sum of the whole row in front of it.
 //
@@ -354,93 +415,67 @@ __global__ __launch_bounds__(64 * WAVES) void decode_gates_kernel(const DecodeK 
     for (int e = 0; e < 8; ++e) part_acc[wave][ch * 8 + e] = acc[e];
   }
   __syncthreads();
-  if (tid >= LPR) return;
-  m = part_m[0];
-  l = part_l[0];
-  double shift = part_g[0];
+  if (tid < LPR) {
+    m = part_m[0];
+    l = part_l[0];
+    double shift = part_g[0];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) acc[e] = part_acc[0][ch * 8 + e];
+    for (int e = 0; e < 8; ++e) acc[e] = part_acc[0][ch * 8 + e];
 #pragma unroll
-  for (int w = 1; w < WAVES; ++w) {
-    float acc2[8];
+    for (int w = 1; w < WAVES; ++w) {
+      float acc2[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc2[e] = part_acc[w][ch * 8 + e];
-    merge_state(m, l, acc, part_m[w] + (float)shift * kLog2e, part_l[w], acc2);
-    shift += part_g[w];
-  }
+      for (int e = 0; e < 8; ++e) acc2[e] = part_acc[w][ch * 8 + e];
+      merge_state(m, l, acc, part_m[w] + (float)shift * kLog2e, part_l[w], acc2);
+      shift += part_g[w];
+    }
 
-  if (a.splits > 1) {  // partial result of this split: accumulator, maximum and sum relative to its last key, sum of its gates
-    const int64_t row = (int64_t)bh * a.splits + sp;
-    float* wo = a.ws_o + row * D + ch * 8;
-    const f32x4 w0 = {acc[0], acc[1], acc[2], acc[3]}, w1 = {acc[4], acc[5], acc[6], acc[7]};
-    *reinterpret_cast<f32x4*>(wo) = w0;
-    *reinterpret_cast<f32x4*>(wo + 4) = w1;
-    if (ch == 0) a.ws_p[row] = DecodePartial{shift, m, l};
-    return;
-  }
-  const bool empty = lo >= N;  // every key is left padding: o = 0, lse = -inf (:679-685)
-  const float inv = empty ? 0.f : 1.0f / l;
-  uint16_t* op = const_cast<uint16_t*>(a.o.ptr) + b * a.o.sb + h * a.o.sh + ch * 8;
-  u32x4 w;
+    if (a.splits > 1) {  // partial result of this split: accumulator, maximum and sum relative to its last key, sum of its gates
+      const int64_t row = (int64_t)bh * a.splits + sp;
+      float* wo = a.ws_o + row * D + ch * 8;
+      if (WAVES == 4 && a.arrived) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) w[e] = Tr::pack2(acc[2 * e] * inv, acc[2 * e + 1] * inv);
-  *reinterpret_cast<u32x4*>(op) = w;
-  if (ch == 0 && a.lse) a.lse[bh] = empty ? -INFINITY : m * kLn2 + __logf(l);
+        for (int e = 0; e < 8; ++e) store_agent(wo + e, acc[e]);
+        if (ch == 0) {
+          store_agent(&a.ws_p[row].g, shift);
+          store_agent(&a.ws_p[row].m, m);
+          store_agent(&a.ws_p[row].l, l);
+        }
+      } else {
+        const f32x4 w0 = {acc[0], acc[1], acc[2], acc[3]}, w1 = {acc[4], acc[5], acc[6], acc[7]};
+        *reinterpret_cast<f32x4*>(wo) = w0;
+        *reinterpret_cast<f32x4*>(wo + 4) = w1;
+        if (ch == 0) a.ws_p[row] = DecodePartial{shift, m, l};
+      }
+    } else {
+      const bool empty = lo >= N;  // every key is left padding: o = 0, lse = -inf (:679-685)
+      const float inv = empty ? 0.f : 1.0f / l;
+      uint16_t* op = const_cast<uint16_t*>(a.o.ptr) + b * a.o.sb + h * a.o.sh + ch * 8;
+      u32x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = Tr::pack2(acc[2 * e] * inv, acc[2 * e + 1] * inv);
+      *reinterpret_cast<u32x4*>(op) = w;
+      if (ch == 0 && a.lse) a.lse[bh] = empty ? -INFINITY : m * kLn2 + __logf(l);
+    }
+  }
+  if constexpr (WAVES == 4) {   // the last of the splits merges them (decode_merges)
+    if (a.splits <= 1 || !a.arrived) return;
+    __shared__ bool last;
+    if (wave == 0) {   // the wave that stored the partials
+      stores_complete();
+      if (lane == 0) last = arrive(&a.arrived[bh]) == (uint32_t)a.splits - 1u;
+    }
+    __syncthreads();
+    if (!last) return;
+    decode_merge<Tr, D, true>(a, bh);
+    if (tid == 0) __hip_atomic_store(&a.arrived[bh], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
-// Merge of the splits of decode_gates_kernel: one workgroup per (batch, head), every partial in flight at once (at most
-// kDecodeMaxSplits of them, one round trip; a thread that walks the splits one after the other pays one per split).
+// decode_merge as a launch of its own
 template <typename Tr, int D>
 __global__ __launch_bounds__(256) void decode_combine_kernel(const DecodeK a) {
-  constexpr int TPR = D / 4, GROUPS = 256 / TPR, PER = (kDecodeMaxSplits + GROUPS - 1) / GROUPS;
-  __shared__ float weight[kDecodeMaxSplits];
-  __shared__ float l_tot, m_tot;
-  __shared__ __align__(16) float part[GROUPS][D];
-  const int tid = threadIdx.x, bh = blockIdx.x, b = bh / a.H, h = bh % a.H, splits = a.splits;
-  const int grp = tid / TPR, d = (tid % TPR) * 4;
-  const float* wo = a.ws_o + (int64_t)bh * splits * D + d;
-  f32x4 x[PER];
-#pragma unroll
-  for (int i = 0; i < PER; ++i) x[i] = *reinterpret_cast<const f32x4*>(wo + (int64_t)min(grp + i * GROUPS, splits - 1) * D);
-  if (tid < kWave) {   // one lane per split (counted from the last keys): its maximum moves by the gates of the splits behind it
-    const DecodePartial p = a.ws_p[(int64_t)bh * splits + min(tid, splits - 1)];
-    double incl = tid < splits ? p.g : 0.0;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const double up = __shfl_up(incl, off);
-      if (tid >= off) incl += up;
-    }
-    const double excl = __shfl_up(incl, 1);
-    const float m = tid == 0 ? p.m : tid < splits ? p.m + (float)excl * kLog2e : -INFINITY;
-    float mx = m;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-    const float w = __builtin_amdgcn_exp2f(m - mx);
-    float l = p.l * w;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off);
-    weight[tid] = w;
-    if (tid == 0) { l_tot = l; m_tot = mx; }
-  }
-  __syncthreads();
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < PER; ++i)
-    if (grp + i * GROUPS < splits) acc += x[i] * weight[grp + i * GROUPS];
-  *reinterpret_cast<f32x4*>(&part[grp][d]) = acc;
-  __syncthreads();
-  if (tid >= TPR) return;
-  acc = *reinterpret_cast<const f32x4*>(&part[0][d]);
-  const int used = min(GROUPS, splits);
-  for (int i = 1; i < used; ++i) acc += *reinterpret_cast<const f32x4*>(&part[i][d]);
-  const bool empty = a.seq_start && a.seq_start[b] >= a.N;
-  const float inv = empty ? 0.f : 1.0f / l_tot;
-  uint16_t* op = const_cast<uint16_t*>(a.o.ptr) + b * a.o.sb + h * a.o.sh + d;
-  u32x2 w;
-  w[0] = Tr::pack2(acc[0] * inv, acc[1] * inv);
-  w[1] = Tr::pack2(acc[2] * inv, acc[3] * inv);
-  *reinterpret_cast<u32x2*>(op) = w;
-  if (d == 0 && a.lse) a.lse[bh] = empty ? -INFINITY : m_tot * kLn2 + __logf(l_tot);
+  decode_merge<Tr, D, false>(a, blockIdx.x);
 }
 
 // Whether one workgroup of sixteen waves takes a (batch, head) whole, which saves the merge of splits and its launch.  The line
@@ -462,7 +497,7 @@ static hipError_t launch_decode_gates_d(const DecodeK& a, hipStream_t s) {
   }
   hipLaunchKernelGGL((decode_gates_kernel<Tr, D, 4>), dim3((unsigned)(a.splits * a.B * a.H)), dim3(256), 0, s, a);
   const hipError_t e = hipGetLastError();
-  if (e != hipSuccess || a.splits <= 1) return e;
+  if (e != hipSuccess || a.splits <= 1 || a.arrived) return e;
   hipLaunchKernelGGL((decode_combine_kernel<Tr, D>), dim3((unsigned)(a.B * a.H)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
@@ -493,6 +528,12 @@ int decode_splits(int B, int H, int N, int D) {
   splits = splits > kDecodeMaxSplits ? kDecodeMaxSplits : splits;
   return splits < 1 ? 1 : (int)splits;
 }
+
+// Whether the split that arrives last merges the others, where there are counters.  The kernels take no less time that way (partials past the L2, a
+// counter, partials back: three round trips to memory against a launch boundary), but the call is a launch shorter: us of GPU / of host time, two
+// launches and one: B1 H12 N1500 D64 8.0 / 9.1 and 8.4 / 4.6, B1 H1 N5000 D128 7.8 / 9.2 and 9.0 / 4.8.  A generation step of one user waits for the host.  With more
+// workgroups than CUs the step is the GPU's, and the round trips add up: B4 H12 N3000 D64 11.3 and 12.4, B1 H16 N8000 D128 14.6 and 25.9.
+bool decode_merges(int B, int H, int splits) { return splits > 1 && (int64_t)B * H * splits <= kCus; }
 
 // ---------------------------------------------------------------------------
 // New tokens into a layer's cache: keys, values and log gates in one launch.  One 16-byte piece of K and the same piece of V per

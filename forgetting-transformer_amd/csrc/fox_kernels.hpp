@@ -69,6 +69,7 @@ struct DecodeK {
   int splits;
   float* ws_o;               // (B, H, splits, D) partial accumulators
   DecodePartial* ws_p;       // (B, H, splits)
+  uint32_t* arrived;         // null, or (B, H) zeros: the split that arrives last merges them and leaves a zero
 };
 constexpr int kDecodeMaxSplits = 64;                     // one lane of a wave each in the merge
 template <int D> constexpr int kDecodeBatchKeys = 4096 / D;   // keys a wave holds in flight: 8 KiB of K and 8 KiB of V
@@ -195,6 +196,7 @@ hipError_t launch_fwd_decode(const FwdK& a, int D, int dtype, hipStream_t s);  /
 hipError_t launch_decode_gates(const DecodeK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_cache_append(const CacheAppendK& a, hipStream_t s);
 int decode_splits(int B, int H, int N, int D);
+bool decode_merges(int B, int H, int splits);
 hipError_t launch_norm_gate(const NormGateK& a, int D, int dtype, bool bwd, int act, hipStream_t s);  // act: FOX_ACT_*
 int64_t norm_gate_workspace_rows(int64_t rows);
 hipError_t launch_shift_fwd(const ShiftK& a, int D, int dtype, hipStream_t s);
