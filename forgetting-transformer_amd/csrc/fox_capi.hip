@@ -316,6 +316,13 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
   return check_hip(fox::launch_fwd_gates(k, args->dims.D, args->dims.dtype, (hipStream_t)stream), what);
 }
 
+int check_gates(const fox_gates* gates) {
+  if (!gates || !gates->g) return fail(FOX_E_ARG, "gates and its g must not be NULL");
+  if (gates->is_logit ? gates->dtype < FOX_DTYPE_BF16 || gates->dtype > FOX_DTYPE_FP32 : gates->dtype != FOX_DTYPE_FP32)
+    return fail(FOX_E_ARG, "gates: dtype must be FOX_DTYPE_BF16, FP16 or FP32 for logits and FP32 for log gates (got %d)", gates->dtype);
+  return FOX_OK;
+}
+
 int check_epilogue(const fox_fwd_args* args, const fox_fwd_epilogue* epi) {
   if (!args || !epi) return fail(FOX_E_ARG, "args and epilogue must not be NULL");
   if (epi->activation != FOX_ACT_SIGMOID && epi->activation != FOX_ACT_SWISH && epi->activation != FOX_ACT_NONE)
@@ -394,11 +401,9 @@ int fox_attn_fwd_takes_gates(const fox_dims* dims, int32_t pruned, int32_t* yes)
 }
 
 int fox_attn_fwd_gates(const fox_fwd_args* args, const fox_gates* gates, const fox_fwd_epilogue* epi, void* stream) {
-  if (!args || !gates) return fail(FOX_E_ARG, "args and gates must not be NULL");
+  if (!args) return fail(FOX_E_ARG, "args is NULL");
   if (epi) FOX_TRY(check_epilogue(args, epi));
-  if (!gates->g) return fail(FOX_E_ARG, "g is NULL");
-  if (gates->is_logit ? gates->dtype < FOX_DTYPE_BF16 || gates->dtype > FOX_DTYPE_FP32 : gates->dtype != FOX_DTYPE_FP32)
-    return fail(FOX_E_ARG, "gates: dtype must be FOX_DTYPE_BF16, FP16 or FP32 for logits and FP32 for log gates (got %d)", gates->dtype);
+  FOX_TRY(check_gates(gates));
   int32_t yes = 0;
   FOX_TRY(fox_attn_fwd_takes_gates(&args->dims, args->threshold != nullptr, &yes));
   if (!yes) return fail(FOX_E_ARG, "fox_attn_fwd_gates does not take this shape (fox_attn_fwd_takes_gates)");
@@ -482,8 +487,27 @@ int fox_auto_threshold(const fox_dims* dims, const fox_view* q, const fox_view* 
   FOX_TRY(check_view(k, "k"));
   if (!thr || !norm_scratch) return fail(FOX_E_ARG, "thr and norm_scratch must not be NULL");
   return check_hip(fox::launch_auto_threshold(to_view(*q), to_view(*k), dims->B, dims->H, dims->M, dims->N, dims->D,
-                                              dims->dtype, sm_scale, thr, norm_scratch, (hipStream_t)stream),
+                                              dims->dtype, sm_scale, thr, norm_scratch, nullptr, nullptr, (hipStream_t)stream),
                    "fox_auto_threshold");
+}
+
+int fox_auto_threshold_scan(const fox_dims* dims, const fox_view* q, const fox_view* k, float sm_scale, float* thr, uint32_t* norm_scratch,
+                            const fox_gates* gates, const int64_t* seq_start, float* c, void* stream) {
+  FOX_TRY(check_dims(dims));
+  FOX_TRY(check_view(q, "q"));
+  FOX_TRY(check_view(k, "k"));
+  if (!thr || !norm_scratch || !c) return fail(FOX_E_ARG, "thr, norm_scratch and c must not be NULL");
+  FOX_TRY(check_gates(gates));
+  const fox::GateK t{gates->g, gates->stride_b, gates->stride_h, gates->stride_n, gates->is_logit ? gates->dtype : fox::kGateLog, c,
+                     gates->is_logit ? gates->log_fgate : nullptr};
+  if (fox::threshold_scans(dims->B, dims->H, dims->M, dims->N, dims->D))
+    return check_hip(fox::launch_auto_threshold(to_view(*q), to_view(*k), dims->B, dims->H, dims->M, dims->N, dims->D, dims->dtype, sm_scale, thr,
+                                                norm_scratch, &t, seq_start, (hipStream_t)stream), "fox_auto_threshold_scan");
+  FOX_TRY(fox_auto_threshold(dims, q, k, sm_scale, thr, norm_scratch, stream));
+  if (gates->is_logit)
+    return fox_gate_cumsum_fwd(gates->g, gates->dtype, gates->stride_b, gates->stride_h, gates->stride_n, seq_start, t.log_fgate, c, dims->B, dims->H,
+                               dims->N, stream);
+  return fox_cumsum_fwd((const float*)gates->g, gates->stride_b, gates->stride_h, gates->stride_n, seq_start, c, dims->B, dims->H, dims->N, stream);
 }
 
 int fox_qk_norm_threshold(const float* q_weight, const float* k_weight, int32_t H, int32_t D, double seq_len, double tolerance, float* thr,

@@ -213,6 +213,7 @@ hipError_t launch_cumsum_bwd(const float* dc, float* dg, int64_t db, int64_t dh,
 hipError_t launch_mfma_probe(const void* operands, float* sink, int workgroups, int iters, hipStream_t s);  // fox_probe.hip
 hipError_t launch_qk_norm_threshold(const float* wq, const float* wk, int H, int D, double seq_len, double tolerance, float* thr, hipStream_t s);
 hipError_t launch_auto_threshold(const View& q, const View& k, int B, int H, int M, int N, int D, int dtype, float sm_scale,
-                                 float* thr, uint32_t* scratch, hipStream_t s);
+                                 float* thr, uint32_t* scratch, const GateK* t, const int64_t* seq_start, hipStream_t s);   // t: null, or scanned as well
+bool threshold_scans(int B, int H, int M, int N, int D);
 
 }  // namespace fox

@@ -254,17 +254,17 @@ __global__ void zero_u32_kernel(uint32_t* p, int n) {
   if (i < n) p[i] = 0u;
 }
 
-// grid (row blocks, B*H, 2): z = 0 scans q (T = M), z = 1 scans k (T = N).  scratch holds, per (batch, head), the two
+// One workgroup: rows block * 512 .. of q (which = 0, T = M) or of k (which = 1, T = N) of one (batch, head), `blocks` workgroups each.  scratch holds, per (batch, head), the two
 // running maxima (float bits) and the number of workgroups that have added theirs; the workgroup that arrives last
 // turns the maxima into the threshold, so no kernel of its own is needed for that.
 template <typename Tr, int D>
-__global__ __launch_bounds__(256) void norm_max_kernel(View q, View k, int H, int M, int N, uint32_t* scratch, float* thr,
-                                                       float sm_scale, float log_n) {
+__device__ __forceinline__ void norm_max(const View& q, const View& k, int H, int M, int N, uint32_t* scratch, float* thr, float sm_scale,
+                                         float log_n, int block, int blocks, int bh, int which) {
   constexpr int LPR = D / 8, RPP = 256 / LPR, ROWS = 512;
   const int tid = threadIdx.x;
-  const int bh = blockIdx.y, b = bh / H, h = bh % H;
-  const View& t = blockIdx.z == 0 ? q : k;
-  const int T = blockIdx.z == 0 ? M : N;
+  const int b = bh / H, h = bh % H;
+  const View& t = which == 0 ? q : k;
+  const int T = which == 0 ? M : N;
   const uint16_t* p = t.ptr + b * t.sb + h * t.sh;
   const int ch = tid % LPR;
   float best = 0.f;
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(256) void norm_max_kernel(View q, View k, int H, in
     u32x4 x[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int row = min(blockIdx.x * ROWS + (pass + u) * RPP + tid / LPR, T - 1);  // rows past the end repeat the last one
+      const int row = min(block * ROWS + (pass + u) * RPP + tid / LPR, T - 1);  // rows past the end repeat the last one
       x[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + (int64_t)row * t.st + ch * 8));
     }
 #pragma unroll
@@ -297,10 +297,10 @@ __global__ __launch_bounds__(256) void norm_max_kernel(View q, View k, int H, in
   // Non-negative floats order like uints.  The arrival is counted only after the maximum has been applied: the count's
   // operand depends on the value the first atomic returns, and a returning atomic has been carried out where all
   // workgroups' atomics meet.  (No fence: a device-wide release would write back the whole L2 once per workgroup.)
-  const uint32_t before = atomicMax(&mine[blockIdx.z], __float_as_uint(best));
+  const uint32_t before = atomicMax(&mine[which], __float_as_uint(best));
   uint32_t one = 1u;
   asm volatile("" : "+v"(one) : "v"(before));
-  if (atomicAdd(&mine[2], one) != gridDim.x * 2u - 1u) return;
+  if (atomicAdd(&mine[2], one) != (uint32_t)blocks * 2u - 1u) return;
   // the last workgroup of this (batch, head): every maximum has been added (read through the atomic unit as well)
   const float qn = __uint_as_float(atomicMax(&mine[0], 0u)), kn = __uint_as_float(atomicMax(&mine[1], 0u));
   // every tensor op of the reference rounds to the input dtype
@@ -311,6 +311,44 @@ __global__ __launch_bounds__(256) void norm_max_kernel(View q, View k, int H, in
   th = -th;
   th = round16<Tr>(th - 10.f);
   thr[bh] = th;
+}
+
+// grid (row blocks, B*H, 2)
+template <typename Tr, int D>
+__global__ __launch_bounds__(256) void norm_max_kernel(View q, View k, int H, int M, int N, uint32_t* scratch, float* thr, float sm_scale, float log_n) {
+  norm_max<Tr, D>(q, k, H, M, N, scratch, thr, sm_scale, log_n, blockIdx.x, gridDim.x, blockIdx.y, blockIdx.z);
+}
+
+// The same with the forward scan of the gates beside it, one workgroup per row in front of the others: the scan is a chain of one workgroup's barriers
+// (20 us in a step at B4 T16384 H16) that needs none of the bandwidth the norms stream at (88 us), and needs no threshold.
+template <typename Tr, int D, int KIND>
+__global__ __launch_bounds__(256) void norm_max_scan_kernel(View q, View k, int H, int M, int N, uint32_t* scratch, float* thr, float sm_scale, float log_n,
+                                                            GateK t, const int64_t* __restrict__ seq_start, int rows, int blocks) {
+  if ((int)blockIdx.x >= rows) {
+    const int id = blockIdx.x - rows, pair = id / blocks;
+    norm_max<Tr, D>(q, k, H, M, N, scratch, thr, sm_scale, log_n, id - pair * blocks, blocks, pair % rows, pair / rows);
+    return;
+  }
+  const int bh = blockIdx.x, b = bh / H, h = bh % H;
+  int seq = 0;
+  if (seq_start) {
+    const int64_t s64 = seq_start[b];
+    seq = (int)(s64 < 0 ? 0 : (s64 > N ? N : s64));
+  }
+  const int64_t base = b * t.sb + h * t.sh;
+  float *dst = t.c + (int64_t)bh * N, *lg = t.log_fgate ? t.log_fgate + (int64_t)bh * N : nullptr;
+  scan_row<false, 256>(
+      N,
+      [&](int idx) {
+        if constexpr (KIND == kGateLog) {
+          return idx >= seq ? reinterpret_cast<const float*>(t.g)[base + (int64_t)idx * t.sn] : 0.f;
+        } else {
+          const float g = log_sigmoid(load_logit<KIND>(t.g, base + (int64_t)idx * t.sn));
+          if (lg) lg[idx] = g;
+          return idx >= seq ? g : 0.f;
+        }
+      },
+      [&](int idx, float sum) { dst[idx] = sum; });
 }
 
 // Threshold per head from the QK-norm weights: -(2 * max|w_q| * max|w_k| * sqrt(D) + log T) + tolerance, every operation
@@ -346,27 +384,49 @@ hipError_t launch_qk_norm_threshold(const float* wq, const float* wk, int H, int
   return hipGetLastError();
 }
 
-template <typename Tr>
-static hipError_t auto_threshold_t(const View& q, const View& k, int B, int H, int M, int N, int D, float sm_scale, float* thr,
-                                   uint32_t* scratch, hipStream_t s) {
-  const int n_bh = B * H;
-  hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)((3 * n_bh + 255) / 256)), dim3(256), 0, s, scratch, 3 * n_bh);
-  const dim3 grid((unsigned)((N + 511) / 512), (unsigned)n_bh, 2u);
+template <typename Tr, int D>
+static hipError_t auto_threshold_d(const View& q, const View& k, int B, int H, int M, int N, float sm_scale, float* thr, uint32_t* scratch,
+                                   const GateK* t, const int64_t* seq_start, hipStream_t s) {
+  const int n_bh = B * H, blocks = (N + 511) / 512;
   const float log_n = (float)log((double)N);
-  switch (D) {
-    case 16: hipLaunchKernelGGL((norm_max_kernel<Tr, 16>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n); break;
-    case 32: hipLaunchKernelGGL((norm_max_kernel<Tr, 32>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n); break;
-    case 64: hipLaunchKernelGGL((norm_max_kernel<Tr, 64>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n); break;
-    case 128: hipLaunchKernelGGL((norm_max_kernel<Tr, 128>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n); break;
+  hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)((3 * n_bh + 255) / 256)), dim3(256), 0, s, scratch, 3 * n_bh);
+  if (!t) {
+    hipLaunchKernelGGL((norm_max_kernel<Tr, D>), dim3((unsigned)blocks, (unsigned)n_bh, 2u), dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n);
+    return hipGetLastError();
+  }
+  const dim3 grid((unsigned)n_bh * (1u + 2u * (unsigned)blocks));
+  switch (t->kind) {
+    case kGateLog: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, kGateLog>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, n_bh, blocks); break;
+    case 0: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, 0>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, n_bh, blocks); break;
+    case 1: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, 1>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, n_bh, blocks); break;
+    case 2: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, 2>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, n_bh, blocks); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
+template <typename Tr>
+static hipError_t auto_threshold_t(const View& q, const View& k, int B, int H, int M, int N, int D, float sm_scale, float* thr, uint32_t* scratch,
+                                   const GateK* t, const int64_t* seq_start, hipStream_t s) {
+  switch (D) {
+    case 16: return auto_threshold_d<Tr, 16>(q, k, B, H, M, N, sm_scale, thr, scratch, t, seq_start, s);
+    case 32: return auto_threshold_d<Tr, 32>(q, k, B, H, M, N, sm_scale, thr, scratch, t, seq_start, s);
+    case 64: return auto_threshold_d<Tr, 64>(q, k, B, H, M, N, sm_scale, thr, scratch, t, seq_start, s);
+    case 128: return auto_threshold_d<Tr, 128>(q, k, B, H, M, N, sm_scale, thr, scratch, t, seq_start, s);
+    default: return hipErrorInvalidValue;
+  }
+}
 
 hipError_t launch_auto_threshold(const View& q, const View& k, int B, int H, int M, int N, int D, int dtype, float sm_scale,
-                                 float* thr, uint32_t* scratch, hipStream_t s) {
-  return dtype == 0 ? auto_threshold_t<Bf16>(q, k, B, H, M, N, D, sm_scale, thr, scratch, s)
-                    : auto_threshold_t<Fp16>(q, k, B, H, M, N, D, sm_scale, thr, scratch, s);
+                                 float* thr, uint32_t* scratch, const GateK* t, const int64_t* seq_start, hipStream_t s) {
+  return dtype == 0 ? auto_threshold_t<Bf16>(q, k, B, H, M, N, D, sm_scale, thr, scratch, t, seq_start, s)
+                    : auto_threshold_t<Fp16>(q, k, B, H, M, N, D, sm_scale, thr, scratch, t, seq_start, s);
+}
+
+// Whether the scan goes beside the norms: where they stream for longer (at about 6 TB/s) than its 256 threads take (about 1 us per 1024 elements and 2
+// to start; the scan of its own has 1024).  "auto" forward, two launches / one, us: B4 T16384 H16 D128 345 / 329, B4 T4096 H32 D64 107 / 99, B2 T8192 H16 D64 68.4 /
+// 62.5, B8 T700 H32 D32 29.6 / 26.9.
+bool threshold_scans(int B, int H, int M, int N, int D) {
+  return (int64_t)B * H * ((int64_t)M + N) * D * 2 >= 6000 * ((int64_t)N + 2000) && (int64_t)B * H * (1 + 2 * (int64_t)((N + 511) / 512)) < (int64_t)1 << 31;
 }
 
 }  // namespace fox

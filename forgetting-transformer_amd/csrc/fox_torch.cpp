@@ -127,11 +127,10 @@ Forward run_forward(Attention& a, const Tensor& q, const Tensor& k, const Tensor
   void* stream = stream_of(q);
   const fox_dims dims = a.dims(q);
   const fox_view qv = view_of(q, a.head_first), kv = view_of(k, a.head_first), vv = view_of(v, a.head_first);
+  Tensor norm_scratch;
   if (a.auto_threshold) {
     a.threshold = at::empty({a.B, a.H}, q.options().dtype(at::kFloat));
-    Tensor scratch = at::empty({a.B, a.H, 3}, q.options().dtype(at::kInt));
-    check(fox_auto_threshold(&dims, &qv, &kv, (float)a.sm_scale, a.threshold.mutable_data_ptr<float>(),
-                             (uint32_t*)scratch.mutable_data_ptr(), stream), "fox_auto_threshold");
+    norm_scratch = at::empty({a.B, a.H, 3}, q.options().dtype(at::kInt));
   }
   // log_lambda (B,H,N) and the log-normaliser (B,H,M) come from one allocation, which the backward keeps; key splits have their own
   int64_t ws_bytes = 0;
@@ -150,7 +149,12 @@ Forward run_forward(Attention& a, const Tensor& q, const Tensor& k, const Tensor
     f.log_fgate = at::empty({a.B, a.H, a.N}, q.options().dtype(at::kFloat));
     gates.log_fgate = f.log_fgate.mutable_data_ptr<float>();
   }
-  if (!from_gates && a.is_logit) {
+  if (a.auto_threshold) {
+    float* thr = a.threshold.mutable_data_ptr<float>();
+    uint32_t* scratch = (uint32_t*)norm_scratch.mutable_data_ptr();
+    if (from_gates) check(fox_auto_threshold(&dims, &qv, &kv, (float)a.sm_scale, thr, scratch, stream), "fox_auto_threshold");
+    else check(fox_auto_threshold_scan(&dims, &qv, &kv, (float)a.sm_scale, thr, scratch, &gates, a.seq_ptr(), base, stream), "fox_auto_threshold_scan");
+  } else if (!from_gates && a.is_logit) {
     check(fox_gate_cumsum_fwd(gates.g, gates.dtype, gates.stride_b, gates.stride_h, gates.stride_n, a.seq_ptr(), gates.log_fgate, base, dims.B,
                               dims.H, dims.N, stream), "fox_gate_cumsum_fwd");
   } else if (!from_gates) {

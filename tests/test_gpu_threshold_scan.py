@@ -1,0 +1,47 @@
+"""The "auto" threshold with the scan of the gates beside it (fox_auto_threshold_scan), against the two on their own, bit for bit.  The first shape streams
+too little for that and takes the two launches; the others have rows of one and several spans of its 256 threads, with ends inside a span."""
+import ctypes as C
+
+import pytest
+import torch
+
+from conftest import make_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("logit", [None, torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B,H,M,N,D,dtype,padded", [(2, 3, 200, 300, 64, torch.bfloat16, False), (16, 32, 500, 513, 32, torch.float16, True),
+                                                    (8, 16, 1000, 1000, 128, torch.bfloat16, False), (3, 60, 2048, 2049, 64, torch.bfloat16, True),
+                                                    (4, 100, 4100, 4100, 16, torch.bfloat16, False)])
+def test_against_the_two_launches(B, H, M, N, D, dtype, padded, logit):
+    from forgetting_transformer.ops import _lib
+    from forgetting_transformer.ops.forgetting_attention import _view
+    lib = _lib.load()
+    q, k, _, g, _, ss = make_inputs(B, H, M, N, D, dtype=dtype, device="cuda", seed=N, gate_mean=1.0, head_first=False,
+                                    seq_start=[(N * b) // B for b in range(B)] if padded else None)
+    q, k, g = (x.transpose(1, 2) for x in (q, k, g))   # strided gates
+    kind = {None: 2, torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}[logit]
+    if logit is not None:
+        g = (g * 3 + 2).to(logit)
+    dims = _lib.Dims(B, H, M, N, D, 0 if dtype == torch.bfloat16 else 1)
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ssp = None if ss is None else ss.data_ptr()
+    res = []
+    for together in (False, True):
+        thr, scratch = torch.full((B, H), float("nan"), device="cuda"), torch.full((B, H, 3), -1, dtype=torch.int32, device="cuda")
+        c, lg = (torch.full((B, H, N), float("nan"), device="cuda") for _ in range(2))
+        views = C.byref(_view(q)), C.byref(_view(k))
+        if together:
+            gates = _lib.Gates(g.data_ptr(), logit is not None, kind, *g.stride(), lg.data_ptr() if logit is not None else None)
+            _lib.check(lib.fox_auto_threshold_scan(C.byref(dims), *views, D ** -0.5, thr.data_ptr(), scratch.data_ptr(), C.byref(gates), ssp,
+                                                   c.data_ptr(), stream), "together")
+        else:
+            _lib.check(lib.fox_auto_threshold(C.byref(dims), *views, D ** -0.5, thr.data_ptr(), scratch.data_ptr(), stream), "threshold")
+            if logit is None:
+                _lib.check(lib.fox_cumsum_fwd(g.data_ptr(), *g.stride(), ssp, c.data_ptr(), B, H, N, stream), "scan")
+            else:
+                _lib.check(lib.fox_gate_cumsum_fwd(g.data_ptr(), kind, *g.stride(), ssp, lg.data_ptr(), c.data_ptr(), B, H, N, stream), "scan")
+        res.append((thr, c) + ((lg,) if logit is not None else ()))
+    for a, b in zip(*res):
+        assert torch.isfinite(b).all() and torch.equal(a, b)
