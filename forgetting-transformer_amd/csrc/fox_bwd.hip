@@ -329,6 +329,8 @@ __device__ __forceinline__ void dkdv_body(const BwdK& a, int bh, int nt, const D
   const float c_ref = c_row[n0];
   const float c_key = c_row[min(n, N - 1)];
   const float c_last = c_row[min(N - 1, n0 + BN - 1)];  // for the pruning bound below
+  float drow_key = 0.f;   // (the split variant is short: the row sum for its dc is requested here, not waited for at the end)
+  if constexpr (DSPLIT) drow_key = a.drow[(int64_t)bh * M + min(max(n - p_seq, 0), M - 1)];
   const float qk_scale = nonzero_scale(a.sm_scale * kLog2e), inv_scale = 1.0f / qk_scale;
 
   // Per-row terms of a step: the loads are requested here, the arithmetic on them is done where the values
@@ -392,7 +394,7 @@ __device__ __forceinline__ void dkdv_body(const BwdK& a, int bh, int nt, const D
       kreg[kk] = lds_row_operand<D>(q_tile0, 32 * kb + i, 2 * kk + g);
       vreg[kk] = lds_row_operand<D>(do_tile0, 32 * kb + i, 2 * kk + g);
     }
-    __syncthreads();   // buffer set 0 is free for the second step's tiles
+    // (the barrier in front of the first step frees buffer set 0 for the second step's tiles)
   }
 
   // The long-loop kernel (head dim 128, one workgroup per CU).  Phase 1: the steps that touch the tile's
@@ -502,7 +504,7 @@ __device__ __forceinline__ void dkdv_body(const BwdK& a, int bh, int nt, const D
   if (n < N && g == 0 && dh == 0) {  // (the two waves of a split pair hold the same column sums)
     float rtot = 0.f;   // (beside the dQ kernel: the reverse scan adds it)
     if constexpr (!OWN_DELTA) {
-      if (n >= p_seq) rtot = a.drow[(int64_t)bh * M + (n - p_seq)];
+      if (n >= p_seq) rtot = DSPLIT ? drow_key : a.drow[(int64_t)bh * M + (n - p_seq)];
     }
     a.dc[(int64_t)bh * N + n] = rtot - ctot;
   }
@@ -510,9 +512,19 @@ __device__ __forceinline__ void dkdv_body(const BwdK& a, int bh, int nt, const D
   // wave's DW columns)
   static_assert(2 * kStoreStageBytes<DW> <= Tile<D>::bytes(BMQ), "two waves stage in one tile buffer");
   __syncthreads();  // every wave is done with the tiles of the last step
-  char* stage = (wave < 2 ? q_tile0 : do_tile0) + (wave & 1) * kStoreStageBytes<DW>;
-  store_rows_via_lds<Tr, DW>(stage, dkacc, a.sm_scale, dkp + dh * DW, a.dk.st, n_w0, N, lane);
-  store_rows_via_lds<Tr, DW>(stage, dvacc, 1.0f, dvp + dh * DW, a.dv.st, n_w0, N, lane);
+  if constexpr (DSPLIT) {   // both at once, a tile buffer per wave: one pass through LDS instead of two
+    static_assert(2 * kStoreStageBytes<DW> <= Tile<D>::bytes(BMQ), "a wave stages both in one tile buffer");
+    char* stage = wave == 0 ? q_tile0 : wave == 1 ? q_tile1 : wave == 2 ? do_tile0 : do_tile1;
+    stage_rows<Tr, DW>(stage, dkacc, a.sm_scale, lane);
+    stage_rows<Tr, DW>(stage + kStoreStageBytes<DW>, dvacc, 1.0f, lane);
+    staged_rows_visible();
+    store_staged_rows<Tr, DW>(stage, dkp + dh * DW, a.dk.st, n_w0, N, lane);
+    store_staged_rows<Tr, DW>(stage + kStoreStageBytes<DW>, dvp + dh * DW, a.dv.st, n_w0, N, lane);
+  } else {
+    char* stage = (wave < 2 ? q_tile0 : do_tile0) + (wave & 1) * kStoreStageBytes<DW>;
+    store_rows_via_lds<Tr, DW>(stage, dkacc, a.sm_scale, dkp + dh * DW, a.dk.st, n_w0, N, lane);
+    store_rows_via_lds<Tr, DW>(stage, dvacc, 1.0f, dvp + dh * DW, a.dv.st, n_w0, N, lane);
+  }
 }
 
 template <typename Tr, int D, bool DSPLIT>

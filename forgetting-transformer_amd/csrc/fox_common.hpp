@@ -379,9 +379,8 @@ template <int D>
 constexpr int kStoreStageBytes = 32 * (2 * D + 16);
 
 template <typename Tr, int D>
-__device__ __forceinline__ void store_rows_via_lds(char* stage, const f32x16 (&acc)[(D + 31) / 32], float mul, uint16_t* dst,
-                                                   int64_t row_stride, int row0, int row_limit, int lane) {
-  constexpr int DB = (D + 31) / 32, CH = D / 8, RS = 2 * D + 16;
+__device__ __forceinline__ void stage_rows(char* stage, const f32x16 (&acc)[(D + 31) / 32], float mul, int lane) {
+  constexpr int DB = (D + 31) / 32, RS = 2 * D + 16;
   const int g = lane >> 5, i = lane & 31;
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -395,9 +394,15 @@ __device__ __forceinline__ void store_rows_via_lds(char* stage, const f32x16 (&a
         *reinterpret_cast<u32x2*>(stage + i * RS + 2 * d) = w;
       }
     }
+}
+__device__ __forceinline__ void staged_rows_visible() {   // to the wave that staged them
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+template <typename Tr, int D>
+__device__ __forceinline__ void store_staged_rows(const char* stage, uint16_t* dst, int64_t row_stride, int row0, int row_limit, int lane) {
+  constexpr int CH = D / 8, RS = 2 * D + 16;
 #pragma unroll
   for (int idx0 = 0; idx0 < 32 * CH; idx0 += kWave) {
     const int idx = idx0 + lane, row = idx / CH, ch = idx % CH;
@@ -408,6 +413,13 @@ __device__ __forceinline__ void store_rows_via_lds(char* stage, const f32x16 (&a
       __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst + (int64_t)(row0 + row) * row_stride + 8 * ch));
     }
   }
+}
+template <typename Tr, int D>
+__device__ __forceinline__ void store_rows_via_lds(char* stage, const f32x16 (&acc)[(D + 31) / 32], float mul, uint16_t* dst,
+                                                   int64_t row_stride, int row0, int row_limit, int lane) {
+  stage_rows<Tr, D>(stage, acc, mul, lane);
+  staged_rows_visible();
+  store_staged_rows<Tr, D>(stage, dst, row_stride, row0, row_limit, lane);
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();   // the staging area may be rewritten after this
 }
