@@ -8,7 +8,7 @@
 //                  registers as MFMA B operands; dK^T, dV^T accumulators) and
 //                  walks the query tiles below its diagonal; writes dk, dv and
 //                  dc[n] = drow[n - (N - M)] - sum_i dS[i,n].
-//   bwd_kernel   : both kinds of workgroups in one launch, for small grids (bwd_together).
+//                  With BOTH the launch holds the workgroups of either kernel, for small grids (bwd_together).
 //   delta_kernel : delta alone (a stage of its own for callers that want it;
 //                  the backward does not launch it).
 // Every kernel only stores: no read-modify-write of anything another kernel wrote,
@@ -226,7 +226,7 @@ __device__ __forceinline__ void dkdv_step_interior(const char* q_tile, const cha
 // workgroups (two waves per SIMD) share a CU.
 //
 // OWN_DELTA: the body forms delta = sum_d o_id * do_id for the rows of a step itself instead of reading what the dQ kernel left, so
-// that it can run beside it (bwd_kernel).  A wave takes the rows whose dO it has brought into LDS: its own wait is enough to read
+// that it can run beside it (dq_kernel with BOTH).  A wave takes the rows whose dO it has brought into LDS: its own wait is enough to read
 // them, and the barrier that publishes the step's tiles publishes their delta as well.
 template <int D, bool DSPLIT>
 struct DkdvLds {
@@ -592,17 +592,48 @@ __device__ __forceinline__ void dq_tile(const char* k_tile, const char* v_tile, 
   }
 }
 
-template <int D>
-struct DqLds {
-  char *k_tile0, *k_tile1, *v_tile0, *v_tile1;   // Tile<D>::bytes(kFwdBN) each
-  float *cn_s0, *cn_s1;                          // kFwdBN each
-};
-template <typename Tr, int D>
-__device__ __forceinline__ void dq_body(const BwdK& a, int bh, int mt, const DqLds<D>& lds) {
-  constexpr int BM = kFwdBM, BN = kFwdBN;
+// The kernel's argument block behind a pointer the compiler cannot see through: each kind of workgroup loads its arguments where it needs
+// them (loaded at entry, those of both would not fit the scalar registers).
+__device__ __forceinline__ const BwdK& own_arguments() {
+  typedef const BwdK __attribute__((address_space(4)))* kernarg;
+  kernarg p = (kernarg)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const BwdK*)p;
+}
+
+// BOTH: dQ and dK/dV in one launch, for small grids of head dims up to 64 (bwd_together): workgroups of either kind side by side, the heaviest of either
+// kind first.  One after the other, each of the two kernels waits for its longest walk on a chip that is mostly idle.  (The dQ walk is part of the
+// kernel and not a function both kernels call: that way the compiler waits for LDS eight times more often in it, and at D = 128 it took 5-10 % longer.)
+template <typename Tr, int D, bool BOTH>
+__global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK args) {
+  constexpr int BM = kFwdBM, BN = kFwdBN, ROWS = BOTH ? kKvBM : kFwdBN;   // rows of a tile buffer: the dK/dV walk needs the larger ones
   constexpr int KK = D / 16, DB = (D + 31) / 32;
-  char *k_tile0 = lds.k_tile0, *k_tile1 = lds.k_tile1, *v_tile0 = lds.v_tile0, *v_tile1 = lds.v_tile1;
-  float *cn_s0 = lds.cn_s0, *cn_s1 = lds.cn_s1;
+  static_assert(!BOTH || (D <= 64 && kKvBM >= kFwdBN), "two workgroups of either kind per CU; the dQ walk fits the buffers of the dK/dV walk");
+  __shared__ __align__(16) char k_tile0[Tile<D>::bytes(ROWS)];
+  __shared__ __align__(16) char k_tile1[Tile<D>::bytes(ROWS)];
+  __shared__ __align__(16) char v_tile0[Tile<D>::bytes(ROWS)];
+  __shared__ __align__(16) char v_tile1[Tile<D>::bytes(ROWS)];
+  __shared__ __align__(16) float cn_s0[ROWS];
+  __shared__ __align__(16) float cn_s1[ROWS];
+  int bh, mt;
+  if constexpr (BOTH) {
+    __shared__ __align__(16) float row2[ROWS];
+    __shared__ __align__(16) float row3[ROWS];
+    const int q_tiles = (args.M + BM - 1) / BM;
+    int t;
+    decode_block(blockIdx.x, 2 * args.n_tiles, args.B * args.H, args.groups, !args.even, false, bh, t);
+    if (!(t & 1)) {
+#ifdef __HIP_DEVICE_COMPILE__
+      dkdv_body<Tr, D, false, true>(own_arguments(), bh, args.n_tiles - 1 - t / 2, {k_tile0, k_tile1, v_tile0, v_tile1, cn_s0, cn_s1, row2, row3});
+#endif
+      return;
+    }
+    mt = t / 2 - (args.n_tiles - q_tiles);   // (fewer query tiles than key tiles where M < N)
+    if (mt < 0) return;
+  } else {
+    decode_block(blockIdx.x, args.n_tiles, args.B * args.H, args.groups, !args.even, true, bh, mt);
+  }
+  const BwdK& a = BOTH ? own_arguments() : args;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 5, i = lane & 31;
   const int b = bh / a.H, h = bh % a.H;
@@ -752,57 +783,6 @@ __device__ __forceinline__ void dq_body(const BwdK& a, int bh, int mt, const DqL
   store_rows_via_lds<Tr, D>(stage, dqacc, a.sm_scale, dqp, a.dq.st, m0 + 32 * wave, M, lane);
 }
 
-template <typename Tr, int D>
-__global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK a) {
-  __shared__ __align__(16) char k_tile0[Tile<D>::bytes(kFwdBN)];
-  __shared__ __align__(16) char k_tile1[Tile<D>::bytes(kFwdBN)];
-  __shared__ __align__(16) char v_tile0[Tile<D>::bytes(kFwdBN)];
-  __shared__ __align__(16) char v_tile1[Tile<D>::bytes(kFwdBN)];
-  __shared__ __align__(16) float cn_s0[kFwdBN];
-  __shared__ __align__(16) float cn_s1[kFwdBN];
-#ifdef __HIP_DEVICE_COMPILE__
-  int bh, mt;
-  decode_block(blockIdx.x, a.n_tiles, a.B * a.H, a.groups, !a.even, true, bh, mt);
-  dq_body<Tr, D>(a, bh, mt, {k_tile0, k_tile1, v_tile0, v_tile1, cn_s0, cn_s1});
-#endif
-}
-
-// ---------------------------------------------------------------------------
-// The kernel's argument block behind a pointer the compiler cannot see through: each kind of workgroup loads its arguments where it needs
-// them (loaded at entry, those of both would not fit the scalar registers).
-__device__ __forceinline__ const BwdK& own_arguments() {
-  typedef const BwdK __attribute__((address_space(4)))* kernarg;
-  kernarg p = (kernarg)__builtin_amdgcn_kernarg_segment_ptr();
-  asm volatile("" : "+s"(p));
-  return *(const BwdK*)p;
-}
-
-// dQ and dK/dV in one launch, for small grids of head dims up to 64: workgroups of either kind side by side, the heaviest of either kind first.
-// One after the other, each of the two kernels waits for its longest walk on a chip that is mostly idle.
-template <typename Tr, int D>
-__global__ __launch_bounds__(256, 2) void bwd_kernel(const BwdK a) {
-  static_assert(D <= 64 && kKvBM >= kFwdBN, "two workgroups of either kind per CU; the dQ walk fits the buffers of the dK/dV walk");
-  __shared__ __align__(16) char tile0[Tile<D>::bytes(kKvBM)];
-  __shared__ __align__(16) char tile1[Tile<D>::bytes(kKvBM)];
-  __shared__ __align__(16) char tile2[Tile<D>::bytes(kKvBM)];
-  __shared__ __align__(16) char tile3[Tile<D>::bytes(kKvBM)];
-  __shared__ __align__(16) float row0[kKvBM];
-  __shared__ __align__(16) float row1[kKvBM];
-  __shared__ __align__(16) float row2[kKvBM];
-  __shared__ __align__(16) float row3[kKvBM];
-#ifdef __HIP_DEVICE_COMPILE__
-  const int q_tiles = (a.M + kFwdBM - 1) / kFwdBM;
-  int bh, t;
-  decode_block(blockIdx.x, 2 * a.n_tiles, a.B * a.H, a.groups, !a.even, false, bh, t);
-  if (t & 1) {
-    const int mt = t / 2 - (a.n_tiles - q_tiles);   // (fewer query tiles than key tiles where M < N)
-    if (mt >= 0) dq_body<Tr, D>(own_arguments(), bh, mt, {tile0, tile1, tile2, tile3, row0, row1});
-  } else {
-    dkdv_body<Tr, D, false, true>(own_arguments(), bh, a.n_tiles - 1 - t / 2, {tile0, tile1, tile2, tile3, row0, row1, row2, row3});
-  }
-#endif
-}
-
 // explicit instantiations: every (dtype, head dim) pair the dispatchers can reach
 #define FOX_INSTANTIATE_BWD(KERNEL, TR)                      \
   template __global__ void KERNEL<TR, 16>(const BwdK);       \
@@ -819,11 +799,16 @@ FOX_INSTANTIATE_BWD(delta_kernel, Fp16)
   template __global__ void dkdv_kernel<TR, 128, true>(const BwdK);
 FOX_INSTANTIATE_DKDV(Bf16)
 FOX_INSTANTIATE_DKDV(Fp16)
-FOX_INSTANTIATE_BWD(dq_kernel, Bf16)
-FOX_INSTANTIATE_BWD(dq_kernel, Fp16)
-#define FOX_INSTANTIATE_BOTH(TR)                               template __global__ void bwd_kernel<TR, 16>(const BwdK);     template __global__ void bwd_kernel<TR, 32>(const BwdK);     template __global__ void bwd_kernel<TR, 64>(const BwdK);
-FOX_INSTANTIATE_BOTH(Bf16)
-FOX_INSTANTIATE_BOTH(Fp16)
+#define FOX_INSTANTIATE_DQ(TR)                                       \
+  template __global__ void dq_kernel<TR, 16, false>(const BwdK);     \
+  template __global__ void dq_kernel<TR, 32, false>(const BwdK);     \
+  template __global__ void dq_kernel<TR, 64, false>(const BwdK);     \
+  template __global__ void dq_kernel<TR, 128, false>(const BwdK);    \
+  template __global__ void dq_kernel<TR, 16, true>(const BwdK);      \
+  template __global__ void dq_kernel<TR, 32, true>(const BwdK);      \
+  template __global__ void dq_kernel<TR, 64, true>(const BwdK);
+FOX_INSTANTIATE_DQ(Bf16)
+FOX_INSTANTIATE_DQ(Fp16)
 
 // ---------------------------------------------------------------------------
 #define FOX_DISPATCH_D(KERNEL, GRID, SMEM)                                                        \
@@ -870,7 +855,13 @@ static hipError_t dq_t(const BwdK& a0, int D, hipStream_t s) {
   a.groups = order_groups(a.B * a.H, a.n_tiles, a.M, a.N, D, a.k.st, a.thr != nullptr);
   a.even = even_tiles(a.M, a.N);
   const dim3 grid((unsigned)(a.n_tiles * a.B * a.H));
-  FOX_DISPATCH_D(dq_kernel, grid, 0)
+  switch (D) {
+    case 16: hipLaunchKernelGGL((dq_kernel<Tr, 16, false>), grid, dim3(256), 0, s, a); break;
+    case 32: hipLaunchKernelGGL((dq_kernel<Tr, 32, false>), grid, dim3(256), 0, s, a); break;
+    case 64: hipLaunchKernelGGL((dq_kernel<Tr, 64, false>), grid, dim3(256), 0, s, a); break;
+    case 128: hipLaunchKernelGGL((dq_kernel<Tr, 128, false>), grid, dim3(256), 0, s, a); break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
 
@@ -882,9 +873,9 @@ static hipError_t bwd_t(const BwdK& a0, int D, hipStream_t s) {
   a.even = even_tiles(a.M, a.N);
   const dim3 grid((unsigned)(2 * a.n_tiles * a.B * a.H));
   switch (D) {
-    case 16: hipLaunchKernelGGL((bwd_kernel<Tr, 16>), grid, dim3(256), 0, s, a); break;
-    case 32: hipLaunchKernelGGL((bwd_kernel<Tr, 32>), grid, dim3(256), 0, s, a); break;
-    case 64: hipLaunchKernelGGL((bwd_kernel<Tr, 64>), grid, dim3(256), 0, s, a); break;
+    case 16: hipLaunchKernelGGL((dq_kernel<Tr, 16, true>), grid, dim3(256), 0, s, a); break;
+    case 32: hipLaunchKernelGGL((dq_kernel<Tr, 32, true>), grid, dim3(256), 0, s, a); break;
+    case 64: hipLaunchKernelGGL((dq_kernel<Tr, 64, true>), grid, dim3(256), 0, s, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -898,7 +889,7 @@ hipError_t launch_bwd_delta(const BwdK& a, int D, int dtype, hipStream_t s) {
 hipError_t launch_bwd_dkdv(const BwdK& a, int D, int dtype, hipStream_t s) {
   return dtype == 0 ? dkdv_t<Bf16>(a, D, s) : dkdv_t<Fp16>(a, D, s);
 }
-// Whether dQ and dK/dV go out as one launch (bwd_kernel).  One after the other, each waits for the longest walk of a grid that fills the chip
+// Whether dQ and dK/dV go out as one launch (dq_kernel with BOTH).  One after the other, each waits for the longest walk of a grid that fills the chip
 // once or less; side by side the two waits are one, and so are two launches and the drain between them.  Backward, one after the other / together, us:
 // D 64 B1 H5 T3000 118 / 80, B2 H8 T2000 82 / 60, B4 H12 T512 31.9 / 27.8, B16 H16 T250 35.0 / 32.0, B2 H12 T2048 at -60 45.4 / 44.4; D 32 B3 H5 T777 34.6 / 29.3,
 // D 16 B4 H16 T1000 42.8 / 33.7.  Against it stand delta, formed anew for every step, and the LDS of the dK/dV walk, which the dQ walk does not
