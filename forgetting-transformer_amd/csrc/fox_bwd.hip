@@ -540,7 +540,7 @@ __global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(
   __shared__ __align__(16) float dl_s1[BMQ];
 #ifdef __HIP_DEVICE_COMPILE__
   int bh, nt;
-  decode_block(blockIdx.x, a.n_tiles, a.B * a.H, a.groups, !a.even && (D <= 64 || DSPLIT), false, bh, nt);
+  decode_block(blockIdx.x, a.order, false, bh, nt);
   nt = a.n_tiles - 1 - nt;  // the first key tiles see the most query rows: start them first
   dkdv_body<Tr, D, DSPLIT, false>(a, bh, nt, {q_tile0, q_tile1, do_tile0, do_tile1, rc_s0, rc_s1, dl_s0, dl_s1});
 #endif
@@ -621,7 +621,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK args) {
     __shared__ __align__(16) float row3[ROWS];
     const int q_tiles = (args.M + BM - 1) / BM;
     int t;
-    decode_block(blockIdx.x, 2 * args.n_tiles, args.B * args.H, args.groups, !args.even, false, bh, t);
+    decode_block(blockIdx.x, args.order, false, bh, t);
     if (!(t & 1)) {
 #ifdef __HIP_DEVICE_COMPILE__
       dkdv_body<Tr, D, false, true>(own_arguments(), bh, args.n_tiles - 1 - t / 2, {k_tile0, k_tile1, v_tile0, v_tile1, cn_s0, cn_s1, row2, row3});
@@ -631,12 +631,12 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK args) {
     mt = t / 2 - (args.n_tiles - q_tiles);   // (fewer query tiles than key tiles where M < N)
     if (mt < 0) return;
   } else {
-    decode_block(blockIdx.x, args.n_tiles, args.B * args.H, args.groups, !args.even, true, bh, mt);
+    decode_block(blockIdx.x, args.order, true, bh, mt);
   }
   const BwdK& a = BOTH ? own_arguments() : args;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 5, i = lane & 31;
-  const int b = bh / a.H, h = bh % a.H;
+  const int b = divide(bh, a.order.by_heads), h = bh - b * a.H;
   const int M = a.M, N = a.N, p_seq = N - M;
   const int m0 = mt * BM;
   const float* c_row = a.c + (int64_t)bh * N;
@@ -829,15 +829,17 @@ static hipError_t delta_t(const BwdK& a, int D, hipStream_t s) {
 template <typename Tr>
 static hipError_t dkdv_t(const BwdK& a0, int D, hipStream_t s) {
   BwdK a = a0;
-  a.groups = order_groups(a.B * a.H, (a.N + kKvBN - 1) / kKvBN, a.M, a.N, D, a.k.st, a.thr != nullptr);
-  a.even = even_tiles(a.M, a.N);
+  const int groups = order_groups(a.B * a.H, (a.N + kKvBN - 1) / kKvBN, a.M, a.N, D, a.k.st, a.thr != nullptr);
+  const bool fold = !even_tiles(a.M, a.N) && (D <= 64 || a.cls == kClassLight);   // (two workgroups per CU)
   if (a.cls == kClassLight) {  // the split variant: 64 keys per workgroup
     if (!dkdv_split_supports(D)) return hipErrorInvalidValue;
     a.n_tiles = (a.N + 63) / 64;
+    a.order = block_order(a.B, a.H, a.n_tiles, groups, fold);
     hipLaunchKernelGGL((dkdv_kernel<Tr, 128, true>), dim3((unsigned)(a.n_tiles * a.B * a.H)), dim3(256), 0, s, a);
     return hipGetLastError();
   }
   a.n_tiles = (a.N + kKvBN - 1) / kKvBN;
+  a.order = block_order(a.B, a.H, a.n_tiles, groups, fold);
   const dim3 grid((unsigned)(a.n_tiles * a.B * a.H));
   switch (D) {
     case 16: hipLaunchKernelGGL((dkdv_kernel<Tr, 16, false>), grid, dim3(256), 0, s, a); break;
@@ -852,8 +854,7 @@ template <typename Tr>
 static hipError_t dq_t(const BwdK& a0, int D, hipStream_t s) {
   BwdK a = a0;
   a.n_tiles = (a.M + kFwdBM - 1) / kFwdBM;
-  a.groups = order_groups(a.B * a.H, a.n_tiles, a.M, a.N, D, a.k.st, a.thr != nullptr);
-  a.even = even_tiles(a.M, a.N);
+  a.order = block_order(a.B, a.H, a.n_tiles, order_groups(a.B * a.H, a.n_tiles, a.M, a.N, D, a.k.st, a.thr != nullptr), !even_tiles(a.M, a.N));
   const dim3 grid((unsigned)(a.n_tiles * a.B * a.H));
   switch (D) {
     case 16: hipLaunchKernelGGL((dq_kernel<Tr, 16, false>), grid, dim3(256), 0, s, a); break;
@@ -869,8 +870,7 @@ template <typename Tr>
 static hipError_t bwd_t(const BwdK& a0, int D, hipStream_t s) {
   BwdK a = a0;
   a.n_tiles = (a.N + kKvBN - 1) / kKvBN;
-  a.groups = order_groups(a.B * a.H, a.n_tiles, a.M, a.N, D, a.k.st, a.thr != nullptr);
-  a.even = even_tiles(a.M, a.N);
+  a.order = block_order(a.B, a.H, 2 * a.n_tiles, order_groups(a.B * a.H, a.n_tiles, a.M, a.N, D, a.k.st, a.thr != nullptr), !even_tiles(a.M, a.N));
   const dim3 grid((unsigned)(2 * a.n_tiles * a.B * a.H));
   switch (D) {
     case 16: hipLaunchKernelGGL((dq_kernel<Tr, 16, true>), grid, dim3(256), 0, s, a); break;

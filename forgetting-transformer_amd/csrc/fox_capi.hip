@@ -266,11 +266,12 @@ int fwd_impl(const fox_fwd_args* args, void* workspace, int64_t workspace_bytes,
   k.B = args->dims.B; k.H = args->dims.H; k.M = args->dims.M; k.N = args->dims.N;
   k.sm_scale = args->sm_scale;
   k.n_mtiles = (args->dims.M + fox::kFwdBM - 1) / fox::kFwdBM;
-  k.groups = fox::order_groups(k.B * k.H, k.n_mtiles, k.M, k.N, args->dims.D, k.k.st, k.thr != nullptr);
-  k.even = fox::even_tiles(k.M, k.N);
   const FwdPlan plan = plan_fwd(args->dims, k.thr != nullptr, workspace != nullptr || gates);   // (with gates: pairs in place of splits, or neither)
   k.splits = plan.splits;
   k.pair = plan.pair;
+  k.order = fox::block_order(k.B, k.H, k.n_mtiles * k.splits, fox::order_groups(k.B * k.H, k.n_mtiles, k.M, k.N, args->dims.D, k.k.st, k.thr != nullptr),
+                             !fox::even_tiles(k.M, k.N) && !(k.pair && k.splits <= 1));   // (paired: one workgroup per CU)
+  k.by_splits = fox::divisor(k.splits);
   k.stream = k.n_mtiles == 1 && (int64_t)k.B * k.H * k.N * args->dims.D * 4 >= g_stream_min_kv_bytes.load(std::memory_order_relaxed);
   if (workspace) {
     const int64_t need = split_bytes(args->dims, plan.wanted);
@@ -598,6 +599,8 @@ int fox_attn_decode_counted(const fox_fwd_args* args, const float* g, int64_t g_
       if (fox::decode_merges(k.B, k.H, k.splits)) k.arrived = arrived;
     }
   }
+  k.by_splits = fox::divisor(k.splits);
+  k.by_heads = fox::divisor(k.H);
   return check_hip(fox::launch_decode_gates(k, args->dims.D, args->dims.dtype, (hipStream_t)stream), "fox_attn_decode");
 }
 

@@ -9,6 +9,8 @@
 #include <type_traits>
 #include <utility>
 
+#include "fox_kernels.hpp"
+
 namespace fox {
 
 // Compile-time loop: f(std::integral_constant<int, I>{}) for I = BEGIN .. END-1, so that everything
@@ -515,43 +517,6 @@ __device__ __forceinline__ f32x16 acc_init(const float* t, int row0, int g) {
 // magnitude is replaced by 1e-30, for which scale * (q.k) still rounds to nothing against
 // the bias.
 __device__ __forceinline__ float nonzero_scale(float s) { return fabsf(s) < 1e-30f ? 1e-30f : s; }
-
-// Workgroup id -> (bh, tile).  Every tile of one (batch, head) goes to one XCD when the count allows it (the hardware
-// deals consecutive workgroup ids round-robin over the 8 XCDs, each with its own L2).  Within an XCD the (batch, head)
-// pairs are taken in `groups` groups of nearly equal size, and inside a group the tiles come heaviest first (largest index
-// under a causal mask) with the pairs of the group in turn.  One pair after the other would start the last pair's
-// heaviest tile when the chip is about to run empty; all pairs at once would stream more K and V than an L2 holds.
-// order_groups() on the host picks the number of groups.
-// `fold`: when the whole grid is resident at two workgroups per CU, the second workgroup of a CU is the one that arrives
-// kCus ids after the first.  Taken in the same order both would be heavy on one CU and both light on another; from
-// workgroup kCus on the list is therefore walked from its light end (forward B1 H16 T4096 D128: 109 -> 84 us, dQ 152 -> 116 us).
-// `last_first`: the pairs from the last to the first.  The dQ kernel takes them so, between a forward and a dK/dV kernel that start with the
-// first: each of the three then opens on the tensors its predecessor touched last, which are still in the 256 MiB last-level cache.
-// Backward with dQ ascending / descending: B4 T16384 H16 D128 "auto" 731 / 710 us, B16 H16 T4096 D64 "auto" 516 / 491,
-// B4 H32 T4096 D64 at -10 240 / 229, without a threshold 963 / 953.
-constexpr int kXcds = 8, kCus = 256;
-__device__ __forceinline__ void decode_block(int wid, int n_tiles, int n_bh, int groups, bool fold, bool last_first, int& bh, int& tile) {
-  const bool by_xcd = n_bh % kXcds == 0;
-  const int nb = by_xcd ? n_bh / kXcds : n_bh, cus = by_xcd ? kCus / kXcds : kCus;
-  const int total = n_tiles * nb;
-  int r = by_xcd ? wid / kXcds : wid;
-  if (fold && r >= cus && total <= 2 * cus) r = total - 1 - (r - cus);
-  int b;
-  if (groups == 1) {   // the usual case of a small grid, where the divisions below would show
-    const int t = r / nb;
-    b = r - t * nb;
-    tile = n_tiles - 1 - t;
-  } else {             // the first nb % groups groups hold one pair more than the others
-    const int small = nb / groups, extra = nb % groups, big_end = extra * (small + 1) * n_tiles;
-    const bool big = r < big_end;
-    const int size = big ? small + 1 : small;
-    const int q = big ? r : r - big_end, grp = q / (size * n_tiles), in = q - grp * size * n_tiles;
-    b = (big ? 0 : extra * (small + 1)) + grp * size + in % size;
-    tile = n_tiles - 1 - in / size;
-  }
-  if (last_first) b = nb - 1 - b;
-  bh = by_xcd ? b * kXcds + wid % kXcds : b;
-}
 
 // Adaptive Computation Pruning, query-side bound: the first key block of width BN
 // in [0, t_max] whose largest decay  c_out - c[last column of the block]  is not

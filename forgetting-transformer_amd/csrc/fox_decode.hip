@@ -53,8 +53,8 @@ __global__ __launch_bounds__(256) void decode_kernel(const FwdK a) {
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int ch = lane % LPR, r = lane / LPR;
-  const int sp = blockIdx.x % a.splits, bh = blockIdx.x / a.splits;
-  const int b = bh / a.H, h = bh % a.H;
+  const int bh = divide(blockIdx.x, a.by_splits), sp = blockIdx.x - bh * a.splits;
+  const int b = divide(bh, a.order.by_heads), h = bh - b * a.H;
   const int N = a.N;
   const float* c_row = a.c + (int64_t)bh * N;
   const uint16_t* qp = a.q.ptr + b * a.q.sb + h * a.q.sh;
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256) void decode_kernel(const FwdK a) {
 
   // this workgroup's share of [lo, N): whole rounds of 4 waves x KPB keys
   const int n_keys = N - lo;
-  int per = (n_keys + a.splits - 1) / a.splits;
+  int per = divide(n_keys + a.splits - 1, a.by_splits);
   per = (per + 4 * KPB - 1) / (4 * KPB) * (4 * KPB);
   const int k0 = min(N, lo + sp * per), k1 = min(N, k0 + per);
 
@@ -228,7 +228,7 @@ __device__ __forceinline__ void decode_merge(const DecodeK& a, int bh) {
   __shared__ float weight[kDecodeMaxSplits];
   __shared__ float l_tot, m_tot;
   __shared__ __align__(16) float part[GROUPS][D];
-  const int tid = threadIdx.x, b = bh / a.H, h = bh % a.H, splits = a.splits;
+  const int tid = threadIdx.x, b = divide(bh, a.by_heads), h = bh - b * a.H, splits = a.splits;
   const int grp = tid / TPR, d = (tid % TPR) * 4;
   const float* wo = a.ws_o + (int64_t)bh * splits * D + d;
   f32x4 x[PER];
@@ -303,8 +303,8 @@ __global__ __launch_bounds__(64 * WAVES) void decode_gates_kernel(const DecodeK 
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ch = lane % LPR, r = lane / LPR;
-  const int sp = blockIdx.x % a.splits, bh = blockIdx.x / a.splits;
-  const int b = bh / a.H, h = bh % a.H;
+  const int bh = divide(blockIdx.x, a.by_splits), sp = blockIdx.x - bh * a.splits;
+  const int b = divide(bh, a.by_heads), h = bh - b * a.H;
   const int N = a.N;
   const float* gp = a.g + b * a.g_sb + h * a.g_sh;
   const uint16_t* qp = a.q.ptr + b * a.q.sb + h * a.q.sh;
@@ -317,8 +317,8 @@ __global__ __launch_bounds__(64 * WAVES) void decode_gates_kernel(const DecodeK 
     lo = (int)(s64 < 0 ? 0 : (s64 > N ? N : s64));
   }
   // run gw of the splits * WAVES runs, counted from the last key: whole batches, the first one excepted
-  const int runs = a.splits * WAVES, gw = sp * WAVES + wave;
-  int per = (N - lo + runs - 1) / runs;
+  const int gw = sp * WAVES + wave;
+  int per = divide((N - lo + WAVES - 1) / WAVES + a.splits - 1, a.by_splits);
   per = (per + KPB - 1) / KPB * KPB;
   const int64_t back = (int64_t)gw * per;
   const int k1 = back < N - lo ? N - (int)back : lo, k0 = k1 - lo > per ? k1 - per : lo;

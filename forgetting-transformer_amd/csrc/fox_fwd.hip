@@ -346,13 +346,13 @@ __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's o
   int bh, mt, sp = 0;
   if constexpr (SPLIT) {  // (query tile, key split) pairs take the place of query tiles
     int mts;
-    decode_block(blockIdx.x, a.n_mtiles * a.splits, a.B * a.H, a.groups, !a.even, false, bh, mts);
-    mt = mts / a.splits;
-    sp = mts % a.splits;
+    decode_block(blockIdx.x, a.order, false, bh, mts);
+    mt = divide(mts, a.by_splits);
+    sp = mts - mt * a.splits;
   } else {
-    decode_block(blockIdx.x, a.n_mtiles, a.B * a.H, a.groups, !a.even && !PAIR, false, bh, mt);   // paired: one workgroup per CU
+    decode_block(blockIdx.x, a.order, false, bh, mt);
   }
-  const int b = bh / a.H, h = bh % a.H;
+  const int b = divide(bh, a.order.by_heads), h = bh - b * a.H;
   const int M = a.M, N = a.N, p_seq = N - M;
   const int m0 = mt * BM;
   __shared__ float c_s[SCAN ? kOwnScanMaxKeys : 1];
@@ -478,7 +478,7 @@ __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's o
   if (a.first_block && tid == 0 && sp == 0) a.first_block[(int64_t)bh * a.n_mtiles + mt] = lo / BN;
   int n_tiles = (hi - lo + BN - 1) / BN;  // walked from the last (diagonal) tile down to lo
   if constexpr (SPLIT) {  // this workgroup's contiguous share of the key tiles
-    const int per = (n_tiles + a.splits - 1) / a.splits;
+    const int per = divide(n_tiles + a.splits - 1, a.by_splits);
     const int t0 = min(n_tiles, sp * per), t1 = min(n_tiles, t0 + per);
     lo += t0 * BN;
     n_tiles = t1 - t0;

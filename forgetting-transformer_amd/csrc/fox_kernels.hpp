@@ -32,6 +32,29 @@ struct GateK {
 enum : int { kGateLog = -1 };            // else 0 bf16, 1 fp16, 2 fp32 logits
 constexpr int kOwnScanMaxKeys = 3584;    // what fits beside the tiles in LDS at every head dim and occupancy
 
+// Division by a number that is fixed for a launch, n / d = n * mul >> shift, exact for 0 <= n < 2^31: mul is 2^shift / d rounded up, by less than
+// one, so the quotient is too large by less than n / 2^shift <= 1 / d.  (A division of scalars is some twenty dependent instructions.)
+struct Divisor {
+  uint32_t mul;
+  int32_t shift;
+};
+constexpr Divisor divisor(int32_t d) {
+  int32_t shift = 31;
+  while (((int64_t)1 << (shift - 31)) < d) ++shift;
+  return {(uint32_t)((((uint64_t)1 << shift) + d - 1) / d), shift};
+}
+__host__ __device__ __forceinline__ int divide(int n, Divisor d) { return (int)(((uint64_t)(uint32_t)n * d.mul) >> d.shift); }
+
+// Launch order of the attention kernels, made by block_order(), read by decode_block().
+struct BlockOrder {
+  int32_t tiles;              // of a (batch, head) pair
+  int32_t nb;                 // pairs per XCD, or of the launch where 8 does not divide them
+  int32_t size, extra;        // groups of pairs: the first `extra` hold size + 1, the others size
+  Divisor by_size[2], by_group[2];   // by the pairs and by the workgroups of a group; [1]: of a larger one
+  Divisor by_heads;           // pair -> batch
+  int32_t by_xcd, fold;
+};
+
 struct FwdK {
   View q, k, v, o;
   const float* c;
@@ -42,9 +65,9 @@ struct FwdK {
   int B, H, M, N;
   float sm_scale;
   int n_mtiles;
-  int groups;      // (batch, head) groups of the launch order (order_groups)
-  bool even;       // the tiles weigh about the same (even_tiles)
   int splits;      // key splits of the forward (1 = none)
+  BlockOrder order;
+  Divisor by_splits;
   bool pair;       // two groups of waves share every query tile's walk (fwd_pairs)
   float* ws_o;     // (splits, B, H, M, D) partial accumulators
   float* ws_ml;    // (splits, B, H, M, 2) partial row maximum and row sum
@@ -67,6 +90,7 @@ struct DecodeK {
   int B, H, N;
   float sm_scale;
   int splits;
+  Divisor by_splits, by_heads;
   float* ws_o;               // (B, H, splits, D) partial accumulators
   DecodePartial* ws_p;       // (B, H, splits)
   uint32_t* arrived;         // null, or (B, H) zeros: the split that arrives last merges them and leaves a zero
@@ -96,8 +120,7 @@ struct BwdK {
   int B, H, M, N;
   float sm_scale;
   int n_tiles;
-  int groups;      // (batch, head) groups of the launch order (order_groups), set by the launchers
-  bool even;       // the tiles weigh about the same (even_tiles), set by the launchers
+  BlockOrder order;   // set by the launchers
   int cls;         // kClassAll, or the class of key tiles this dK/dV launch handles (fox_common.hpp)
   int light_limit; // distance from the diagonal, in keys, that separates the two classes
   int32_t* q_first_block;  // optional (B,H,ceil(M/kFwdBM)): first key block (of kFwdBN keys) each query tile of the dQ kernel visits
@@ -143,6 +166,7 @@ struct NormGateK {
 };
 
 // Tile sizes (see fox_tile_config in the public header)
+constexpr int kXcds = 8, kCus = 256;
 constexpr int kFwdBM = 128;
 constexpr int kFwdBN = 64;
 constexpr int kKvBN = 128;   // key rows per workgroup in the dK/dV kernel
@@ -179,6 +203,52 @@ constexpr int order_groups(int n_bh, int tiles, int M, int N, int D, int64_t row
   if (even_tiles(M, N)) per = 1;
   const int64_t groups = nb / (by_xcd ? per : per * 8);
   return groups < 1 ? 1 : (int)groups;
+}
+// The divisions of decode_block and their operands.  `fold` asks for the folded order, which a grid gets that is resident at once.
+constexpr BlockOrder block_order(int B, int H, int tiles, int groups, bool fold) {
+  BlockOrder o{};
+  const int n_bh = B * H;
+  o.tiles = tiles;
+  o.by_xcd = n_bh % kXcds == 0;
+  o.nb = o.by_xcd ? n_bh / kXcds : n_bh;
+  o.size = o.nb / groups;
+  o.extra = o.nb % groups;
+  for (int i = 0; i < 2; ++i) {
+    o.by_size[i] = divisor(o.size + i);
+    o.by_group[i] = divisor((o.size + i) * tiles);
+  }
+  o.by_heads = divisor(H);
+  o.fold = fold && (int64_t)tiles * o.nb <= 2 * (o.by_xcd ? kCus / kXcds : kCus);
+  return o;
+}
+
+// Workgroup id -> (bh, tile).  Every tile of one (batch, head) goes to one XCD when the count allows it (the hardware
+// deals consecutive workgroup ids round-robin over the 8 XCDs, each with its own L2).  Within an XCD the (batch, head)
+// pairs are taken in groups of nearly equal size, and inside a group the tiles come heaviest first (largest index
+// under a causal mask) with the pairs of the group in turn.  One pair after the other would start the last pair's
+// heaviest tile when the chip is about to run empty; all pairs at once would stream more K and V than an L2 holds.
+// order_groups() picks the number of groups, block_order() makes the operands.
+// Folded: when the whole grid is resident at two workgroups per CU, the second workgroup of a CU is the one that arrives
+// kCus ids after the first.  Taken in the same order both would be heavy on one CU and both light on another; from
+// workgroup kCus on the list is therefore walked from its light end (forward B1 H16 T4096 D128: 109 -> 84 us, dQ 152 -> 116 us).
+// `last_first`: the pairs from the last to the first.  The dQ kernel takes them so, between a forward and a dK/dV kernel that start with the
+// first: each of the three then opens on the tensors its predecessor touched last, which are still in the 256 MiB last-level cache.
+// Backward with dQ ascending / descending: B4 T16384 H16 D128 "auto" 731 / 710 us, B16 H16 T4096 D64 "auto" 516 / 491,
+// B4 H32 T4096 D64 at -10 240 / 229, without a threshold 963 / 953.
+// What is divided by is the same for a whole launch: six divisions by Divisor instead of the compiler's take some 130 instructions off the front of a
+// kernel, which is what a workgroup of a pruned walk and one that finds nothing to do notice (figures: PENDING).
+__host__ __device__ __forceinline__ void decode_block(uint32_t wid, const BlockOrder& o, bool last_first, int& bh, int& tile) {
+  int r = (int)(o.by_xcd ? wid / kXcds : wid);
+  const int cus = o.by_xcd ? kCus / kXcds : kCus;
+  if (o.fold && r >= cus) r = o.tiles * o.nb - 1 - (r - cus);
+  const int big_pairs = o.extra * (o.size + 1);
+  const int big = r < big_pairs * o.tiles, size = o.size + big;
+  const Divisor by_group = big ? o.by_group[1] : o.by_group[0], by_size = big ? o.by_size[1] : o.by_size[0];
+  const int q = big ? r : r - big_pairs * o.tiles, grp = divide(q, by_group), in = q - grp * size * o.tiles, t = divide(in, by_size);
+  int b = (big ? 0 : big_pairs) + grp * size + in - t * size;
+  tile = o.tiles - 1 - t;
+  if (last_first) b = o.nb - 1 - b;
+  bh = o.by_xcd ? b * kXcds + (int)(wid % kXcds) : b;
 }
 
 hipError_t launch_fwd(const FwdK& a, int D, int dtype, hipStream_t s);

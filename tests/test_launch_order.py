@@ -1,0 +1,61 @@
+"""The launch order of the attention kernels: what decode_block gives with the operands block_order prepares, against plain divisions."""
+import pathlib
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = pathlib.Path(__file__).resolve().parents[1]
+
+PROGRAM = r"""
+#include "fox_kernels.hpp"
+#include <cstdio>
+using namespace fox;
+int main() {
+  const int dividends[] = {0, 1, 2, 127, 128, 65535, 1 << 24, (1 << 25) - 1, 1 << 30, 2147483646, 2147483647};
+  for (int d : {1, 2, 3, 5, 7, 12, 60, 127, 128, 129, 641, 65535, 65537, (1 << 25) - 1, 1 << 30, (1 << 30) + 1, 2147483647})
+    for (int n : dividends)
+      for (int near = -1; near <= 1; ++near) {   // also on either side of a multiple of d
+        const int64_t x = near ? (int64_t)(n / d) * d + near : n;
+        if (x >= 0 && x <= 2147483647 && divide((int)x, divisor(d)) != (int)x / d) return std::printf("%lld / %d\n", (long long)x, d), 1;
+      }
+  // pairs that 8 divides or not, one group, several of one or two sizes, one pair a group, resident grids or not
+  const int shapes[][4] = {{1, 12, 1, 1}, {1, 12, 4, 1}, {3, 5, 7, 1}, {4, 16, 128, 4}, {4, 15, 64, 60}, {5, 16, 33, 3}, {7, 9, 10, 5}, {1, 1, 4096, 1}, {2, 16, 16, 2}, {8, 64, 3, 64}, {4, 12, 8, 1}};
+  for (auto& s : shapes)
+    for (int v = 0; v < 4; ++v) {
+      const int B = s[0], H = s[1], tiles = s[2], groups = s[3], n_bh = B * H;
+      const bool fold = v & 1, last_first = v & 2, by_xcd = n_bh % 8 == 0;
+      const int nb = by_xcd ? n_bh / 8 : n_bh, cus = by_xcd ? 32 : 256, total = nb * tiles;
+      const BlockOrder o = block_order(B, H, tiles, groups, fold);
+      for (int xcd = 0; xcd < (by_xcd ? 8 : 1); ++xcd) {
+        int place = 0;
+        for (int first = 0, g = 0; g < groups; ++g) {   // the order in words: group by group, heaviest tile first, the pairs of the group in turn
+          const int size = nb / groups + (g < nb % groups);
+          for (int tile = tiles - 1; tile >= 0; --tile)
+            for (int pair = first; pair < first + size; ++pair, ++place) {
+              const int r = fold && total <= 2 * cus && place >= cus ? total - 1 - (place - cus) : place;   // (folding is its own inverse)
+              int bh, t;
+              decode_block(by_xcd ? r * 8 + xcd : r, o, last_first, bh, t);
+              const int want = last_first ? nb - 1 - pair : pair;
+              if (t != tile || bh != (by_xcd ? want * 8 + xcd : want) || divide(bh, o.by_heads) != bh / H)
+                return std::printf("B%d H%d tiles %d groups %d variant %d place %d\n", B, H, tiles, groups, v, r), 1;
+            }
+          first += size;
+        }
+        if (place != total) return 1;
+      }
+    }
+}
+"""
+
+
+def test_launch_order_without_divisions(tmp_path):
+    hipcc = shutil.which("hipcc") or shutil.which("/opt/rocm/bin/hipcc")
+    if hipcc is None:
+        pytest.skip("no hipcc")
+    src, exe = tmp_path / "order.hip", tmp_path / "order"
+    src.write_text(PROGRAM)
+    csrc = ROOT / "forgetting-transformer_amd" / "csrc"
+    subprocess.run([hipcc, "-std=c++17", "-O1", "--offload-arch=gfx950", "-Wno-unused-command-line-argument", f"-I{csrc}", str(src), "-o", str(exe)], check=True)
+    done = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert done.returncode == 0, done.stdout
