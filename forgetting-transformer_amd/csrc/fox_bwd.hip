@@ -227,7 +227,14 @@ __device__ __forceinline__ void dkdv_step_interior(const char* q_tile, const cha
 //
 // OWN_DELTA: the body forms delta = sum_d o_id * do_id for the rows of a step itself instead of reading what the dQ kernel left, so
 // that it can run beside it (dq_kernel with BOTH).  A wave takes the rows whose dO it has brought into LDS: its own wait is enough to read
-// them, and the barrier that publishes the step's tiles publishes their delta as well.
+// them, and the barrier that publishes the step's tiles publishes their delta as well.  The sum is the dQ walk's, bit for bit: the gradient of the
+// gates is the difference of the row sums of dS there and the column sums here, and is only as good as the two see one delta.
+
+// Two elements' part of delta.  (One expression for both walks, with the rounding spelled out.)
+template <typename Tr>
+__device__ __forceinline__ float delta_term(uint32_t o, uint32_t d_o) {
+  return __builtin_fmaf(Tr::lo(o), Tr::lo(d_o), Tr::hi(o) * Tr::hi(d_o));
+}
 template <int D, bool DSPLIT>
 struct DkdvLds {
   static constexpr int BMQ = DSPLIT ? 64 : kKvBM;
@@ -278,32 +285,40 @@ __device__ __forceinline__ void dkdv_body(const BwdK& a, int bh, int nt, const D
   // Everything the workgroup needs first is requested before anything is waited for: the tile of the
   // first diagonal step (it does not depend on the pruning bound), K and V, then the per-row terms.
   const DirectTileLoader<D, BMQ> qld(a.q.st, wave, lane), dold(a.d_o.st, wave, lane);
-  // The wave's own rows of a step: its j-th load brings one 1 KiB block of the tile into LDS, 16 bytes per lane in lane order, and o is
-  // fetched in the same order, so that the CH lanes of a row hold matching pieces of o and dO (whole rows: operand-shaped loads move a
-  // quarter of the bytes per clock).
+  // The wave's own rows of a step: its j-th load brings one 1 KiB block of the tile, the rows of which the CH lanes of a row read back chunk by
+  // chunk; o is fetched in the same shape (whole rows: operand-shaped loads move a quarter of the bytes per clock).
   constexpr int CH = D / 8, OPER = OWN_DELTA ? DirectTileLoader<D, BMQ>::PER : 0, ORPB = Tile<D>::RPB;
   static_assert(!OWN_DELTA || DirectTileLoader<D, BMQ>::NBLK % 4 == 0, "every wave has whole blocks of the step");
-  const DirectTileLoader<D, BMQ> old(a.o.st, wave, lane);
+  static_assert(!OWN_DELTA || CH <= 16, "the lanes of a row lie in one DPP row");
+  const int o_row = wave * ORPB + lane / CH, o_ch = lane % CH;   // of block 0; the j-th block is 4 * ORPB rows further down each
   u32x4 o_raw[OPER > 0 ? OPER : 1];
   auto issue_o = [&](int ms) {
     if constexpr (OWN_DELTA) {
       const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<uint16_t*>(op + (int64_t)ms * a.o.st), 0, old.extent(a.o.st, ms, M), 0x00020000);
+          const_cast<uint16_t*>(op + (int64_t)ms * a.o.st), 0, dold.extent(a.o.st, ms, M), 0x00020000);
 #pragma unroll
-      for (int j = 0; j < OPER; ++j) o_raw[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, old.voff[j], 0, 0));
+      for (int j = 0; j < OPER; ++j)
+        o_raw[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)((o_row + 4 * ORPB * j) * a.o.st * 2) + 16 * o_ch, 0, 0));
     }
   };
-  auto store_own_delta = [&](const char* dot, float* dl) {   // after the wave's own loads have landed; rows past M are zeros
+  // After the wave's own loads have landed; rows past M are zeros.  The bits of delta are those of the dQ walk: its two halves of the wave add the
+  // terms of the even and of the odd chunks of a row one after the other, and the halves are added last.  Here a chunk is a lane, so the running sum
+  // goes from lane to lane, two lanes further with every chunk; the last two lanes of the row end up with the two halves.
+  auto store_own_delta = [&](const char* dot, float* dl) {
     if constexpr (OWN_DELTA) {
-      const int line = lane >> 4, row0 = (line * 16 + ((lane & 15) ^ (line << 2))) / CH;
 #pragma unroll
       for (int j = 0; j < OPER; ++j) {
-        const u32x4 x = *reinterpret_cast<const u32x4*>(dot + (wave + 4 * j) * Tile<D>::BLOCK_BYTES + 16 * lane);
+        const int row = o_row + 4 * ORPB * j;
+        const u32x4 x = lds_row_operand<D>(dot, row, o_ch);
         float part = 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) part += Tr::lo(o_raw[j][e]) * Tr::lo(x[e]) + Tr::hi(o_raw[j][e]) * Tr::hi(x[e]);
-        part = row_sum<CH>(part);
-        if (lane % CH == 0) dl[(wave + 4 * j) * ORPB + row0] = -part;
+        for (int kk = 0; kk < KK; ++kk) {
+          if (kk > 0) part = dpp_take<0x112>(part);   // row_shr 2
+#pragma unroll
+          for (int e = 0; e < 4; ++e) part += delta_term<Tr>(o_raw[j][e], x[e]);
+        }
+        part = row_sum<2>(part);
+        if (o_ch == CH - 1) dl[row] = -part;
       }
     }
   };
@@ -733,8 +748,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK args) {
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        part += Tr::lo(oreg[kk][e]) * Tr::lo(doreg[kk][e]) + Tr::hi(oreg[kk][e]) * Tr::hi(doreg[kk][e]);
+      for (int e = 0; e < 4; ++e) part += delta_term<Tr>(oreg[kk][e], doreg[kk][e]);
     delta = half_sum(part);
     if (m < M && g == 0) a.delta[(int64_t)bh * M + m] = delta;
   }

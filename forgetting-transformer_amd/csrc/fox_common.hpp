@@ -341,12 +341,13 @@ __device__ __forceinline__ double of_lane(double x, int lane) {   // lane: wave-
   return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
 }
 
-// x + (x of the lane selected by a DPP control), as one v_add_f32 with a DPP operand
+// x of the lane selected by a DPP control (zero where there is none); with an addition one v_add_f32 with a DPP operand
 template <int CTRL>
-__device__ __forceinline__ float dpp_add(float x) {
-  const int y = __builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true);
-  return x + __int_as_float(y);
+__device__ __forceinline__ float dpp_take(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
 }
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) { return x + dpp_take<CTRL>(x); }
 
 // Sum over the LPR (2, 4, 8 or 16) consecutive lanes that hold one key row; every lane gets the total.
 template <int LPR>
