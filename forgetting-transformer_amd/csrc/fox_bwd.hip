@@ -517,7 +517,7 @@ __device__ __forceinline__ void dkdv_body(const BwdK& a, int bh, int nt, const D
   // gradient w.r.t. the cumulative sum: the row sum the dQ kernel left for the query row that sits at this key
   // position (none left of the first query row) minus this key's column sum
   if (n < N && g == 0 && dh == 0) {  // (the two waves of a split pair hold the same column sums)
-    float rtot = 0.f;   // (beside the dQ kernel: the reverse scan adds it)
+    float rtot = 0.f;   // (beside the dQ walk: the reverse scan adds it)
     if constexpr (!OWN_DELTA) {
       if (n >= p_seq) rtot = DSPLIT ? drow_key : a.drow[(int64_t)bh * M + (n - p_seq)];
     }
@@ -789,7 +789,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK args) {
   }
 
   const float rtot = half_sum(rsum);
-  if (m < M && g == 0) a.drow[(int64_t)bh * M + m] = rtot;  // the dK/dV kernel, next on this stream, folds it into dc
+  if (m < M && g == 0) a.drow[(int64_t)bh * M + m] = rtot;  // for dc: the dK/dV kernel, next on this stream, adds it, or with BOTH the reverse scan
   // dQ leaves through LDS (the tile buffers are free now, one per wave) so that the global stores are whole rows
   static_assert(kStoreStageBytes<D> <= Tile<D>::bytes(BN), "one wave stages in one tile buffer");
   __syncthreads();  // every wave is done with the last tile

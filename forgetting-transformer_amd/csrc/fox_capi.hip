@@ -337,7 +337,7 @@ int check_epilogue(const fox_fwd_args* args, const fox_fwd_epilogue* epi) {
 }
 
 // dq, dk, dv and dlog_lambda, by the two stages one after the other or side by side in one launch.  In the latter case dlog_lambda
-// lacks the row sums of dS: *drow is where they are, for the scan that follows (null otherwise).
+// lacks the row sums of dS: *drow is where they are, for the scan that follows, which adds them (null otherwise).
 int bwd_products(const fox_bwd_args* args, void* stream, const float** drow) {
   fox::BwdK k;
   FOX_TRY(make_bwd(args, k, true));
@@ -467,7 +467,7 @@ int fox_gate_cumsum_bwd(const float* dc, const void* logits, int32_t logits_dtyp
   if (B <= 0 || H <= 0 || N <= 0) return fail(FOX_E_ARG, "B, H, N must be positive");
   if (logits_dtype < FOX_DTYPE_BF16 || logits_dtype > FOX_DTYPE_FP32) return fail(FOX_E_ARG, "logits_dtype must be FOX_DTYPE_BF16, FP16 or FP32 (got %d)", logits_dtype);
   if ((const void*)dc == dlogits || logits == dlogits) return fail(FOX_E_ARG, "dlogits must not alias dc or logits");
-  return check_hip(fox::launch_gate_cumsum_bwd(dc, logits, logits_dtype, sb, sh, sn, seq_start, dlogits, db, dh, dn, B, H, N,
+  return check_hip(fox::launch_gate_cumsum_bwd(const_cast<float*>(dc), logits, logits_dtype, sb, sh, sn, seq_start, dlogits, db, dh, dn, B, H, N,
                                                nullptr, N, (hipStream_t)stream),
                    "fox_gate_cumsum_bwd");
 }
@@ -478,7 +478,7 @@ int fox_cumsum_bwd(const float* dc, float* dg, int64_t dg_sb, int64_t dg_sh, int
   if (B <= 0 || H <= 0 || N <= 0) return fail(FOX_E_ARG, "B, H, N must be positive");
   if (dc == dg) return fail(FOX_E_ARG, "dc and dg must not alias");
   if (dg_sb == 0 && dg_sh == 0 && dg_sn == 0) { dg_sb = (int64_t)H * N; dg_sh = N; dg_sn = 1; }   // contiguous (B,H,N)
-  return check_hip(fox::launch_cumsum_bwd(dc, dg, dg_sb, dg_sh, dg_sn, seq_start, B, H, N, nullptr, N, (hipStream_t)stream), "fox_cumsum_bwd");
+  return check_hip(fox::launch_cumsum_bwd(const_cast<float*>(dc), dg, dg_sb, dg_sh, dg_sn, seq_start, B, H, N, nullptr, N, (hipStream_t)stream), "fox_cumsum_bwd");
 }
 
 int fox_auto_threshold(const fox_dims* dims, const fox_view* q, const fox_view* k, float sm_scale, float* thr,

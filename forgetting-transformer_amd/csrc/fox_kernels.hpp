@@ -275,10 +275,11 @@ hipError_t launch_cumsum_fwd(const float* g, int64_t sb, int64_t sh, int64_t sn,
                              int H, int N, hipStream_t s);
 hipError_t launch_gate_cumsum_fwd(const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn, const int64_t* seq_start,
                                   float* log_fgate, float* c, int B, int H, int N, hipStream_t s);
-hipError_t launch_gate_cumsum_bwd(const float* dc, const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn,
+// drow: null (dc is only read), or (B,H,M) added to the last M of dc, in memory as well
+hipError_t launch_gate_cumsum_bwd(float* dc, const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn,
                                   const int64_t* seq_start, void* dlogits, int64_t db, int64_t dh, int64_t dn, int B, int H, int N,
-                                  const float* drow, int M, hipStream_t s);   // drow: null, or (B,H,M) added to the last M of dc
-hipError_t launch_cumsum_bwd(const float* dc, float* dg, int64_t db, int64_t dh, int64_t dn, const int64_t* seq_start, int B, int H,
+                                  const float* drow, int M, hipStream_t s);
+hipError_t launch_cumsum_bwd(float* dc, float* dg, int64_t db, int64_t dh, int64_t dn, const int64_t* seq_start, int B, int H,
                              int N, const float* drow, int M, hipStream_t s);
 hipError_t launch_mfma_probe(const void* operands, float* sink, int workgroups, int iters, hipStream_t s);  // fox_probe.hip
 hipError_t launch_qk_norm_threshold(const float* wq, const float* wk, int H, int D, double seq_len, double tolerance, float* thr, hipStream_t s);

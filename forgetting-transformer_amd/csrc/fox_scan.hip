@@ -23,8 +23,12 @@ namespace fox {
 // Rows of 77 to 2048 elements: 5.1 us a call with 1024 threads, 3.9 with as many as the row needs.  Rows cut over several
 // workgroups, each adding up what lies in front of its piece, were slower wherever there were enough of them to count (64 rows of 16384 8.5 -> 10.4
 // us, 256 rows of 32768 17 -> 28 us).
-template <bool REVERSE, int NT, typename Load, typename Store>
-__device__ __forceinline__ void scan_row(int N, Load load, Store store) {
+// keep(idx, x): what load() gave, once it is there.
+struct KeepNone {
+  __device__ __forceinline__ void operator()(int, float) const {}
+};
+template <bool REVERSE, int NT, typename Load, typename Store, typename Keep = KeepNone>
+__device__ __forceinline__ void scan_row(int N, Load load, Store store, Keep keep = {}) {
   constexpr int PER = 8, SPAN = PER * NT, WAVES = NT / kWave;
   __shared__ double wave_tot[WAVES];
   __shared__ __align__(16) float stage[SPAN];
@@ -42,7 +46,11 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store) {
   fetch(0, x);
   for (int base = 0; base < N; base += SPAN) {
 #pragma unroll
-    for (int e = 0; e < PER; ++e) stage[e * NT + tid] = x[e];
+    for (int e = 0; e < PER; ++e) {
+      stage[e * NT + tid] = x[e];
+      const int pos = base + e * NT + tid;
+      if (pos < N) keep(REVERSE ? N - 1 - pos : pos, x[e]);
+    }
     if (base + SPAN < N) fetch(base + SPAN, x_next);   // in flight while this span is scanned
     __syncthreads();
     const f32x4 lo4 = *reinterpret_cast<const f32x4*>(stage + tid * PER), hi4 = *reinterpret_cast<const f32x4*>(stage + tid * PER + 4);
@@ -105,7 +113,8 @@ inline unsigned scan_blocks(int rows) { return (unsigned)((rows + kXcds - 1) / k
 inline int scan_threads(int N) { return N <= 8 * 64 ? 64 : N <= 8 * 256 ? 256 : 1024; }
 
 // Gradient of the cumulative sum at position idx of a row: minus its column sum of dS and, where the backward ran in one launch
-// (drow not null: M row sums, of the last M positions), plus its row sum.  (Every load is issued: none behind a branch of its own.)
+// (drow not null: M row sums, of the last M positions), plus its row sum; in that case the sum also goes back into dc, which then holds
+// what the dK/dV kernel leaves there on its own.  (Every load is issued: none behind a branch of its own.)
 __device__ __forceinline__ float load_dc(const float* dc_row, const float* drow_row, int p_seq, int idx) {
   if (!drow_row) return dc_row[idx];
   const float x = dc_row[idx], r = drow_row[max(idx - p_seq, 0)];
@@ -113,14 +122,16 @@ __device__ __forceinline__ float load_dc(const float* dc_row, const float* drow_
 }
 
 template <bool REVERSE, int NT>
-__global__ __launch_bounds__(NT) void scan_kernel(const float* __restrict__ in, int64_t sb, int64_t sh, int64_t sn,
+__global__ __launch_bounds__(NT) void scan_kernel(const float* in, int64_t sb, int64_t sh, int64_t sn,
                                                    const int64_t* __restrict__ seq_start, float* __restrict__ out, int64_t ob,
-                                                   int64_t oh, int64_t on, int rows, int H, int N, const float* __restrict__ drow, int M) {
+                                                   int64_t oh, int64_t on, int rows, int H, int N, const float* __restrict__ drow, int M,
+                                                   float* dc) {
   const int bh = REVERSE ? scan_row_of_block(rows, on != 1) : blockIdx.x, b = bh / H, h = bh % H;
   if (REVERSE && bh >= rows) return;
   const float* src = in + b * sb + h * sh;
   float* dst = out + b * ob + h * oh;
   const float* dr = REVERSE && drow ? drow + (int64_t)bh * M : nullptr;
+  float* dc_row = dr ? dc + (int64_t)bh * N : nullptr;
   int seq = 0;
   if (seq_start) {
     const int64_t s64 = seq_start[b];
@@ -131,7 +142,8 @@ __global__ __launch_bounds__(NT) void scan_kernel(const float* __restrict__ in, 
   // forward); it is stored as an exact zero instead of the rounding noise of that sum.
   scan_row<REVERSE, NT>(
       N, [&](int idx) { return REVERSE ? load_dc(src, dr, N - M, idx) : idx >= seq ? src[(int64_t)idx * sn] : 0.f; },
-      [&](int idx, float sum) { dst[(int64_t)idx * on] = (REVERSE && idx <= seq) ? 0.f : sum; });
+      [&](int idx, float sum) { dst[(int64_t)idx * on] = (REVERSE && idx <= seq) ? 0.f : sum; },
+      [&](int idx, float x) { if (REVERSE && dc_row) dc_row[idx] = x; });
 }
 
 template <int DT>
@@ -171,13 +183,13 @@ __global__ __launch_bounds__(NT) void gate_scan_fwd_kernel(const void* __restric
 // dlogit[l] = (sum_{n>=l} dc[n]) * d logsigmoid(x_l)/dx = dg[l] * (1 - sigmoid(x_l)), stored in the
 // dtype and layout of the logits.
 template <int DT, int NT>
-__global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(const float* __restrict__ dc, const void* __restrict__ logits,
+__global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(float* dc, const void* __restrict__ logits,
                                                             int64_t sb, int64_t sh, int64_t sn, const int64_t* __restrict__ seq_start,
                                                             void* __restrict__ dlogits, int64_t db, int64_t dh, int64_t dn,
                                                             int rows, int H, int N, const float* __restrict__ drow, int M) {
   const int bh = scan_row_of_block(rows, dn != 1), b = bh / H, h = bh % H;
   if (bh >= rows) return;
-  const float* src = dc + (int64_t)bh * N;
+  float* src = dc + (int64_t)bh * N;
   const float* dr = drow ? drow + (int64_t)bh * M : nullptr;
   const int64_t lbase = b * sb + h * sh, dbase = b * db + h * dh;
   int seq = 0;
@@ -193,7 +205,8 @@ __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(const float* __restri
         const float r = __fdividef(z, 1.f + z);              // sigmoid(-|x|)
         // positions up to and including seq: an exact zero, as in scan_kernel<true>
         store_logit<DT>(dlogits, dbase + (int64_t)idx * dn, idx <= seq ? 0.f : sum * (x < 0.f ? 1.f - r : r));
-      });
+      },
+      [&](int idx, float x) { if (dr) src[idx] = x; });
 }
 
 // KERNEL<ARG, threads for rows of N elements>, BLOCKS workgroups, one per row of the B x H.
@@ -215,7 +228,7 @@ hipError_t launch_gate_cumsum_fwd(const void* logits, int dtype, int64_t sb, int
   return hipGetLastError();
 }
 
-hipError_t launch_gate_cumsum_bwd(const float* dc, const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn,
+hipError_t launch_gate_cumsum_bwd(float* dc, const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn,
                                   const int64_t* seq_start, void* dlogits, int64_t db, int64_t dh, int64_t dn, int B, int H, int N,
                                   const float* drow, int M, hipStream_t s) {
   switch (dtype) {
@@ -230,14 +243,14 @@ hipError_t launch_gate_cumsum_bwd(const float* dc, const void* logits, int dtype
 hipError_t launch_cumsum_fwd(const float* g, int64_t sb, int64_t sh, int64_t sn, const int64_t* seq_start, float* c, int B,
                              int H, int N, hipStream_t s) {
   FOX_LAUNCH_SCAN(scan_kernel, false, (unsigned)(B * H), g, sb, sh, sn, seq_start, c,
-                     (int64_t)H * N, (int64_t)N, (int64_t)1, B * H, H, N, nullptr, N)
+                     (int64_t)H * N, (int64_t)N, (int64_t)1, B * H, H, N, nullptr, N, nullptr)
   return hipGetLastError();
 }
 
-hipError_t launch_cumsum_bwd(const float* dc, float* dg, int64_t db, int64_t dh, int64_t dn, const int64_t* seq_start, int B, int H,
+hipError_t launch_cumsum_bwd(float* dc, float* dg, int64_t db, int64_t dh, int64_t dn, const int64_t* seq_start, int B, int H,
                              int N, const float* drow, int M, hipStream_t s) {
   FOX_LAUNCH_SCAN(scan_kernel, true, scan_blocks(B * H), dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
-                     seq_start, dg, db, dh, dn, B * H, H, N, drow, M)
+                     seq_start, dg, db, dh, dn, B * H, H, N, drow, M, dc)
   return hipGetLastError();
 }
 

@@ -238,7 +238,7 @@ typedef struct fox_bwd_args {
   float sm_scale;
   float* delta;               /* (B,H,M) workspace, written by the dQ stage: rowsum(o * do) */
   float* drow;                /* (B,H,M) workspace, written by the dQ stage, read by the dK/dV stage: row sums of dS */
-  float* dlog_lambda;         /* (B,H,N) workspace, written: gradient w.r.t. c (by fox_attn_bwd for small grids: without the row sums) */
+  float* dlog_lambda;         /* (B,H,N) workspace, written: gradient w.r.t. c */
   float* dlog_fgate;          /* (B,H,N) written: gradient w.r.t. log_fgate */
   int64_t dlog_fgate_stride_b, dlog_fgate_stride_h, dlog_fgate_stride_n;  /* its element strides; all 0 = contiguous */
   /* Optional outputs (NULL = not wanted): the pruning bounds the two kernels worked with, the counterparts of
@@ -259,8 +259,8 @@ typedef struct fox_bwd_args {
  *   fox_attn_bwd_dkdv  : dk, dv, dlog_lambda[n] = drow[n-(N-M)] - sum_i dS[i,n]; reads delta and drow
  *                        (_find_end_index_kernel :747-795 + _bwd_kv_kernel :956-1143)
  *   fox_cumsum_bwd     : dlog_fgate from dlog_lambda                (:390-392)
- * fox_attn_bwd runs all three (ForgettingAttention.backward :232-400); for small grids the first two as one launch, which leaves the row
- * sums to the scan: dlog_lambda then holds only -sum_i dS[i,n].  The reference launches the key/value
+ * fox_attn_bwd runs all three (ForgettingAttention.backward :232-400), for small grids the first two as one launch, after which the
+ * scan adds the row sums to dlog_lambda; every buffer ends up with the same bits either way.  The reference launches the key/value
  * kernel first and lets the query kernel add its row sums into the same buffer (:1334-1344); here every stage
  * only stores, so repeating a stage (or timing it alone) leaves the result unchanged, and only the order
  * dq before dkdv matters.  fox_attn_bwd_delta writes `delta` alone (_bwd_preprocess as a stage of its own; only

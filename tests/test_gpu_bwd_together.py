@@ -39,8 +39,8 @@ def _run(B, H, M, N, D, dtype, thr, seq, head_first):
             _lib.check(lib.fox_attn_bwd_dq(C.byref(args), stream), "dq")
             _lib.check(lib.fox_attn_bwd_dkdv(C.byref(args), stream), "dkdv")
             _lib.check(lib.fox_cumsum_bwd(tmp[2].data_ptr(), dg.data_ptr(), *dg.stride(), ptr(ss), B, H, N, stream), "scan")
-        res.append((dq, dk, dv, dg, tmp[0]))
-    for name, a, b in zip(("dq", "dk", "dv", "dlog_fgate", "delta"), *res):
+        res.append((dq, dk, dv, dg, *tmp))
+    for name, a, b in zip(("dq", "dk", "dv", "dlog_fgate", "delta", "drow", "dlog_lambda"), *res):
         assert torch.isfinite(b).all()
         assert torch.equal(a, b), name
     # (One or two query rows: a gradient is one or two products of three 16-bit roundings each, 3 * 2^-9 = 6e-3 and up to twice that of a scale that
