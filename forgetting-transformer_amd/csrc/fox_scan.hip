@@ -13,6 +13,27 @@
 
 namespace fox {
 
+// The gradient of a cumulative sum at one position is its row sum of dS minus its column sum.  Where the backward ran in one launch the dK/dV walk
+// could not wait for the row sums (drow, of the last M positions of the row): the reverse scan adds them, and stores the sum back into dc, which then
+// holds what the dK/dV kernel leaves there on its own.  The loads are a loop of their own under one branch: in a branch per element every one of them was
+// waited for before the next was sent (4 rows of 16384 positions 15.1 us, so 12.3; without row sums 9.9; 24 rows of 2048 6.0, 4.5 and 4.1).
+struct RowSums {
+  const float* drow;   // (M) or null
+  float* dc;
+  int p_seq;
+  __device__ __forceinline__ bool any() const { return drow != nullptr; }
+  __device__ __forceinline__ float load(int idx) const {
+    const float r = drow[max(idx - p_seq, 0)];
+    return idx >= p_seq ? r : 0.f;
+  }
+  __device__ __forceinline__ void keep(int idx, float x) const { dc[idx] = x; }
+};
+struct NoRows {
+  __device__ __forceinline__ constexpr bool any() const { return false; }
+  __device__ __forceinline__ float load(int) const { return 0.f; }
+  __device__ __forceinline__ void keep(int, float) const {}
+};
+
 // Scan of one row: element idx is produced by load(idx) and the running sum up to and including
 // it is handed to store(idx, sum).  REVERSE walks the row from its last element to its first.
 // A span of 8 x NT elements moves between memory and LDS with consecutive lanes on consecutive
@@ -23,35 +44,39 @@ namespace fox {
 // Rows of 77 to 2048 elements: 5.1 us a call with 1024 threads, 3.9 with as many as the row needs.  Rows cut over several
 // workgroups, each adding up what lies in front of its piece, were slower wherever there were enough of them to count (64 rows of 16384 8.5 -> 10.4
 // us, 256 rows of 32768 17 -> 28 us).
-// keep(idx, x): what load() gave, once it is there.
-struct KeepNone {
-  __device__ __forceinline__ void operator()(int, float) const {}
-};
-template <bool REVERSE, int NT, typename Load, typename Store, typename Keep = KeepNone>
-__device__ __forceinline__ void scan_row(int N, Load load, Store store, Keep keep = {}) {
+// rows: a second addend of the last M positions (RowSums), or nothing.
+template <bool REVERSE, int NT, typename Load, typename Store, typename Rows = NoRows>
+__device__ __forceinline__ void scan_row(int N, Load load, Store store, Rows rows = {}) {
   constexpr int PER = 8, SPAN = PER * NT, WAVES = NT / kWave;
   __shared__ double wave_tot[WAVES];
   __shared__ __align__(16) float stage[SPAN];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   double carry = 0.0;
-  float x[PER], x_next[PER];
-  auto fetch = [&](int base, float (&dst)[PER]) {  // element e of a thread sits at position base + e*NT + tid of the scan order
+  float x[PER], x_next[PER], r[PER] = {}, r_next[PER] = {};
+  auto fetch = [&](int base, float (&dst)[PER], float (&dst_r)[PER]) {  // element e of a thread sits at position base + e*NT + tid of the scan order
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
       const int pos = base + e * NT + tid;
       const int idx = REVERSE ? N - 1 - pos : pos;
       dst[e] = pos < N ? load(idx) : 0.f;
     }
+    if (rows.any()) {
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        const int pos = base + e * NT + tid, in = min(pos, N - 1);
+        const float y = rows.load(REVERSE ? N - 1 - in : in);
+        dst_r[e] = pos < N ? y : 0.f;
+      }
+    }
   };
-  fetch(0, x);
+  fetch(0, x, r);
   for (int base = 0; base < N; base += SPAN) {
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
+      if (rows.any()) x[e] += r[e];
       stage[e * NT + tid] = x[e];
-      const int pos = base + e * NT + tid;
-      if (pos < N) keep(REVERSE ? N - 1 - pos : pos, x[e]);
     }
-    if (base + SPAN < N) fetch(base + SPAN, x_next);   // in flight while this span is scanned
+    if (base + SPAN < N) fetch(base + SPAN, x_next, r_next);   // in flight while this span is scanned
     __syncthreads();
     const f32x4 lo4 = *reinterpret_cast<const f32x4*>(stage + tid * PER), hi4 = *reinterpret_cast<const f32x4*>(stage + tid * PER + 4);
     double v[PER];
@@ -94,8 +119,18 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store, Keep kee
       const int idx = REVERSE ? N - 1 - pos : pos;
       if (pos < N) store(idx, stage[e * NT + tid]);
     }
+    if (rows.any()) {
 #pragma unroll
-    for (int e = 0; e < PER; ++e) x[e] = x_next[e];
+      for (int e = 0; e < PER; ++e) {
+        const int pos = base + e * NT + tid;
+        if (pos < N) rows.keep(REVERSE ? N - 1 - pos : pos, x[e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      x[e] = x_next[e];
+      r[e] = r_next[e];
+    }
     __syncthreads();  // the span has left LDS before the next one is written
   }
 }
@@ -110,16 +145,13 @@ __device__ __forceinline__ int scan_row_of_block(int rows, bool neighbours) {
 }
 inline unsigned scan_blocks(int rows) { return (unsigned)((rows + kXcds - 1) / kXcds * kXcds); }
 
-inline int scan_threads(int N) { return N <= 8 * 64 ? 64 : N <= 8 * 256 ? 256 : 1024; }
-
-// Gradient of the cumulative sum at position idx of a row: minus its column sum of dS and, where the backward ran in one launch
-// (drow not null: M row sums, of the last M positions), plus its row sum; in that case the sum also goes back into dc, which then holds
-// what the dK/dV kernel leaves there on its own.  (Every load is issued: none behind a branch of its own.)
-__device__ __forceinline__ float load_dc(const float* dc_row, const float* drow_row, int p_seq, int idx) {
-  if (!drow_row) return dc_row[idx];
-  const float x = dc_row[idx], r = drow_row[max(idx - p_seq, 0)];
-  return idx >= p_seq ? x + r : x;
+template <bool REVERSE>
+__device__ __forceinline__ auto row_sums(const float* drow, float* dc, int bh, int M, int N) {   // of the row of pair bh
+  if constexpr (REVERSE) return RowSums{drow ? drow + (int64_t)bh * M : nullptr, dc + (int64_t)bh * N, N - M};
+  else return NoRows{};
 }
+
+inline int scan_threads(int N) { return N <= 8 * 64 ? 64 : N <= 8 * 256 ? 256 : 1024; }
 
 template <bool REVERSE, int NT>
 __global__ __launch_bounds__(NT) void scan_kernel(const float* in, int64_t sb, int64_t sh, int64_t sn,
@@ -130,8 +162,6 @@ __global__ __launch_bounds__(NT) void scan_kernel(const float* in, int64_t sb, i
   if (REVERSE && bh >= rows) return;
   const float* src = in + b * sb + h * sh;
   float* dst = out + b * ob + h * oh;
-  const float* dr = REVERSE && drow ? drow + (int64_t)bh * M : nullptr;
-  float* dc_row = dr ? dc + (int64_t)bh * N : nullptr;
   int seq = 0;
   if (seq_start) {
     const int64_t s64 = seq_start[b];
@@ -141,9 +171,9 @@ __global__ __launch_bounds__(NT) void scan_kernel(const float* in, int64_t sb, i
   // arithmetic (those gates shift every cumulative sum the kernels see by the same amount, or are zeroed by the
   // forward); it is stored as an exact zero instead of the rounding noise of that sum.
   scan_row<REVERSE, NT>(
-      N, [&](int idx) { return REVERSE ? load_dc(src, dr, N - M, idx) : idx >= seq ? src[(int64_t)idx * sn] : 0.f; },
+      N, [&](int idx) { return (REVERSE || idx >= seq) ? src[(int64_t)idx * sn] : 0.f; },
       [&](int idx, float sum) { dst[(int64_t)idx * on] = (REVERSE && idx <= seq) ? 0.f : sum; },
-      [&](int idx, float x) { if (REVERSE && dc_row) dc_row[idx] = x; });
+      row_sums<REVERSE>(drow, dc, bh, M, N));
 }
 
 template <int DT>
@@ -189,8 +219,7 @@ __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(float* dc, const void
                                                             int rows, int H, int N, const float* __restrict__ drow, int M) {
   const int bh = scan_row_of_block(rows, dn != 1), b = bh / H, h = bh % H;
   if (bh >= rows) return;
-  float* src = dc + (int64_t)bh * N;
-  const float* dr = drow ? drow + (int64_t)bh * M : nullptr;
+  const float* src = dc + (int64_t)bh * N;
   const int64_t lbase = b * sb + h * sh, dbase = b * db + h * dh;
   int seq = 0;
   if (seq_start) {
@@ -198,7 +227,7 @@ __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(float* dc, const void
     seq = (int)(s64 < 0 ? 0 : (s64 > N ? N : s64));
   }
   scan_row<true, NT>(
-      N, [&](int idx) { return load_dc(src, dr, N - M, idx); },
+      N, [&](int idx) { return src[idx]; },
       [&](int idx, float sum) {
         const float x = load_logit<DT>(logits, lbase + (int64_t)idx * sn);
         const float z = __expf(-fabsf(x));
@@ -206,7 +235,7 @@ __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(float* dc, const void
         // positions up to and including seq: an exact zero, as in scan_kernel<true>
         store_logit<DT>(dlogits, dbase + (int64_t)idx * dn, idx <= seq ? 0.f : sum * (x < 0.f ? 1.f - r : r));
       },
-      [&](int idx, float x) { if (dr) src[idx] = x; });
+      row_sums<true>(drow, dc, bh, M, N));
 }
 
 // KERNEL<ARG, threads for rows of N elements>, BLOCKS workgroups, one per row of the B x H.
