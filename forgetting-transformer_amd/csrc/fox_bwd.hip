@@ -634,17 +634,16 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK args) {
   if constexpr (BOTH) {
     __shared__ __align__(16) float row2[ROWS];
     __shared__ __align__(16) float row3[ROWS];
-    const int q_tiles = (args.M + BM - 1) / BM;
     int t;
     decode_block(blockIdx.x, args.order, false, bh, t);
-    if (!(t & 1)) {
+    const BothTile w = both_tile(t, args.n_tiles, (args.M + BM - 1) / BM);
+    if (!w.query) {
 #ifdef __HIP_DEVICE_COMPILE__
-      dkdv_body<Tr, D, false, true>(own_arguments(), bh, args.n_tiles - 1 - t / 2, {k_tile0, k_tile1, v_tile0, v_tile1, cn_s0, cn_s1, row2, row3});
+      dkdv_body<Tr, D, false, true>(own_arguments(), bh, w.tile, {k_tile0, k_tile1, v_tile0, v_tile1, cn_s0, cn_s1, row2, row3});
 #endif
       return;
     }
-    mt = t / 2 - (args.n_tiles - q_tiles);   // (fewer query tiles than key tiles where M < N)
-    if (mt < 0) return;
+    mt = w.tile;
   } else {
     decode_block(blockIdx.x, args.order, true, bh, mt);
   }
@@ -884,8 +883,12 @@ template <typename Tr>
 static hipError_t bwd_t(const BwdK& a0, int D, hipStream_t s) {
   BwdK a = a0;
   a.n_tiles = (a.N + kKvBN - 1) / kKvBN;
-  a.order = block_order(a.B, a.H, 2 * a.n_tiles, order_groups(a.B * a.H, a.n_tiles, a.M, a.N, D, a.k.st, a.thr != nullptr), !even_tiles(a.M, a.N));
-  const dim3 grid((unsigned)(2 * a.n_tiles * a.B * a.H));
+  const int q_tiles = (a.M + kFwdBM - 1) / kFwdBM, tiles = a.n_tiles + q_tiles;
+  // M < N: the query tiles of all pairs first.  Each has the longest walk there is, and with the pairs one after the other those of the next pair would
+  // join those of the one before on their CUs.
+  const int groups = q_tiles < a.n_tiles ? 1 : order_groups(a.B * a.H, a.n_tiles, a.M, a.N, D, a.k.st, a.thr != nullptr);
+  a.order = block_order(a.B, a.H, tiles, groups, !even_tiles(a.M, a.N));
+  const dim3 grid((unsigned)(tiles * a.B * a.H));
   switch (D) {
     case 16: hipLaunchKernelGGL((dq_kernel<Tr, 16, true>), grid, dim3(256), 0, s, a); break;
     case 32: hipLaunchKernelGGL((dq_kernel<Tr, 32, true>), grid, dim3(256), 0, s, a); break;

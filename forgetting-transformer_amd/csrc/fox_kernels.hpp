@@ -251,6 +251,19 @@ __host__ __device__ __forceinline__ void decode_block(uint32_t wid, const BlockO
   bh = o.by_xcd ? b * kXcds + (int)(wid % kXcds) : b;
 }
 
+// Tile t of a (batch, head) pair in the one-launch backward (dq_kernel with BOTH), which holds key_tiles + query_tiles of them (M <= N, so there are at
+// least as many of the former).  From the last to the first: query and key tiles in turn, heaviest first, then the key tiles left over.
+struct BothTile {
+  bool query;
+  int tile;
+};
+__host__ __device__ __forceinline__ BothTile both_tile(int t, int key_tiles, int query_tiles) {
+  const int rest = key_tiles - query_tiles, u = t - rest;
+  if (u >= 0 && (u & 1)) return {true, u >> 1};
+  const int rank = u < 0 ? t : rest + (u >> 1);   // of the key tile, from the one with the fewest rows to walk
+  return {false, key_tiles - 1 - rank};
+}
+
 hipError_t launch_fwd(const FwdK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_fwd_gates(const FwdK& a, int D, int dtype, hipStream_t s);   // unsplit, at most kOwnScanMaxKeys keys, M > 1
 bool fwd_scans(int B, int H, int M, int N, int splits);

@@ -45,6 +45,16 @@ int main() {
         if (place != total) return 1;
       }
     }
+  // one-launch backward: as many workgroups as there are tiles, each tile once, the heaviest of either kind first
+  for (int keys = 1; keys < 20; ++keys)
+    for (int queries = 1; queries <= keys; ++queries) {
+      int next_query = queries - 1, next_key = 0;
+      for (int t = keys + queries - 1; t >= 0; --t) {
+        const BothTile w = both_tile(t, keys, queries);
+        if (w.tile != (w.query ? next_query-- : next_key++)) return std::printf("%d key tiles, %d query tiles, place %d\n", keys, queries, t), 1;
+      }
+      if (next_query != -1 || next_key != keys) return 1;
+    }
 }
 """
 
