@@ -907,15 +907,24 @@ hipError_t launch_bwd_dkdv(const BwdK& a, int D, int dtype, hipStream_t s) {
   return dtype == 0 ? dkdv_t<Bf16>(a, D, s) : dkdv_t<Fp16>(a, D, s);
 }
 // Whether dQ and dK/dV go out as one launch (dq_kernel with BOTH).  One after the other, each waits for the longest walk of a grid that fills the chip
-// once or less; side by side the two waits are one, and so are two launches and the drain between them.  Backward, one after the other / together, us:
-// D 64 B1 H5 T3000 118 / 80, B2 H8 T2000 82 / 60, B4 H12 T512 31.9 / 27.8, B16 H16 T250 35.0 / 32.0, B2 H12 T2048 at -60 45.4 / 44.4; D 32 B3 H5 T777 34.6 / 29.3,
-// D 16 B4 H16 T1000 42.8 / 33.7.  Against it stand delta, formed anew for every step, and the LDS of the dK/dV walk, which the dQ walk does not
-// need: with more than 512 tiles of either kind at D 64 it goes either way (768: B12 H16 T500 51.2 / 50.3, B16 H24 T250 38.1 / 40.5; 2048: B8 H32 T1000
-// "auto" 87 / 99; 4096: B4 H32 T4096 980 / 1130).  Head dims up to 32 hold three workgroups per CU: 768 tiles B4 H24 T1000 at -10 35.1 / 32.7 and
-// 35.4 / 31.6, 2048 tiles B8 H16 T2048 D16 151 / 200.
+// once or less; side by side the two waits are one, and so are two launches and the drain between them.  Forward and backward, the latter one after the
+// other / together, us: D 64 B2 H12 T2048 117 / 98, B4 H12 T512 43.7 / 36.1, B16 H16 T250 42.2 / 41.6, B1 H16 M256 N4096 114 / 106; D 32 B3 H5 T777 49.7 / 38.1,
+// D 16 B16 H16 T250 34.2 / 29.3.  Against it stand delta, formed anew for every step, the row sums that the reverse scan has to add, and the LDS of the
+// dK/dV walk, which the dQ walk does not need.
+// - With more than 512 tiles of either kind at D 64 it goes either way (backward alone, 768: B12 H16 T500 51.2 / 50.3, B16 H24 T250 38.1 / 40.5; 2048: B8 H32
+//   T1000 "auto" 87 / 99; 4096: B4 H32 T4096 980 / 1130).  Head dims up to 32 hold three workgroups per CU: 768 tiles B3 H32 T1000 D32 at -10 57.3 / 52.3 and
+//   D16 54.9 / 48.5, 2048 tiles B8 H16 T2048 D16, backward alone, 151 / 200.
+// - Long rows.  The reverse scan of few long rows is a chain that the row sums make longer, and under a threshold walks are short and have little to overlap,
+//   so that the grid has to leave room: D 64 at -10, T4096 with 320 tiles 53.5 / 53.1, 384 55.2 / 56.1, 448 57.3 / 59.1, 512 55.6 / 59.2; T16384 with 256 59.2 / 57.4,
+//   384 60.8 / 65.4, 512 68.1 / 76.0; D 32 T16384 with 256 51.7 / 49.3, 512 61.3 / 64.8.  Rows up to 2048 (D 64) and 8192 are past that: B2 H12 T2048 48.5 / 47.7,
+//   D 32 B1 H12 T8192 68.0 / 66.8.  Without a threshold D 64 T4096 gains with 448 tiles, 221 / 195, not with 512, 226 / 230 (T16384 818 / 833); D 32 gains with 768, 805 / 747.
+//   Where M < N the tiles of both kinds count: B1 H16 M300 N4096 at -10 (560 of them) 52.4 / 47.7.
 bool bwd_together(const BwdK& a, int D) {
   if (D > 64 || a.o.st <= 0 || ((int64_t)kKvBM * a.o.st + D) * 2 >= (int64_t)1 << 31) return false;   // o through 32-bit offsets
-  return (int64_t)((a.N + kKvBN - 1) / kKvBN) * a.B * a.H <= (D == 64 ? 2 : 3) * kCus;
+  const int64_t pairs = (int64_t)a.B * a.H, keys = pairs * ((a.N + kKvBN - 1) / kKvBN), both = keys + pairs * ((a.M + kFwdBM - 1) / kFwdBM);
+  if (keys > (D == 64 ? 2 : 3) * kCus) return false;
+  if (a.N <= (D == 64 ? 2048 : 8192)) return true;
+  return a.thr ? 2 * both <= 5 * kCus : D < 64 || 2 * both <= 7 * kCus;
 }
 hipError_t launch_bwd(const BwdK& a, int D, int dtype, hipStream_t s) {
   return dtype == 0 ? bwd_t<Bf16>(a, D, s) : bwd_t<Fp16>(a, D, s);

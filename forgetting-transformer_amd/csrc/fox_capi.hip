@@ -363,8 +363,9 @@ int bwd_products(const fox_bwd_args* args, void* stream, const float** drow) {
 extern "C" {
 
 // 0.2.x: fox_bwd_args and the scan entry points differ from 0.1.0; 0.2.1 adds fox_set_stream_min_kv_bytes and fox_probe_mfma, 0.2.2
-// fox_attn_decode, fox_cache_append, fox_qk_norm_threshold and fox_attn_fwd_plan, 0.2.3 fox_attn_fwd_gates and fox_attn_fwd_takes_gates
-int fox_version(void) { return 203; }
+// fox_attn_decode, fox_cache_append, fox_qk_norm_threshold and fox_attn_fwd_plan, 0.2.3 fox_attn_fwd_gates, fox_attn_fwd_takes_gates,
+// fox_auto_threshold_scan, fox_attn_decode_counted and fox_attn_bwd_logits, 0.2.4 fox_attn_bwd_one_launch
+int fox_version(void) { return 204; }
 
 const char* fox_last_error(void) { return g_err; }
 
@@ -658,6 +659,14 @@ int fox_attn_bwd_dq(const fox_bwd_args* args, void* stream) {
   FOX_TRY(check_view(&args->dq, "dq"));
   k.dq = to_view(args->dq);
   return check_hip(fox::launch_bwd_dq(k, args->dims.D, args->dims.dtype, (hipStream_t)stream), "fox_attn_bwd_dq");
+}
+
+int fox_attn_bwd_one_launch(const fox_bwd_args* args, int32_t* yes) {
+  fox::BwdK k;
+  FOX_TRY(make_bwd(args, k, true));
+  if (!yes) return fail(FOX_E_ARG, "yes is NULL");
+  *yes = fox::bwd_together(k, args->dims.D);
+  return FOX_OK;
 }
 
 int fox_attn_bwd(const fox_bwd_args* args, void* stream) {

@@ -157,6 +157,7 @@ SIGNATURES = {
     "fox_attn_bwd_dkdv": (C.c_int, [C.POINTER(BwdArgs), C.c_void_p]),
     "fox_attn_bwd_dq": (C.c_int, [C.POINTER(BwdArgs), C.c_void_p]),
     "fox_attn_bwd": (C.c_int, [C.POINTER(BwdArgs), C.c_void_p]),
+    "fox_attn_bwd_one_launch": (C.c_int, [C.POINTER(BwdArgs), C.POINTER(C.c_int32)]),
     "fox_attn_bwd_logits": (C.c_int, [C.POINTER(BwdArgs), C.c_void_p, C.c_int32] + [C.c_int64] * 3 + [C.c_void_p] + [C.c_int64] * 3 +
                             [C.c_void_p]),
     "fox_norm_gate_fwd": (C.c_int, [C.POINTER(NormGateArgs), C.c_void_p]),

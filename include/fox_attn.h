@@ -270,6 +270,8 @@ int fox_attn_bwd_delta(const fox_bwd_args* args, void* stream);
 int fox_attn_bwd_dkdv(const fox_bwd_args* args, void* stream);
 int fox_attn_bwd_dq(const fox_bwd_args* args, void* stream);
 int fox_attn_bwd(const fox_bwd_args* args, void* stream);
+/* Whether fox_attn_bwd and fox_attn_bwd_logits run the first two stages of these arguments as one launch. */
+int fox_attn_bwd_one_launch(const fox_bwd_args* args, int32_t* yes);
 
 /*
  * fox_attn_bwd for a forward from the gate logits (fox_gate_cumsum_fwd): dlogits in place of dlog_fgate, with the dtype of the

@@ -40,6 +40,11 @@ class _Problem:
                               *(x.data_ptr() for x in tmp), _ptr(dg), *(dg.stride() if dg is not None else (0, 0, 0)), None, None)
         return a, grads, tmp
 
+    def one_launch(self, args):
+        yes = C.c_int32(-1)
+        self._lib.check(self.lib.fox_attn_bwd_one_launch(C.byref(args), C.byref(yes)), "fox_attn_bwd_one_launch")
+        return yes.value == 1
+
     def call(self, name, *args):
         self._lib.check(getattr(self.lib, name)(*args, self.stream), name)
 
@@ -55,6 +60,7 @@ def _run(B, H, M, N, D, dtype, thr, seq, head_first):
         dg = torch.full((B, H, N), float("nan"), device="cuda")
         args, grads, tmp = p.args(dg)
         if together:
+            assert p.one_launch(args)
             p.call("fox_attn_bwd", C.byref(args))
         else:
             p.call("fox_attn_bwd_dq", C.byref(args))
@@ -98,6 +104,7 @@ def test_strided_gate_gradients(B, H, M, N, seq, logit):
     for together in (False, True):
         dg = as_bth(torch.full((B, H, N), float("nan"), device="cuda", dtype=logit or torch.float32))
         args, _, tmp = p.args(dg if logit is None else None)
+        assert p.one_launch(args)
         if not together:
             p.call("fox_attn_bwd_dq", C.byref(args))
             p.call("fox_attn_bwd_dkdv", C.byref(args))

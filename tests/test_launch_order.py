@@ -1,4 +1,5 @@
 """The launch order of the attention kernels: what decode_block gives with the operands block_order prepares, against plain divisions."""
+import ctypes as C
 import pathlib
 import shutil
 import subprocess
@@ -69,3 +70,20 @@ def test_launch_order_without_divisions(tmp_path):
     subprocess.run([hipcc, "-std=c++17", "-O1", "--offload-arch=gfx950", "-Wno-unused-command-line-argument", f"-I{csrc}", str(src), "-o", str(exe)], check=True)
     done = subprocess.run([str(exe)], capture_output=True, text=True)
     assert done.returncode == 0, done.stdout
+
+
+@pytest.mark.parametrize("B,H,M,N,D,pruned,yes", [
+    (4, 12, 512, 512, 64, False, 1), (2, 32, 1000, 1000, 64, True, 1), (2, 16, 2048, 2048, 64, True, 1), (16, 16, 257, 257, 64, False, 0), (1, 1, 100, 100, 128, False, 0),
+    (3, 32, 1000, 1000, 32, True, 1), (1, 6, 16384, 16384, 16, False, 1), (49, 16, 100, 100, 32, False, 0), (48, 16, 100, 100, 32, True, 1),
+    # long rows: room on the chip, more of it under a threshold
+    (1, 10, 4096, 4096, 64, True, 1), (1, 11, 4096, 4096, 64, True, 0), (1, 14, 4096, 4096, 64, False, 1), (1, 15, 4096, 4096, 64, False, 0),
+    (1, 2, 16384, 16384, 32, True, 1), (1, 4, 16384, 16384, 32, True, 0), (1, 12, 8192, 8192, 32, True, 1),
+    (1, 16, 300, 4096, 64, True, 1), (1, 16, 2048, 4096, 64, True, 0), (1, 16, 2048, 4096, 64, False, 1)])
+def test_grids_of_the_one_launch_backward(B, H, M, N, D, pruned, yes):
+    from forgetting_transformer.ops import _lib
+    x = 1 << 20   # (never read: host arithmetic only)
+    got = C.c_int32(-1)
+    view = _lib.View(x, H * N * D, N * D, D)
+    args = _lib.BwdArgs(_lib.Dims(B, H, M, N, D, 0), *[view] * 8, x, x, None, x if pruned else None, 0.1, x, x + 64, x, x, 0, 0, 0, None, None)
+    _lib.check(_lib.load().fox_attn_bwd_one_launch(C.byref(args), C.byref(got)), "fox_attn_bwd_one_launch")
+    assert got.value == yes
