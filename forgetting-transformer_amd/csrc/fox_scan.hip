@@ -1,7 +1,7 @@
 // Row scans and the "auto" pruning threshold for gfx950.
 //
-//   scan_kernel<false> : c[n]  = sum_{l<=n} g[l], with g[l] := 0 for l < seq_start
-//   scan_kernel<true>  : dg[l] = sum_{n>=l} dc[n]
+//   scan_kernel<kForward> : c[n]  = sum_{l<=n} g[l], with g[l] := 0 for l < seq_start
+//   scan_kernel<kReverse> : dg[l] = sum_{n>=l} dc[n]
 //   gate_scan_fwd/bwd  : the same two scans fused with logsigmoid of the gate logits and its derivative
 //   norm_max_kernel    : the "auto" threshold from the largest row L2 norms of q and k.
 //
@@ -15,13 +15,14 @@ namespace fox {
 
 // The gradient of a cumulative sum at one position is its row sum of dS minus its column sum.  Where the backward ran in one launch the dK/dV walk
 // could not wait for the row sums (drow, of the last M positions of the row): the reverse scan adds them, and stores the sum back into dc, which then
-// holds what the dK/dV kernel leaves there on its own.  The loads are a loop of their own under one branch: in a branch per element every one of them was
-// waited for before the next was sent (4 rows of 16384 positions 15.1 us, so 12.3; without row sums 9.9; 24 rows of 2048 6.0, 4.5 and 4.1).
+// holds what the dK/dV kernel leaves there on its own.  The loads are a loop of their own, without a branch: in a branch per element every one of them was
+// waited for before the next was sent (2 rows of 16384 positions 12.5 us, so 11.2, without row sums 8.6; 48 rows of 512 5.1, 4.0 and 4.0).  A variant
+// of its own: as a branch at run time it cost the other scans 0.3 to 0.6 us.
 struct RowSums {
-  const float* drow;   // (M) or null
+  static constexpr bool kAny = true;
+  const float* drow;   // (M)
   float* dc;
   int p_seq;
-  __device__ __forceinline__ bool any() const { return drow != nullptr; }
   __device__ __forceinline__ float load(int idx) const {
     const float r = drow[max(idx - p_seq, 0)];
     return idx >= p_seq ? r : 0.f;
@@ -29,7 +30,7 @@ struct RowSums {
   __device__ __forceinline__ void keep(int idx, float x) const { dc[idx] = x; }
 };
 struct NoRows {
-  __device__ __forceinline__ constexpr bool any() const { return false; }
+  static constexpr bool kAny = false;
   __device__ __forceinline__ float load(int) const { return 0.f; }
   __device__ __forceinline__ void keep(int, float) const {}
 };
@@ -52,7 +53,7 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store, Rows row
   __shared__ __align__(16) float stage[SPAN];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   double carry = 0.0;
-  float x[PER], x_next[PER], r[PER] = {}, r_next[PER] = {};
+  float x[PER], x_next[PER], r[PER], r_next[PER];   // (r: Rows::kAny only)
   auto fetch = [&](int base, float (&dst)[PER], float (&dst_r)[PER]) {  // element e of a thread sits at position base + e*NT + tid of the scan order
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
@@ -60,7 +61,7 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store, Rows row
       const int idx = REVERSE ? N - 1 - pos : pos;
       dst[e] = pos < N ? load(idx) : 0.f;
     }
-    if (rows.any()) {
+    if constexpr (Rows::kAny) {
 #pragma unroll
       for (int e = 0; e < PER; ++e) {
         const int pos = base + e * NT + tid, in = min(pos, N - 1);
@@ -73,7 +74,7 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store, Rows row
   for (int base = 0; base < N; base += SPAN) {
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-      if (rows.any()) x[e] += r[e];
+      if constexpr (Rows::kAny) x[e] += r[e];
       stage[e * NT + tid] = x[e];
     }
     if (base + SPAN < N) fetch(base + SPAN, x_next, r_next);   // in flight while this span is scanned
@@ -119,7 +120,7 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store, Rows row
       const int idx = REVERSE ? N - 1 - pos : pos;
       if (pos < N) store(idx, stage[e * NT + tid]);
     }
-    if (rows.any()) {
+    if constexpr (Rows::kAny) {
 #pragma unroll
       for (int e = 0; e < PER; ++e) {
         const int pos = base + e * NT + tid;
@@ -129,7 +130,7 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store, Rows row
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
       x[e] = x_next[e];
-      r[e] = r_next[e];
+      if constexpr (Rows::kAny) r[e] = r_next[e];
     }
     __syncthreads();  // the span has left LDS before the next one is written
   }
@@ -145,19 +146,21 @@ __device__ __forceinline__ int scan_row_of_block(int rows, bool neighbours) {
 }
 inline unsigned scan_blocks(int rows) { return (unsigned)((rows + kXcds - 1) / kXcds * kXcds); }
 
-template <bool REVERSE>
+template <bool ROWS>
 __device__ __forceinline__ auto row_sums(const float* drow, float* dc, int bh, int M, int N) {   // of the row of pair bh
-  if constexpr (REVERSE) return RowSums{drow ? drow + (int64_t)bh * M : nullptr, dc + (int64_t)bh * N, N - M};
+  if constexpr (ROWS) return RowSums{drow + (int64_t)bh * M, dc + (int64_t)bh * N, N - M};
   else return NoRows{};
 }
 
 inline int scan_threads(int N) { return N <= 8 * 64 ? 64 : N <= 8 * 256 ? 256 : 1024; }
 
-template <bool REVERSE, int NT>
+enum : int { kForward = 0, kReverse = 1, kReverseRows = 2 };   // kinds of scan_kernel; the last with row sums to add
+template <int KIND, int NT>
 __global__ __launch_bounds__(NT) void scan_kernel(const float* in, int64_t sb, int64_t sh, int64_t sn,
                                                    const int64_t* __restrict__ seq_start, float* __restrict__ out, int64_t ob,
                                                    int64_t oh, int64_t on, int rows, int H, int N, const float* __restrict__ drow, int M,
                                                    float* dc) {
+  constexpr bool REVERSE = KIND != kForward;
   const int bh = REVERSE ? scan_row_of_block(rows, on != 1) : blockIdx.x, b = bh / H, h = bh % H;
   if (REVERSE && bh >= rows) return;
   const float* src = in + b * sb + h * sh;
@@ -173,7 +176,7 @@ __global__ __launch_bounds__(NT) void scan_kernel(const float* in, int64_t sb, i
   scan_row<REVERSE, NT>(
       N, [&](int idx) { return (REVERSE || idx >= seq) ? src[(int64_t)idx * sn] : 0.f; },
       [&](int idx, float sum) { dst[(int64_t)idx * on] = (REVERSE && idx <= seq) ? 0.f : sum; },
-      row_sums<REVERSE>(drow, dc, bh, M, N));
+      row_sums<KIND == kReverseRows>(drow, dc, bh, M, N));
 }
 
 template <int DT>
@@ -212,11 +215,13 @@ __global__ __launch_bounds__(NT) void gate_scan_fwd_kernel(const void* __restric
 
 // dlogit[l] = (sum_{n>=l} dc[n]) * d logsigmoid(x_l)/dx = dg[l] * (1 - sigmoid(x_l)), stored in the
 // dtype and layout of the logits.
-template <int DT, int NT>
+constexpr int kRows = 4;   // with row sums to add
+template <int DT_ROWS, int NT>
 __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(float* dc, const void* __restrict__ logits,
                                                             int64_t sb, int64_t sh, int64_t sn, const int64_t* __restrict__ seq_start,
                                                             void* __restrict__ dlogits, int64_t db, int64_t dh, int64_t dn,
                                                             int rows, int H, int N, const float* __restrict__ drow, int M) {
+  constexpr int DT = DT_ROWS & 3;
   const int bh = scan_row_of_block(rows, dn != 1), b = bh / H, h = bh % H;
   if (bh >= rows) return;
   const float* src = dc + (int64_t)bh * N;
@@ -232,10 +237,10 @@ __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(float* dc, const void
         const float x = load_logit<DT>(logits, lbase + (int64_t)idx * sn);
         const float z = __expf(-fabsf(x));
         const float r = __fdividef(z, 1.f + z);              // sigmoid(-|x|)
-        // positions up to and including seq: an exact zero, as in scan_kernel<true>
+        // positions up to and including seq: an exact zero, as in scan_kernel
         store_logit<DT>(dlogits, dbase + (int64_t)idx * dn, idx <= seq ? 0.f : sum * (x < 0.f ? 1.f - r : r));
       },
-      row_sums<true>(drow, dc, bh, M, N));
+      row_sums<(DT_ROWS & kRows) != 0>(drow, dc, bh, M, N));
 }
 
 // KERNEL<ARG, threads for rows of N elements>, BLOCKS workgroups, one per row of the B x H.
@@ -260,10 +265,13 @@ hipError_t launch_gate_cumsum_fwd(const void* logits, int dtype, int64_t sb, int
 hipError_t launch_gate_cumsum_bwd(float* dc, const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn,
                                   const int64_t* seq_start, void* dlogits, int64_t db, int64_t dh, int64_t dn, int B, int H, int N,
                                   const float* drow, int M, hipStream_t s) {
-  switch (dtype) {
+  switch (drow ? dtype | kRows : dtype) {
     case 0: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 0, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
     case 1: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 1, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
     case 2: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 2, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 0 | kRows: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, (0 | kRows), scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 1 | kRows: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, (1 | kRows), scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 2 | kRows: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, (2 | kRows), scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -271,15 +279,20 @@ hipError_t launch_gate_cumsum_bwd(float* dc, const void* logits, int dtype, int6
 
 hipError_t launch_cumsum_fwd(const float* g, int64_t sb, int64_t sh, int64_t sn, const int64_t* seq_start, float* c, int B,
                              int H, int N, hipStream_t s) {
-  FOX_LAUNCH_SCAN(scan_kernel, false, (unsigned)(B * H), g, sb, sh, sn, seq_start, c,
+  FOX_LAUNCH_SCAN(scan_kernel, kForward, (unsigned)(B * H), g, sb, sh, sn, seq_start, c,
                      (int64_t)H * N, (int64_t)N, (int64_t)1, B * H, H, N, nullptr, N, nullptr)
   return hipGetLastError();
 }
 
 hipError_t launch_cumsum_bwd(float* dc, float* dg, int64_t db, int64_t dh, int64_t dn, const int64_t* seq_start, int B, int H,
                              int N, const float* drow, int M, hipStream_t s) {
-  FOX_LAUNCH_SCAN(scan_kernel, true, scan_blocks(B * H), dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
-                     seq_start, dg, db, dh, dn, B * H, H, N, drow, M, dc)
+  if (drow) {
+    FOX_LAUNCH_SCAN(scan_kernel, kReverseRows, scan_blocks(B * H), dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
+                       seq_start, dg, db, dh, dn, B * H, H, N, drow, M, dc)
+  } else {
+    FOX_LAUNCH_SCAN(scan_kernel, kReverse, scan_blocks(B * H), dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
+                       seq_start, dg, db, dh, dn, B * H, H, N, nullptr, N, nullptr)
+  }
   return hipGetLastError();
 }
 
