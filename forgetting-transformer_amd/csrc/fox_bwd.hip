@@ -306,10 +306,13 @@ __device__ __forceinline__ void dkdv_body(const BwdK& a, int bh, int nt, const D
   // goes from lane to lane, two lanes further with every chunk; the last two lanes of the row end up with the two halves.
   auto store_own_delta = [&](const char* dot, float* dl) {
     if constexpr (OWN_DELTA) {
+      // Tile<D>::off() within a block, written out, and here: as a call, or as a value of the function above, it changes what the compiler makes of the
+      // addresses in dkdv_kernel at head dims 32 and 64, which does not even come here (25 more additions; B3 H16 T1536 at -60 79.3 -> 80.7 us).
+      const int o_at = 16 * ((lane & 48) | ((lane & 15) ^ (lane >> 4 << 2)));
 #pragma unroll
       for (int j = 0; j < OPER; ++j) {
         const int row = o_row + 4 * ORPB * j;
-        const u32x4 x = lds_row_operand<D>(dot, row, o_ch);
+        const u32x4 x = *reinterpret_cast<const u32x4*>(dot + (wave + 4 * j) * Tile<D>::BLOCK_BYTES + o_at);
         float part = 0.f;
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
