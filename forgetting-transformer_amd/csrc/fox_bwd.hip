@@ -648,7 +648,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK args) {
     }
     mt = w.tile;
   } else {
-    decode_block(blockIdx.x, args.order, true, bh, mt);
+    decode_block(blockIdx.x, args.order, args.last_first, bh, mt);
   }
   const BwdK& a = BOTH ? own_arguments() : args;
 
@@ -871,6 +871,9 @@ static hipError_t dq_t(const BwdK& a0, int D, hipStream_t s) {
   BwdK a = a0;
   a.n_tiles = (a.M + kFwdBM - 1) / kFwdBM;
   a.order = block_order(a.B, a.H, a.n_tiles, order_groups(a.B * a.H, a.n_tiles, a.M, a.N, D, a.k.st, a.thr != nullptr), !even_tiles(a.M, a.N));
+  // Not under a threshold on a grid that is resident at once: all pairs start together, and where 8 does not divide them the turned order puts each on another
+  // XCD than its forward (turned / not, whole step: B1 H12 T4096 D64 at -10 56.5 / 55.5 us, B1 H6 T8192 57.0 / 56.4; without a threshold B1 H1 T16384 D128 804 / 809).
+  a.last_first = !a.thr || a.n_tiles * a.B * a.H > 2 * kCus;
   const dim3 grid((unsigned)(a.n_tiles * a.B * a.H));
   switch (D) {
     case 16: hipLaunchKernelGGL((dq_kernel<Tr, 16, false>), grid, dim3(256), 0, s, a); break;

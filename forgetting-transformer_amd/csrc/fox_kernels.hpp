@@ -121,6 +121,7 @@ struct BwdK {
   float sm_scale;
   int n_tiles;
   BlockOrder order;   // set by the launchers
+  bool last_first;    // dQ: pairs from the last to the first, set by its launcher
   int cls;         // kClassAll, or the class of key tiles this dK/dV launch handles (fox_common.hpp)
   int light_limit; // distance from the diagonal, in keys, that separates the two classes
   int32_t* q_first_block;  // optional (B,H,ceil(M/kFwdBM)): first key block (of kFwdBN keys) each query tile of the dQ kernel visits
@@ -231,12 +232,13 @@ constexpr BlockOrder block_order(int B, int H, int tiles, int groups, bool fold)
 // Folded: when the whole grid is resident at two workgroups per CU, the second workgroup of a CU is the one that arrives
 // kCus ids after the first.  Taken in the same order both would be heavy on one CU and both light on another; from
 // workgroup kCus on the list is therefore walked from its light end (forward B1 H16 T4096 D128: 109 -> 84 us, dQ 152 -> 116 us).
-// `last_first`: the pairs from the last to the first.  The dQ kernel takes them so, between a forward and a dK/dV kernel that start with the
+// `last_first`: the pairs from the last to the first.  The dQ kernel takes them so (with one exception, dq_t), between a forward and a dK/dV kernel that start with the
 // first: each of the three then opens on the tensors its predecessor touched last, which are still in the 256 MiB last-level cache.
 // Backward with dQ ascending / descending: B4 T16384 H16 D128 "auto" 731 / 710 us, B16 H16 T4096 D64 "auto" 516 / 491,
 // B4 H32 T4096 D64 at -10 240 / 229, without a threshold 963 / 953.
 // What is divided by is the same for a whole launch: six divisions by Divisor instead of the compiler's take some 130 instructions off the front of a
-// kernel, which is what a workgroup of a pruned walk and one that finds nothing to do notice (figures: PENDING).
+// kernel, which is what a workgroup of a pruned walk and one that finds nothing to do notice (at -10: the dK/dV class without a tile, B4 T4096 H16 D128, 6.9 -> 5.6 us, forward
+// B4 T4096 H32 D64 57.9 -> 56.5; other kernels and dense walks within the runs' spread).
 __host__ __device__ __forceinline__ void decode_block(uint32_t wid, const BlockOrder& o, bool last_first, int& bh, int& tile) {
   int r = (int)(o.by_xcd ? wid / kXcds : wid);
   const int cus = o.by_xcd ? kCus / kXcds : kCus;
