@@ -398,7 +398,7 @@ int fox_attn_fwd_takes_gates(const fox_dims* dims, int32_t pruned, int32_t* yes)
   FOX_TRY(check_dims(dims));
   if (!yes) return fail(FOX_E_ARG, "yes is NULL");
   const FwdPlan p = plan_fwd(*dims, pruned != 0, true);
-  *yes = fox::fwd_scans(dims->B, dims->H, dims->M, dims->N, p.splits);
+  *yes = fox::fwd_scans(dims->B, dims->H, dims->M, dims->N, dims->D, pruned != 0, p.splits);
   return FOX_OK;
 }
 

@@ -859,13 +859,24 @@ hipError_t launch_fwd_gates(const FwdK& a, int D, int dtype, hipStream_t s) {
 
 // Whether the forward forms the cumulative sums itself (fwd_scan_kernel) instead of reading what a scan left.  The scan is a launch and
 // 3 to 6 us of one workgroup per row; own sums cost a workgroup 1 to 2 us, most of it while its first tiles arrive, but every workgroup.
-// Forward with its scan / with own sums, us.  Resident grids (up to two workgroups per CU), any row: B1 H12 N77 D64 8.9 / 6.9, B4 H12 N512 14.7 / 12.8,
-// B1 H16 N3001 D128 57.0 / 54.2, B2 H12 N2048 D64 at -10 15.0 / 13.5, B1 H16 N3500 D128 at -10 22.9 / 19.7.  Up to four per CU: short rows, B8 H16 N768 D64 22.9 / 21.5,
-// B16 H32 N256 20.8 / 20.5, not long ones (B4 H16 N1500 D128 55.8 / 55.8).  Beyond that every round repeats the sums: B8 H12 N2048 D64 70.6 / 71.4,
-// B16 H16 N3500 475 / 499.
-bool fwd_scans(int B, int H, int M, int N, int splits) {
-  const int64_t wgs = (int64_t)((M + kFwdBM - 1) / kFwdBM) * B * H;
-  return M > 1 && splits <= 1 && N <= kOwnScanMaxKeys && (wgs <= 2 * kCus || (wgs <= 4 * kCus && N <= 1024));
+// Forward with its scan / with own sums, us, on inputs that the caches hold; on fresh ones the gates of (B, T, H) memory, a line per token and workgroup,
+// come from further away and the longest rows gain nothing (B1 T3001 H16 D128).
+// - Resident grids (up to two workgroups per CU): B16 H16 N250 D64 12.5 / 10.4, B4 H32 N500 16.1 / 14.6, B2 H12 N2048 D128 43.6 / 42.4, B1 H16 N3500 66.4 / 64.3,
+//   at -10 B2 H32 N1000 D64 17.4 / 15.5, B1 H16 N3500 18.8 / 16.6.  Without a threshold the walks of head dims up to 64 hide little of it; they lose on long rows of many
+//   heads: B1 H32 N1900 D16 28.9 / 30.2, D32 30.3 / 31.6, D64 33.9 / 34.6 (H16 N2048 24.3 / 24.1, 25.6 / 24.9, 29.0 / 28.7).
+// - Fewer queries than keys: every query tile of a pair repeats almost the whole row, B8 H32 M130 N3500 D64 at -10 23.7 / 25.9, M400 B4 22.6 / 24.6, M130 N1600 18.6 /
+//   19.2.  The line lies at 2900 keys summed up per CU (B8 H32 M130 N1200 17.9 / 17.8); a pair's only tile repeats nothing
+//   (B16 H32 M128 N3500 34.0 / 28.4).
+// - Up to four workgroups per CU: short rows, at -10 B4 H32 N1000 D64 25.1 / 24.2, without a threshold up to 3.5 (B4 H28 N1000 30.8 / 29.5, B4 H32 N1000 34.3 / 35.5, B8 H32
+//   N500 25.1 / 25.7) or very short ones (B16 H32 N256 20.5 / 20.0, D128 31.3 / 30.2; D128 B8 H24 N500 31.6 / 32.8).  Not long ones (B4 H16 N1500 D128 55.8 / 55.8).
+// - Beyond that every round repeats the sums: B8 H12 N2048 D64 70.6 / 71.4, B16 H16 N3500 475 / 499.
+bool fwd_scans(int B, int H, int M, int N, int D, bool pruned, int splits) {
+  const int64_t pairs = (int64_t)B * H, tiles = (M + kFwdBM - 1) / kFwdBM, wgs = tiles * pairs;
+  if (M <= 1 || splits > 1 || N > kOwnScanMaxKeys) return false;
+  if (tiles > 1 && M < N && wgs * (2 * (int64_t)N - M) > 2 * 2900 * kCus) return false;
+  if (wgs <= 2 * kCus) return pruned || D > 64 || N <= 1024 || 4 * wgs <= 5 * kCus || pairs < 24;
+  if (wgs > 4 * kCus || N > 1024) return false;
+  return pruned || N <= 384 || (D <= 64 && 2 * wgs <= 7 * kCus);
 }
 
 // Whether the forward takes the paired variant (fwd_pair_kernel): less than two query tiles per CU under a causal triangle, where the

@@ -87,3 +87,18 @@ def test_grids_of_the_one_launch_backward(B, H, M, N, D, pruned, yes):
     args = _lib.BwdArgs(_lib.Dims(B, H, M, N, D, 0), *[view] * 8, x, x, None, x if pruned else None, 0.1, x, x + 64, x, x, 0, 0, 0, None, None)
     _lib.check(_lib.load().fox_attn_bwd_one_launch(C.byref(args), C.byref(got)), "fox_attn_bwd_one_launch")
     assert got.value == yes
+
+
+@pytest.mark.parametrize("B,H,M,N,D,pruned,yes", [
+    (1, 1, 2, 3584, 64, False, 0), (2, 16, 2048, 2048, 128, False, 1), (2, 16, 2048, 2048, 64, False, 0), (2, 16, 2048, 2048, 64, True, 1), (2, 9, 3583, 3583, 16, False, 1),
+    (4, 32, 500, 500, 32, False, 1), (8, 32, 400, 1000, 64, True, 0),
+    # several query tiles behind many keys repeat the row, one does not
+    (8, 32, 130, 1200, 64, True, 1), (8, 32, 130, 1600, 64, True, 0), (8, 32, 130, 1600, 128, False, 0), (16, 32, 128, 3500, 64, True, 1), (8, 32, 130, 1500, 64, True, 1),
+    # more than two workgroups per CU
+    (4, 28, 1000, 1000, 64, False, 1), (4, 32, 1000, 1000, 64, False, 0), (4, 32, 1000, 1000, 64, True, 1), (16, 32, 256, 256, 128, False, 1), (8, 24, 500, 500, 128, False, 0),
+    (3, 16, 1536, 1536, 64, True, 0), (32, 33, 128, 128, 64, True, 0)])
+def test_grids_that_form_their_own_sums(B, H, M, N, D, pruned, yes):
+    from forgetting_transformer.ops import _lib
+    got = C.c_int32(-1)
+    _lib.check(_lib.load().fox_attn_fwd_takes_gates(C.byref(_lib.Dims(B, H, M, N, D, 0)), pruned, C.byref(got)), "fox_attn_fwd_takes_gates")
+    assert got.value == yes
