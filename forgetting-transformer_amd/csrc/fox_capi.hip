@@ -364,7 +364,7 @@ extern "C" {
 
 // 0.2.x: fox_bwd_args and the scan entry points differ from 0.1.0; 0.2.1 adds fox_set_stream_min_kv_bytes and fox_probe_mfma, 0.2.2
 // fox_attn_decode, fox_cache_append, fox_qk_norm_threshold and fox_attn_fwd_plan, 0.2.3 fox_attn_fwd_gates, fox_attn_fwd_takes_gates,
-// fox_auto_threshold_scan, fox_attn_decode_counted and fox_attn_bwd_logits, 0.2.4 fox_attn_bwd_one_launch
+// fox_auto_threshold_scan, fox_attn_decode_counted and fox_attn_bwd_logits, 0.2.4 fox_attn_bwd_one_launch and fox_attn_decode_counters
 int fox_version(void) { return 204; }
 
 const char* fox_last_error(void) { return g_err; }
@@ -559,6 +559,14 @@ int fox_attn_decode_workspace_bytes(const fox_dims* dims, int64_t* bytes) {
   if (dims->M != 1) return fail(FOX_E_ARG, "fox_attn_decode takes one query row (M = %d)", dims->M);
   const int splits = fox::decode_splits(dims->B, dims->H, dims->N, dims->D);
   *bytes = splits <= 1 ? 0 : (int64_t)splits * dims->B * dims->H * (int64_t)(dims->D * sizeof(float) + sizeof(fox::DecodePartial));
+  return FOX_OK;
+}
+
+int fox_attn_decode_counters(const fox_dims* dims, int32_t* counters) {
+  FOX_TRY(check_dims(dims));
+  if (!counters) return fail(FOX_E_ARG, "counters is NULL");
+  if (dims->M != 1) return fail(FOX_E_ARG, "fox_attn_decode takes one query row (M = %d)", dims->M);
+  *counters = fox::decode_merges(dims->B, dims->H, fox::decode_splits(dims->B, dims->H, dims->N, dims->D)) ? dims->B * dims->H : 0;
   return FOX_OK;
 }
 

@@ -62,22 +62,23 @@ Tensor empty_floats(const Tensor& t, int64_t n) { return at::empty({n}, t.option
 // Arrival counters for kernels whose last workgroup finishes the work of all: kCounters zeros per stream, which every such kernel leaves zero
 // again.  Launches on one stream follow each other, so the block of a stream has one user at a time, whichever threads feed the stream.  Only
 // for torch's own streams, which live as long as the process (the handle of another stream may come back as a different stream), at most
-// kCounterBlocks of them, and not during capture (a graph may be replayed beside its stream).  Null: the caller takes the way without counters.
-constexpr int64_t kCounters = 4096;
+// kCounterBlocks of them per device, and not during capture (a graph may be replayed beside its stream).  Null: the caller takes the way without
+// counters.  kCounters is the most that fox_attn_decode_counters asks for: at least two workgroups for each, on at most as many as there are CUs.
+constexpr int64_t kCounters = 128;
 constexpr size_t kCounterBlocks = 64;
 uint32_t* arrival_counters(const Tensor& like, int64_t n) {
   const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream(like.device().index());
   const bool torch_owned = stream.id() == 0 || (stream.id() & 1);
   if (n > kCounters || !torch_owned || c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return nullptr;
   static std::mutex mutex;
-  static auto* blocks = new std::map<std::pair<int, int64_t>, Tensor>;   // (not destroyed: the device may be gone before static objects are)
+  static auto* devices = new std::map<int, std::map<int64_t, Tensor>>;   // (not destroyed: the device may be gone before static objects are)
   const std::lock_guard<std::mutex> lock(mutex);
-  const std::pair<int, int64_t> key(like.device().index(), stream.id());
-  auto it = blocks->find(key);
-  if (it == blocks->end()) {
-    if (blocks->size() >= kCounterBlocks) return nullptr;
+  auto& blocks = (*devices)[like.device().index()];
+  auto it = blocks.find(stream.id());
+  if (it == blocks.end()) {
+    if (blocks.size() >= kCounterBlocks) return nullptr;
     const c10::InferenceMode no_inference(false);
-    it = blocks->emplace(key, at::zeros({kCounters}, like.options().dtype(at::kInt))).first;
+    it = blocks.emplace(stream.id(), at::zeros({kCounters}, like.options().dtype(at::kInt))).first;
   }
   return (uint32_t*)it->second.mutable_data_ptr();
 }
@@ -222,7 +223,9 @@ Tensor run_decode(const Attention& a, const Tensor& q, const Tensor& k, const Te
     args.workspace = ws.mutable_data_ptr();
     args.workspace_bytes = ws_bytes;
   }
-  uint32_t* arrived = ws_bytes > 0 ? arrival_counters(q, a.B * a.H) : nullptr;
+  int32_t counters = 0;
+  check(fox_attn_decode_counters(&args.dims, &counters), "fox_attn_decode_counters");
+  uint32_t* arrived = counters > 0 ? arrival_counters(q, counters) : nullptr;
   check(fox_attn_decode_counted(&args, g.const_data_ptr<float>(), g.stride(0), a.gs_h(g), a.gs_n(g), arrived, stream_of(q)), "fox_attn_decode");
   return out;
 }

@@ -149,6 +149,7 @@ SIGNATURES = {
     "fox_attn_fwd_plan": (C.c_int, [C.POINTER(Dims), C.c_int32, C.POINTER(C.c_int32), C.POINTER(C.c_int32), C.POINTER(C.c_int64)]),
     "fox_attn_decode": (C.c_int, [C.POINTER(FwdArgs), C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p]),
     "fox_attn_decode_counted": (C.c_int, [C.POINTER(FwdArgs), C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p, C.c_void_p]),
+    "fox_attn_decode_counters": (C.c_int, [C.POINTER(Dims), C.POINTER(C.c_int32)]),
     "fox_attn_decode_workspace_bytes": (C.c_int, [C.POINTER(Dims), C.POINTER(C.c_int64)]),
     "fox_attn_fwd_gates": (C.c_int, [C.POINTER(FwdArgs), C.POINTER(Gates), C.POINTER(FwdEpilogue), C.c_void_p]),
     "fox_attn_fwd_takes_gates": (C.c_int, [C.POINTER(Dims), C.c_int32, C.POINTER(C.c_int32)]),

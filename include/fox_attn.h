@@ -204,10 +204,13 @@ int fox_attn_fwd_noalloc(const fox_fwd_args* args, void* stream);
  */
 int fox_attn_decode(const fox_fwd_args* args, const float* g, int64_t g_stride_b, int64_t g_stride_h, int64_t g_stride_n,
                     void* stream);
-/* The same, with B*H zeros in `arrived` (NULL = fox_attn_decode): where it is the faster way, the split that arrives last merges the partial
- * results, without a launch of its own.  The counters are zero again when the call's work is done; calls that may overlap need their own. */
+/* The same, with zeros in `arrived` (NULL = fox_attn_decode): where it is the faster way, the split that arrives last merges the partial
+ * results, without a launch of its own.  fox_attn_decode_counters says how many zeros that takes (B*H, or 0 where the shape does not merge this
+ * way and `arrived` is not touched; never more than 128).  The counters are zero again when the call's work is done; calls that may overlap need
+ * their own. */
 int fox_attn_decode_counted(const fox_fwd_args* args, const float* g, int64_t g_stride_b, int64_t g_stride_h, int64_t g_stride_n,
                             uint32_t* arrived, void* stream);
+int fox_attn_decode_counters(const fox_dims* dims, int32_t* counters);
 int fox_attn_decode_workspace_bytes(const fox_dims* dims, int64_t* bytes);
 
 /*

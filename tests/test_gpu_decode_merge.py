@@ -18,7 +18,9 @@ def ft():
     return ft
 
 
-SHAPES = [(1, 12, 1500, 64), (1, 1, 5000, 128), (2, 3, 4000, 16), (1, 5, 700, 32), (4, 32, 600, 64), (4, 32, 700, 64)]   # the last two: 256 workgroups and more
+SHAPES = [(1, 12, 1500, 64), (1, 1, 5000, 128), (2, 3, 4000, 16), (1, 5, 700, 32), (4, 32, 600, 64), (4, 32, 700, 64),   # (the last three: one workgroup a pair)
+          (1, 64, 1000, 64), (1, 4, 8192, 128), (1, 64, 1200, 64)]   # 256 workgroups in splits of 4 and of 64, the most of either, and more than 256
+MERGES = {(1, 12, 1500, 64), (1, 1, 5000, 128), (2, 3, 4000, 16), (1, 64, 1000, 64), (1, 4, 8192, 128)}
 
 
 def _inputs(shape, seq=None):
@@ -43,12 +45,31 @@ def _two_launches(q, k, v, g, ss, counters=None):
     return o, lse
 
 
+def _counters(shape):
+    from forgetting_transformer.ops import _lib
+    B, H, N, D = shape
+    n = C.c_int32(-1)
+    _lib.check(_lib.load().fox_attn_decode_counters(C.byref(_lib.Dims(B, H, 1, N, D, 0)), C.byref(n)), "fox_attn_decode_counters")
+    return n.value
+
+
+def test_no_counters_where_the_splits_do_not_merge(ft):
+    """A step of more workgroups than CUs allocates its output and its workspace, and no block of counters on a stream that has none."""
+    q, k, v, g, _ = _inputs((1, 64, 1200, 64))
+    with torch.no_grad(), torch.cuda.stream(torch.cuda.Stream()):
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        ft.forgetting_attention(q, k, v, g, head_first=True)
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == 2
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("padded", [False, True])
 def test_same_bits_and_zero_counters(ft, shape, padded):
     B, H, N, D = shape
     ins = _inputs(shape, [(N * (b + 1)) // B for b in range(B)] if padded else None)   # the last one: nothing but padding
     want = _two_launches(*ins)
+    assert _counters(shape) == (B * H if shape in MERGES else 0)
     counters = torch.zeros(B * H, dtype=torch.int32, device="cuda")
     for _ in range(3):
         got = _two_launches(*ins, counters=counters)
@@ -62,7 +83,7 @@ def test_same_bits_and_zero_counters(ft, shape, padded):
 
 
 def test_streams_threads_and_graphs(ft):
-    ins = [_inputs(s) for s in SHAPES[:4]]
+    ins = [_inputs(s) for s in (*SHAPES[:3], SHAPES[7])]
     want = [_two_launches(*x)[0] for x in ins]
     torch.cuda.synchronize()
     bad = []

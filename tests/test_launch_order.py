@@ -102,3 +102,13 @@ def test_grids_that_form_their_own_sums(B, H, M, N, D, pruned, yes):
     got = C.c_int32(-1)
     _lib.check(_lib.load().fox_attn_fwd_takes_gates(C.byref(_lib.Dims(B, H, M, N, D, 0)), pruned, C.byref(got)), "fox_attn_fwd_takes_gates")
     assert got.value == yes
+
+
+@pytest.mark.parametrize("B,H,N,D,counters", [(1, 12, 1500, 64, 12), (1, 64, 1000, 64, 64), (1, 64, 1200, 64, 0), (1, 4, 8192, 128, 4), (1, 5, 8192, 128, 0), (1, 5, 700, 32, 0),
+                                              (1, 128, 600, 64, 0), (1, 128, 1500, 16, 128), (1, 129, 1500, 16, 0), (16, 16, 32768, 128, 0)])
+def test_counters_of_a_generation_step(B, H, N, D, counters):
+    from forgetting_transformer.ops import _lib
+    got = C.c_int32(-1)
+    _lib.check(_lib.load().fox_attn_decode_counters(C.byref(_lib.Dims(B, H, 1, N, D, 0)), C.byref(got)), "fox_attn_decode_counters")
+    assert got.value == counters <= 128
+    assert _lib.load().fox_attn_decode_counters(C.byref(_lib.Dims(B, H, 2, N, D, 0)), C.byref(got)) == -1
