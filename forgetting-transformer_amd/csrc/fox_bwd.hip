@@ -621,7 +621,8 @@ __device__ __forceinline__ const BwdK& own_arguments() {
 
 // BOTH: dQ and dK/dV in one launch, for small grids of head dims up to 64 (bwd_together): workgroups of either kind side by side, the heaviest of either
 // kind first.  One after the other, each of the two kernels waits for its longest walk on a chip that is mostly idle.  (The dQ walk is part of the
-// kernel and not a function both kernels call: that way the compiler waits for LDS eight times more often in it, and at D = 128 it took 5-10 % longer.)
+// kernel and not a function both kernels call: that way the compiler put eight more waits for LDS into it, 213 instead of 205, and unpruned dQ at D = 128 took 2 to
+// 10 % longer: B4 H16 T4096 365 -> 373 us, B8 H3 T3309 111 -> 119, B2 H16 T2048 67 -> 74.)
 template <typename Tr, int D, bool BOTH>
 __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK args) {
   constexpr int BM = kFwdBM, BN = kFwdBN, ROWS = BOTH ? kKvBM : kFwdBN;   // rows of a tile buffer: the dK/dV walk needs the larger ones

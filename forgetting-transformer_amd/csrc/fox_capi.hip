@@ -364,7 +364,8 @@ extern "C" {
 
 // 0.2.x: fox_bwd_args and the scan entry points differ from 0.1.0; 0.2.1 adds fox_set_stream_min_kv_bytes and fox_probe_mfma, 0.2.2
 // fox_attn_decode, fox_cache_append, fox_qk_norm_threshold and fox_attn_fwd_plan, 0.2.3 fox_attn_fwd_gates, fox_attn_fwd_takes_gates,
-// fox_auto_threshold_scan, fox_attn_decode_counted and fox_attn_bwd_logits, 0.2.4 fox_attn_bwd_one_launch and fox_attn_decode_counters
+// fox_auto_threshold_scan, fox_attn_decode_counted and fox_attn_bwd_logits, 0.2.4 fox_attn_bwd_one_launch,
+// fox_auto_threshold_scan_one_launch and fox_attn_decode_counters
 int fox_version(void) { return 204; }
 
 const char* fox_last_error(void) { return g_err; }
@@ -510,6 +511,13 @@ int fox_auto_threshold_scan(const fox_dims* dims, const fox_view* q, const fox_v
     return fox_gate_cumsum_fwd(gates->g, gates->dtype, gates->stride_b, gates->stride_h, gates->stride_n, seq_start, t.log_fgate, c, dims->B, dims->H,
                                dims->N, stream);
   return fox_cumsum_fwd((const float*)gates->g, gates->stride_b, gates->stride_h, gates->stride_n, seq_start, c, dims->B, dims->H, dims->N, stream);
+}
+
+int fox_auto_threshold_scan_one_launch(const fox_dims* dims, int32_t* yes) {
+  FOX_TRY(check_dims(dims));
+  if (!yes) return fail(FOX_E_ARG, "yes is NULL");
+  *yes = fox::threshold_scans(dims->B, dims->H, dims->M, dims->N, dims->D);
+  return FOX_OK;
 }
 
 int fox_qk_norm_threshold(const float* q_weight, const float* k_weight, int32_t H, int32_t D, double seq_len, double tolerance, float* thr,

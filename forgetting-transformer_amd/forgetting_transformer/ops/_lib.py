@@ -141,6 +141,7 @@ SIGNATURES = {
                                      C.c_void_p]),
     "fox_auto_threshold_scan": (C.c_int, [C.POINTER(Dims), C.POINTER(View), C.POINTER(View), C.c_float, C.c_void_p, C.c_void_p, C.POINTER(Gates),
                                           C.c_void_p, C.c_void_p, C.c_void_p]),
+    "fox_auto_threshold_scan_one_launch": (C.c_int, [C.POINTER(Dims), C.POINTER(C.c_int32)]),
     "fox_qk_norm_threshold": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int32, C.c_int32, C.c_double, C.c_double, C.c_void_p, C.c_void_p]),
     "fox_attn_fwd": (C.c_int, [C.POINTER(FwdArgs), C.c_void_p]),
     "fox_attn_fwd_noalloc": (C.c_int, [C.POINTER(FwdArgs), C.c_void_p]),

@@ -415,6 +415,8 @@ int fox_attn_fwd_takes_gates(const fox_dims* dims, int32_t pruned, int32_t* yes)
  * longer than the scan. */
 int fox_auto_threshold_scan(const fox_dims* dims, const fox_view* q, const fox_view* k, float sm_scale, float* thr, uint32_t* norm_scratch,
                             const fox_gates* gates, const int64_t* seq_start, float* c, void* stream);
+/* Whether fox_auto_threshold_scan takes one launch for this shape. */
+int fox_auto_threshold_scan_one_launch(const fox_dims* dims, int32_t* yes);
 
 #ifdef __cplusplus
 }

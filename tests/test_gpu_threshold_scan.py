@@ -25,6 +25,9 @@ def test_against_the_two_launches(B, H, M, N, D, dtype, padded, logit):
     if logit is not None:
         g = (g * 3 + 2).to(logit)
     dims = _lib.Dims(B, H, M, N, D, 0 if dtype == torch.bfloat16 else 1)
+    one_launch = C.c_int32(-1)
+    _lib.check(lib.fox_auto_threshold_scan_one_launch(C.byref(dims), C.byref(one_launch)), "one launch")
+    assert one_launch.value == (N != 300)
     stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
     ssp = None if ss is None else ss.data_ptr()
     res = []

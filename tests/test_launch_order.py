@@ -112,3 +112,12 @@ def test_counters_of_a_generation_step(B, H, N, D, counters):
     _lib.check(_lib.load().fox_attn_decode_counters(C.byref(_lib.Dims(B, H, 1, N, D, 0)), C.byref(got)), "fox_attn_decode_counters")
     assert got.value == counters <= 128
     assert _lib.load().fox_attn_decode_counters(C.byref(_lib.Dims(B, H, 2, N, D, 0)), C.byref(got)) == -1
+
+
+@pytest.mark.parametrize("B,H,M,N,D,yes", [(1, 17, 4096, 4096, 128, 0), (1, 18, 4096, 4096, 128, 1), (8, 22, 700, 700, 32, 0), (8, 23, 700, 700, 32, 1),
+                                           (4, 64, 128, 32768, 16, 1), (1, 64, 128, 32768, 16, 0)])
+def test_thresholds_with_the_scan_beside_the_norms(B, H, M, N, D, yes):
+    from forgetting_transformer.ops import _lib
+    got = C.c_int32(-1)
+    _lib.check(_lib.load().fox_auto_threshold_scan_one_launch(C.byref(_lib.Dims(B, H, M, N, D, 0)), C.byref(got)), "fox_auto_threshold_scan_one_launch")
+    assert got.value == yes
