@@ -574,7 +574,7 @@ int fox_attn_decode_counters(const fox_dims* dims, int32_t* counters) {
   FOX_TRY(check_dims(dims));
   if (!counters) return fail(FOX_E_ARG, "counters is NULL");
   if (dims->M != 1) return fail(FOX_E_ARG, "fox_attn_decode takes one query row (M = %d)", dims->M);
-  *counters = fox::decode_merges(dims->B, dims->H, fox::decode_splits(dims->B, dims->H, dims->N, dims->D)) ? dims->B * dims->H : 0;
+  *counters = fox::decode_merges(dims->B, dims->H, dims->N, dims->D, fox::decode_splits(dims->B, dims->H, dims->N, dims->D)) ? dims->B * dims->H : 0;
   return FOX_OK;
 }
 
@@ -613,7 +613,7 @@ int fox_attn_decode_counted(const fox_fwd_args* args, const float* g, int64_t g_
       k.splits = fox::decode_splits(k.B, k.H, k.N, args->dims.D);
       k.ws_o = (float*)args->workspace;
       k.ws_p = (fox::DecodePartial*)(k.ws_o + (int64_t)k.splits * k.B * k.H * args->dims.D);   // (D is a multiple of 4: 16-byte aligned)
-      if (fox::decode_merges(k.B, k.H, k.splits)) k.arrived = arrived;
+      if (fox::decode_merges(k.B, k.H, k.N, args->dims.D, k.splits)) k.arrived = arrived;
     }
   }
   k.by_splits = fox::divisor(k.splits);

@@ -529,11 +529,17 @@ int decode_splits(int B, int H, int N, int D) {
   return splits < 1 ? 1 : (int)splits;
 }
 
-// Whether the split that arrives last merges the others, where there are counters.  The kernels take no less time that way (partials past the L2, a
-// counter, partials back: three round trips to memory against a launch boundary), but the call is a launch shorter: us of GPU / of host time, two
-// launches and one: B1 H12 N1500 D64 8.0 / 9.1 and 8.4 / 4.6, B1 H1 N5000 D128 7.8 / 9.2 and 9.0 / 4.8.  A generation step of one user waits for the host.  With more
-// workgroups than CUs the step is the GPU's, and the round trips add up: B4 H12 N3000 D64 11.3 and 12.4, B1 H16 N8000 D128 14.6 and 25.9.
-bool decode_merges(int B, int H, int splits) { return splits > 1 && (int64_t)B * H * splits <= kCus; }
+// Whether the split that arrives last merges the others, where there are counters.  The kernels take longer that way (partials past the L2, a counter,
+// partials back: three round trips to memory against a launch boundary), but the call is a launch and 4.5 us of host time shorter, and a generation step of one
+// user waits for the host.  GPU, two launches / one, us: B1 H12 N1500 D64 8.0 / 8.3, B1 H4 N8192 D128 8.3 / 11.5, with more workgroups than CUs B4 H12 N3000 D64
+// 11.0 / 12.2, B1 H16 N8000 D128 14.1 / 26.2.  A token, cache append and attention call: B1 H12 N1200 D64 14.2 / 12.3, H2 N32000 14.3 / 13.3, D128 H12 N2000
+// 14.7 / 13.6, H4 N8000 14.2 / 14.2, H1 N16000 14.6 / 13.4.  Where the splits have several batches of keys a wave the step is the GPU's again: D128 H1
+// N24000 14.4 / 14.4, H4 N12000 14.3 / 14.9, H4 N24000 15.4 / 17.7, D64 H4 N32000 14.4 / 14.8.  (Calls back to back with nothing between them are the GPU's
+// as well: up to 0.5 us more at head dims up to 64 with few workgroups, 1 to 3 us at 128.)
+bool decode_merges(int B, int H, int N, int D, int splits) {
+  const int64_t wgs = (int64_t)B * H * splits, batches = decode_batches(N, D);
+  return splits > 1 && wgs <= kCus && (batches <= kDecodeMaxSplits || (2 * wgs <= kCus && batches <= 2 * kDecodeMaxSplits));
+}
 
 // ---------------------------------------------------------------------------
 // New tokens into a layer's cache: keys, values and log gates in one launch.  One 16-byte piece of K and the same piece of V per

@@ -105,7 +105,9 @@ def test_grids_that_form_their_own_sums(B, H, M, N, D, pruned, yes):
 
 
 @pytest.mark.parametrize("B,H,N,D,counters", [(1, 12, 1500, 64, 12), (1, 64, 1000, 64, 64), (1, 64, 1200, 64, 0), (1, 4, 8192, 128, 4), (1, 5, 8192, 128, 0), (1, 5, 700, 32, 0),
-                                              (1, 128, 600, 64, 0), (1, 128, 1500, 16, 128), (1, 129, 1500, 16, 0), (16, 16, 32768, 128, 0)])
+                                              (1, 128, 600, 64, 0), (1, 128, 1500, 16, 128), (1, 129, 1500, 16, 0), (16, 16, 32768, 128, 0),
+                                              # several batches of keys a wave: up to two, and with half a chip of workgroups
+                                              (1, 4, 8193, 128, 0), (1, 2, 8193, 128, 2), (1, 2, 16384, 128, 2), (1, 1, 16385, 128, 0), (1, 2, 32768, 64, 2), (1, 3, 32768, 64, 0)])
 def test_counters_of_a_generation_step(B, H, N, D, counters):
     from forgetting_transformer.ops import _lib
     got = C.c_int32(-1)
