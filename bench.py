@@ -201,9 +201,11 @@ def event_time(fn, iters, warmup=2):
     return start.elapsed_time(end) * 1e-3 / iters
 
 
-def stage_times(w, tensors, iters, threshold=None):
+def stage_times(w, tensors, iters, threshold=None, joined=False):
     """Time every kernel of the path alone through the C ABI (launches go to torch's current stream).
-    threshold: optional pruning threshold, a float applied to every (batch, head) or a (B, H) fp32 tensor."""
+    threshold: optional pruning threshold, a float applied to every (batch, head) or a (B, H) fp32 tensor.
+    joined: also what the operator runs in place of several of them where the shape is small: `fwd_gates`, the forward that
+    forms the cumulative sums itself, and `bwd`, dQ and dK/dV as one launch with the scan behind it."""
     from forgetting_transformer.ops import _lib
     from forgetting_transformer.ops.forgetting_attention import _view
 
@@ -255,6 +257,12 @@ def stage_times(w, tensors, iters, threshold=None):
     scan()
     out["cumsum_fwd"] = event_time(scan, iters)
     out["fwd"] = event_time(f, iters)
+    yes = C.c_int32(0)
+    if joined:
+        _lib.check(lib.fox_attn_fwd_takes_gates(C.byref(dims), thr is not None, C.byref(yes)), "takes gates")
+        if yes.value:
+            gates = _lib.Gates(log_fgate.data_ptr(), 0, _lib.DTYPE_FP32, *log_fgate.stride(), None)
+            out["fwd_gates"] = event_time(lambda: _lib.check(lib.fox_attn_fwd_gates(C.byref(fwd), C.byref(gates), None, stream), "fwd gates"), iters)
     if w["fwd_only"]:
         return out
     delta = torch.empty((2,) + tuple(lse.shape), dtype=torch.float32, device=dev)
@@ -268,6 +276,10 @@ def stage_times(w, tensors, iters, threshold=None):
         out[name] = event_time(lambda fn=fn, name=name: _lib.check(fn(C.byref(bwd), stream), name), iters)
     out["cumsum_bwd"] = event_time(
         lambda: _lib.check(lib.fox_cumsum_bwd(dc.data_ptr(), dg.data_ptr(), 0, 0, 0, None, B, H, N, stream), "cumsum_bwd"), iters)
+    if joined:
+        _lib.check(lib.fox_attn_bwd_one_launch(C.byref(bwd), C.byref(yes)), "one launch")
+        if yes.value:
+            out["bwd"] = event_time(lambda: _lib.check(lib.fox_attn_bwd(C.byref(bwd), stream), "bwd"), iters)
     return out
 
 
@@ -496,7 +508,7 @@ def head_dim_report(steps, warmup, name="c3d64"):
 def small_shape_report(steps, warmup):
     """The library-example shape (B4 T512 H12 D64 bf16 fwd+bwd): launch-latency-bound.  Wall time per step of the
     operator (Python, autograd, allocations, launches), the same step replayed from a HIP graph, and the sum of
-    its kernels timed alone."""
+    the launches it consists of, timed alone."""
     from forgetting_transformer import forgetting_attention
 
     w = WORKLOADS["c2"]
@@ -509,8 +521,8 @@ def small_shape_report(steps, warmup):
         q.grad = k.grad = v.grad = log_fgate.grad = None
     t = time_steps(step, max(steps, 300), max(warmup, 30))
     t_graph = graph_time(step, max(steps, 300))
-    st = stage_times(w, tensors, max(steps, 20))
-    path = ("cumsum_fwd", "fwd", "bwd_dq", "bwd_dkdv", "cumsum_bwd")
+    st = stage_times(w, tensors, max(steps, 20), joined=True)
+    path = (("fwd_gates",) if "fwd_gates" in st else ("cumsum_fwd", "fwd")) + (("bwd",) if "bwd" in st else ("bwd_dq", "bwd_dkdv", "cumsum_bwd"))
     return {"workload": "B4 T512 H12 D64 bf16 fwd+bwd, gate logits N(0,1)", "wall_ms_per_step": t * 1e3,
             "graph_replay_ms_per_step": t_graph * 1e3, "kernel_sum_ms": sum(st[n] for n in path) * 1e3,
             "kernels_ms": {n: st[n] * 1e3 for n in path}}
