@@ -8,10 +8,12 @@
 //                  registers as MFMA B operands; dK^T, dV^T accumulators) and
 //                  walks the query tiles below its diagonal; writes dk, dv and
 //                  dc[n] = drow[n - (N - M)] - sum_i dS[i,n].
-//                  With BOTH the launch holds the workgroups of either kernel, for small grids (bwd_together).
+//   dq_kernel with BOTH : the workgroups of either kind in one launch, for small
+//                  grids (bwd_together); dc then lacks drow, which the reverse
+//                  scan behind it adds (fox_scan.hip).
 //   delta_kernel : delta alone (a stage of its own for callers that want it;
 //                  the backward does not launch it).
-// Every kernel only stores: no read-modify-write of anything another kernel wrote,
+// Every kernel here only stores: no read-modify-write of anything another kernel wrote,
 // so a stage may be repeated or timed alone without changing the result.
 //
 // Probabilities are rebuilt from the stored log-normaliser:

@@ -286,7 +286,7 @@ __device__ __forceinline__ void decode_merge(const DecodeK& a, int bh) {
 // The score of key n needs the sum of the gates behind it, not the two ends of a sum from the row's start.  Every wave owns
 // a contiguous run of keys, walks it from its end and carries that sum (fp64, rounded once per key) relative to the end of
 // its own run; the runs' totals then shift the partial maxima where partials are merged: four waves in LDS, splits in
-// decode_combine_kernel.  A gate is read once, by the wave that reads its key; the row scan this replaces (one workgroup per
+// decode_merge, by the one that arrives last or in a launch of its own.  A gate is read once, by the wave that reads its key; the row scan this replaces (one workgroup per
 // row, a chain of barriers per 8192 keys) took 20 us of a 600 us step at B16 H16 N32768 D128 and 5.7 us of 36 at
 // B1 H12 N1500 D64.  Bound by HBM where the cache is long, by one round trip per batch where it is short.
 template <typename Tr, int D, int WAVES>
