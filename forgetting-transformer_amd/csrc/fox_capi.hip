@@ -407,9 +407,10 @@ int fox_attn_fwd_gates(const fox_fwd_args* args, const fox_gates* gates, const f
   if (!args) return fail(FOX_E_ARG, "args is NULL");
   if (epi) FOX_TRY(check_epilogue(args, epi));
   FOX_TRY(check_gates(gates));
-  int32_t yes = 0;
-  FOX_TRY(fox_attn_fwd_takes_gates(&args->dims, args->threshold != nullptr, &yes));
-  if (!yes) return fail(FOX_E_ARG, "fox_attn_fwd_gates does not take this shape (fox_attn_fwd_takes_gates)");
+  FOX_TRY(check_dims(&args->dims));
+  const fox_dims& d = args->dims;
+  if (!fox::fwd_can_scan(d.B, d.H, d.M, d.N, plan_fwd(d, args->threshold != nullptr, true).splits))
+    return fail(FOX_E_ARG, "fox_attn_fwd_gates does not take this shape (fox_attn_fwd_takes_gates)");
   return fwd_impl(args, nullptr, 0, stream, "fox_attn_fwd_gates", epi, gates);
 }
 

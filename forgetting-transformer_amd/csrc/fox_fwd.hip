@@ -857,6 +857,12 @@ hipError_t launch_fwd_gates(const FwdK& a, int D, int dtype, hipStream_t s) {
   return dtype == 0 ? launch_fwd_gates_t<Bf16>(a, D, s) : launch_fwd_gates_t<Fp16>(a, D, s);
 }
 
+// What fox_attn_fwd_gates accepts.
+bool fwd_can_scan(int B, int H, int M, int N, int splits) {
+  const int64_t wgs = (int64_t)((M + kFwdBM - 1) / kFwdBM) * B * H;
+  return M > 1 && splits <= 1 && N <= kOwnScanMaxKeys && wgs <= (N <= 1024 ? 4 : 2) * kCus;
+}
+
 // Whether the forward forms the cumulative sums itself (fwd_scan_kernel) instead of reading what a scan left.  The scan is a launch and
 // 3 to 6 us of one workgroup per row; own sums cost a workgroup 1 to 2 us, most of it while its first tiles arrive, but every workgroup.
 // Forward with its scan / with own sums, us, on inputs that the caches hold; on fresh ones the gates of (B, T, H) memory, a line per token and workgroup,
@@ -872,10 +878,9 @@ hipError_t launch_fwd_gates(const FwdK& a, int D, int dtype, hipStream_t s) {
 // - Beyond that every round repeats the sums: B8 H12 N2048 D64 70.6 / 71.4, B16 H16 N3500 475 / 499.
 bool fwd_scans(int B, int H, int M, int N, int D, bool pruned, int splits) {
   const int64_t pairs = (int64_t)B * H, tiles = (M + kFwdBM - 1) / kFwdBM, wgs = tiles * pairs;
-  if (M <= 1 || splits > 1 || N > kOwnScanMaxKeys) return false;
+  if (!fwd_can_scan(B, H, M, N, splits)) return false;
   if (tiles > 1 && M < N && wgs * (2 * (int64_t)N - M) > 2 * 2900 * kCus) return false;
   if (wgs <= 2 * kCus) return pruned || D > 64 || N <= 1024 || 4 * wgs <= 5 * kCus || pairs < 24;
-  if (wgs > 4 * kCus || N > 1024) return false;
   return pruned || N <= 384 || (D <= 64 && 2 * wgs <= 7 * kCus);
 }
 

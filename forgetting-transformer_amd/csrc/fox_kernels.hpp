@@ -268,6 +268,7 @@ __host__ __device__ __forceinline__ BothTile both_tile(int t, int key_tiles, int
 
 hipError_t launch_fwd(const FwdK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_fwd_gates(const FwdK& a, int D, int dtype, hipStream_t s);   // unsplit, at most kOwnScanMaxKeys keys, M > 1
+bool fwd_can_scan(int B, int H, int M, int N, int splits);
 bool fwd_scans(int B, int H, int M, int N, int D, bool pruned, int splits);
 int fwd_key_splits(int B, int H, int M, int N, int D);
 bool fwd_pairs(int B, int H, int M, int N, int D, bool pruned, int splits);

@@ -399,8 +399,8 @@ int fox_attn_fwd_norm_gate(const fox_fwd_args* args, const fox_fwd_epilogue* epi
 /*
  * The forward straight from the gates: what fox_cumsum_fwd or fox_gate_cumsum_fwd followed by fox_attn_fwd or, with an epilogue,
  * fox_attn_fwd_norm_gate compute, in one launch.  Of args, log_lambda is written (NULL = not wanted) and the workspace is not used.
- * For the shapes that fox_attn_fwd_takes_gates names only, FOX_E_ARG otherwise: every workgroup repeats the sum of the gates in front of its
- * rows, which pays for short rows and small grids.
+ * Every workgroup repeats the sum of the gates in front of its rows, which pays for short rows and small grids: fox_attn_fwd_takes_gates names the
+ * shapes for which this is the faster way, and all of those are taken.  Others may be refused with FOX_E_ARG.
  */
 typedef struct fox_gates {
   const void* g;                         /* (B,H,N): fp32 log forget gates, or their logits */

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 DTYPES = {None: 2, torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
 
-def _both(B, H, M, N, D, dtype, thr, seq, logit, strided):
+def _both(B, H, M, N, D, dtype, thr, seq, logit, strided, faster=1):
     from forgetting_transformer.ops import _lib
     from forgetting_transformer.ops.forgetting_attention import _view
     lib = _lib.load()
@@ -27,7 +27,7 @@ def _both(B, H, M, N, D, dtype, thr, seq, logit, strided):
     stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
     yes, need = C.c_int32(-1), C.c_int64(0)
     _lib.check(lib.fox_attn_fwd_takes_gates(C.byref(dims), thr is not None, C.byref(yes)), "takes_gates")
-    assert yes.value == 1
+    assert yes.value == faster
     _lib.check(lib.fox_attn_fwd_workspace_bytes(C.byref(dims), C.byref(need)), "workspace")
     ws = torch.empty(max(need.value, 16), dtype=torch.uint8, device="cuda")
     t = None if thr is None else torch.full((B, H), thr, device="cuda")
@@ -70,6 +70,11 @@ def test_against_the_scan(N, M, D, dtype):
 def test_from_logits_and_pruned(B, H, M, N, D, logit, thr):
     _both(B, H, M, N, D, torch.bfloat16, thr, None, logit, True)
     _both(B, H, M, N, D, torch.bfloat16, thr, [min(n, N) for n in range(0, 97 * B, 97)], None, False)
+
+
+@pytest.mark.parametrize("B,H,M,N,D,thr", [(8, 32, 130, 1600, 64, None), (2, 16, 2048, 2048, 64, None), (8, 24, 500, 500, 128, None), (8, 32, 130, 3500, 64, -10.0)])
+def test_shapes_it_takes_where_a_scan_is_faster(B, H, M, N, D, thr):
+    _both(B, H, M, N, D, torch.bfloat16, thr, None, None, True, faster=0)
 
 
 def test_shapes_it_does_not_take():
