@@ -560,7 +560,7 @@ __global__ __launch_bounds__(256, (D <= 64 || DSPLIT) ? 2 : 1) void dkdv_kernel(
   __shared__ __align__(16) float dl_s1[BMQ];
 #ifdef __HIP_DEVICE_COMPILE__
   int bh, nt;
-  decode_block(blockIdx.x, a.order, false, bh, nt);
+  decode_block(block_id(a), a.order, false, bh, nt);
   nt = a.n_tiles - 1 - nt;  // the first key tiles see the most query rows: start them first
   dkdv_body<Tr, D, DSPLIT, false>(a, bh, nt, {q_tile0, q_tile1, do_tile0, do_tile1, rc_s0, rc_s1, dl_s0, dl_s1});
 #endif
@@ -651,7 +651,7 @@ __global__ __launch_bounds__(256, 2) void dq_kernel(const BwdK args) {
     }
     mt = w.tile;
   } else {
-    decode_block(blockIdx.x, args.order, args.last_first, bh, mt);
+    decode_block(block_id(args), args.order, args.last_first, bh, mt);
   }
   const BwdK& a = BOTH ? own_arguments() : args;
 
