@@ -926,14 +926,15 @@ hipError_t launch_bwd_dkdv(const BwdK& a, int D, int dtype, hipStream_t s) {
 // - Long rows.  The reverse scan of few long rows is a chain that the row sums make longer, and under a threshold walks are short and have little to overlap,
 //   so that the grid has to leave room: D 64 at -10, T4096 with 320 tiles 53.5 / 53.1, 384 55.2 / 56.1, 448 57.3 / 59.1, 512 55.6 / 59.2; T16384 with 256 59.2 / 57.4,
 //   384 60.8 / 65.4, 512 68.1 / 76.0; D 32 T16384 with 256 51.7 / 49.3, 512 61.3 / 64.8.  Rows up to 2048 (D 64) and 8192 are past that: B2 H12 T2048 48.5 / 47.7,
-//   D 32 B1 H12 T8192 68.0 / 66.8.  Without a threshold D 64 T4096 gains with 448 tiles, 221 / 195, not with 512, 226 / 230 (T16384 818 / 833); D 32 gains with 768, 805 / 747.
+//   D 32 B1 H12 T8192 68.0 / 66.8.  Without a threshold D 64 gains until both kinds fill the chip to the last
+//   place: 480 tiles B3 H5 T4000 222 / 197, 510 B1 H10 T6500 346 / 311, 504 B1 H8 T8000 405 / 396, 512 B1 H16 T4000 225 / 223 and 226 / 230, H4 T16384 818 / 833; D 32 gains with 768, 805 / 747.
 //   Where M < N the tiles of both kinds count: B1 H16 M300 N4096 at -10 (560 of them) 52.4 / 47.7.
 bool bwd_together(const BwdK& a, int D) {
   if (D > 64 || a.o.st <= 0 || ((int64_t)kKvBM * a.o.st + D) * 2 >= (int64_t)1 << 31) return false;   // o through 32-bit offsets
   const int64_t pairs = (int64_t)a.B * a.H, keys = pairs * ((a.N + kKvBN - 1) / kKvBN), both = keys + pairs * ((a.M + kFwdBM - 1) / kFwdBM);
   if (keys > (D == 64 ? 2 : 3) * kCus) return false;
   if (a.N <= (D == 64 ? 2048 : 8192)) return true;
-  return a.thr ? 2 * both <= 5 * kCus : D < 64 || 2 * both <= 7 * kCus;
+  return a.thr ? 2 * both <= 5 * kCus : D < 64 || both < 4 * kCus;
 }
 hipError_t launch_bwd(const BwdK& a, int D, int dtype, hipStream_t s) {
   return dtype == 0 ? bwd_t<Bf16>(a, D, s) : bwd_t<Fp16>(a, D, s);

@@ -76,7 +76,7 @@ def test_launch_order_without_divisions(tmp_path):
     (4, 12, 512, 512, 64, False, 1), (2, 32, 1000, 1000, 64, True, 1), (2, 16, 2048, 2048, 64, True, 1), (16, 16, 257, 257, 64, False, 0), (1, 1, 100, 100, 128, False, 0),
     (3, 32, 1000, 1000, 32, True, 1), (1, 6, 16384, 16384, 16, False, 1), (49, 16, 100, 100, 32, False, 0), (48, 16, 100, 100, 32, True, 1),
     # long rows: room on the chip, more of it under a threshold
-    (1, 10, 4096, 4096, 64, True, 1), (1, 11, 4096, 4096, 64, True, 0), (1, 14, 4096, 4096, 64, False, 1), (1, 15, 4096, 4096, 64, False, 0),
+    (1, 10, 4096, 4096, 64, True, 1), (1, 11, 4096, 4096, 64, True, 0), (1, 15, 4096, 4096, 64, False, 1), (1, 16, 4096, 4096, 64, False, 0),
     (1, 2, 16384, 16384, 32, True, 1), (1, 4, 16384, 16384, 32, True, 0), (1, 12, 8192, 8192, 32, True, 1),
     (1, 16, 300, 4096, 64, True, 1), (1, 16, 2048, 4096, 64, True, 0), (1, 16, 2048, 4096, 64, False, 1)])
 def test_grids_of_the_one_launch_backward(B, H, M, N, D, pruned, yes):
