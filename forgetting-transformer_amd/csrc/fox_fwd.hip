@@ -350,7 +350,7 @@ __device__ __forceinline__ void fwd_body(const FwdK& a) {   // a: the kernel's o
     mt = divide(mts, a.by_splits);
     sp = mts - mt * a.splits;
   } else {
-    decode_block(PAIR ? blockIdx.x : block_id(a), a.order, false, bh, mt);
+    decode_block(PAIR || SCAN ? blockIdx.x : block_id(a), a.order, false, bh, mt);
   }
   const int b = divide(bh, a.order.by_heads), h = bh - b * a.H;
   const int M = a.M, N = a.N, p_seq = N - M;

@@ -255,7 +255,8 @@ __host__ __device__ __forceinline__ void decode_block(uint32_t wid, const BlockO
 
 // blockIdx.x, once the lines of the argument block that a kernel opens with are there.  Left to the compiler the order's operands are loaded first and the
 // sizes only where they are needed, a round trip to memory further on, which a short walk notices (sizes later / together: dQ B1 H8 T2870 D128 68.4 / 67.5 us, B2 H3 T3000
-// 71.2 / 70.2, forward B1 H8 T7200 D64 at -10 12.1 / 11.8).  Not in the paired and the split forward, which lose by it (B2 H3 T1794 D128 25.1 / 25.5).
+// 71.2 / 70.2, forward B1 H8 T7200 D64 at -10 12.1 / 11.8).  Not in the paired and the split forward and the one with its own sums, which lose by
+// it (B2 H3 T1794 D128 25.1 / 25.5, B1 H12 T77 D64 6.5 / 6.6).
 template <typename K>
 __device__ __forceinline__ uint32_t block_id(const K& a) {
   uint32_t id = blockIdx.x;
