@@ -566,7 +566,7 @@ int fox_attn_decode_workspace_bytes(const fox_dims* dims, int64_t* bytes) {
   FOX_TRY(check_dims(dims));
   if (!bytes) return fail(FOX_E_ARG, "bytes is NULL");
   if (dims->M != 1) return fail(FOX_E_ARG, "fox_attn_decode takes one query row (M = %d)", dims->M);
-  const int splits = fox::decode_splits(dims->B, dims->H, dims->N, dims->D);
+  const int splits = fox::decode_splits(dims->B, dims->H, dims->N, dims->D, true);   // (never fewer than without seq_start)
   *bytes = splits <= 1 ? 0 : (int64_t)splits * dims->B * dims->H * (int64_t)(dims->D * sizeof(float) + sizeof(fox::DecodePartial));
   return FOX_OK;
 }
@@ -575,7 +575,7 @@ int fox_attn_decode_counters(const fox_dims* dims, int32_t* counters) {
   FOX_TRY(check_dims(dims));
   if (!counters) return fail(FOX_E_ARG, "counters is NULL");
   if (dims->M != 1) return fail(FOX_E_ARG, "fox_attn_decode takes one query row (M = %d)", dims->M);
-  *counters = fox::decode_merges(dims->B, dims->H, dims->N, dims->D, fox::decode_splits(dims->B, dims->H, dims->N, dims->D)) ? dims->B * dims->H : 0;
+  *counters = fox::decode_merges(dims->B, dims->H, dims->N, dims->D, fox::decode_splits(dims->B, dims->H, dims->N, dims->D, true)) ? dims->B * dims->H : 0;
   return FOX_OK;
 }
 
@@ -611,7 +611,7 @@ int fox_attn_decode_counted(const fox_fwd_args* args, const float* g, int64_t g_
     if (need > 0) {
       if (args->workspace_bytes < need) return fail(FOX_E_ARG, "workspace too small: %lld < %lld bytes", (long long)args->workspace_bytes, (long long)need);
       if (((uintptr_t)args->workspace & 15) != 0) return fail(FOX_E_ALIGN, "workspace must be 16-byte aligned");
-      k.splits = fox::decode_splits(k.B, k.H, k.N, args->dims.D);
+      k.splits = fox::decode_splits(k.B, k.H, k.N, args->dims.D, args->seq_start != nullptr);
       k.ws_o = (float*)args->workspace;
       k.ws_p = (fox::DecodePartial*)(k.ws_o + (int64_t)k.splits * k.B * k.H * args->dims.D);   // (D is a multiple of 4: 16-byte aligned)
       if (fox::decode_merges(k.B, k.H, k.N, args->dims.D, k.splits)) k.arrived = arrived;

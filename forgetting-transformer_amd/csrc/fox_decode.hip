@@ -517,16 +517,30 @@ hipError_t launch_decode_gates(const DecodeK& a, int D, int dtype, hipStream_t s
   return dtype == 0 ? launch_decode_gates_t<Bf16>(a, D, s) : launch_decode_gates_t<Fp16>(a, D, s);
 }
 
-// Splits of launch_decode_gates: about eight workgroups per CU, but no wave with less than a whole batch of keys (16 KiB of K and V):
-// a step over a short cache is a chain of round trips, one per batch a wave walks.  B1 H12 N1500 D64: two splits 7.9 us
-// (three batches a wave), six 4.6.
-int decode_splits(int B, int H, int N, int D) {
-  const int64_t bh = (int64_t)B * H, batches = decode_batches(N, D);
-  if (decode_one_workgroup(bh, batches, D)) return 1;
-  int64_t splits = (2048 + bh - 1) / bh;
-  splits = splits > batches ? batches : splits;
-  splits = splits > kDecodeMaxSplits ? kDecodeMaxSplits : splits;
-  return splits < 1 ? 1 : (int)splits;
+// Splits of launch_decode_gates: about eight workgroups per CU, a wave's run being a whole number `per` of batches of keys, and as many splits as the runs of a row without
+// padding need.  (More than that are not just idle: consecutive workgroups go round the XCDs, so with twelve of sixteen splits in use four of the eight XCDs got two
+// thirds of the rows.)  us, 2048 workgroups whatever the row / now:
+// - A run of a few batches: the number with which the CUs get the most even share of them, one batch a wave where that is no worse, so that no wave waits for its second.
+//   D 128, 128 pairs N3000 41.6 / 35.0 (twelve splits of two batches 36.1), 64 pairs N5000 32.6 / 29.7, D 64, 128 pairs N5000 33.2 / 29.0.
+// - One split, and no merge, where every CU, or three of four, has one pair, or all have nearly the same number: one workgroup a CU asks for as much as the memory gives.
+//   D 128, 192 pairs N1700 31.3 / 28.9, N32768 491 / 448, 256 pairs N1700 42.9 / 35.6, N15000 298 / 286, D 64, 512 pairs N500 13.7 / 10.5, N15000 301 / 289.  128 pairs
+//   N24000 (243 / 295) and 320 (582 / 688) lose, and so do 192 pairs of head dims below 64 (D 16 N15000 36.5 / 41.1).  Not with padding, which differs from row to row: the longest row would be left to one CU.
+// - With padding the rows' own lengths decide what a split gets, and the number is not made even (D 128, 128 pairs N15000, padded by up to all of it, 16 / 15 splits 90.8 / 95.0).
+// - With padding, long rows of many pairs: half as many workgroups; they start and end less often, and are still few batches of the whole (D 128, 256 pairs N32768, padded
+//   by up to a quarter 577 / 567, by up to all of it 398 / 372; shorter rows lose the balance: N5000 54.9 / 56.7, 512 pairs N5000 99 / 104).
+int decode_splits(int B, int H, int N, int D, bool padded) {
+  const int64_t bh = (int64_t)B * H, batches = decode_batches(N, D), rounds = (bh + kCus - 1) / kCus;
+  if (batches <= 1 || decode_one_workgroup(bh, batches, D)) return 1;
+  if (!padded && (bh <= kCus && D >= 64 ? 4 * bh >= 3 * kCus : 10 * bh >= 9 * rounds * kCus)) return 1;
+  const int64_t most = batches < kDecodeMaxSplits ? batches : kDecodeMaxSplits;
+  const int64_t wgs = padded && bh >= kCus && batches >= 128 ? 4 * kCus : 8 * kCus, even = (wgs + bh - 1) / bh, splits = even < most ? even : most;
+  int64_t per = (batches + splits - 1) / splits;
+  auto runs = [&](int64_t p) { return (batches + p - 1) / p; };
+  auto heaviest = [&](int64_t p) { return p * ((bh * runs(p) + kCus - 1) / kCus); };   // CU's share, in batches a wave
+  if (per <= 4)
+    for (int64_t p = per - 1; p >= 1 && runs(p) <= most && bh * runs(p) <= 16 * kCus; --p)
+      if (heaviest(p) < heaviest(per) || (p == 1 && heaviest(p) == heaviest(per))) per = p;
+  return (int)(padded && per > 1 ? splits : runs(per));
 }
 
 // Whether the split that arrives last merges the others, where there are counters.  The kernels take longer that way (partials past the L2, a counter,

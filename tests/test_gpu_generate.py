@@ -49,6 +49,19 @@ def test_single_query_behind_a_closed_gate(ft, N, at):
     assert_parity("out", out, ref)
 
 
+# how many splits a row is cut into (decode_splits): 192 pairs are the fewest that go without a merge, 191 and 257 are not enough and too many, 461 and 512
+# fill the CUs twice; one batch of keys a wave or several; with padding, which never goes without
+@pytest.mark.parametrize("B,H,N,D", [(1, 191, 700, 128), (1, 192, 700, 128), (16, 16, 1409, 64), (1, 257, 641, 128), (1, 460, 700, 64), (1, 461, 700, 64), (4, 128, 520, 128),
+                                     (3, 16, 2049, 128), (3, 16, 9000, 16), (8, 12, 2300, 64)])
+@pytest.mark.parametrize("padded", [False, True])
+def test_single_query_splits(ft, B, H, N, D, padded):
+    ss = [(N * i) // B for i in range(B)] if padded else None
+    q, k, v, g, _, ss = make_inputs(B, H, 1, N, D, device="cuda", head_first=True, seq_start=ss, seed=N + H, gate_mean=2.0)
+    with torch.no_grad():
+        out = ft.forgetting_attention(q, k, v, g, head_first=True, seq_start=ss)
+    assert_parity("out", out, O.forgetting_attention_ref(q, k, v, g, head_first=True, seq_start=ss))
+
+
 # one workgroup of sixteen waves takes a (batch, head) whole: two batches of keys with few heads, up to four with many, and
 # the first sizes beyond
 @pytest.mark.parametrize("B,H,N,D", [(2, 3, 257, 64), (2, 3, 512, 64), (2, 3, 513, 64), (1, 3, 129, 128), (2, 2, 2048, 16), (2, 2, 600, 32),
