@@ -309,40 +309,65 @@ __global__ void zero_u32_kernel(uint32_t* p, int n) {
   if (i < n) p[i] = 0u;
 }
 
-// One workgroup: rows block * 512 .. of q (which = 0, T = M) or of k (which = 1, T = N) of one (batch, head), `blocks` workgroups each.  scratch holds, per (batch, head), the two
+// The threshold from the largest norms; every tensor op of the reference rounds to the input dtype.
+template <typename Tr>
+__device__ __forceinline__ float threshold_of_norms(float qn, float kn, float sm_scale, float log_n) {
+  float ub = round16<Tr>(qn * kn);
+  ub = round16<Tr>(ub * sm_scale);
+  float th = round16<Tr>(2.f * ub);
+  th = round16<Tr>(th + log_n);
+  th = -th;
+  return round16<Tr>(th - 10.f);
+}
+// Norm of a row of which this lane holds eight elements, its D / 8 lanes the others.
+template <typename Tr, int LPR>
+__device__ __forceinline__ float row_norm(const u32x4& x) {
+  float acc = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc += Tr::lo(x[e]) * Tr::lo(x[e]) + Tr::hi(x[e]) * Tr::hi(x[e]);
+#pragma unroll
+  for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
+  return round16<Tr>(sqrtf(acc));
+}
+__device__ __forceinline__ float wave_max(float x) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) x = fmaxf(x, __shfl_xor(x, off));
+  return x;
+}
+
+// Workgroup `id` of those of all q, w.q_blocks for each (batch, head), and then of all k: kNormRows rows of one of them.  scratch holds, per (batch, head), the two
 // running maxima (float bits) and the number of workgroups that have added theirs; the workgroup that arrives last
 // turns the maxima into the threshold, so no kernel of its own is needed for that.
+constexpr int kNormRows = 512;
+struct NormBlocks {
+  int pairs, q_blocks, k_blocks;
+  Divisor by_q, by_k, by_heads;
+};
 template <typename Tr, int D>
 __device__ __forceinline__ void norm_max(const View& q, const View& k, int H, int M, int N, uint32_t* scratch, float* thr, float sm_scale,
-                                         float log_n, int block, int blocks, int bh, int which) {
-  constexpr int LPR = D / 8, RPP = 256 / LPR, ROWS = 512;
+                                         float log_n, int id, const NormBlocks& w) {
+  constexpr int LPR = D / 8, RPP = 256 / LPR;
   const int tid = threadIdx.x;
-  const int b = bh / H, h = bh % H;
-  const View& t = which == 0 ? q : k;
-  const int T = which == 0 ? M : N;
+  const int which = id >= w.pairs * w.q_blocks;   // 1: k
+  if (which) id -= w.pairs * w.q_blocks;
+  const int bh = divide(id, which ? w.by_k : w.by_q), block = id - bh * (which ? w.k_blocks : w.q_blocks), b = divide(bh, w.by_heads), h = bh - b * H;
+  const View& t = which ? k : q;
+  const int T = which ? N : M;
   const uint16_t* p = t.ptr + b * t.sb + h * t.sh;
   const int ch = tid % LPR;
   float best = 0.f;
-  constexpr int U = (ROWS / RPP) < 8 ? (ROWS / RPP) : 8;  // rows in flight per thread
-  for (int pass = 0; pass < ROWS / RPP; pass += U) {
+  constexpr int U = (kNormRows / RPP) < 8 ? (kNormRows / RPP) : 8;  // rows in flight per thread
+  for (int pass = 0; pass < kNormRows / RPP; pass += U) {
     u32x4 x[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int row = min(block * ROWS + (pass + u) * RPP + tid / LPR, T - 1);  // rows past the end repeat the last one
+      const int row = min(block * kNormRows + (pass + u) * RPP + tid / LPR, T - 1);  // rows past the end repeat the last one
       x[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + (int64_t)row * t.st + ch * 8));
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      float acc = 0.f;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc += Tr::lo(x[u][e]) * Tr::lo(x[u][e]) + Tr::hi(x[u][e]) * Tr::hi(x[u][e]);
-#pragma unroll
-      for (int off = LPR / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-      best = fmaxf(best, round16<Tr>(sqrtf(acc)));
-    }
+    for (int u = 0; u < U; ++u) best = fmaxf(best, row_norm<Tr, LPR>(x[u]));
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) best = fmaxf(best, __shfl_xor(best, off));
+  best = wave_max(best);
   __shared__ float wave_best[4];
   if ((tid & 63) == 0) wave_best[tid >> 6] = best;
   __syncthreads();
@@ -355,33 +380,61 @@ __device__ __forceinline__ void norm_max(const View& q, const View& k, int H, in
   const uint32_t before = atomicMax(&mine[which], __float_as_uint(best));
   uint32_t one = 1u;
   asm volatile("" : "+v"(one) : "v"(before));
-  if (atomicAdd(&mine[2], one) != (uint32_t)blocks * 2u - 1u) return;
+  if (atomicAdd(&mine[2], one) != (uint32_t)(w.q_blocks + w.k_blocks) - 1u) return;
   // the last workgroup of this (batch, head): every maximum has been added (read through the atomic unit as well)
   const float qn = __uint_as_float(atomicMax(&mine[0], 0u)), kn = __uint_as_float(atomicMax(&mine[1], 0u));
-  // every tensor op of the reference rounds to the input dtype
-  float ub = round16<Tr>(qn * kn);
-  ub = round16<Tr>(ub * sm_scale);
-  float th = round16<Tr>(2.f * ub);
-  th = round16<Tr>(th + log_n);
-  th = -th;
-  th = round16<Tr>(th - 10.f);
-  thr[bh] = th;
+  thr[bh] = threshold_of_norms<Tr>(qn, kn, sm_scale, log_n);
 }
 
-// grid (row blocks, B*H, 2)
 template <typename Tr, int D>
-__global__ __launch_bounds__(256) void norm_max_kernel(View q, View k, int H, int M, int N, uint32_t* scratch, float* thr, float sm_scale, float log_n) {
-  norm_max<Tr, D>(q, k, H, M, N, scratch, thr, sm_scale, log_n, blockIdx.x, gridDim.x, blockIdx.y, blockIdx.z);
+__global__ __launch_bounds__(256) void norm_max_kernel(View q, View k, int H, int M, int N, uint32_t* scratch, float* thr, float sm_scale, float log_n, NormBlocks w) {
+  norm_max<Tr, D>(q, k, H, M, N, scratch, thr, sm_scale, log_n, blockIdx.x, w);
 }
 
-// The same with the forward scan of the gates beside it, one workgroup per row in front of the others: the scan is a chain of one workgroup's barriers
+// Short rows: one workgroup takes q and k of a (batch, head) whole, up to 128 KB in flight, and there is nothing to clear, to count or to wait for: a single
+// round trip and a reduction (12 pairs T256 D128: 12.7 us for zeroing, norms and atomics, 6.2 now).
+template <typename Tr, int D>
+__global__ __launch_bounds__(1024) void norm_max_pair_kernel(View q, View k, int H, int M, int N, float* thr, float sm_scale, float log_n) {
+  constexpr int LPR = D / 8, RPP = 1024 / LPR, U = 8;
+  const int tid = threadIdx.x, bh = blockIdx.x, b = bh / H, h = bh % H, ch = tid % LPR;
+  const uint16_t *qp = q.ptr + b * q.sb + h * q.sh + ch * 8, *kp = k.ptr + b * k.sb + h * k.sh + ch * 8;
+  float best_q = 0.f, best_k = 0.f;
+  for (int row0 = tid / LPR; row0 < M + N; row0 += U * RPP) {   // (the lanes of a row together)
+    u32x4 x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int row = min(row0 + u * RPP, M + N - 1);   // rows of q, then those of k
+      const uint16_t* p = row < M ? qp + (int64_t)row * q.st : kp + (int64_t)(row - M) * k.st;
+      x[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float n = row_norm<Tr, LPR>(x[u]);
+      if (row0 + u * RPP < M) best_q = fmaxf(best_q, n);
+      else best_k = fmaxf(best_k, n);
+    }
+  }
+  best_q = wave_max(best_q);
+  best_k = wave_max(best_k);
+  __shared__ float wave_q[16], wave_k[16];
+  if ((tid & 63) == 0) {
+    wave_q[tid >> 6] = best_q;
+    wave_k[tid >> 6] = best_k;
+  }
+  __syncthreads();
+  if (tid >= kWave) return;
+  best_q = wave_max(wave_q[tid & 15]);
+  best_k = wave_max(wave_k[tid & 15]);
+  if (tid == 0) thr[bh] = threshold_of_norms<Tr>(best_q, best_k, sm_scale, log_n);
+}
+
+// norm_max_kernel with the forward scan of the gates beside it, one workgroup per row in front of the others: the scan is a chain of one workgroup's barriers
 // (20 us in a step at B4 T16384 H16) that needs none of the bandwidth the norms stream at (88 us), and needs no threshold.
 template <typename Tr, int D, int KIND>
 __global__ __launch_bounds__(256) void norm_max_scan_kernel(View q, View k, int H, int M, int N, uint32_t* scratch, float* thr, float sm_scale, float log_n,
-                                                            GateK t, const int64_t* __restrict__ seq_start, int rows, int blocks) {
-  if ((int)blockIdx.x >= rows) {
-    const int id = blockIdx.x - rows, pair = id / blocks;
-    norm_max<Tr, D>(q, k, H, M, N, scratch, thr, sm_scale, log_n, id - pair * blocks, blocks, pair % rows, pair / rows);
+                                                            GateK t, const int64_t* __restrict__ seq_start, NormBlocks w) {
+  if ((int)blockIdx.x >= w.pairs) {
+    norm_max<Tr, D>(q, k, H, M, N, scratch, thr, sm_scale, log_n, blockIdx.x - w.pairs, w);
     return;
   }
   const int bh = blockIdx.x, b = bh / H, h = bh % H;
@@ -439,22 +492,32 @@ hipError_t launch_qk_norm_threshold(const float* wq, const float* wk, int H, int
   return hipGetLastError();
 }
 
+// Whether one workgroup takes a (batch, head) whole, where that is no longer a chain than the launch that clears the scratch and the three atomics behind each
+// other.  us, with them / whole: D 128 T64 9.8 / 6.0, T512 9.4 .. 11.7 / 9.0 .. 9.5, T1024 9.4 / 15.3, D 64 T512 8.4 / 6.0, T1024 7.9 / 9.1, D 32 and 16 T512 7.4 / 5.9 and
+// 7.4 / 6.3, T1024 7.6 / 7.3 and 7.5 / 7.2; 512 pairs D 128 T512 26.8 / 23.6.
+static bool threshold_pairs(int M, int N) { return (int64_t)M + N <= 1024; }
+
 template <typename Tr, int D>
 static hipError_t auto_threshold_d(const View& q, const View& k, int B, int H, int M, int N, float sm_scale, float* thr, uint32_t* scratch,
                                    const GateK* t, const int64_t* seq_start, hipStream_t s) {
-  const int n_bh = B * H, blocks = (N + 511) / 512;
+  const int n_bh = B * H, q_blocks = (M + kNormRows - 1) / kNormRows, k_blocks = (N + kNormRows - 1) / kNormRows;
+  const NormBlocks w{n_bh, q_blocks, k_blocks, divisor(q_blocks), divisor(k_blocks), divisor(H)};
   const float log_n = (float)log((double)N);
-  hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)((3 * n_bh + 255) / 256)), dim3(256), 0, s, scratch, 3 * n_bh);
-  if (!t) {
-    hipLaunchKernelGGL((norm_max_kernel<Tr, D>), dim3((unsigned)blocks, (unsigned)n_bh, 2u), dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n);
+  if (!t && threshold_pairs(M, N)) {
+    hipLaunchKernelGGL((norm_max_pair_kernel<Tr, D>), dim3((unsigned)n_bh), dim3(1024), 0, s, q, k, H, M, N, thr, sm_scale, log_n);
     return hipGetLastError();
   }
-  const dim3 grid((unsigned)n_bh * (1u + 2u * (unsigned)blocks));
+  hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)((3 * n_bh + 255) / 256)), dim3(256), 0, s, scratch, 3 * n_bh);
+  const dim3 norms((unsigned)n_bh * (unsigned)(q_blocks + k_blocks)), grid(norms.x + (unsigned)n_bh);
+  if (!t) {
+    hipLaunchKernelGGL((norm_max_kernel<Tr, D>), norms, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, w);
+    return hipGetLastError();
+  }
   switch (t->kind) {
-    case kGateLog: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, kGateLog>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, n_bh, blocks); break;
-    case 0: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, 0>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, n_bh, blocks); break;
-    case 1: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, 1>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, n_bh, blocks); break;
-    case 2: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, 2>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, n_bh, blocks); break;
+    case kGateLog: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, kGateLog>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, w); break;
+    case 0: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, 0>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, w); break;
+    case 1: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, 1>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, w); break;
+    case 2: hipLaunchKernelGGL((norm_max_scan_kernel<Tr, D, 2>), grid, dim3(256), 0, s, q, k, H, M, N, scratch, thr, sm_scale, log_n, *t, seq_start, w); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -477,11 +540,14 @@ hipError_t launch_auto_threshold(const View& q, const View& k, int B, int H, int
                     : auto_threshold_t<Fp16>(q, k, B, H, M, N, D, sm_scale, thr, scratch, t, seq_start, s);
 }
 
-// Whether the scan goes beside the norms: where they stream for longer (at about 6 TB/s) than its 256 threads take (about 1 us per 1024 elements and 2
-// to start; the scan of its own has 1024).  "auto" forward, two launches / one, us: B4 T16384 H16 D128 345 / 329, B4 T4096 H32 D64 107 / 99, B2 T8192 H16 D64 68.4 /
-// 62.5, B8 T700 H32 D32 29.6 / 26.9.
+// Whether the scan goes beside the norms.  There it has 256 threads (2 us and 1 us per 1024 elements), on its own 1024 (about 4 us and 1 us per 2100) and a launch; the norms take 8 us
+// and stream at about 6 TB/s.  So always, but for a row that takes longer than all of that and is alone.  us, two launches / one: B4 T16384 H16 D128 forward "auto" 345 / 329; threshold
+// and scan alone, 12 pairs D128 M = N = 4096 17.5 / 12.8, M8 N9000 21.1 / 12.6, 32 pairs M4 N29333 D64 56 / 45, 128 pairs D16 M8 N4000 16.6 / 13.6, 2 pairs N32768 D16 21.8 / 26.1, 12
+// pairs N32768 D64 38.1 / 39.7, D128 45.7 / 43.7.  Rows that norm_max_pair_kernel takes stay with it, unless there are so many that the norms stream for longer than the scan takes.
 bool threshold_scans(int B, int H, int M, int N, int D) {
-  return (int64_t)B * H * ((int64_t)M + N) * D * 2 >= 6000 * ((int64_t)N + 2000) && (int64_t)B * H * (1 + 2 * (int64_t)((N + 511) / 512)) < (int64_t)1 << 31;
+  const int64_t pairs = (int64_t)B * H, bytes = pairs * ((int64_t)M + N) * D * 2;
+  const bool beside = threshold_pairs(M, N) ? bytes >= 6000 * ((int64_t)N + 2000) : bytes >= 6000000 * ((int64_t)N / 1400 - 11);
+  return beside && pairs * (1 + 2 * (int64_t)((N + kNormRows - 1) / kNormRows)) < (int64_t)1 << 31;
 }
 
 }  // namespace fox
