@@ -76,15 +76,32 @@ std::atomic<int> g_light_limit{256};   // measured crossover of the two kernels 
 // when the next call on them comes (32-270 MB, called in a loop: 5-14 % faster with cached loads).
 std::atomic<int64_t> g_stream_min_kv_bytes{(int64_t)512 << 20};
 
+// Whether the split variant of the dK/dV kernel takes every tile, with or without a threshold.  Its 64-key tiles fit twice on a CU and
+// start and end sooner, the 128-key tiles of the other variant read dO and Q half as often.  dK/dV at D 128, other variant / split, us:
+// - Rows shorter than 512 keys, whatever the grid: 1 tile N64 10.0 / 5.6, 512 tiles N64 21.4 / 8.8, 768 tiles N320 44.4 / 35.5, 1536 tiles N320
+//   91.4 / 67.4 and N384 97.3 / 89.2, 2048 tiles N448 132.4 / 113.0; not N512 with 512 tiles 33.9 / 35.7.
+// - Where no CU gets a second 128-key tile, up to 896 keys: 256 tiles N512 20.8 / 19.5, 160 tiles N640 23.3 / 21.3, 192 tiles N768 26.1 / 24.6;
+//   not 320 tiles N600 25.6 / 26.2, 256 tiles N1024 32.2 / 33.6.
+// Under a threshold it saves the launch for the tiles far from the diagonal, of which there are few or none: at -10 12 tiles N128 9.2 / 7.7, 768 tiles
+// N320 34.7 / 32.0, 256 tiles N512 17.2 / 15.1.
+bool split_takes_all(int B, int H, int N) {
+  const int64_t tiles = (int64_t)B * H * ((N + 127) / 128);
+  return N < 512 || (N <= 896 && tiles <= fox::kCus);
+}
+
 // The tile classes of a call: *first and *second are the classes of the launches to make (kClassAll alone,
 // kClassLight alone, or kClassLight then kClassHeavy), *limit the distance handed to the kernels.
-void tile_classes(bool pruned, bool light_ok, int* first, int* second, int* limit) {
+void tile_classes(bool pruned, bool light_ok, bool light_all, int* first, int* second, int* limit) {
   const int lim = g_light_limit.load(std::memory_order_relaxed);
   *first = fox::kClassAll;
   *second = -1;
   *limit = lim;
   if (!light_ok || lim == 0) return;
-  if (lim < 0) { *first = fox::kClassLight; return; }
+  if (lim < 0 || light_all) {
+    *first = fox::kClassLight;
+    *limit = -1;
+    return;
+  }
   if (!pruned) return;
   *first = fox::kClassLight;
   *second = fox::kClassHeavy;
@@ -662,7 +679,7 @@ int fox_attn_bwd_dkdv(const fox_bwd_args* args, void* stream) {
   k.dk = to_view(args->dk);
   k.dv = to_view(args->dv);
   int first, second;
-  tile_classes(k.thr != nullptr, fox::dkdv_split_supports(args->dims.D), &first, &second, &k.light_limit);
+  tile_classes(k.thr != nullptr, fox::dkdv_split_supports(args->dims.D), split_takes_all(k.B, k.H, k.N), &first, &second, &k.light_limit);
   k.cls = first;
   FOX_TRY(check_hip(fox::launch_bwd_dkdv(k, args->dims.D, args->dims.dtype, (hipStream_t)stream), "fox_attn_bwd_dkdv"));
   if (second < 0) return FOX_OK;

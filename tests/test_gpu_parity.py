@@ -417,6 +417,17 @@ def test_dkdv_kernel_variants(fa, limit, B, H, M, N, seq, thr, gates):
         assert lib.fox_set_acp_light_limit(prev) == limit
 
 
+@pytest.mark.parametrize("B,H,M,N,seq,thr,dtype", [
+    (1, 2, 64, 64, None, None, torch.bfloat16), (16, 20, 65, 65, None, -10.0, torch.bfloat16), (2, 3, 511, 511, [0, 300], -10.0, torch.float16),
+    (12, 8, 511, 511, None, None, torch.bfloat16), (8, 8, 512, 512, None, None, torch.bfloat16), (5, 13, 512, 512, None, -10.0, torch.bfloat16),
+    (1, 3, 896, 896, None, -10.0, torch.bfloat16), (1, 2, 200, 897, None, None, torch.float16)])
+def test_dkdv_kernel_of_short_rows(fa, B, H, M, N, seq, thr, dtype):
+    """Head dim 128, at the edges of the rule that hands every tile to the split dK/dV kernel: rows below 512 keys on any grid,
+    up to 896 keys with at most 256 tiles of 128 (8 * 8 * 4 of them; 5 * 13 * 4 are too many), one key more than either."""
+    run_case(fa, B, H, M, N, 128, dtype=dtype, seq_start=seq, thr=thr, tol=REL_TOL if dtype == torch.bfloat16 else 1e-2, gate_mean=0.0,
+             seed=B + N, qkv_std=0.7)
+
+
 def test_in_op_timers_fill_the_info_table(fa):
     """The reference's hidden timing flags (:45-70, :176-181, :217-222): same results, and the class-level table
     gets the elapsed milliseconds and call counts under the caller's key."""
