@@ -37,24 +37,27 @@ struct NoRows {
 
 // Scan of one row: element idx is produced by load(idx) and the running sum up to and including
 // it is handed to store(idx, sum).  REVERSE walks the row from its last element to its first.
-// A span of 8 x NT elements moves between memory and LDS with consecutive lanes on consecutive
+// A span of PER x NT elements moves between memory and LDS with consecutive lanes on consecutive
 // elements (whole cache lines per wave instruction, whatever the caller's stride), and between LDS and
-// registers with eight consecutive elements per thread, the order the scan wants.
+// registers with PER consecutive elements per thread, the order the scan wants.  The totals of the threads meet by DPP (wave_scan): through
+// shuffles, twelve trips through LDS one after the other, 12 rows of 4096 took 5.4 / 4.7 us.
 // Bound by latency: one workgroup per row, few rows.  A long row gets the widest workgroup there is; a row that a single span of
 // fewer waves covers gets just those (scan_threads), and the barriers between sixteen waves and the chain over their totals go.
 // Rows of 77 to 2048 elements: 5.1 us a call with 1024 threads, 3.9 with as many as the row needs.  Rows cut over several
 // workgroups, each adding up what lies in front of its piece, were slower wherever there were enough of them to count (64 rows of 16384 8.5 -> 10.4
 // us, 256 rows of 32768 17 -> 28 us).
 // rows: a second addend of the last M positions (RowSums), or nothing.
-template <bool REVERSE, int NT, typename Load, typename Store, typename Rows = NoRows>
+template <bool REVERSE, int NT, int PER, typename Load, typename Store, typename Rows = NoRows>
 __device__ __forceinline__ void scan_row(int N, Load load, Store store, Rows rows = {}) {
-  constexpr int PER = 8, SPAN = PER * NT, WAVES = NT / kWave;
+  static_assert(PER % 4 == 0);
+  constexpr int SPAN = PER * NT, WAVES = NT / kWave;
   __shared__ double wave_tot[WAVES];
   __shared__ __align__(16) float stage[SPAN];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   double carry = 0.0;
   float x[PER], x_next[PER], r[PER], r_next[PER];   // (r: Rows::kAny only)
   auto fetch = [&](int base, float (&dst)[PER], float (&dst_r)[PER]) {  // element e of a thread sits at position base + e*NT + tid of the scan order
+    asm volatile("" : "+s"(base));   // (one address after the other: as pointers that a loop moves on they took 32 registers and spilt)
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
       const int pos = base + e * NT + tid;
@@ -79,21 +82,17 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store, Rows row
     }
     if (base + SPAN < N) fetch(base + SPAN, x_next, r_next);   // in flight while this span is scanned
     __syncthreads();
-    const f32x4 lo4 = *reinterpret_cast<const f32x4*>(stage + tid * PER), hi4 = *reinterpret_cast<const f32x4*>(stage + tid * PER + 4);
+    f32x4* const own = reinterpret_cast<f32x4*>(stage + tid * PER);
     double v[PER];
     double run = 0.0;
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      run += (double)(e < 4 ? lo4[e & 3] : hi4[e & 3]);
-      v[e] = run;
+    for (int i = 0; i < PER / 4; ++i) {
+      const f32x4 y = own[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[4 * i + e] = run += (double)y[e];
     }
     // inclusive scan of the per-thread totals across the wave, then across waves
-    double incl = run;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const double up = __shfl_up(incl, off);
-      if (lane >= off) incl += up;
-    }
+    const double incl = wave_scan(run);
     if (lane == kWave - 1) wave_tot[wave] = incl;
     __syncthreads();
     double before = carry, total = 0.0;
@@ -104,14 +103,13 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store, Rows row
       total += t;
     }
     before += incl - run;
-    f32x4 o_lo, o_hi;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      o_lo[e] = (float)(before + v[e]);
-      o_hi[e] = (float)(before + v[4 + e]);
+    for (int i = 0; i < PER / 4; ++i) {
+      f32x4 y;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = (float)(before + v[4 * i + e]);
+      own[i] = y;   // each thread overwrites the values it read
     }
-    *reinterpret_cast<f32x4*>(stage + tid * PER) = o_lo;   // each thread overwrites the eight values it read
-    *reinterpret_cast<f32x4*>(stage + tid * PER + 4) = o_hi;
     carry += total;
     __syncthreads();
 #pragma unroll
@@ -153,9 +151,18 @@ __device__ __forceinline__ auto row_sums(const float* drow, float* dc, int bh, i
 }
 
 inline int scan_threads(int N) { return N <= 8 * 64 ? 64 : N <= 8 * 256 ? 256 : 1024; }
+// Whether a thread of the widest workgroup takes sixteen elements of a span in place of eight: rows of more than 8192 positions have half as
+// many spans then, each a chain through LDS, the waves' totals and three barriers.  us, eight and shuffles / sixteen and DPP (a row of one span gains 0.3 to 0.7
+// from the latter alone): 15 rows of 12242 forward 7.9 / 6.5, reverse 8.1 / 6.8; 64 rows of 16384 8.5 / 6.9 and 9.1 / 7.7; reverse, 64 rows of 32768, 16.0 / 13.3.
+// Against it stand the loads of a row's next span, sent while one is scanned.  Eight / sixteen, both by DPP: forward 64 rows of 20000 9.4 / 10.7, 256 rows of
+// 32768 14.7 / 15.4, 512 rows of 16384 16.1 / 17.1; reverse 512 rows of 20000 22.2 / 26.2, 16384 18.6 / 18.6.
+inline bool scan_deep(int N, int64_t rows, bool reverse) {
+  if (N <= 8 * 1024) return false;
+  return reverse ? rows <= kCus || N <= 16 * 1024 : rows <= kCus && N <= 16 * 1024;
+}
 
 enum : int { kForward = 0, kReverse = 1, kReverseRows = 2 };   // kinds of scan_kernel; the last with row sums to add
-template <int KIND, int NT>
+template <int KIND, int NT, int PER>
 __global__ __launch_bounds__(NT) void scan_kernel(const float* in, int64_t sb, int64_t sh, int64_t sn,
                                                    const int64_t* __restrict__ seq_start, float* __restrict__ out, int64_t ob,
                                                    int64_t oh, int64_t on, int rows, int H, int N, const float* __restrict__ drow, int M,
@@ -173,8 +180,9 @@ __global__ __launch_bounds__(NT) void scan_kernel(const float* in, int64_t sb, i
   // Reverse: the gradient of every gate up to and including position seq is the sum of all dc, zero in exact
   // arithmetic (those gates shift every cumulative sum the kernels see by the same amount, or are zeroed by the
   // forward); it is stored as an exact zero instead of the rounding noise of that sum.
-  scan_row<REVERSE, NT>(
-      N, [&](int idx) { return (REVERSE || idx >= seq) ? src[(int64_t)idx * sn] : 0.f; },
+  scan_row<REVERSE, NT, PER>(
+      N,
+      [&](int idx) { return (REVERSE || idx >= seq) ? src[(int64_t)idx * sn] : 0.f; },
       [&](int idx, float sum) { dst[(int64_t)idx * on] = (REVERSE && idx <= seq) ? 0.f : sum; },
       row_sums<KIND == kReverseRows>(drow, dc, bh, M, N));
 }
@@ -188,7 +196,7 @@ __device__ __forceinline__ void store_logit(void* p, int64_t i, float x) {
 
 // c[n] = sum_{seq_start <= l <= n} logsigmoid(x[l]) in one pass over the logits; optionally also
 // stores log_fgate[n] = logsigmoid(x[n]) (the decode cache of the FoX layer keeps it).
-template <int DT, int NT>
+template <int DT, int NT, int PER>
 __global__ __launch_bounds__(NT) void gate_scan_fwd_kernel(const void* __restrict__ logits, int64_t sb, int64_t sh, int64_t sn,
                                                             const int64_t* __restrict__ seq_start,
                                                             float* __restrict__ log_fgate, float* __restrict__ out, int H,
@@ -202,7 +210,7 @@ __global__ __launch_bounds__(NT) void gate_scan_fwd_kernel(const void* __restric
     const int64_t s64 = seq_start[b];
     seq = (int)(s64 < 0 ? 0 : (s64 > N ? N : s64));
   }
-  scan_row<false, NT>(
+  scan_row<false, NT, PER>(
       N,
       [&](int idx) {
         const float x = load_logit<DT>(logits, base + (int64_t)idx * sn);
@@ -216,7 +224,7 @@ __global__ __launch_bounds__(NT) void gate_scan_fwd_kernel(const void* __restric
 // dlogit[l] = (sum_{n>=l} dc[n]) * d logsigmoid(x_l)/dx = dg[l] * (1 - sigmoid(x_l)), stored in the
 // dtype and layout of the logits.
 constexpr int kRows = 4;   // with row sums to add
-template <int DT_ROWS, int NT>
+template <int DT_ROWS, int NT, int PER>
 __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(float* dc, const void* __restrict__ logits,
                                                             int64_t sb, int64_t sh, int64_t sn, const int64_t* __restrict__ seq_start,
                                                             void* __restrict__ dlogits, int64_t db, int64_t dh, int64_t dn,
@@ -231,7 +239,7 @@ __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(float* dc, const void
     const int64_t s64 = seq_start[b];
     seq = (int)(s64 < 0 ? 0 : (s64 > N ? N : s64));
   }
-  scan_row<true, NT>(
+  scan_row<true, NT, PER>(
       N, [&](int idx) { return src[idx]; },
       [&](int idx, float sum) {
         const float x = load_logit<DT>(logits, lbase + (int64_t)idx * sn);
@@ -244,19 +252,21 @@ __global__ __launch_bounds__(NT) void gate_scan_bwd_kernel(float* dc, const void
 }
 
 // KERNEL<ARG, threads for rows of N elements>, BLOCKS workgroups, one per row of the B x H.
-#define FOX_LAUNCH_SCAN(KERNEL, ARG, BLOCKS, ...)                                                                      \
-  switch (scan_threads(N)) {                                                                                    \
-    case 64: hipLaunchKernelGGL((KERNEL<ARG, 64>), dim3(BLOCKS), dim3(64), 0, s, __VA_ARGS__); break;    \
-    case 256: hipLaunchKernelGGL((KERNEL<ARG, 256>), dim3(BLOCKS), dim3(256), 0, s, __VA_ARGS__); break; \
-    default: hipLaunchKernelGGL((KERNEL<ARG, 1024>), dim3(BLOCKS), dim3(1024), 0, s, __VA_ARGS__);       \
+#define FOX_LAUNCH_SCAN(KERNEL, ARG, REVERSE, BLOCKS, ...)                                                                      \
+  switch (scan_threads(N)) {                                                                                                     \
+    case 64: hipLaunchKernelGGL((KERNEL<ARG, 64, 8>), dim3(BLOCKS), dim3(64), 0, s, __VA_ARGS__); break;                         \
+    case 256: hipLaunchKernelGGL((KERNEL<ARG, 256, 8>), dim3(BLOCKS), dim3(256), 0, s, __VA_ARGS__); break;                      \
+    default:                                                                                                                     \
+      if (scan_deep(N, (int64_t)B * H, REVERSE)) hipLaunchKernelGGL((KERNEL<ARG, 1024, 16>), dim3(BLOCKS), dim3(1024), 0, s, __VA_ARGS__);                \
+      else hipLaunchKernelGGL((KERNEL<ARG, 1024, 8>), dim3(BLOCKS), dim3(1024), 0, s, __VA_ARGS__);                              \
   }
 
 hipError_t launch_gate_cumsum_fwd(const void* logits, int dtype, int64_t sb, int64_t sh, int64_t sn, const int64_t* seq_start,
                                   float* log_fgate, float* c, int B, int H, int N, hipStream_t s) {
   switch (dtype) {
-    case 0: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 0, (unsigned)(B * H), logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
-    case 1: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 1, (unsigned)(B * H), logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
-    case 2: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 2, (unsigned)(B * H), logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
+    case 0: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 0, false, (unsigned)(B * H), logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
+    case 1: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 1, false, (unsigned)(B * H), logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
+    case 2: FOX_LAUNCH_SCAN(gate_scan_fwd_kernel, 2, false, (unsigned)(B * H), logits, sb, sh, sn, seq_start, log_fgate, c, H, N) break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -266,12 +276,12 @@ hipError_t launch_gate_cumsum_bwd(float* dc, const void* logits, int dtype, int6
                                   const int64_t* seq_start, void* dlogits, int64_t db, int64_t dh, int64_t dn, int B, int H, int N,
                                   const float* drow, int M, hipStream_t s) {
   switch (drow ? dtype | kRows : dtype) {
-    case 0: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 0, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
-    case 1: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 1, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
-    case 2: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 2, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
-    case 0 | kRows: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, (0 | kRows), scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
-    case 1 | kRows: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, (1 | kRows), scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
-    case 2 | kRows: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, (2 | kRows), scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 0: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 0, true, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 1: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 1, true, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 2: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, 2, true, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 0 | kRows: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, (0 | kRows), true, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 1 | kRows: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, (1 | kRows), true, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
+    case 2 | kRows: FOX_LAUNCH_SCAN(gate_scan_bwd_kernel, (2 | kRows), true, scan_blocks(B * H), dc, logits, sb, sh, sn, seq_start, dlogits, db, dh, dn, B * H, H, N, drow, M) break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -279,7 +289,7 @@ hipError_t launch_gate_cumsum_bwd(float* dc, const void* logits, int dtype, int6
 
 hipError_t launch_cumsum_fwd(const float* g, int64_t sb, int64_t sh, int64_t sn, const int64_t* seq_start, float* c, int B,
                              int H, int N, hipStream_t s) {
-  FOX_LAUNCH_SCAN(scan_kernel, kForward, (unsigned)(B * H), g, sb, sh, sn, seq_start, c,
+  FOX_LAUNCH_SCAN(scan_kernel, kForward, false, (unsigned)(B * H), g, sb, sh, sn, seq_start, c,
                      (int64_t)H * N, (int64_t)N, (int64_t)1, B * H, H, N, nullptr, N, nullptr)
   return hipGetLastError();
 }
@@ -287,10 +297,10 @@ hipError_t launch_cumsum_fwd(const float* g, int64_t sb, int64_t sh, int64_t sn,
 hipError_t launch_cumsum_bwd(float* dc, float* dg, int64_t db, int64_t dh, int64_t dn, const int64_t* seq_start, int B, int H,
                              int N, const float* drow, int M, hipStream_t s) {
   if (drow) {
-    FOX_LAUNCH_SCAN(scan_kernel, kReverseRows, scan_blocks(B * H), dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
+    FOX_LAUNCH_SCAN(scan_kernel, kReverseRows, true, scan_blocks(B * H), dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
                        seq_start, dg, db, dh, dn, B * H, H, N, drow, M, dc)
   } else {
-    FOX_LAUNCH_SCAN(scan_kernel, kReverse, scan_blocks(B * H), dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
+    FOX_LAUNCH_SCAN(scan_kernel, kReverse, true, scan_blocks(B * H), dc, (int64_t)H * N, (int64_t)N, (int64_t)1,
                        seq_start, dg, db, dh, dn, B * H, H, N, nullptr, N, nullptr)
   }
   return hipGetLastError();
@@ -445,7 +455,7 @@ __global__ __launch_bounds__(256) void norm_max_scan_kernel(View q, View k, int 
   }
   const int64_t base = b * t.sb + h * t.sh;
   float *dst = t.c + (int64_t)bh * N, *lg = t.log_fgate ? t.log_fgate + (int64_t)bh * N : nullptr;
-  scan_row<false, 256>(
+  scan_row<false, 256, 8>(
       N,
       [&](int idx) {
         if constexpr (KIND == kGateLog) {

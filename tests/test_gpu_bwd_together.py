@@ -123,3 +123,9 @@ def test_strided_gate_gradients(B, H, M, N, seq, logit):
         res.append((dg, tmp[1], tmp[2]))
     for a, b in zip(*res):
         assert torch.isfinite(a).all() and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("logit", [None, torch.float16])
+def test_strided_gate_gradients_of_long_rows(logit):
+    """The same where a row is two spans of sixteen positions a thread."""
+    test_strided_gate_gradients(1, 2, 300, 16500, [17], logit)

@@ -651,6 +651,12 @@ def test_cumsum_kernels_at_the_edges_of_their_workgroups(fa, N):
     assert ((dx.double() - ref).abs() <= 2e-6 * ref.abs() + 1e-12).all()   # hardware exp and reciprocal: a few ulp
 
 
+@pytest.mark.parametrize("N", [8192, 16383, 16384, 16385, 32769])
+def test_cumsum_kernels_with_sixteen_positions_a_thread(fa, N):
+    """Rows around one and two spans of 8 * 1024 and of 16 * 1024 positions, which the scans choose between."""
+    test_cumsum_kernels_at_the_edges_of_their_workgroups(fa, N)
+
+
 def test_mfma_probe_runs(fa):
     """The measuring-stick loop of the power report: launches, returns, leaves its sink alone."""
     from forgetting_transformer.ops import _lib
