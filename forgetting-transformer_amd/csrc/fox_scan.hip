@@ -112,16 +112,18 @@ __device__ __forceinline__ void scan_row(int N, Load load, Store store, Rows row
     }
     carry += total;
     __syncthreads();
+    int out = base;
+    if constexpr (Rows::kAny) asm volatile("" : "+s"(out));   // (as in fetch; the others have the registers for it)
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-      const int pos = base + e * NT + tid;
+      const int pos = out + e * NT + tid;
       const int idx = REVERSE ? N - 1 - pos : pos;
       if (pos < N) store(idx, stage[e * NT + tid]);
     }
     if constexpr (Rows::kAny) {
 #pragma unroll
       for (int e = 0; e < PER; ++e) {
-        const int pos = base + e * NT + tid;
+        const int pos = out + e * NT + tid;
         if (pos < N) rows.keep(REVERSE ? N - 1 - pos : pos, x[e]);
       }
     }
