@@ -928,17 +928,10 @@ bool fwd_scans(int B, int H, int M, int N, int D, bool pruned, int splits) {
 // - Smaller grids with fewer keys than are split: from 512 keys on.  D 64: N300 11.6 / 12.0, N512 15.6 / 14.5, N777 19.3 / 17.1.
 // - Two key splits cost a pass over fp32 partials and a merge launch, which pays for longer walks only.  D 128 and 64: B2 H12 N1024
 //   33.2 / 25.3 and 24.6 / 19.4, B1 H16 N2048 44.3 / 38.2 and 34.3 / 29.3, B1 H10 N2900 53.4 / 55.1 and 38.2 / 39.0.
-// - Under a pruning threshold the walks are short as a rule, and what there is to save is the launches of the scan in front and the
-//   merge behind two or three key splits: the pair, with its own sums, is one launch.  Split / paired at -10 (gates of mean 0 and 3)
-//   and with a threshold that prunes nothing: D 128 H10 N1700 24.8 / 11.8, 26.0 / 14.4 and 33.6 / 29; H16 N1700 26.8 / 11.9, 28.2 / 14.3
-//   and 39.0 / 30; D 64 H12 N2200 20.8 / 10.5.  36 such shapes geomean 0.60 and 0.88, "auto" 0.83 and 0.93; the worst one where nothing is
-//   pruned D 32 B2 H5 N2800 29.0 / 32.0.  More splits than that, and grids of less than a quarter of the CUs, gain as much where pruning
-//   bites and lose where it does not (H3 N3500 36 / 56, D 64 N1000 "auto" 20.7 / 23.1).  Unsplit grids have too many short walks to gain.
-// - Head dim 16 has no room to hand the accumulators over.
+// - Under a pruning threshold the walks are short whatever the shape; head dim 16 has no room to hand the accumulators over.
 bool fwd_pairs(int B, int H, int M, int N, int D, bool pruned, int splits) {
   const int64_t wgs = (int64_t)((M + kFwdBM - 1) / kFwdBM) * B * H;
-  if (D < 32 || even_tiles(M, N) || wgs >= 2 * kCus || N < 512) return false;
-  if (pruned) return N <= kOwnScanMaxKeys && ((splits == 2 && 4 * wgs >= kCus) || (splits == 3 && 2 * wgs > kCus));
+  if (D < 32 || pruned || even_tiles(M, N) || wgs >= 2 * kCus || N < 512) return false;
   if (splits > 1) return splits == 2 && N <= 2560;
   return N >= 16 * (wgs - kCus);
 }

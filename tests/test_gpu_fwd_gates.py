@@ -77,23 +77,6 @@ def test_shapes_it_takes_where_a_scan_is_faster(B, H, M, N, D, thr):
     _both(B, H, M, N, D, torch.bfloat16, thr, None, None, True, faster=0)
 
 
-# Under a threshold the paired kernel takes grids that would have two key splits (from 129 query tiles, or 64 with 961 to 1472 keys), or three that fill the chip: little pruned, or
-# all but the tiles at the diagonal
-@pytest.mark.parametrize("B,H,M,N,D", [(2, 5, 1100, 1100, 64), (1, 8, 1025, 1400, 128), (1, 16, 2048, 2048, 128), (1, 10, 2817, 2817, 32), (2, 4, 3584, 3584, 64)])
-@pytest.mark.parametrize("thr,gate_mean", [(-40.0, 3.0), (-30.0, -2.0)])
-@pytest.mark.parametrize("padded", [False, True])
-def test_pruned_pairs(B, H, M, N, D, thr, gate_mean, padded):
-    from forgetting_transformer import forgetting_attention
-    from forgetting_transformer.ops import _lib
-    splits, paired = C.c_int32(-1), C.c_int32(-1)
-    _lib.check(_lib.load().fox_attn_fwd_plan(C.byref(_lib.Dims(B, H, M, N, D, 0)), 1, C.byref(splits), C.byref(paired), None), "plan")
-    assert (splits.value, paired.value) == (1, 1)
-    q, k, v, g, _, ss = make_inputs(B, H, M, N, D, device="cuda", seed=N + D, gate_mean=gate_mean, seq_start=[N - 70 * (b + 1) for b in range(B)] if padded else None)
-    with torch.no_grad():
-        out = forgetting_attention(q, k, v, g, head_first=True, seq_start=ss, adaptive_threshold=thr)
-    assert_parity("out", out, O.forgetting_attention_ref(q, k, v, g, head_first=True, seq_start=ss))   # what is pruned weighs less than exp(-20)
-
-
 def test_shapes_it_does_not_take():
     from forgetting_transformer.ops import _lib
     lib = _lib.load()
