@@ -11,6 +11,7 @@
 #include <mutex>
 
 #include "fox_common.hpp"
+#include "fox_decode_plan.hpp"
 #include "fox_kernels.hpp"
 
 // Library-owned scratch of fox_attn_fwd_noalloc: the partial (max, sum, accumulator) results of a key-split
@@ -583,8 +584,7 @@ int fox_attn_decode_workspace_bytes(const fox_dims* dims, int64_t* bytes) {
   FOX_TRY(check_dims(dims));
   if (!bytes) return fail(FOX_E_ARG, "bytes is NULL");
   if (dims->M != 1) return fail(FOX_E_ARG, "fox_attn_decode takes one query row (M = %d)", dims->M);
-  const int splits = fox::decode_splits(dims->B, dims->H, dims->N, dims->D, true);   // (never fewer than without seq_start)
-  *bytes = splits <= 1 ? 0 : (int64_t)splits * dims->B * dims->H * (int64_t)(dims->D * sizeof(float) + sizeof(fox::DecodePartial));
+  *bytes = fox::decode_workspace_bytes(dims->B, dims->H, dims->N, dims->D);
   return FOX_OK;
 }
 
@@ -592,7 +592,7 @@ int fox_attn_decode_counters(const fox_dims* dims, int32_t* counters) {
   FOX_TRY(check_dims(dims));
   if (!counters) return fail(FOX_E_ARG, "counters is NULL");
   if (dims->M != 1) return fail(FOX_E_ARG, "fox_attn_decode takes one query row (M = %d)", dims->M);
-  *counters = fox::decode_merges(dims->B, dims->H, dims->N, dims->D, fox::decode_splits(dims->B, dims->H, dims->N, dims->D, true)) ? dims->B * dims->H : 0;
+  *counters = fox::decode_merges(dims->B, dims->H, dims->N, dims->D, fox::decode_plan(dims->B, dims->H, dims->N, dims->D, true).splits) ? dims->B * dims->H : 0;
   return FOX_OK;
 }
 
@@ -623,16 +623,15 @@ int fox_attn_decode_counted(const fox_fwd_args* args, const float* g, int64_t g_
   k.sm_scale = args->sm_scale;
   k.splits = 1;
   if (args->workspace) {
-    int64_t need = 0;
-    FOX_TRY(fox_attn_decode_workspace_bytes(&args->dims, &need));
-    if (need > 0) {
-      if (args->workspace_bytes < need) return fail(FOX_E_ARG, "workspace too small: %lld < %lld bytes", (long long)args->workspace_bytes, (long long)need);
-      if (((uintptr_t)args->workspace & 15) != 0) return fail(FOX_E_ALIGN, "workspace must be 16-byte aligned");
-      k.splits = fox::decode_splits(k.B, k.H, k.N, args->dims.D, args->seq_start != nullptr);
-      k.ws_o = (float*)args->workspace;
-      k.ws_p = (fox::DecodePartial*)(k.ws_o + (int64_t)k.splits * k.B * k.H * args->dims.D);   // (D is a multiple of 4: 16-byte aligned)
-      if (fox::decode_merges(k.B, k.H, k.N, args->dims.D, k.splits)) k.arrived = arrived;
-    }
+    const int D = args->dims.D;
+    const bool padded = args->seq_start != nullptr, aligned = ((uintptr_t)args->workspace & 15) == 0;
+    const int64_t need = fox::decode_bytes(k.B, k.H, D, fox::decode_plan(k.B, k.H, k.N, D, padded).least);
+    if (need > 0 && args->workspace_bytes < need) return fail(FOX_E_ARG, "workspace too small: %lld < %lld bytes", (long long)args->workspace_bytes, (long long)need);
+    if (need > 0 && !aligned) return fail(FOX_E_ALIGN, "workspace must be 16-byte aligned");
+    k.splits = fox::decode_splits(k.B, k.H, k.N, D, padded, aligned ? args->workspace_bytes : 0);
+    k.ws_o = (float*)args->workspace;
+    k.ws_p = (fox::DecodePartial*)(k.ws_o + (int64_t)k.splits * k.B * k.H * D);   // (D is a multiple of 4: 16-byte aligned)
+    if (fox::decode_merges(k.B, k.H, k.N, D, k.splits)) k.arrived = arrived;
   }
   k.by_splits = fox::divisor(k.splits);
   k.by_heads = fox::divisor(k.H);

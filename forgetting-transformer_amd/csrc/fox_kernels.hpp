@@ -292,8 +292,6 @@ hipError_t launch_bwd_dq(const BwdK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_fwd_decode(const FwdK& a, int D, int dtype, hipStream_t s);  // M == 1, without the merge of the splits
 hipError_t launch_decode_gates(const DecodeK& a, int D, int dtype, hipStream_t s);
 hipError_t launch_cache_append(const CacheAppendK& a, hipStream_t s);
-int decode_splits(int B, int H, int N, int D, bool padded);
-bool decode_merges(int B, int H, int N, int D, int splits);
 hipError_t launch_norm_gate(const NormGateK& a, int D, int dtype, bool bwd, int act, hipStream_t s);  // act: FOX_ACT_*
 int64_t norm_gate_workspace_rows(int64_t rows);
 hipError_t launch_shift_fwd(const ShiftK& a, int D, int dtype, hipStream_t s);

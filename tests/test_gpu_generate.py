@@ -62,6 +62,35 @@ def test_single_query_splits(ft, B, H, N, D, padded):
     assert_parity("out", out, O.forgetting_attention_ref(q, k, v, g, head_first=True, seq_start=ss))
 
 
+# shapes whose number of splits is another with padding than without; the scratch lies inside a larger allocation, of the size that the query asks for
+# and one piece smaller, where the call makes do with fewer splits
+@pytest.mark.parametrize("B,H,N,D", [(4, 12, 16384, 128), (8, 12, 8192, 128), (8, 16, 6500, 128), (16, 8, 10000, 64), (4, 16, 13000, 128), (4, 16, 9232, 128),
+                                     (10, 32, 16384, 128), (12, 32, 16384, 128), (10, 32, 1808, 128), (33, 1, 64513, 16), (2, 520, 16384, 128)])
+@pytest.mark.parametrize("padded", [False, True])
+def test_splits_stay_inside_their_scratch(ft, B, H, N, D, padded):
+    from forgetting_transformer.ops import _lib
+    from forgetting_transformer.ops.forgetting_attention import _view
+    lib, stream = _lib.load(), C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    gen = torch.Generator(device="cuda").manual_seed(N)   # (up to 2 * 10^9 elements: drawn there)
+    q, k, v = (torch.randn(B, H, T, D, generator=gen, device="cuda", dtype=torch.bfloat16) for T in (1, N, N))
+    g = torch.nn.functional.logsigmoid(torch.randn(B, H, N, generator=gen, device="cuda") + 2.0)
+    ss = torch.tensor([(N * i) // (4 * B) for i in range(B)], device="cuda") if padded else None
+    ref = O.forgetting_attention_ref(q, k, v, g, head_first=True, seq_start=ss)
+    dims, need = _lib.Dims(B, H, 1, N, D, _lib.DTYPE_BF16), C.c_int64(0)
+    _lib.check(lib.fox_attn_decode_workspace_bytes(C.byref(dims), C.byref(need)), "fox_attn_decode_workspace_bytes")
+    guard = 4 << 20   # more than the partial results of 64 splits of any of these shapes would run over
+    for room in (need.value, need.value - 16):
+        block, o = torch.full((guard + need.value + guard,), 0xA5, dtype=torch.uint8, device="cuda"), torch.full_like(q, float("nan"))
+        args = _lib.FwdArgs(dims, _view(q), _view(k), _view(v), _view(o), None, None, None if ss is None else ss.data_ptr(), None, D ** -0.5, None,
+                            block.data_ptr() + guard, room)
+        _lib.check(lib.fox_attn_decode(C.byref(args), g.data_ptr(), *g.stride(), stream), "fox_attn_decode")
+        assert (block[:guard] == 0xA5).all() and (block[guard + room:] == 0xA5).all()
+        assert_parity("out", o, ref)
+        if room == need.value:
+            with torch.no_grad():
+                assert torch.equal(ft.forgetting_attention(q, k, v, g, head_first=True, seq_start=ss), o)
+
+
 # one workgroup of sixteen waves takes a (batch, head) whole: two batches of keys with few heads, up to four with many, and
 # the first sizes beyond
 @pytest.mark.parametrize("B,H,N,D", [(2, 3, 257, 64), (2, 3, 512, 64), (2, 3, 513, 64), (1, 3, 129, 128), (2, 2, 2048, 16), (2, 2, 600, 32),
