@@ -592,7 +592,7 @@ int fox_attn_decode_counters(const fox_dims* dims, int32_t* counters) {
   FOX_TRY(check_dims(dims));
   if (!counters) return fail(FOX_E_ARG, "counters is NULL");
   if (dims->M != 1) return fail(FOX_E_ARG, "fox_attn_decode takes one query row (M = %d)", dims->M);
-  *counters = fox::decode_merges(dims->B, dims->H, dims->N, dims->D, fox::decode_plan(dims->B, dims->H, dims->N, dims->D, true).splits) ? dims->B * dims->H : 0;
+  *counters = fox::decode_counters(dims->B, dims->H, dims->N, dims->D);
   return FOX_OK;
 }
 

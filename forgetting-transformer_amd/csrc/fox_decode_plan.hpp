@@ -70,9 +70,16 @@ inline int decode_splits(int B, int H, int N, int D, bool padded, int64_t bytes)
 // 14.7 / 13.6, H4 N8000 14.2 / 14.2, H1 N16000 14.6 / 13.4.  Where the splits have several batches of keys a wave the step is the GPU's again: D128 H1
 // N24000 14.4 / 14.4, H4 N12000 14.3 / 14.9, H4 N24000 15.4 / 17.7, D64 H4 N32000 14.4 / 14.8.  (Calls back to back with nothing between them are the GPU's
 // as well: up to 0.5 us more at head dims up to 64 with few workgroups, 1 to 3 us at 128.)
-inline bool decode_merges(int B, int H, int N, int D, int splits) {
+inline bool decode_merge_pays(int B, int H, int N, int D, int splits) {
   const int64_t wgs = (int64_t)B * H * splits, batches = decode_batches(N, D);
   return splits > 1 && wgs <= kCus && (batches <= kDecodeMaxSplits || (2 * wgs <= kCus && batches <= 2 * kDecodeMaxSplits));
+}
+// Counters that a shape's calls may touch.  A few shapes pay without left padding only (3 pairs of 16385 to 21504 keys at head dim 64), and stay with two launches.
+inline int decode_counters(int B, int H, int N, int D) {
+  return decode_merge_pays(B, H, N, D, decode_plan(B, H, N, D, true).splits) ? B * H : 0;
+}
+inline bool decode_merges(int B, int H, int N, int D, int splits) {
+  return decode_merge_pays(B, H, N, D, splits) && decode_counters(B, H, N, D) > 0;
 }
 
 }  // namespace fox

@@ -1,5 +1,5 @@
 """The key splits of a generation step, on the host: the scratch that the query asks for holds what any call launches, and a call with less
-scratch than that launches no more than fits."""
+scratch than that launches no more than fits; counters are touched where the query asks for them."""
 import pathlib
 import shutil
 import subprocess
@@ -37,6 +37,8 @@ int main() {
               const int n = decode_splits(1, bh, N, D, padded, bytes);
               if (decode_bytes(1, bh, D, n) > bytes || (bytes >= room && n != p.splits) || (n != p.splits && n != p.least))
                 return std::printf("%d pairs N%d D%d padded %d: %d splits in %lld bytes\n", bh, N, D, padded, n, (long long)bytes), 1;
+              if (decode_merges(1, bh, N, D, n) && (decode_counters(1, bh, N, D) != bh || bh > 128))
+                return std::printf("%d pairs N%d D%d padded %d: %d splits merge, %d counters\n", bh, N, D, padded, n, decode_counters(1, bh, N, D)), 1;
             }
           }
           more[0] += splits[0] > splits[1];

@@ -82,6 +82,16 @@ def test_same_bits_and_zero_counters(ft, shape, padded):
         assert torch.equal(out, want[0])
 
 
+@pytest.mark.parametrize("shape", [(1, 3, 16391, 64), (1, 3, 67584, 16), (3, 1, 10240, 128), (1, 64, 1200, 64)])
+def test_counters_are_left_alone_where_none_are_asked_for(ft, shape):
+    """Also where the plan without padding would merge in the launch and the one with it would not."""
+    ins = _inputs(shape)
+    assert _counters(shape) == 0
+    counters = torch.full((shape[0] * shape[1],), 7, dtype=torch.int32, device="cuda")
+    want, got = _two_launches(*ins), _two_launches(*ins, counters=counters)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and (counters == 7).all()
+
+
 def test_streams_threads_and_graphs(ft):
     ins = [_inputs(s) for s in (*SHAPES[:3], SHAPES[7])]
     want = [_two_launches(*x)[0] for x in ins]
