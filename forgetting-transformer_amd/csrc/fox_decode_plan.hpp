@@ -21,7 +21,8 @@ inline bool decode_one_workgroup(int64_t bh, int64_t batches, int D) {
 // padding need.  (More than that are not just idle: consecutive workgroups go round the XCDs, so with twelve of sixteen splits in use four of the eight XCDs got two
 // thirds of the rows.)  us, 2048 workgroups whatever the row / now:
 // - A run of a few batches: the number with which the CUs get the most even share of them, one batch a wave where that is no worse, so that no wave waits for its second.
-//   D 128, 128 pairs N3000 41.6 / 35.0 (twelve splits of two batches 36.1), 64 pairs N5000 32.6 / 29.7, D 64, 128 pairs N5000 33.2 / 29.0.
+//   D 128, 128 pairs N3000 41.6 / 35.0 (twelve splits of two batches 36.1), 64 pairs N5000 32.6 / 29.7, D 64, 128 pairs N5000 33.2 / 29.0.  Not from one split, which needs no merge
+//   (2048 pairs N1700 D16, padded by up to a quarter, one split 35.4, two 44.1).
 // - One split, and no merge, where every CU, or three of four, has one pair, or all have nearly the same number: one workgroup a CU asks for as much as the memory gives.
 //   D 128, 192 pairs N1700 31.3 / 28.9, N32768 491 / 448, 256 pairs N1700 42.9 / 35.6, N15000 298 / 286, D 64, 512 pairs N500 13.7 / 10.5, N15000 301 / 289.  128 pairs
 //   N24000 (243 / 295) and 320 (582 / 688) lose, and so do 192 pairs of head dims below 64 (D 16 N15000 36.5 / 41.1).  Not with padding, which differs from row to row: the longest row would be left to one CU.
@@ -42,7 +43,7 @@ inline DecodePlan decode_plan(int B, int H, int N, int D, bool padded) {
   int64_t per = (batches + splits - 1) / splits;
   auto runs = [&](int64_t p) { return (batches + p - 1) / p; };
   auto heaviest = [&](int64_t p) { return p * ((bh * runs(p) + kCus - 1) / kCus); };   // CU's share, in batches a wave
-  if (per <= 4)
+  if (splits > 1 && per <= 4)
     for (int64_t p = per - 1; p >= 1 && runs(p) <= most && bh * runs(p) <= 16 * kCus; --p)
       if (heaviest(p) < heaviest(per) || (p == 1 && heaviest(p) == heaviest(per))) per = p;
   return {(int)(padded && per > 1 ? splits : runs(per)), (int)fewer};

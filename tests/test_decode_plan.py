@@ -15,7 +15,7 @@ PROGRAM = r"""
 using namespace fox;
 int main() {
   int more[2] = {0, 0};   // shapes where the call without padding, and the one with it, has the more splits
-  for (int bh = 1; bh <= 2100; bh += bh < 1100 ? 1 : 7)
+  for (int bh = 1; bh <= 2100; bh += bh < 1100 ? 1 : 4)
     for (int D : {16, 32, 64, 128})
       for (int64_t batch = 1; batch <= 512; batch += batch < 140 ? 1 : 5)
         for (int past = 0; past <= 1; ++past) {
@@ -29,7 +29,7 @@ int main() {
             // the number before it was made even: at most 2048 workgroups, which is what a caller's scratch always had to hold at most
             const int64_t even = std::min(std::min((2048 + bh - 1) / (int64_t)bh, decode_batches(N, D)), (int64_t)kDecodeMaxSplits);
             const bool whole = decode_batches(N, D) <= 1 || decode_one_workgroup(bh, decode_batches(N, D), D);
-            if (p.splits < 1 || p.splits > kDecodeMaxSplits || p.least < 1 || p.least > (whole ? 1 : even) || need > room || (whole && room))
+            if (p.splits < 1 || p.splits > kDecodeMaxSplits || p.least < 1 || p.least > (whole ? 1 : even) || (even == 1 && p.splits > 1) || need > room || (whole && room))
               return std::printf("%d pairs N%d D%d padded %d: %d splits, %d at least, room %lld\n", bh, N, D, padded, p.splits, p.least, (long long)room), 1;
             splits[padded] = p.splits;
             for (const int64_t bytes : {room, need, room - 1, (need + room) / 2, decode_bytes(1, bh, D, (int)even)}) {
