@@ -69,7 +69,8 @@ int check_extent(const fox_view* v, int rows, int D, const char* name) {
 // Distance from the diagonal, in keys, within which the pruning bound of a 128-key tile must lie for the tile to go
 // to the split variant of the dK/dV kernel (fox_set_acp_light_limit): 0 = never, negative = every tile of every
 // call that the variant supports.
-std::atomic<int> g_light_limit{256};   // measured crossover of the two kernels at head dim 128
+constexpr int kLightLimit = 256;   // measured crossover of the two kernels at head dim 128
+std::atomic<int> g_light_limit{kLightLimit};
 
 // Bytes of K and V together from which on a forward with one query tile per (batch, head) loads its K and V tiles
 // with the non-temporal hint (fox_set_stream_min_kv_bytes).  Such a call reads every tile once; the hint pays
@@ -77,7 +78,7 @@ std::atomic<int> g_light_limit{256};   // measured crossover of the two kernels 
 // when the next call on them comes (32-270 MB, called in a loop: 5-14 % faster with cached loads).
 std::atomic<int64_t> g_stream_min_kv_bytes{(int64_t)512 << 20};
 
-// Whether the split variant of the dK/dV kernel takes every tile, with or without a threshold.  Its 64-key tiles fit twice on a CU and
+// Whether the split variant of the dK/dV kernel takes every tile, with or without a threshold, where no caller has set another limit.  Its 64-key tiles fit twice on a CU and
 // start and end sooner, the 128-key tiles of the other variant read dO and Q half as often.  dK/dV at D 128, other variant / split, us:
 // - Rows shorter than 512 keys, whatever the grid: 1 tile N64 10.0 / 5.6, 512 tiles N64 21.4 / 8.8, 768 tiles N320 44.4 / 35.5, 1536 tiles N320
 //   91.4 / 67.4 and N384 97.3 / 89.2, 2048 tiles N448 132.4 / 113.0; not N512 with 512 tiles 33.9 / 35.7.
@@ -98,7 +99,7 @@ void tile_classes(bool pruned, bool light_ok, bool light_all, int* first, int* s
   *second = -1;
   *limit = lim;
   if (!light_ok || lim == 0) return;
-  if (lim < 0 || light_all) {
+  if (lim < 0 || (light_all && lim == kLightLimit)) {
     *first = fox::kClassLight;
     *limit = -1;
     return;

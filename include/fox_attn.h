@@ -72,7 +72,7 @@ int fox_probe_mfma(const void* operands, float* sink, int32_t workgroups, int32_
  * splits the head dim over two waves and runs two workgroups per CU, the others to the kernel built for long
  * loops.  This sets `keys` (256 by default, the measured crossover) for all later calls of the process and returns the previous value: 0 = the long-loop
  * kernel only, negative = the split variant for every tile of every call it supports (head dim 128), with or
- * without a threshold.  Where it is positive, rows of fewer than 512 keys, and of up to 896 keys where the call has at
+ * without a threshold.  At its default, rows of fewer than 512 keys, and of up to 896 keys where the call has at
  * most 256 tiles of 128 keys, take the split variant for every tile as well, with or without a threshold.  The results obey the same contract either way.  Like the reference's tile pickers,
  * which "can be overwritten at runtime" (get_bwd_kv_config, :838).
  */

@@ -417,6 +417,34 @@ def test_dkdv_kernel_variants(fa, limit, B, H, M, N, seq, thr, gates):
         assert lib.fox_set_acp_light_limit(prev) == limit
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N", [(515, 515), (300, 457)])
+def test_dkdv_limit_of_a_caller_holds_for_short_rows(fa, M, N, dtype):
+    """Rows that the split dK/dV kernel takes whole at the default limit: one key as the limit leaves all tiles but the last to the other kernel, which 0 leaves all of them to."""
+    from forgetting_transformer.ops import _lib
+    from forgetting_transformer.ops.forgetting_attention import record_pruning_bounds
+    lib = _lib.load()
+    q, k, v, g, do, _ = make_inputs(2, 3, M, N, 128, dtype=dtype, device="cuda", seed=M, head_first=True, gate_mean=1.0)
+    leaves = [x.requires_grad_() for x in (q, k, v, g)]
+
+    def run(limit):
+        prev = None if limit is None else lib.fox_set_acp_light_limit(limit)
+        try:
+            with record_pruning_bounds() as rec:
+                grads = torch.autograd.grad(fa(*leaves, head_first=True, adaptive_threshold=-10.0), leaves, do)
+        finally:
+            if prev is not None:
+                lib.fox_set_acp_light_limit(prev)
+        return (*grads, rec[-1]["kv_end_row"])
+
+    whole, none, one = run(-1), run(0), run(1)
+    assert all(torch.equal(a, b) for a, b in zip(run(None), whole))
+    cut = (N - 1) // 128 * 128
+    (_, dk, dv, _, end), (_, dk0, dv0, _, end0) = one, none
+    assert torch.equal(dk[:, :, :cut], dk0[:, :, :cut]) and torch.equal(dv[:, :, :cut], dv0[:, :, :cut]) and torch.equal(end[..., :cut // 64], end0[..., :cut // 64])
+    assert not torch.equal(whole[-1][..., :cut // 64], end0[..., :cut // 64])   # steps of 64 rows from 64 keys, and from 128
+
+
 @pytest.mark.parametrize("B,H,M,N,seq,thr,dtype", [
     (1, 2, 64, 64, None, None, torch.bfloat16), (16, 20, 65, 65, None, -10.0, torch.bfloat16), (2, 3, 511, 511, [0, 300], -10.0, torch.float16),
     (12, 8, 511, 511, None, None, torch.bfloat16), (8, 8, 512, 512, None, None, torch.bfloat16), (5, 13, 512, 512, None, -10.0, torch.bfloat16),
