@@ -159,7 +159,7 @@ inline int scan_threads(int N) { return N <= 8 * 64 ? 64 : N <= 8 * 256 ? 256 : 
 // Against it stand the loads of a row's next span, sent while one is scanned.  Eight / sixteen, both by DPP: forward 64 rows of 20000 9.4 / 10.7, 256 rows of
 // 32768 14.7 / 15.4, 512 rows of 16384 16.1 / 17.1; reverse 512 rows of 20000 22.2 / 26.2, 16384 18.6 / 18.6.
 inline bool scan_deep(int N, int64_t rows, bool reverse) {
-  if (N <= 8 * 1024) return false;
+  if (N <= 8 * 1024 || N > 1 << 30) return false;   // (the end of a span stays below 2^31: rows up to 2^31 - 8 * 1024 have always been taken)
   return reverse ? rows <= kCus || N <= 16 * 1024 : rows <= kCus && N <= 16 * 1024;
 }
 

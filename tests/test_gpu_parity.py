@@ -685,6 +685,20 @@ def test_cumsum_kernels_with_sixteen_positions_a_thread(fa, N):
     test_cumsum_kernels_at_the_edges_of_their_workgroups(fa, N)
 
 
+def test_reverse_scan_of_the_longest_row(fa):
+    """A span of sixteen positions a thread would end beyond 2^31: such rows go by spans of eight."""
+    from forgetting_transformer.ops import _lib
+    lib, N = _lib.load(), (1 << 31) - 9000
+    dc, dg = torch.zeros(1, 1, N, device="cuda"), torch.full((1, 1, N), float("nan"), device="cuda")
+    at = [5000, 1 << 20, (1 << 30) + 1, N - 16384, N - 1]
+    dc[0, 0, at] = torch.tensor([1.0, 2.0, 4.0, 8.0, 16.0], device="cuda")
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.check(lib.fox_cumsum_bwd(dc.data_ptr(), dg.data_ptr(), 0, 0, 0, None, 1, 1, N, stream), "cumsum_bwd")
+    for i, (first, last) in enumerate(zip([1] + [p + 1 for p in at], at)):
+        low, high = dg[0, 0, first:last + 1].aminmax()   # the sum of what lies at or behind the position
+        assert low.item() == high.item() == 31 - (2 ** i - 1), (first, last)
+
+
 def test_mfma_probe_runs(fa):
     """The measuring-stick loop of the power report: launches, returns, leaves its sink alone."""
     from forgetting_transformer.ops import _lib
