@@ -442,8 +442,11 @@ __global__ __launch_bounds__(1024) void norm_max_pair_kernel(View q, View k, int
 
 // norm_max_kernel with the forward scan of the gates beside it, one workgroup per row in front of the others: the scan is a chain of one workgroup's barriers
 // (20 us in a step at B4 T16384 H16) that needs none of the bandwidth the norms stream at (88 us), and needs no threshold.
+// At most six waves a SIMD, which is what the registers leave head dims 64 and 128 as well: with eight all norms of a middling call are resident at once and the scan's
+// chain waits behind them.  Eight / six, us: 64 pairs T8192 D32 26.3 / 23.8, 128 pairs T4096 D32 25.4 / 23.3, 512 pairs T16384 D16 287 / 261, T2048 D16 43.7 / 40.7.  Five
+// starve the norms of long rows (256 pairs T8192 D64 117 / 123).
 template <typename Tr, int D, int KIND>
-__global__ __launch_bounds__(256) void norm_max_scan_kernel(View q, View k, int H, int M, int N, uint32_t* scratch, float* thr, float sm_scale, float log_n,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 6))) void norm_max_scan_kernel(View q, View k, int H, int M, int N, uint32_t* scratch, float* thr, float sm_scale, float log_n,
                                                             GateK t, const int64_t* __restrict__ seq_start, NormBlocks w) {
   if ((int)blockIdx.x >= w.pairs) {
     norm_max<Tr, D>(q, k, H, M, N, scratch, thr, sm_scale, log_n, blockIdx.x - w.pairs, w);
