@@ -407,7 +407,7 @@ __global__ __launch_bounds__(256) void norm_max_kernel(View q, View k, int H, in
 // round trip and a reduction (12 pairs T256 D128: 12.7 us for zeroing, norms and atomics, 6.2 now).
 template <typename Tr, int D>
 __global__ __launch_bounds__(1024) void norm_max_pair_kernel(View q, View k, int H, int M, int N, float* thr, float sm_scale, float log_n) {
-  constexpr int LPR = D / 8, RPP = 1024 / LPR, U = 8;
+  constexpr int LPR = D / 8, RPP = 1024 / LPR, U = RPP >= 128 ? 1024 / RPP : 8;   // (threshold_pairs: 1024 rows at most, and no load beyond them)
   const int tid = threadIdx.x, bh = blockIdx.x, b = bh / H, h = bh % H, ch = tid % LPR;
   const uint16_t *qp = q.ptr + b * q.sb + h * q.sh + ch * 8, *kp = k.ptr + b * k.sb + h * k.sh + ch * 8;
   float best_q = 0.f, best_k = 0.f;
@@ -508,8 +508,8 @@ hipError_t launch_qk_norm_threshold(const float* wq, const float* wk, int H, int
 }
 
 // Whether one workgroup takes a (batch, head) whole, where that is no longer a chain than the launch that clears the scratch and the three atomics behind each
-// other.  us, with them / whole: D 128 T64 9.8 / 6.0, T512 9.4 .. 11.7 / 9.0 .. 9.5, T1024 9.4 / 15.3, D 64 T512 8.4 / 6.0, T1024 7.9 / 9.1, D 32 and 16 T512 7.4 / 5.9 and
-// 7.4 / 6.3, T1024 7.6 / 7.3 and 7.5 / 7.2; 512 pairs D 128 T512 26.8 / 23.6.
+// other.  us, with them / whole: D 128 T64 9.8 / 6.0, T512 9.4 .. 11.7 / 9.0 .. 9.5, T1024 9.4 / 15.3, D 64 T512 8.4 / 6.0, T1024 7.9 / 9.1, D 32 T512 6.8 / 4.6, D 16 6.7 / 3.9
+// (with loads beyond the last row 6.1 and 5.6; M1 N1000, 64 pairs D 16 6.8 / 5.7, with them 7.1); 512 pairs T512, D 128 26.8 / 23.6, D 32 14.8 / 11.9.
 static bool threshold_pairs(int M, int N) { return (int64_t)M + N <= 1024; }
 
 template <typename Tr, int D>
