@@ -95,7 +95,7 @@ def test_against_one_after_the_other(B, H, M, N, thr, seq, head_first, dtype, D)
 
 
 @pytest.mark.parametrize("logit", [None, torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("B,H,M,N,seq", [(2, 3, 130, 300, [0, 200]), (1, 3, 700, 1500, None), (1, 2, 1000, 8300, [17])])   # a row of one span, of one span at each width, of two
+@pytest.mark.parametrize("B,H,M,N,seq", [(2, 3, 130, 300, [0, 200]), (1, 3, 700, 1500, None), (1, 2, 1000, 8300, [17])])   # one span of each width: 256 threads, 1024, 1024 with sixteen positions each
 def test_strided_gate_gradients(B, H, M, N, seq, logit):
     """The reverse scan with the row sums added, into gates and logits that lie as (B, T, H), against the stages on their own."""
     p = _Problem(B, H, M, N, 32, torch.bfloat16, None, seq, False)
@@ -125,7 +125,7 @@ def test_strided_gate_gradients(B, H, M, N, seq, logit):
         assert torch.isfinite(a).all() and torch.equal(a, b)
 
 
-@pytest.mark.parametrize("logit", [None, torch.float16])
+@pytest.mark.parametrize("logit", [None, torch.bfloat16, torch.float16, torch.float32])
 def test_strided_gate_gradients_of_long_rows(logit):
     """The same where a row is two spans of sixteen positions a thread."""
     test_strided_gate_gradients(1, 2, 300, 16500, [17], logit)

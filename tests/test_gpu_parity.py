@@ -649,14 +649,13 @@ def test_cumsum_kernels(fa):
 
 
 @pytest.mark.parametrize("N", [1, 64, 511, 512, 513, 2047, 2048, 2049, 8193])   # one, four and sixteen waves a row, one span and two
-def test_cumsum_kernels_at_the_edges_of_their_workgroups(fa, N):
+def test_cumsum_kernels_at_the_edges_of_their_workgroups(fa, N, B=2, H=3):
     from forgetting_transformer.ops import _lib
     lib = _lib.load()
     stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
-    B, H = 2, 3
     x = (torch.randn(B, N, H, device="cuda") * 2).transpose(1, 2)
     g = F.logsigmoid(x.double())
-    ss = torch.tensor([0, N // 3], device="cuda")
+    ss = torch.tensor([0, N // 3], device="cuda")[-B:]
     keep = torch.arange(N, device="cuda") >= ss[:, None, None]
     c, c_gate, lg, dg = (torch.full((B, H, N), float("nan"), device="cuda") for _ in range(4))
     g32 = g.float()
@@ -683,6 +682,12 @@ def test_cumsum_kernels_at_the_edges_of_their_workgroups(fa, N):
 def test_cumsum_kernels_with_sixteen_positions_a_thread(fa, N):
     """Rows around one and two spans of 8 * 1024 and of 16 * 1024 positions, which the scans choose between."""
     test_cumsum_kernels_at_the_edges_of_their_workgroups(fa, N)
+
+
+@pytest.mark.parametrize("N", [8193, 16385, 20000])
+def test_cumsum_kernels_with_more_rows_than_cus(fa, N):
+    """257 rows: several spans of eight positions a thread, forward from 8193 positions on, reverse from 16385 (one span of sixteen up to there)."""
+    test_cumsum_kernels_at_the_edges_of_their_workgroups(fa, N, B=1, H=257)
 
 
 def test_reverse_scan_of_the_longest_row(fa):
