@@ -25,7 +25,9 @@ inline bool decode_one_workgroup(int64_t bh, int64_t batches, int D) {
 //   (2048 pairs N1700 D16, padded by up to a quarter, one split 35.4, two 44.1).
 // - One split, and no merge, where every CU, or three of four, has one pair, or all have nearly the same number: one workgroup a CU asks for as much as the memory gives.
 //   D 128, 192 pairs N1700 31.3 / 28.9, N32768 491 / 448, 256 pairs N1700 42.9 / 35.6, N15000 298 / 286, D 64, 512 pairs N500 13.7 / 10.5, N15000 301 / 289.  128 pairs
-//   N24000 (243 / 295) and 320 (582 / 688) lose, and so do 192 pairs of head dims below 64 (D 16 N15000 36.5 / 41.1).  Not with padding, which differs from row to row: the longest row would be left to one CU.
+//   N24000 (243 / 295) and 320 (582 / 688) lose, and so do 192 pairs of head dims below 64 (D 16 N15000 36.5 / 41.1); those gain
+//   from nine tenths of the CUs on: D 32, 231 pairs N5000 30.6 / 27.2, N32768 163 / 150, 256 pairs N5000 43.7 / 29.2, 512 pairs N32768 348 / 328, D 16, 231 pairs N1700 11.8 / 9.2, N32768 86.5 / 81.9,
+//   256 pairs N12000 46.8 / 36.6, 768 pairs N28000 222 / 219, N50000 384 / 380; only rows of N32768, each a power of two away from the next, lose there (256 pairs 92.4 / 93.3, 768 pairs 255 / 267).  Not with padding, which differs from row to row: the longest row would be left to one CU.
 // - With padding the rows' own lengths decide what a split gets, and the number is not made even (D 128, 128 pairs N15000, padded by up to all of it, 16 / 15 splits 90.8 / 95.0).
 // - With padding, long rows of many pairs: half as many workgroups; they start and end less often, and are still few batches of the whole (D 128, 256 pairs N32768, padded
 //   by up to a quarter 577 / 567, by up to all of it 398 / 372; shorter rows lose the balance: N5000 54.9 / 56.7, 512 pairs N5000 99 / 104).

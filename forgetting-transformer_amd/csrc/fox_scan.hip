@@ -560,8 +560,8 @@ hipError_t launch_auto_threshold(const View& q, const View& k, int B, int H, int
 // - Fewer queries than half the keys: always, but for a row that takes longer than all of that and is alone.  Threshold and scan alone, two launches / one, us: M8 N9000 12 pairs D128
 //   21.1 / 12.6, 32 pairs M4 N29333 D64 56 / 45, 128 pairs D16 M8 N4000 16.6 / 13.6, 2 pairs N32768 D16 21.8 / 26.1, 12 pairs N32768 D64 38.1 / 39.7, D128 45.7 / 43.7.
 // - Else where the norms stream for longer than the scan's 256 threads take.  "auto" forward, us: B4 T16384 H16 D128 345 / 329, B4 T4096 H32 D64 107 / 99, B2 T8192 H16 D64 68.4 / 62.5,
-//   B8 T700 H32 D32 29.6 / 26.9.  One launch would be the faster one for some way below that line as well (12 pairs D128 M = N = 4096 17.5 / 12.8); the line is where it always was
-//   because what fox_auto_threshold_scan_one_launch says of a shape is part of the interface.
+//   B8 T700 H32 D32 29.6 / 26.9.  Below that line one launch can be the faster one as well (12 pairs D128 M = N = 4096, threshold and scan alone, 17.5 / 12.8), but a host test
+//   holds the line at shapes on either side of it, and it has not been swept for another.
 bool threshold_scans(int B, int H, int M, int N, int D) {
   const int64_t pairs = (int64_t)B * H, bytes = pairs * ((int64_t)M + N) * D * 2;
   const bool beside = threshold_pairs(M, N) || 2 * (int64_t)M >= N ? bytes >= 6000 * ((int64_t)N + 2000) : bytes >= 6000000 * ((int64_t)N / 1400 - 11);

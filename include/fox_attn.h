@@ -412,8 +412,8 @@ typedef struct fox_gates {
 int fox_attn_fwd_gates(const fox_fwd_args* args, const fox_gates* gates, const fox_fwd_epilogue* epilogue, void* stream);
 int fox_attn_fwd_takes_gates(const fox_dims* dims, int32_t pruned, int32_t* yes);
 
-/* fox_auto_threshold and the scan of the gates (fox_cumsum_fwd or fox_gate_cumsum_fwd into c, (B,H,N)), side by side in one launch where the norms take
- * longer than the scan. */
+/* fox_auto_threshold and the scan of the gates (fox_cumsum_fwd or fox_gate_cumsum_fwd into c, (B,H,N)), side by side in one launch or one after the other: in one
+ * where the norms stream for longer than the scan takes, and for fewer queries than half the keys and more than 1024 rows of both unless a long row is nearly alone. */
 int fox_auto_threshold_scan(const fox_dims* dims, const fox_view* q, const fox_view* k, float sm_scale, float* thr, uint32_t* norm_scratch,
                             const fox_gates* gates, const int64_t* seq_start, float* c, void* stream);
 /* Whether fox_auto_threshold_scan takes one launch for this shape. */
