@@ -29,8 +29,10 @@ inline bool decode_one_workgroup(int64_t bh, int64_t batches, int D) {
 //   from nine tenths of the CUs on: D 32, 231 pairs N5000 30.6 / 27.2, N32768 163 / 150, 256 pairs N5000 43.7 / 29.2, 512 pairs N32768 348 / 328, D 16, 231 pairs N1700 11.8 / 9.2, N32768 86.5 / 81.9,
 //   256 pairs N12000 46.8 / 36.6, 768 pairs N28000 222 / 219, N50000 384 / 380; only rows of N32768, each a power of two away from the next, lose there (256 pairs 92.4 / 93.3, 768 pairs 255 / 267).  Not with padding, which differs from row to row: the longest row would be left to one CU.
 // - With padding the rows' own lengths decide what a split gets, and the number is not made even (D 128, 128 pairs N15000, padded by up to all of it, 16 / 15 splits 90.8 / 95.0).
-// - With padding, long rows of many pairs: half as many workgroups; they start and end less often, and are still few batches of the whole (D 128, 256 pairs N32768, padded
-//   by up to a quarter 577 / 567, by up to all of it 398 / 372; shorter rows lose the balance: N5000 54.9 / 56.7, 512 pairs N5000 99 / 104).
+// - With padding, long rows, the same number of pairs on every CU and four splits left of eight: half as many workgroups; they start and end less often, and are still few batches of
+//   the whole (D 128, 256 pairs N32768, padded by up to a quarter 577 / 567, by up to all of it 398 / 372; shorter rows lose the balance: N5000 54.9 / 56.7, 512 pairs N5000 99 / 104).
+//   Not where the CUs' shares become less even (N32768 D 64, 320 pairs, seven splits / four, 349 / 361, D 128 padded by up to all of it 323 / 353, 1040 pairs N20000, two / one, 1324 / 1379 and 783 / 889),
+//   nor with fewer than four pieces of a row (512 pairs N20000 D 128 padded by up to all of it, four / two, 412 / 462; N32768 513 / 482).
 struct DecodePlan {
   int splits;   // what a call takes
   int least;    // what its scratch must have room for: before the number is made even, which may take more
@@ -40,7 +42,7 @@ inline DecodePlan decode_plan(int B, int H, int N, int D, bool padded) {
   if (batches <= 1 || decode_one_workgroup(bh, batches, D)) return {1, 1};
   const int64_t most = batches < kDecodeMaxSplits ? batches : kDecodeMaxSplits;
   auto of = [&](int64_t wgs) { const int64_t even = (wgs + bh - 1) / bh; return even < most ? even : most; };
-  const int64_t fewer = of(bh >= kCus && batches >= 128 ? 4 * kCus : 8 * kCus), splits = padded ? fewer : of(8 * kCus);
+  const int64_t fewer = of(bh >= kCus && batches >= 128 ? 4 * kCus : 8 * kCus), splits = padded && bh % kCus == 0 && fewer >= 4 ? fewer : of(8 * kCus);
   if (!padded && (bh <= kCus && D >= 64 ? 4 * bh >= 3 * kCus : 10 * bh >= 9 * rounds * kCus)) return {1, (int)fewer};
   int64_t per = (batches + splits - 1) / splits;
   auto runs = [&](int64_t p) { return (batches + p - 1) / p; };

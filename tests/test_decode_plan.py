@@ -32,6 +32,8 @@ int main() {
             if (p.splits < 1 || p.splits > kDecodeMaxSplits || p.least < 1 || p.least > (whole ? 1 : even) || (even == 1 && p.splits > 1) || need > room || (whole && room))
               return std::printf("%d pairs N%d D%d padded %d: %d splits, %d at least, room %lld\n", bh, N, D, padded, p.splits, p.least, (long long)room), 1;
             splits[padded] = p.splits;
+            // padded rows give up splits only where four are left and every CU has as many pairs as the others
+            if (padded && p.splits < even && (bh % kCus || p.splits < 4) && !whole) return std::printf("%d pairs N%d D%d: %d splits of %lld\n", bh, N, D, p.splits, (long long)even), 1;
             for (const int64_t bytes : {room, need, room - 1, (need + room) / 2, decode_bytes(1, bh, D, (int)even)}) {
               if (bytes < need) continue;   // refused
               const int n = decode_splits(1, bh, N, D, padded, bytes);
